@@ -54,7 +54,10 @@ constexpr int bwd_fused_waves(int D, bool causal) { return D <= 32 ? 2 : 1; }
 // halves of the score and dP tiles are exchanged through LDS and added (both wavefronts then hold
 // bit-identical sums, so their softmax statistics agree).  The two are a workgroup of their own,
 // so that its barrier couples nobody else.
-template <typename T, int D, bool CAUSAL, int SB, int NBW, int SPLIT>
+//
+// PART: part heads (hsa_attn_tile.h), p.dh channels laid out like D; with SPLIT = 2 the second
+// wavefront owns the channels from 64 on, of which dh - 64 exist.
+template <typename T, int D, bool CAUSAL, int SB, int NBW, int SPLIT, bool PART = false>
 __global__ void __launch_bounds__((SPLIT == 2 ? 2 : BWD_WPB) * 64)
 __attribute__((amdgpu_waves_per_eu(bwd_fused_waves(D / SPLIT, CAUSAL))))
 attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
@@ -121,13 +124,17 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
     const int strip = (unit / H) % NS;
     const int b = unit / (H * NS);
     const int blk0 = strip * SB;
-    const size_t rs = (size_t)H * D;
-    const size_t qo = ((size_t)b * N * H + h) * D + half * HD, ko = ((size_t)b * p.M * H + h) * D + half * HD;
+    const int dh = PART ? p.dh : D;
+    const int dw = PART ? (SPLIT == 2 ? (half ? dh - HD : HD) : dh) : HD;  // channels of the head this wavefront owns
+    const size_t rs = (size_t)H * dh;
+    const size_t qo = ((size_t)b * N * H + h) * dh + half * HD, ko = ((size_t)b * p.M * H + h) * dh + half * HD;
+    const int pchk = PART ? min(lchk, dw / 8 - 1) : lchk;  // the piece this lane fetches
+    const bool own_piece = !PART || 8 * lchk < dw;         // the piece exists: this lane stores it
     const uint16_t *Q0 = p.q + qo, *G0 = p.dout + qo, *O0 = fp.out + qo;
     const uint16_t *K0 = p.k + ko, *V0 = p.v + ko;
-    const uint16_t *Kb = K0 + 8 * lchk, *Vb = V0 + 8 * lchk;
-    uint16_t *dKb = p.dk + ko + 8 * lchk;
-    uint16_t *dVb = p.dv + ko + 8 * lchk;
+    const uint16_t *Kb = K0 + 8 * pchk, *Vb = V0 + 8 * pchk;
+    uint16_t *dKb = p.dk + ko + 8 * pchk;
+    uint16_t *dVb = p.dv + ko + 8 * pchk;
     // key / value blocks in operand form: the leaf blocks a query block reaches (they slide along
     // the strip), the near tree block, the far tree block
     u32x4_t Kc[NKB][KS], Vc[NKB][KS];
@@ -154,8 +161,13 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
     // the two contraction steps, and its own 16 bytes of a transfer
     const uint32_t stg_base = lds_address(stage_mem) + wave * WAVE_STG;
     int pc8[NLD];
+    bool stage_piece[NLD];  // ... and whether it exists (a part head's missing pieces repeat the last one)
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) pc8[i] = 8 * (lchk ^ (((i * RPI + lrow) / RPB) % CPR));
+    for (int i = 0; i < NLD; ++i) {
+        const int pc = lchk ^ (((i * RPI + lrow) / RPB) % CPR);
+        stage_piece[i] = !PART || 8 * pc < dw;
+        pc8[i] = 8 * (PART ? min(pc, dw / 8 - 1) : pc);
+    }
     const uint32_t opa0 = stg_base + r16 * RB + ((g ^ ((r16 / RPB) % CPR)) << 4);
     const uint32_t opa1 = stg_base + r16 * RB + ((((4 + g) % CPR) ^ ((r16 / RPB) % CPR)) << 4);
     const uint32_t lin = stg_base + 16 * bt.lane;
@@ -307,6 +319,10 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
         } else {
             lds_read16_x4<OFF, OFF + ARR, OFF + ARR, OFF + 2 * ARR>(opa0, opa0, lin, lin, Qf[0], Gf[0], gw[0], ow[0]);
         }
+        if constexpr (PART) {
+            bt.clear_behind(Qf, dw);
+            bt.clear_behind(Gf, dw);
+        }
         // the exchanged values: the tiles of the NK key blocks and the rows' sums for delta
         f32x4 xv[2 * NK + 1];
         // the lanes that share a row sum their pieces (both rows carry the same permutation of
@@ -321,6 +337,7 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
                 sd = fmaf(to_float<T>((uint16_t)(a & 0xffffu)), to_float<T>((uint16_t)(o & 0xffffu)), sd);
                 sd = fmaf(to_float<T>((uint16_t)(a >> 16)), to_float<T>((uint16_t)(o >> 16)), sd);
             }
+            if (!stage_piece[i]) sd = 0.f;
 #pragma unroll
             for (int m = 1; m < CPR; m <<= 1) sd += __shfl_xor(sd, m, 64);
             xv[2 * NK][i] = sd;
@@ -348,6 +365,7 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
         uint16_t *dVp = dVb + (size_t)(kb * TILE_Q + lrow) * rs;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
+            if (!own_piece) continue;
             *reinterpret_cast<u32x4_t *>(dKp + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
             *reinterpret_cast<u32x4_t *>(dVp + (size_t)(i * RPI) * rs) = bt.get_row_piece(1, i);
         }
@@ -424,6 +442,10 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
         else wait_vmem_all_but<5 * NLD>();
         if constexpr (KS == 2) lds_read16_6x2<0, ARR>(opa0, opa1, Qf, Gf, Kc[NKL - 1], Vc[NKL - 1], Kc[NKL], Vc[NKL]);
         else lds_read16_6x1<0, ARR>(opa0, Qf, Gf, Kc[NKL - 1], Vc[NKL - 1], Kc[NKL], Vc[NKL]);
+        if constexpr (PART) {
+            bt.clear_behind(Qf, dw);
+            bt.clear_behind(Gf, dw);
+        }
         // the operands are in registers: the area takes the next block's rows, after the last
         // block the neighbour's query blocks (three staged blocks each, in the halves of the area)
         if (it + 1 < SB) {
@@ -544,10 +566,10 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
                 for (int j = 0; j < NJ; ++j) acc[j] = M_::k16(KT[j], dsp, acc[j]);
             }
             bt.put_result(0, acc, 1.0f);
-            uint16_t *optr = p.dq + qo + 8 * lchk + (size_t)(q0 + lrow) * rs;
+            uint16_t *optr = p.dq + qo + 8 * pchk + (size_t)(q0 + lrow) * rs;
 #pragma unroll
             for (int i = 0; i < NLD; ++i)
-                *reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
+                if (own_piece) *reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
         }
 
         // ---- orientation 2: dK^T, dV^T [channel, key] ---------------------------------------------------
@@ -630,7 +652,7 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
 #pragma unroll
                 for (int i = 0; i < NLD; ++i) {
                     const int sl = i * RPI + lrow;
-                    if ((sl < 15 || five_final) && t_row[i] >= 0) {
+                    if ((sl < 15 || five_final) && t_row[i] >= 0 && own_piece) {
                         *reinterpret_cast<u32x4_t *>(dKb + (size_t)t_row[i] * rs) = bt.get_row_piece(0, i);
                         *reinterpret_cast<u32x4_t *>(dVb + (size_t)t_row[i] * rs) = bt.get_row_piece(1, i);
                     }
@@ -661,6 +683,7 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
                         const int ch = 32 * (j >> 1) + 8 * g + 4 * (j & 1);
+                        if (PART && ch >= dw) continue;
                         *reinterpret_cast<u32x2_t *>(p.dk + ro + ch) =
                             u32x2_t{M_::pack(fk[j][0], fk[j][1]), M_::pack(fk[j][2], fk[j][3])};
                         *reinterpret_cast<u32x2_t *>(p.dv + ro + ch) =
@@ -668,13 +691,14 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
                     }
                 } else {
                     const int NR = NB / FAR;
-                    float *far = p.partial + 2 * (size_t)p.B * NB * H * 2 * D;
-                    const size_t po = ((((size_t)b * NR + blk0 / FAR) * H + h) * LF + (lvl - 6)) * D;
+                    float *far = p.partial + 2 * (size_t)p.B * NB * H * 2 * dh;
+                    const size_t po = ((((size_t)b * NR + blk0 / FAR) * H + h) * LF + (lvl - 6)) * dh;
                     float *pkp = far + po + half * HD;
-                    float *pvp = far + (size_t)p.B * NR * H * LF * D + po + half * HD;
+                    float *pvp = far + (size_t)p.B * NR * H * LF * dh + po + half * HD;
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
                         const int ch = 32 * (j >> 1) + 8 * g + 4 * (j & 1);
+                        if (PART && ch >= dw) continue;
                         *reinterpret_cast<f32x4 *>(pkp + ch) = fk[j];
                         *reinterpret_cast<f32x4 *>(pvp + ch) = fv[j];
                     }
@@ -738,59 +762,69 @@ __global__ void __launch_bounds__(BWD_WPB * 64) attn_bwd_reduce_kernel(BwdTilePa
 
 template <typename T, int D>
 int attn_bwd_fused_launch_td(const BwdFusedParams &fp, bool causal, hipStream_t st);
+// part heads on the layout of D channels
+template <typename T, int D>
+int attn_bwd_fused_part_launch_td(const BwdFusedParams &fp, bool causal, hipStream_t st);
 
 // launches one variant: a workgroup is four wavefronts (heads), or the two halves of one head
-template <typename T, int D, bool CAUSAL, int SB, int NBW>
+template <typename T, int D, bool CAUSAL, int SB, int NBW, bool PART>
 static int bwd_fused_launch_one(const BwdFusedParams &q, hipStream_t st) {
     constexpr int SPLIT = D > 64 ? 2 : 1;
     constexpr int WPB = SPLIT == 2 ? 2 : BWD_WPB;
     const int nwg = SPLIT == 2 ? q.t.n_units : (q.t.n_units + WPB - 1) / WPB;
-    attn_bwd_tile_fused_kernel<T, D, CAUSAL, SB, NBW, SPLIT><<<dim3(nwg), dim3(WPB * 64), 0, st>>>(q);
+    attn_bwd_tile_fused_kernel<T, D, CAUSAL, SB, NBW, SPLIT, PART><<<dim3(nwg), dim3(WPB * 64), 0, st>>>(q);
     return check_launch("attn_bwd_tile_fused_kernel");
 }
 
-template <typename T, int D, bool CAUSAL, int NBW>
+template <typename T, int D, bool CAUSAL, int NBW, bool PART>
 static int bwd_fused_launch_sb(const BwdFusedParams &q, int sb, hipStream_t st) {
     switch (sb) {
-        case 32: return bwd_fused_launch_one<T, D, CAUSAL, 32, NBW>(q, st);
-        case 16: return bwd_fused_launch_one<T, D, CAUSAL, 16, NBW>(q, st);
-        case 8: return bwd_fused_launch_one<T, D, CAUSAL, 8, NBW>(q, st);
-        default: return bwd_fused_launch_one<T, D, CAUSAL, 4, NBW>(q, st);
+        case 32: return bwd_fused_launch_one<T, D, CAUSAL, 32, NBW, PART>(q, st);
+        case 16: return bwd_fused_launch_one<T, D, CAUSAL, 16, NBW, PART>(q, st);
+        case 8: return bwd_fused_launch_one<T, D, CAUSAL, 8, NBW, PART>(q, st);
+        default: return bwd_fused_launch_one<T, D, CAUSAL, 4, NBW, PART>(q, st);
     }
 }
 
-#define HSA_BWD_FUSED_INSTANTIATE(T, D)                                                                     \
-    template <>                                                                                             \
-    int attn_bwd_fused_launch_td<T, D>(const BwdFusedParams &fp, bool causal, hipStream_t st) {             \
-        BwdFusedParams q = fp;                                                                              \
-        const int NB = fp.t.N / TILE_Q;                                                                     \
-        /* the longest strips (8, 16, 32 blocks) whose wavefronts still fill the chip once (one per SIMD */ \
-        /* on 256 CUs): fewer halo blocks, more tree levels final inside the strip.  Measured (us, strips */ \
-        /* of 8 / 16 / 32): B8 H8 N4096 D64 93 / 88 / 119, B8 H8 N8192 D64 180 / 173 / 166, B1 H16 N65536 */ \
-        /* D64 348 / 327 / 317, B1 H16 N65536 D128 R32 734 / 679 / 657, B1 H16 N16384 D64 92.6 / 94.2 / 120 */ \
-        const long waves8 = (long)(fp.t.n_units / 8) * (D > 64 ? 2 : 1);                                    \
-        const int knob = bwd_fused_strip_knob();                                                            \
-        int sb = (NB % 8 == 0 && knob != 4 && (knob >= 8 || (D >= 64 && waves8 >= 1024))) ? 8 : 4;          \
-        if (sb == 8 && NB % 16 == 0 && (knob >= 16 || (knob == 0 && waves8 >= 2 * 1024))) sb = 16;          \
-        if (sb == 16 && NB % 32 == 0 && (knob >= 32 || (knob == 0 && waves8 >= 4 * 1024))) sb = 32;         \
-        const int nbw = fp.t.R > TILE_Q ? 2 : 1;                                                            \
-        if (nbw == 2 && !causal) return fail(HSA_ERR_UNSUPPORTED, "one-pass backward: window radius above 16 needs the causal mask"); \
-        q.t.n_units = fp.t.n_units / sb;                                                                    \
-        q.t.red_lg_sb = sb == 32 ? 5 : sb == 16 ? 4 : sb == 8 ? 3 : 2;                                      \
-        {   /* the second launch starts above the levels the strips finish themselves */                    \
-            int first = level_offset(fp.t.N, q.t.red_lg_sb + 5);                                            \
-            if (first > 2 * fp.t.N - 2) first = 2 * fp.t.N - 2;                                             \
-            const size_t threads = (size_t)fp.t.B * (fp.t.M - first) * fp.t.H * (D / 4) * BWD_FUSED_RED_SPLIT; \
-            q.t.red_first_row = first;                                                                      \
-            q.t.red_wgs = (int)((threads + BWD_WPB * 64 - 1) / (BWD_WPB * 64));                             \
-        }                                                                                                   \
-        int rc;                                                                                             \
-        if (nbw == 2) rc = bwd_fused_launch_sb<T, D, true, 2>(q, sb, st);                                   \
-        else if (causal) rc = bwd_fused_launch_sb<T, D, true, 1>(q, sb, st);                                \
-        else rc = bwd_fused_launch_sb<T, D, false, 1>(q, sb, st);                                           \
-        if (rc != HSA_OK || q.t.red_wgs == 0) return rc;                                                    \
-        attn_bwd_reduce_kernel<T><<<q.t.red_wgs, BWD_WPB * 64, 0, st>>>(q.t, D);                            \
-        return check_launch("attn_bwd_reduce_kernel");                                                      \
+// both launches of the one-pass backward on the layout of D channels
+template <typename T, int D, bool PART>
+static int bwd_fused_launch(const BwdFusedParams &fp, bool causal, hipStream_t st) {
+    BwdFusedParams q = fp;
+    const int NB = fp.t.N / TILE_Q, dh = PART ? fp.t.dh : D;
+    // the longest strips (8, 16, 32 blocks) whose wavefronts still fill the chip once (one per SIMD
+    // on 256 CUs): fewer halo blocks, more tree levels final inside the strip.  Measured (us, strips
+    // of 8 / 16 / 32): B8 H8 N4096 D64 93 / 88 / 119, B8 H8 N8192 D64 180 / 173 / 166, B1 H16 N65536
+    // D64 348 / 327 / 317, B1 H16 N65536 D128 R32 734 / 679 / 657, B1 H16 N16384 D64 92.6 / 94.2 / 120
+    const long waves8 = (long)(fp.t.n_units / 8) * (D > 64 ? 2 : 1);
+    const int knob = bwd_fused_strip_knob();
+    int sb = (NB % 8 == 0 && knob != 4 && (knob >= 8 || (D >= 64 && waves8 >= 1024))) ? 8 : 4;
+    if (sb == 8 && NB % 16 == 0 && (knob >= 16 || (knob == 0 && waves8 >= 2 * 1024))) sb = 16;
+    if (sb == 16 && NB % 32 == 0 && (knob >= 32 || (knob == 0 && waves8 >= 4 * 1024))) sb = 32;
+    const int nbw = fp.t.R > TILE_Q ? 2 : 1;
+    if (nbw == 2 && !causal) return fail(HSA_ERR_UNSUPPORTED, "one-pass backward: window radius above 16 needs the causal mask");
+    q.t.n_units = fp.t.n_units / sb;
+    q.t.red_lg_sb = sb == 32 ? 5 : sb == 16 ? 4 : sb == 8 ? 3 : 2;
+    {   // the second launch starts above the levels the strips finish themselves
+        int first = level_offset(fp.t.N, q.t.red_lg_sb + 5);
+        if (first > 2 * fp.t.N - 2) first = 2 * fp.t.N - 2;
+        const size_t threads = (size_t)fp.t.B * (fp.t.M - first) * fp.t.H * (dh / 4) * BWD_FUSED_RED_SPLIT;
+        q.t.red_first_row = first;
+        q.t.red_wgs = (int)((threads + BWD_WPB * 64 - 1) / (BWD_WPB * 64));
+    }
+    int rc;
+    if (nbw == 2) rc = bwd_fused_launch_sb<T, D, true, 2, PART>(q, sb, st);
+    else if (causal) rc = bwd_fused_launch_sb<T, D, true, 1, PART>(q, sb, st);
+    else if constexpr (D <= 64 || !PART) rc = bwd_fused_launch_sb<T, D, false, 1, PART>(q, sb, st);
+    else return fail(HSA_ERR_UNSUPPORTED, "one-pass backward: more than 64 channels per head need the causal mask");
+    if (rc != HSA_OK || q.t.red_wgs == 0) return rc;
+    attn_bwd_reduce_kernel<T><<<q.t.red_wgs, BWD_WPB * 64, 0, st>>>(q.t, dh);
+    return check_launch("attn_bwd_reduce_kernel");
+}
+
+#define HSA_BWD_FUSED_INSTANTIATE(T, D)                                                              \
+    template <>                                                                                      \
+    int attn_bwd_fused_launch_td<T, D>(const BwdFusedParams &fp, bool causal, hipStream_t st) {      \
+        return bwd_fused_launch<T, D, false>(fp, causal, st);                                        \
     }
 
 }  // namespace hsa

@@ -35,6 +35,7 @@ struct BwdTileParams {
     float *stats;   // [B, N, H, 2]: log2-domain lse, delta
     float *partial; // [2, B, N/16, H, L-4, D] fp32 per-block partial rows of dK, dV for levels >= 4
     int B, N, M, H, L, R;
+    int dh;         // channels per head (kernels built for part heads; else the template's D)
     int n_units;
     float scale_log2e, scale;
     // rows the key pass's trailing workgroups finish from the partial rows (none: red_wgs == 0)
@@ -70,10 +71,11 @@ constexpr int bwd_query_waves(int D, int nkl, int sb) {
     return (nkl <= 5 && (D <= 32 || (D <= 64 && (nkl <= 3 || sb == 1)))) ? 2 : 1;
 }
 
-template <typename T, int D>
+// DC > 0: part heads (hsa_attn_tile.h), DC channels of the layout's D in the contractions
+template <typename T, int D, int DC = 0>
 struct BwdTile {
     using M_ = Mma<T>;
-    static constexpr int KS = D / 32, NJ = D / 16, CPR = D / 8, RPI = 64 / CPR, NLD = TILE_Q / RPI;
+    static constexpr int KS = (DC ? DC : D) / 32, NJ = (DC ? DC : D) / 16, CPR = D / 8, RPI = 64 / CPR, NLD = TILE_Q / RPI;
     // a block in LDS: rows back to back, the 16-byte pieces of row r at piece index p ^ swz(r)
     // (conflict-free from both sides, see hsa_attn_tile.h); slots keep the size of a padded block
     static constexpr int RB = D * 2, RPB = RB >= 256 ? 1 : 256 / RB, BLK_BYTES = TILE_Q * (RB + 16);
@@ -112,6 +114,12 @@ struct BwdTile {
         const unsigned char *reg = lds + slot * BLK_BYTES + r16 * RB;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) dst[ks] = *reinterpret_cast<const u32x4_t *>(reg + 16 * ((4 * ks + g) ^ op_swz));
+    }
+    // sets the channels behind a part head to zero (query-side operands: Q and dO)
+    __device__ __forceinline__ void clear_behind(u32x4_t (&x)[KS], int dh) const {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            if (8 * (4 * ks + g) >= dh) x[ks] = u32x4_t{0u, 0u, 0u, 0u};
     }
     // operand rows -> "lane = channel, regs = rows" form
     __device__ __forceinline__ void transpose(const u32x4_t (&op)[KS], u32x2_t (&dst)[NJ]) const {
@@ -154,11 +162,12 @@ struct BwdTile {
 // Partial rows (fp32): level 5 per query block when SB == 1, entry 1 of [2][B][N/16][H][2][D]
 // (dK then dV; entry 0 and, for longer strips, the whole area stay unused); levels >= 6 per
 // strip, [2][B][N/16/SB][H][L-6][D], right behind.
-template <typename T, int D, int NBW, bool CAUSAL, int SB>
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
 __global__ void __launch_bounds__(BWD_WPB * 64)
 __attribute__((amdgpu_waves_per_eu(bwd_query_waves(D, CAUSAL ? NBW + 1 : 2 * NBW + 1, SB))))
 attn_bwd_tile_query_kernel(BwdTileParams p) {
-    using BT = BwdTile<T, D>;
+    using BT = BwdTile<T, D, DC>;
+    constexpr bool PART = DC > 0;
     using M_ = Mma<T>;
     constexpr int KS = BT::KS, NJ = BT::NJ, RPI = BT::RPI, NLD = BT::NLD;
     constexpr int NKL = CAUSAL ? NBW + 1 : 2 * NBW + 1;
@@ -183,13 +192,16 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
     const int b = unit / (H * NS);
     const int blk0 = strip * SB;
     const int qs = blk0 * TILE_Q;  // first query of the strip
-    const size_t rs = (size_t)H * D;
-    const uint16_t *Qb = p.q + ((size_t)b * N * H + h) * D + 8 * lchk;
-    const uint16_t *Gb = p.dout + ((size_t)b * N * H + h) * D + 8 * lchk;
-    const uint16_t *Kb = p.k + ((size_t)b * p.M * H + h) * D + 8 * lchk;
-    const uint16_t *Vb = p.v + ((size_t)b * p.M * H + h) * D + 8 * lchk;
-    uint16_t *dKb = p.dk + ((size_t)b * p.M * H + h) * D + 8 * lchk;
-    uint16_t *dVb = p.dv + ((size_t)b * p.M * H + h) * D + 8 * lchk;
+    const int dh = PART ? p.dh : D;
+    const size_t rs = (size_t)H * dh;
+    const int pchk = PART ? min(lchk, dh / 8 - 1) : lchk;  // the piece this lane fetches
+    const bool own_piece = !PART || 8 * lchk < dh;         // the piece exists: this lane stores it
+    const uint16_t *Qb = p.q + ((size_t)b * N * H + h) * dh + 8 * pchk;
+    const uint16_t *Gb = p.dout + ((size_t)b * N * H + h) * dh + 8 * pchk;
+    const uint16_t *Kb = p.k + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
+    const uint16_t *Vb = p.v + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
+    uint16_t *dKb = p.dk + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
+    uint16_t *dVb = p.dv + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
 
     // ---- tree slot constants (same slot layout as the forward kernel) -------------------------
     int t_lvl[NLD], t_add[NLD], t_xor[NLD], u_row[NLD];  // rows this lane fetches; u_row -1 = no such slot
@@ -298,6 +310,10 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         bt.put(3, sg.v);
         bt.get(0, Qf);
         bt.get(1, Gf);
+        if constexpr (PART) {
+            bt.clear_behind(Qf, dh);
+            bt.clear_behind(Gf, dh);
+        }
         bt.get(2, Kc[NKL - 1]);
         bt.get(3, Vc[NKL - 1]);
         bt.put(2, sg.kt);
@@ -411,10 +427,10 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
                 for (int j = 0; j < NJ; ++j) acc[j] = M_::k16(KT[j], dsp, acc[j]);
             }
             bt.put_result(0, acc, 1.0f);
-            uint16_t *optr = p.dq + ((size_t)b * N * H + h) * D + 8 * lchk + (size_t)(q0 + lrow) * rs;
+            uint16_t *optr = p.dq + ((size_t)b * N * H + h) * dh + 8 * pchk + (size_t)(q0 + lrow) * rs;
 #pragma unroll
             for (int i = 0; i < NLD; ++i)
-                *reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
+                if (own_piece) *reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
         }
 
         // ---- orientation 2 for the tree blocks: dK^T, dV^T [channel, slot] ------------------------------
@@ -475,12 +491,13 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
                     }
                     five_final = (it & 1) != 0;
                 } else if (r16 == 15 && 5 < L) {
-                    const size_t po = ((((size_t)b * NB + blk) * H + h) * 2 + 1) * D;
+                    const size_t po = ((((size_t)b * NB + blk) * H + h) * 2 + 1) * dh;
                     float *pkp = p.partial + po;
-                    float *pvp = p.partial + (size_t)p.B * NB * H * 2 * D + po;
+                    float *pvp = p.partial + (size_t)p.B * NB * H * 2 * dh + po;
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
                         const int ch = 32 * (j >> 1) + 8 * g + 4 * (j & 1);
+                        if (PART && ch >= dh) continue;
                         *reinterpret_cast<f32x4 *>(pkp + ch) = tk[j];
                         *reinterpret_cast<f32x4 *>(pvp + ch) = tv[j];
                     }
@@ -492,7 +509,7 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
 #pragma unroll
                 for (int i = 0; i < NLD; ++i) {
                     const int sl = i * RPI + lrow;
-                    if ((sl < 15 || five_final) && t_row[i] >= 0) {
+                    if ((sl < 15 || five_final) && t_row[i] >= 0 && own_piece) {
                         *reinterpret_cast<u32x4_t *>(dKb + (size_t)t_row[i] * rs) = bt.get_row_piece(0, i);
                         *reinterpret_cast<u32x4_t *>(dVb + (size_t)t_row[i] * rs) = bt.get_row_piece(1, i);
                     }
@@ -519,13 +536,14 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         const int lvl = 6 + r16;
         const int LF = L - 6;
         if (lvl < L) {
-            float *far = p.partial + 2 * (size_t)p.B * NB * H * 2 * D;
-            const size_t po = ((((size_t)b * NS + strip) * H + h) * LF + (lvl - 6)) * D;
+            float *far = p.partial + 2 * (size_t)p.B * NB * H * 2 * dh;
+            const size_t po = ((((size_t)b * NS + strip) * H + h) * LF + (lvl - 6)) * dh;
             float *pkp = far + po;
-            float *pvp = far + (size_t)p.B * NS * H * LF * D + po;
+            float *pvp = far + (size_t)p.B * NS * H * LF * dh + po;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
                 const int ch = 32 * (j >> 1) + 8 * g + 4 * (j & 1);
+                if (PART && ch >= dh) continue;
                 *reinterpret_cast<f32x4 *>(pkp + ch) = fk[j];
                 *reinterpret_cast<f32x4 *>(pvp + ch) = fv[j];
             }
@@ -547,10 +565,12 @@ __device__ __forceinline__ void bwd_reduce_rows(const float *__restrict__ partia
 // The last red_wgs workgroups of the grid do not take key blocks: they sum the query pass's
 // partial rows into the upper tree levels' dK / dV rows (independent of the leaf rows this pass
 // writes), which fills the chip while the key blocks' last loads and stores drain.
-template <typename T, int D, int NBW, bool CAUSAL, int SB>
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
 __global__ void __launch_bounds__(BWD_WPB * 64)
 attn_bwd_tile_key_kernel(BwdTileParams p) {
-    using BT = BwdTile<T, D>;
+    using BT = BwdTile<T, D, DC>;
+    constexpr bool PART = DC > 0;
+    const int dh = PART ? p.dh : D;
     using M_ = Mma<T>;
     constexpr int KS = BT::KS, NJ = BT::NJ, RPI = BT::RPI, NLD = BT::NLD;
     constexpr int NQB = CAUSAL ? NBW + 1 : 2 * NBW + 1;  // query blocks that reach a key block
@@ -561,7 +581,7 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
     const int key_wgs = (int)gridDim.x - p.red_wgs;
     if ((int)blockIdx.x >= key_wgs) {
         using S = typename T::storage;
-        bwd_reduce_rows<T>(p.partial, reinterpret_cast<S *>(p.dk), reinterpret_cast<S *>(p.dv), p.B, p.N, p.M, p.H, D,
+        bwd_reduce_rows<T>(p.partial, reinterpret_cast<S *>(p.dk), reinterpret_cast<S *>(p.dv), p.B, p.N, p.M, p.H, dh,
                            p.L, p.causal, p.red_first_row, p.red_lg_sb,
                            (size_t)((int)blockIdx.x - key_wgs) * (BWD_WPB * 64) + threadIdx.x);
         return;
@@ -579,11 +599,13 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
     const int strip = (unit / H) % NS;
     const int b = unit / (H * NS);
     const int kb0 = strip * SB;
-    const size_t rs = (size_t)H * D;
-    const uint16_t *Qb = p.q + ((size_t)b * N * H + h) * D + 8 * lchk;
-    const uint16_t *Gb = p.dout + ((size_t)b * N * H + h) * D + 8 * lchk;
-    const uint16_t *Kb = p.k + ((size_t)b * p.M * H + h) * D + 8 * lchk;
-    const uint16_t *Vb = p.v + ((size_t)b * p.M * H + h) * D + 8 * lchk;
+    const size_t rs = (size_t)H * dh;
+    const int pchk = PART ? min(lchk, dh / 8 - 1) : lchk;  // the piece this lane fetches
+    const bool own_piece = !PART || 8 * lchk < dh;         // the piece exists: this lane stores it
+    const uint16_t *Qb = p.q + ((size_t)b * N * H + h) * dh + 8 * pchk;
+    const uint16_t *Gb = p.dout + ((size_t)b * N * H + h) * dh + 8 * pchk;
+    const uint16_t *Kb = p.k + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
+    const uint16_t *Vb = p.v + ((size_t)b * p.M * H + h) * dh + 8 * pchk;
 
     auto load_block = [&](const uint16_t *base, int row0, u32x4_t (&dst)[NLD]) {
         const uint16_t *ptr = base + (size_t)(row0 + lrow) * rs;
@@ -620,6 +642,10 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
         bt.put(3, rg);
         bt.get(2, qq.Qf);
         bt.get(3, qq.Gf);
+        if constexpr (PART) {
+            bt.clear_behind(qq.Qf, dh);
+            bt.clear_behind(qq.Gf, dh);
+        }
         bt.transpose(qq.Qf, qq.QT);
         bt.transpose(qq.Gf, qq.GT);
 #pragma unroll
@@ -698,10 +724,11 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
         }
         bt.put_result(0, tk, 1.0f);
         bt.put_result(1, tv, 1.0f);
-        uint16_t *dKp = p.dk + ((size_t)b * p.M * H + h) * D + 8 * lchk + (size_t)(k0 + lrow) * rs;
-        uint16_t *dVp = p.dv + ((size_t)b * p.M * H + h) * D + 8 * lchk + (size_t)(k0 + lrow) * rs;
+        uint16_t *dKp = p.dk + ((size_t)b * p.M * H + h) * dh + 8 * pchk + (size_t)(k0 + lrow) * rs;
+        uint16_t *dVp = p.dv + ((size_t)b * p.M * H + h) * dh + 8 * pchk + (size_t)(k0 + lrow) * rs;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
+            if (!own_piece) continue;
             *reinterpret_cast<u32x4_t *>(dKp + (size_t)(i * RPI) * rs) = bt.get_row_piece(0, i);
             *reinterpret_cast<u32x4_t *>(dVp + (size_t)(i * RPI) * rs) = bt.get_row_piece(1, i);
         }
@@ -817,5 +844,11 @@ __device__ __forceinline__ void bwd_reduce_rows(const float *__restrict__ partia
     *reinterpret_cast<Pack *>(dk + o) = ok;
     *reinterpret_cast<Pack *>(dv + o) = ov;
 }
+
+template <typename T, int D>
+int attn_bwd_tile_launch_td(const BwdTileParams &p, int nbw, bool causal, int sb, hipStream_t st);
+// part heads: layout of D channels, DC of them in the contractions
+template <typename T, int D, int DC>
+int attn_bwd_tile_part_launch_td(const BwdTileParams &p, int nbw, bool causal, int sb, hipStream_t st);
 
 }  // namespace hsa

@@ -1,0 +1,4 @@
+#include "hsa_attn_part_inst.h"
+namespace hsa {
+HSA_PART_INSTANTIATE(BF16, 32, 32)
+}  // namespace hsa

@@ -30,6 +30,15 @@
 // every K/V row is fetched once; later blocks' operands are requested before the current
 // block is computed (the strip loop is fully unrolled, every load has its own registers).
 // Lanes whose tree slot does not exist (level >= L) issue no load.
+//
+// Head sizes between the layouts (any other multiple of 8 up to 120: "part heads", DC > 0): rows
+// are laid out for the next of 32 / 64 / 128 channels, of which DC (a multiple of 32) take part in
+// the contractions and dh exist.  A lane whose 16-byte piece lies behind the head fetches the
+// head's last piece again (the same cache line, no extra traffic), the query operand's missing
+// channels are set to zero once they are in operand form (so whatever the other operand holds
+// there contributes nothing), and nothing is stored behind the head.  The traffic is that of the
+// real head size; only the instruction count is that of the layout.  B3 H8 N2048 D96 R16 causal:
+// 451 us on the gather kernel, 19.3 us here; forward and backward 2089 us -> 119 us a call.
 #pragma once
 
 #include "hsa_common.h"
@@ -72,6 +81,7 @@ struct TileParams {
     int NS;       // strips per sequence
     int n_units;  // B * NS * H
     int runs;     // runs of SB blocks one wavefront walks (a strip is SB * runs blocks): the kernel's RUNS
+    int dh;       // channels per head (kernels built for part heads; else the template's D)
     int xcd_swizzle;
     int alternate;    // neighbouring strips walk in opposite directions
     float scale_log2e;
@@ -100,14 +110,17 @@ template <int D, int NKL = 1> constexpr int tile_max_wpb() { return (D > 64 || N
 // strip of 4 * RUNS blocks instead of once per four; only the far tree block (the same for the 64
 // queries of a run) is exchanged between runs, requested two blocks ahead.  Straight-line code
 // like a single run; two runs are built.
-template <typename T, int D, int NBW, bool CAUSAL, int SB, bool WT = false, bool LSE = false, int RUNS = 1>
+// DC > 0: a part head, p.dh channels laid out like D, DC of them in the contractions.
+template <typename T, int D, int NBW, bool CAUSAL, int SB, bool WT = false, bool LSE = false, int RUNS = 1, int DC = 0>
 __global__ void __launch_bounds__((tile_max_wpb<D, (CAUSAL ? NBW + 1 : 2 * NBW + 1)>() * 64))
 attn_tile_kernel(TileParams p) {
     using M_ = Mma<T>;
     constexpr bool MULTI = RUNS > 1;
     static_assert(!MULTI || (SB == 4 && !WT), "runs are the 64 queries that share a far tree block");
-    constexpr int KS = D / 32;                         // 32-channel steps of the QK contraction
-    constexpr int NJ = D / 16;                         // 16-channel output tiles
+    constexpr bool PART = DC > 0;
+    static_assert(!PART || (!WT && DC % 32 == 0 && DC <= D && 2 * DC > D), "part heads: forward output and log-sum-exp");
+    constexpr int KS = (PART ? DC : D) / 32;           // 32-channel steps of the QK contraction
+    constexpr int NJ = (PART ? DC : D) / 16;           // 16-channel output tiles
     constexpr int NKL = CAUSAL ? NBW + 1 : 2 * NBW + 1;  // leaf key blocks per query block
     constexpr int CPR = D / 8;                         // 16-byte pieces per head-row
     constexpr int RPI = 64 / CPR;                      // rows covered by one load instruction
@@ -151,11 +164,14 @@ attn_tile_kernel(TileParams p) {
     const int NB = N / TILE_Q;
     constexpr int TOT = SB * RUNS;  // blocks per strip
     const int blk0 = s * TOT;       // NB is a multiple of the strip length (powers of two, strip <= NB)
-    const size_t rs = (size_t)p.H * D;  // elements between consecutive rows
-    const uint16_t *Qb = p.q + ((size_t)b * N * p.H + h) * D + 8 * lchk;
-    const uint16_t *Kb = p.k + ((size_t)b * p.M * p.H + h) * D + 8 * lchk;
-    const uint16_t *Vb = p.v + ((size_t)b * p.M * p.H + h) * D + 8 * lchk;
-    uint16_t *Ob = p.out + ((size_t)b * N * p.H + h) * D + 8 * lchk;
+    const int dh = PART ? p.dh : D;
+    const size_t rs = (size_t)p.H * dh;  // elements between consecutive rows
+    const int pchk = PART ? min(lchk, dh / 8 - 1) : lchk;  // the piece this lane fetches
+    const bool own_piece = !PART || 8 * lchk < dh;         // the piece exists: this lane stores it
+    const uint16_t *Qb = p.q + ((size_t)b * N * p.H + h) * dh + 8 * pchk;
+    const uint16_t *Kb = p.k + ((size_t)b * p.M * p.H + h) * dh + 8 * pchk;
+    const uint16_t *Vb = p.v + ((size_t)b * p.M * p.H + h) * dh + 8 * pchk;
+    uint16_t *Ob = p.out + ((size_t)b * N * p.H + h) * dh + 8 * pchk;
 
     // ---- lane constants -------------------------------------------------------------
     // selection matrices: output column n of tile jj picks channel 8*(n/4) + 4*jj + n%4
@@ -383,6 +399,11 @@ attn_tile_kernel(TileParams p) {
         // this block's raw registers are consumed: request a later block's
         if (decltype(always_tag)::value || next_blk >= 0) request(nsg, next_blk);
         lds_get(0, Qf);
+        if constexpr (PART) {  // the channels behind the head contribute nothing to a score
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                if (8 * (4 * ks + g) >= dh) Qf[ks] = u32x4_t{0u, 0u, 0u, 0u};
+        }
         lds_get(1, Kl[NEWI]);
         lds_get(2, Vn);
         lds_get(3, Kt);
@@ -526,6 +547,7 @@ attn_tile_kernel(TileParams p) {
             for (int i = 0; i < NLD; ++i) {
                 const int row = i * RPI + lrow;
                 const u32x4_t val = *reinterpret_cast<const u32x4_t *>(lds + row * RB + 16 * (lchk ^ swz(row)));
+                if (!own_piece) continue;
                 if constexpr ((HSA_TILE_NT & 32) != 0) *reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs) = val;
                 else __builtin_nontemporal_store(val, reinterpret_cast<u32x4_t *>(optr + (size_t)(i * RPI) * rs));
             }
@@ -587,5 +609,16 @@ template <typename T, int D>
 int attn_tile_weights_launch_td(const TileParams &p, int nbw, bool causal, int wpb, hipStream_t st);
 template <typename T, int D>
 int attn_tile_lse_launch_td(const TileParams &p, int nbw, bool causal, int sb, int wpb, hipStream_t st);
+// part heads (layout D, DC channels in the contractions): output, and log-sum-exp where p.lse is set
+template <typename T, int D, int DC>
+int attn_tile_part_launch_td(const TileParams &p, int nbw, bool causal, int sb, int wpb, hipStream_t st);
+
+// Head sizes the 16-bit tile kernels take: 32, 64 and 128 channels, and every other multiple of 8
+// below 128 as a part head on the next layout.
+constexpr bool tile_head_is_part(int D) { return D != 32 && D != 64 && D != 128; }
+constexpr bool tile_head_ok(int D) { return D >= 8 && D <= 128 && D % 8 == 0; }
+constexpr int tile_head_layout(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : 128; }
+// the window radius part heads are built for
+constexpr int TILE_PART_MAX_R = 2 * TILE_Q;
 
 }  // namespace hsa

@@ -57,7 +57,7 @@ bool attn_tile_eligible(int N, int M, int H, int D, int L, int R, int dtype, boo
     // 2R+1+L floats has to fit the operand pitch
     if (want_weights && 2 * R + 1 + L > D * 2 + 16) return false;
     if (dtype != HSA_F16 && dtype != HSA_BF16) return false;
-    if (D != 32 && D != 64 && D != 128) return false;
+    if (!tile_head_ok(D) || (tile_head_is_part(D) && (want_weights || R > TILE_PART_MAX_R))) return false;
     if (N < TILE_Q || ilog2_exact(N) != L || L > TILE_MAX_LEVELS) return false;
     if (M < 2 * N - 1) return false;
     const int nbw = (R + TILE_Q - 1) / TILE_Q;
@@ -84,6 +84,7 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
     // second round of shorter strips loses to one round of longer ones, B1 H16 N4096 D128 R32
     // 26.1 -> 24.0 us)
     const long block_units = (long)B * H * NB;
+    const bool part = tile_head_is_part(D);
     const long slots = D > 64 ? 1024 : 2048;
     int sb = block_units >= 4 * slots ? 4 : (block_units >= 2 * slots ? 2 : 1);
     // long sequences with the causal mask: a wavefront walks two runs of four blocks, the window's
@@ -106,7 +107,7 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
     while (sb > NB) sb >>= 1;  // NB is a power of two
     // runs: strips of four blocks, one or two blocks of neighbours to either side (two: causal), no weights output
     const int nbw_ = (R + TILE_Q - 1) / TILE_Q;
-    if (sb != 4 || weights || nbw_ < 1 || nbw_ > (causal ? 2 : 1)) runs = 1;
+    if (sb != 4 || weights || part || nbw_ < 1 || nbw_ > (causal ? 2 : 1)) runs = 1;
     while (sb * runs > NB) runs >>= 1;
     p.runs = runs;
     p.NS = NB / (sb * runs);
@@ -116,6 +117,7 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
     p.n_units = (int)units;
     p.xcd_swizzle = knobs.swizzle;
     p.alternate = knobs.alternate;
+    p.dh = D;
     p.scale_log2e = 1.4426950408889634f / sqrtf((float)D);
     // wavefronts per workgroup: as many as the variant allows, but a divisor of the head count
     // where one at least half that large exists, so that a workgroup's wavefronts are heads of one
@@ -145,8 +147,19 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
         if (D == 64) return attn_tile_weights_launch_td<F16, 64>(p, nbw, causal != 0, wpb, st);
         return attn_tile_weights_launch_td<F16, 128>(p, nbw, causal != 0, wpb, st);
     }
+    if (lse && weights) return fail(HSA_ERR_UNSUPPORTED, "weights and log-sum-exp outputs together are not built");
+    if (part) {
+        const bool bf = dtype == HSA_BF16, c = causal != 0;
+        if (D < 32) return bf ? attn_tile_part_launch_td<BF16, 32, 32>(p, nbw, c, sb, wpb, st)
+                              : attn_tile_part_launch_td<F16, 32, 32>(p, nbw, c, sb, wpb, st);
+        if (D < 64) return bf ? attn_tile_part_launch_td<BF16, 64, 64>(p, nbw, c, sb, wpb, st)
+                              : attn_tile_part_launch_td<F16, 64, 64>(p, nbw, c, sb, wpb, st);
+        if (D <= 96) return bf ? attn_tile_part_launch_td<BF16, 128, 96>(p, nbw, c, sb, wpb, st)
+                               : attn_tile_part_launch_td<F16, 128, 96>(p, nbw, c, sb, wpb, st);
+        return bf ? attn_tile_part_launch_td<BF16, 128, 128>(p, nbw, c, sb, wpb, st)
+                  : attn_tile_part_launch_td<F16, 128, 128>(p, nbw, c, sb, wpb, st);
+    }
     if (lse) {
-        if (weights) return fail(HSA_ERR_UNSUPPORTED, "weights and log-sum-exp outputs together are not built");
         if (dtype == HSA_BF16) {
             if (D == 32) return attn_tile_lse_launch_td<BF16, 32>(p, nbw, causal != 0, sb, wpb, st);
             if (D == 64) return attn_tile_lse_launch_td<BF16, 64>(p, nbw, causal != 0, sb, wpb, st);

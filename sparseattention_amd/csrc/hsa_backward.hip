@@ -19,9 +19,6 @@
 
 namespace hsa {
 
-template <typename T, int D>
-int attn_bwd_tile_launch_td(const BwdTileParams &p, int nbw, bool causal, int sb, hipStream_t st);
-
 // ---------------------------------------------------------------- parent build
 template <typename T, int VEC> struct BPack { typename T::storage e[VEC]; };
 
@@ -695,7 +692,7 @@ static bool attn_bwd_tile_eligible(int N, int M, int D, int L, int R, int dtype,
     (void)causal;
     if (dtype == HSA_F32) return attn_bwd_tile_f32_eligible(N, M, D, L, R);
     if (dtype != HSA_F16 && dtype != HSA_BF16) return false;
-    if (D != 32 && D != 64 && D != 128) return false;
+    if (!tile_head_ok(D) || (tile_head_is_part(D) && R > TILE_PART_MAX_R)) return false;
     if (N < TILE_Q || ilog2_exact(N) != L || L > TILE_MAX_LEVELS || M < 2 * N - 1) return false;
     const int nbw = (R + TILE_Q - 1) / TILE_Q;
     return nbw <= 4;
@@ -742,6 +739,14 @@ static int attn_bwd_tile_typed(const void *q, const void *k, const void *v, cons
     p.causal = causal != 0;
     p.red_first_row = first;
     p.red_wgs = (int)red_wgs;
+    p.dh = D;
+    if (tile_head_is_part(D)) {
+        const bool c = causal != 0;
+        if (D < 32) return attn_bwd_tile_part_launch_td<T, 32, 32>(p, nbw, c, sb, st);
+        if (D < 64) return attn_bwd_tile_part_launch_td<T, 64, 64>(p, nbw, c, sb, st);
+        if (D <= 96) return attn_bwd_tile_part_launch_td<T, 128, 96>(p, nbw, c, sb, st);
+        return attn_bwd_tile_part_launch_td<T, 128, 128>(p, nbw, c, sb, st);
+    }
     return D == 32 ? attn_bwd_tile_launch_td<T, 32>(p, nbw, causal != 0, sb, st)
          : D == 64 ? attn_bwd_tile_launch_td<T, 64>(p, nbw, causal != 0, sb, st)
                    : attn_bwd_tile_launch_td<T, 128>(p, nbw, causal != 0, sb, st);
@@ -754,14 +759,16 @@ int &bwd_fused_strip_knob() {
 }
 template <typename T, int D>
 int attn_bwd_fused_launch_td(const BwdFusedParams &fp, bool causal, hipStream_t st);
+template <typename T, int D>
+int attn_bwd_fused_part_launch_td(const BwdFusedParams &fp, bool causal, hipStream_t st);
 
 static bool attn_bwd_fused_eligible(int N, int M, int D, int L, int R, int dtype, int causal) {
     if (dtype != HSA_F16 && dtype != HSA_BF16) return false;
-    if (D != 32 && D != 64 && D != 128) return false;
+    if (!tile_head_ok(D)) return false;
     if (N < TILE_Q * BWD_STRIP || ilog2_exact(N) != L || L > TILE_MAX_LEVELS || M < 2 * N - 1) return false;
-    // 128 channels (two wavefronts per head) only with the causal mask: without it the exchange
+    // more than 64 channels (two wavefronts per head) only with the causal mask: without it the exchange
     // buffers leave room for one workgroup per CU
-    if (D == 128 && causal == 0) return false;
+    if (D > 64 && causal == 0) return false;
     // one block of neighbours to either side, or two with the causal mask
     return R <= TILE_Q || (R <= 2 * TILE_Q && causal != 0);
 }
@@ -802,6 +809,11 @@ static int attn_bwd_fused_typed(const void *q, const void *k, const void *v, con
     p.red_first_row = first;
     p.red_wgs = (int)red_wgs;
     p.red_lg_sb = 2;
+    p.dh = D;
+    if (tile_head_is_part(D))
+        return D < 32 ? attn_bwd_fused_part_launch_td<T, 32>(fp, causal != 0, st)
+             : D < 64 ? attn_bwd_fused_part_launch_td<T, 64>(fp, causal != 0, st)
+                      : attn_bwd_fused_part_launch_td<T, 128>(fp, causal != 0, st);
     return D == 32 ? attn_bwd_fused_launch_td<T, 32>(fp, causal != 0, st)
          : D == 64 ? attn_bwd_fused_launch_td<T, 64>(fp, causal != 0, st)
                    : attn_bwd_fused_launch_td<T, 128>(fp, causal != 0, st);
@@ -947,7 +959,7 @@ int hsa_attn_bwd_saved(const void *q, const void *k, const void *v, const void *
     HSA_REQUIRE(R >= 0, "bad R=%d", R);
     if (!hsa::attn_bwd_fused_eligible(N, M, D, L, R, dtype, causal))
         return hsa::fail(HSA_ERR_UNSUPPORTED, "one-pass backward not available for N=%d D=%d L=%d R=%d causal=%d dtype=%d "
-                         "(16-bit types, 32, 64 or 128 channels per head, radius up to 16, or up to 32 with the causal mask, "
+                         "(16-bit types, a multiple of 8 channels per head up to 128, radius up to 16, or up to 32 with the causal mask, "
                          "at least 64 leaves)", N, D, L, R, causal ? 1 : 0, dtype);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)dout |
                            (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv | (uintptr_t)workspace) & 15) == 0;

@@ -1421,3 +1421,52 @@ def test_module_trains_end_to_end_like_the_oracle():
     _grad_close(yd.grad, yr.grad, torch.float32, "dy")
     for name, p in md.named_parameters():
         _grad_close(p.grad, w[name].grad, torch.float32, name)
+
+
+# head sizes between the tile layouts (B, N, H, D, R): the smallest and the largest of each layout, a
+# head that ends inside the second wavefront's half (72, 80), key rows past 2N-1 (M)
+PART_HEAD_CASES = [(1, 16, 2, 8, 1, None), (2, 64, 3, 24, 16, None), (1, 128, 5, 40, 0, None), (2, 256, 2, 48, 17, 600),
+                   (1, 512, 3, 56, 32, None), (2, 64, 2, 72, 16, None), (1, 256, 3, 80, 32, None), (1, 32, 4, 88, 9, 70),
+                   (3, 1024, 4, 96, 16, None), (1, 128, 1, 104, 20, None), (1, 64, 7, 120, 31, None)]
+
+
+@pytest.mark.parametrize("case", PART_HEAD_CASES)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_part_heads_on_the_tile_kernels(case, causal, dtype, tile_knobs):
+    """Head sizes that are a multiple of 8 but not 32 / 64 / 128: forward (every strip length) and
+    the two backward formulations on the tile kernels against the fp64 oracle, and through autograd."""
+    B, N, H, D, R, M = case
+    q, k, v = make_qkv(B, N, H, D, dtype, seed=N + R + D, M=M)
+    go = torch.randn(B, N, H, D, generator=torch.Generator().manual_seed(N + D)).to(dtype)
+    o = oracle.topology_tables(N, causal)
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    want = oracle.attention_ref(qr, kr, vr, o["forward_idx"], o["forward_mask"] if causal else None, R)
+    want.backward(go.double())
+    refs = (qr.grad, kr.grad, vr.grad)
+    qd, kd, vd, gd = q.to(DEV), k.to(DEV), v.to(DEV), go.to(DEV)
+    t = sa.build_tree_topology(N, causal, device=DEV)
+    mask = t["forward_mask"] if causal else None
+    for strip in (0, 1, 2, 4, 8):
+        tile_knobs(strip, -1, -1, -1)
+        out = fn.attention_forward(qd, kd, vd, t["forward_idx"], mask, R, algo="tile")
+        assert_close(out, want.detach(), dtype, "part head, strips of %d" % strip)
+    tile_knobs(0, -1, -1, -1)
+    for name, g, ref in zip(("dQ", "dK", "dV"), fn.attention_backward(gd, qd, kd, vd, R, causal, algo="tile"), refs):
+        _grad_close(g, ref, dtype, name + " two passes")
+    if N >= 64 and (R <= 16 or causal) and (D <= 64 or causal):
+        assert fn.saved_state_backward_available(qd, kd, R, causal)
+        out, lse = fn.attention_forward_lse(qd, kd, vd, R, causal)
+        assert_close(out, want.detach(), dtype, "part head with log-sum-exp")
+        for strip in (4, 8, 16, 32):
+            assert _lib.lib().hsa_attn_bwd_saved_tune(strip) == 0
+            try:
+                got = fn.attention_backward_saved(gd, qd, kd, vd, out, lse, R, causal)
+            finally:
+                _lib.lib().hsa_attn_bwd_saved_tune(0)
+            for name, g, ref in zip(("dQ", "dK", "dV"), got, refs):
+                _grad_close(g, ref, dtype, "%s one pass, strips of %d" % (name, strip))
+    qa, ka, va = (x.clone().requires_grad_(True) for x in (qd, kd, vd))
+    sa.hierarchical_attention(qa, ka, va, t["forward_idx"], t["backward_gather"], mask, R).backward(gd)
+    for name, a, ref in zip(("dQ", "dK", "dV"), (qa, ka, va), refs):
+        _grad_close(a.grad, ref, dtype, name + " autograd")

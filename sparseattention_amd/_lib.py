@@ -104,6 +104,24 @@ def lib():
     return _lib
 
 
+_ext = None
+
+
+def ext():
+    """The extension module with the hot calls in native code (csrc/torch_ops.cpp); raises if it has
+    not been built."""
+    global _ext
+    if _ext is None:
+        lib()  # the library it links against, with the clearer message if nothing has been built
+        try:
+            from . import _hsa_torch
+        except ImportError as exc:
+            raise HsaError("the extension module _hsa_torch is missing (%s). Build it first: "
+                           "python -m sparseattention_amd._build" % exc)
+        _ext = _hsa_torch
+    return _ext
+
+
 def check(rc: int, what: str):
     if rc != 0:
         msg = lib().hsa_last_error().decode("utf-8", "replace")

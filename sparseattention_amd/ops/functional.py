@@ -300,6 +300,9 @@ def build_tree(Q_p, K_p, V_p, K_leaf, V_leaf, out: Optional[torch.Tensor] = None
     `out = K_full[:, N:]`) as long as each batch's rows are dense.  `out2`, if given,
     receives a second copy of the result (for instance `V_full[:, N:]`).
     """
+    res = _lib.ext().build_tree(Q_p, K_p, V_p, K_leaf, V_leaf, out, out2)
+    if res is not None:
+        return res
     _lib.require_gpu(Q_p, K_p, V_p, K_leaf, V_leaf, out, out2)
     B, N, H, D = K_leaf.shape
     assert N >= 2 and (N & (N - 1)) == 0, "leaf count must be a power of 2"
@@ -501,4 +504,10 @@ def hierarchical_attention(Q, K, V, idx_table, gather_table, mask_table=None, wi
     """Each leaf query attends to keys n-R..n+R plus one tree node per level.
     `mask_table is None` selects the non-causal mode; `gather_table` is unused by the
     forward pass."""
+    if one_pass_backward is not False and isinstance(window_size, int):
+        canon = _is_canonical(idx_table, mask_table, Q.shape[1])
+        if canon is not None:
+            out = _lib.ext().span_attention(Q, K, V, canon, window_size)
+            if out is not None:
+                return out
     return HierarchicalAttentionFunc.apply(Q, K, V, idx_table, gather_table, mask_table, window_size)

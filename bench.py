@@ -155,7 +155,7 @@ def cpu_plumbing_case(oracle, cores):
 LIB_LAUNCHERS = ("hsa_attn_fwd", "hsa_build_parents_fwd", "hsa_build_parents_strided_fwd", "hsa_cross_update_top_fwd",
                  "hsa_build_tree_fwd", "hsa_span_input_y", "hsa_topology_device", "hsa_cross_update_pack_weights")
 # the same launches made from the native layer (csrc/torch_ops.cpp)
-EXT_LAUNCHERS = ("span_attention", "build_tree")
+EXT_LAUNCHERS = ("span_attention", "build_tree", "add_layer_norm")
 
 
 def lm_forward_measure(steps, warmup, train_step=True):

@@ -389,6 +389,31 @@ int hsa_attn_bwd_static(const void *q, const void *k, const void *v, const void 
  */
 int hsa_span_input_y_bwd(const void *dy, void *dx, int B, int N, int C, int dtype, void *stream);
 
+/*
+ * Residual sum and layer norm of rows of C channels in one pass: sum = a + b (rounded to the element
+ * type), norm = (sum - mean) / sqrt(var + eps) * gamma + beta; statistics in fp32.  What the
+ * reference's decoder layer does between its blocks
+ * (hierarchical_attention_project/Hierarchical_Transformer_Pretrain.py:375-428) with an addition
+ * and an nn.LayerNorm.
+ *   a, b, sum, norm  [rows, C] dense; b NULL: the norm of a alone, sum NULL then
+ *   gamma, beta      [C] in the same element type
+ *   stats            [rows, 2] fp32 mean and reciprocal standard deviation, for the backward (or NULL)
+ * All tensors 16-byte aligned; hsa_add_layer_norm_ok tells whether C is handled (whole 16-byte
+ * pieces, at most 256 of them: 2048 channels of a 16-bit type).
+ *
+ * Backward, from the gradients of both results: dx (the gradient of a and of b alike) =
+ * dsum + d(norm)/d(sum)^T dnorm, dgamma, dbeta.
+ *   dsum       may be NULL (nothing else uses the sum)
+ *   workspace  hsa_add_layer_norm_bwd_workspace_bytes(rows, C) bytes, written before read
+ */
+int hsa_add_layer_norm_ok(int C, int dtype);
+int hsa_add_layer_norm_fwd(const void *a, const void *b, const void *gamma, const void *beta, void *sum,
+                           void *norm, float *stats, long rows, int C, float eps, int dtype, void *stream);
+size_t hsa_add_layer_norm_bwd_workspace_bytes(long rows, int C);
+int hsa_add_layer_norm_bwd(const void *dnorm, const void *dsum, const void *s, const float *stats,
+                           const void *gamma, void *dx, void *dgamma, void *dbeta, void *workspace,
+                           size_t workspace_bytes, long rows, int C, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -175,9 +175,85 @@ std::optional<Tensor> build_tree(const Tensor &Qp, const Tensor &Kp, const Tenso
     return out;
 }
 
+// ------------------------------------------------------------------ residual sum and layer norm
+struct NormShape {
+    long rows;
+    int C, dtype;
+};
+NormShape norm_shape(const Tensor &a) { return {(long)(a.numel() / a.size(-1)), (int)a.size(-1), type_code(a)}; }
+
+// (sum, norm) of a and b, or (undefined, norm) of a alone; stats may be undefined
+std::pair<Tensor, Tensor> add_norm_plain(const Tensor &a, const Tensor &b, const Tensor &gamma, const Tensor &beta,
+                                         double eps, const Tensor &stats) {
+    const NormShape s = norm_shape(a);
+    Tensor sum = b.defined() ? at::empty_like(a) : Tensor(), norm = at::empty_like(a);
+    c10::DeviceGuard guard(a.device());
+    check(hsa_add_layer_norm_fwd(a.data_ptr(), b.defined() ? b.data_ptr() : nullptr, gamma.data_ptr(), beta.data_ptr(),
+                                 b.defined() ? sum.data_ptr() : nullptr, norm.data_ptr(),
+                                 stats.defined() ? (float *)stats.data_ptr() : nullptr, s.rows, s.C, (float)eps, s.dtype,
+                                 stream_of(a)),
+          "hsa_add_layer_norm_fwd");
+    return {sum, norm};
+}
+
+// outputs: sum, norm (norm alone when there is nothing to add)
+struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &a, const std::optional<Tensor> &b_,
+                                 const Tensor &gamma, const Tensor &beta, double eps) {
+        const Tensor b = b_ ? *b_ : Tensor();
+        Tensor stats = at::empty({norm_shape(a).rows, 2}, a.options().dtype(at::kFloat));
+        auto [sum, norm] = add_norm_plain(a, b, gamma, beta, eps, stats);
+        ctx->set_materialize_grads(false);
+        ctx->saved_data["add"] = b.defined();
+        ctx->save_for_backward({b.defined() ? sum : a, stats, gamma});
+        if (b.defined()) return {sum, norm};
+        return {norm};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const bool add = ctx->saved_data["add"].toBool();
+        const Tensor dsum = add && grads[0].defined() ? grads[0].contiguous() : Tensor();
+        if (!grads.back().defined() || (add && !grads[1].defined()))  // the norm was not used
+            return {dsum, dsum, Tensor(), Tensor(), Tensor()};
+        Tensor dnorm = grads.back().contiguous();
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &stats = saved[1], &gamma = saved[2];
+        const NormShape s = norm_shape(x);
+        Tensor dx = at::empty_like(x), dgamma = at::empty_like(gamma), dbeta = at::empty_like(gamma);
+        Tensor ws = workspace(x, hsa_add_layer_norm_bwd_workspace_bytes(s.rows, s.C));
+        auto aligned = [](const Tensor &t) { return !t.defined() || aligned16(t) ? t : t.clone(); };
+        dnorm = aligned(dnorm);
+        const Tensor ds = aligned(dsum);
+        c10::DeviceGuard guard(x.device());
+        check(hsa_add_layer_norm_bwd(dnorm.data_ptr(), ds.defined() ? ds.data_ptr() : nullptr, x.data_ptr(),
+                                     (const float *)stats.data_ptr(), gamma.data_ptr(), dx.data_ptr(), dgamma.data_ptr(),
+                                     dbeta.data_ptr(), ws.data_ptr(), ws.nbytes(), s.rows, s.C, s.dtype, stream_of(x)),
+              "hsa_add_layer_norm_bwd");
+        return {dx, add ? dx : Tensor(), dgamma, dbeta, Tensor()};
+    }
+};
+
+// (a + b, layer_norm(a + b)), or (None, layer_norm(a)) without b; None where the kernel does not take it
+std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const std::optional<Tensor> &b_,
+                                                        const Tensor &gamma, const Tensor &beta, double eps) {
+    if (!a_.is_cuda() || a_.numel() == 0 || !same_kind(a_, gamma) || !same_kind(a_, beta) || gamma.dim() != 1 ||
+        gamma.size(0) != a_.size(-1) || beta.sizes() != gamma.sizes() || type_code(a_) < 0 ||
+        !hsa_add_layer_norm_ok((int)a_.size(-1), type_code(a_)) || (b_ && (!same_kind(a_, *b_) || b_->sizes() != a_.sizes())) ||
+        !gamma.is_contiguous() || !beta.is_contiguous() || !aligned16(gamma) || !aligned16(beta))
+        return std::nullopt;
+    const Tensor a = a_.contiguous(), b = b_ ? b_->contiguous() : Tensor();
+    if (!aligned16(a) || (b.defined() && !aligned16(b))) return std::nullopt;
+    if (at::GradMode::is_enabled() && (a.requires_grad() || (b.defined() && b.requires_grad()) || gamma.requires_grad() ||
+                                       beta.requires_grad())) {
+        variable_list r = AddLayerNorm::apply(a, b.defined() ? std::optional<Tensor>(b) : std::nullopt, gamma, beta, eps);
+        return std::make_pair(r.size() == 2 ? r[0] : Tensor(), r.back());
+    }
+    return add_norm_plain(a, b, gamma, beta, eps, Tensor());
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_hsa_torch, m) {
     m.def("span_attention", &span_attention);
     m.def("build_tree", &build_tree);
+    m.def("add_layer_norm", &add_layer_norm);
 }

@@ -15,8 +15,35 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .modules import HierarchicalAttention
 from .ops import generate_span_input_Y
+
+
+def _plain_norm(m) -> bool:
+    """An nn.LayerNorm over the last dimension with weight and bias that nobody hooks into."""
+    return (type(m) is nn.LayerNorm and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+
+
+def layer_norm(x, norm):
+    """norm(x) on this package's kernel where it takes the case."""
+    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda"):
+        r = _lib.ext().add_layer_norm(x, None, norm.weight, norm.bias, norm.eps)
+        if r is not None:
+            return r[1]
+    return norm(x)
+
+
+def add_layer_norm(x, branch, norm):
+    """(x + branch, norm(x + branch)): one kernel reads both once and writes both results, where it
+    takes the case (one GPU, one element type; autocast mixes types and keeps the two steps)."""
+    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda"):
+        r = _lib.ext().add_layer_norm(x, branch, norm.weight, norm.bias, norm.eps)
+        if r is not None:
+            return r
+    x = x + branch
+    return x, norm(x)
 
 
 class PositionwiseFeedForward(nn.Module):
@@ -60,17 +87,33 @@ class DecoderLayer(nn.Module):
         self.dropout = nn.Dropout(dropout)
 
     def forward(self, x, y, mask=None, return_attention=False):
-        # span nodes first: un-normalised leaves, normalised nodes; plain residual
-        y = y + self.dropout(self.self_attn.cross_update_Y(x, y_in=self.norm_y(y)))
-        # leaves: pre-norm attention over the window and the updated nodes
-        nx = self.norm1(x)
         if return_attention:
+            # span nodes first: un-normalised leaves, normalised nodes; plain residual
+            y = y + self.dropout(self.self_attn.cross_update_Y(x, y_in=self.norm_y(y)))
+            # leaves: pre-norm attention over the window and the updated nodes
+            nx = self.norm1(x)
             a, w = self.self_attn(nx, nx, nx, y=y, mask=mask, return_attention=True)
-        else:
-            a, w = self.self_attn(nx, nx, nx, y=y, mask=mask), None
-        x = x + self.dropout(a)
-        x = x + self.dropout(self.feed_forward(self.norm2(x)))
-        return (x, y, w) if return_attention else (x, y)
+            x = x + self.dropout(a)
+            x = x + self.dropout(self.feed_forward(self.norm2(x)))
+            return x, y, w
+        return self._chained(x, y, layer_norm(x, self.norm1), layer_norm(y, self.norm_y), mask)[:2]
+
+    def _chained(self, x, y, nx, ny, mask, following=None):
+        """The layer on inputs whose norms are there already (nx = norm1(x), ny = norm_y(y)).  With
+        `following`, the layer that comes next, its norms of the results are taken together with the
+        residual sums and returned as well: (x, y, nx, ny)."""
+        u = self.dropout(self.self_attn.cross_update_Y(x, y_in=ny))
+        y, ny = (y + u, None) if following is None else add_layer_norm(y, u, following.norm_y)
+        a = self.self_attn(nx, nx, nx, y=y, mask=mask)
+        x, n2 = add_layer_norm(x, self.dropout(a), self.norm2)
+        f = self.dropout(self.feed_forward(n2))
+        x, nx = (x + f, None) if following is None else add_layer_norm(x, f, following.norm1)
+        return x, y, nx, ny
+
+    def _may_chain(self) -> bool:
+        """Whether `_chained` may stand in for calling the layer: a plain DecoderLayer without hooks."""
+        return type(self) is DecoderLayer and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
+                                                   or self._backward_pre_hooks)
 
 
 class TransformerLM(nn.Module):
@@ -103,7 +146,13 @@ class TransformerLM(nn.Module):
         x = self.pos_encoding(self.embedding(trg) * math.sqrt(self.d_model))
         y = generate_span_input_Y(x)
         mask = self.make_causal_mask(trg)
-        for layer in self.layers:
+        layers = list(self.layers)
+        if layers and not return_attention and all(type(m) is DecoderLayer and m._may_chain() for m in layers):
+            nx, ny = layer_norm(x, layers[0].norm1), layer_norm(y, layers[0].norm_y)
+            for layer, following in zip(layers, layers[1:] + [None]):
+                x, y, nx, ny = layer._chained(x, y, nx, ny, mask, following)
+            return self.fc_out(x)
+        for layer in layers:
             if return_attention:
                 x, y, _ = layer(x, y, mask=mask, return_attention=True)
             else:

@@ -14,7 +14,9 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/hsa_gfx950.h"
@@ -42,6 +44,19 @@ void check(int rc, const char *what) {
 
 bool same_kind(const Tensor &a, const Tensor &b) {
     return b.defined() && b.is_cuda() && a.device() == b.device() && a.scalar_type() == b.scalar_type();
+}
+
+// Nothing that watches or transforms torch's own calls: no tracing, no dispatch mode, no tensor subclass
+// or functional transform, no forward-mode tangent.  Such calls go the general way, which either
+// supports them or says that it does not.
+bool ordinary(std::initializer_list<const Tensor *> ts) {
+    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                           c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize});
+    if (at::tracer::impl::is_dispatch_enabled() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python))
+        return false;
+    for (const Tensor *t : ts)
+        if (t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
+    return true;
 }
 
 bool aligned16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
@@ -106,7 +121,8 @@ struct SpanAttention : public torch::autograd::Function<SpanAttention> {
     }
 
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
-        const variable_list saved = ctx->get_saved_variables();
+        variable_list saved = ctx->get_saved_variables();
+        for (Tensor &t : saved) t = t.contiguous();  // (saved-tensor hooks may give back another layout)
         const Tensor &Q = saved[0], &K = saved[1], &V = saved[2];
         const bool causal = ctx->saved_data["causal"].toBool();
         const int R = (int)ctx->saved_data["R"].toInt();
@@ -114,7 +130,7 @@ struct SpanAttention : public torch::autograd::Function<SpanAttention> {
         const Tensor G = grads[0].contiguous();
         Tensor dq = at::empty_like(Q), dk = at::empty_like(K), dv = at::empty_like(V);
         c10::DeviceGuard guard(Q.device());
-        if (saved.size() == 5 && aligned16(G)) {
+        if (saved.size() == 5 && aligned16(G) && aligned16(Q) && aligned16(K) && aligned16(V) && aligned16(saved[3])) {
             const size_t bytes = hsa_attn_bwd_saved_workspace_bytes(s.B, s.N, s.M, s.H, s.D, s.L, R, causal, s.dtype);
             Tensor ws = workspace(Q, bytes);
             check(hsa_attn_bwd_saved(Q.data_ptr(), K.data_ptr(), V.data_ptr(), saved[3].data_ptr(),
@@ -139,7 +155,8 @@ struct SpanAttention : public torch::autograd::Function<SpanAttention> {
 std::optional<Tensor> span_attention(const Tensor &Q, const Tensor &K, const Tensor &V, bool causal, int64_t R) {
     if (!Q.is_cuda() || Q.dim() != 4 || K.dim() != 4 || !same_kind(Q, K) || !same_kind(Q, V) || type_code(Q) < 0 ||
         K.sizes() != V.sizes() || K.size(0) != Q.size(0) || K.size(2) != Q.size(2) || K.size(3) != Q.size(3) ||
-        K.size(1) < 2 * Q.size(1) - 1 || Q.numel() == 0 || log2_exact(Q.size(1)) < 0 || R < 0 || R > (1 << 20))
+        K.size(1) < 2 * Q.size(1) - 1 || Q.numel() == 0 || log2_exact(Q.size(1)) < 0 || R < 0 || R > (1 << 20) ||
+        !ordinary({&Q, &K, &V}))
         return std::nullopt;
     if (at::GradMode::is_enabled() && (Q.requires_grad() || K.requires_grad() || V.requires_grad()))
         return SpanAttention::apply(Q, K, V, causal, R);
@@ -215,12 +232,13 @@ struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
         if (!grads.back().defined() || (add && !grads[1].defined()))  // the norm was not used
             return {dsum, dsum, Tensor(), Tensor(), Tensor()};
         Tensor dnorm = grads.back().contiguous();
-        const variable_list saved = ctx->get_saved_variables();
+        auto aligned = [](const Tensor &t) { return !t.defined() || aligned16(t) ? t : t.clone(); };
+        variable_list saved = ctx->get_saved_variables();
+        for (Tensor &t : saved) t = aligned(t.contiguous());  // (saved-tensor hooks may give back another layout)
         const Tensor &x = saved[0], &stats = saved[1], &gamma = saved[2];
         const NormShape s = norm_shape(x);
         Tensor dx = at::empty_like(x), dgamma = at::empty_like(gamma), dbeta = at::empty_like(gamma);
         Tensor ws = workspace(x, hsa_add_layer_norm_bwd_workspace_bytes(s.rows, s.C));
-        auto aligned = [](const Tensor &t) { return !t.defined() || aligned16(t) ? t : t.clone(); };
         dnorm = aligned(dnorm);
         const Tensor ds = aligned(dsum);
         c10::DeviceGuard guard(x.device());
@@ -240,6 +258,7 @@ std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const 
         !hsa_add_layer_norm_ok((int)a_.size(-1), type_code(a_)) || (b_ && (!same_kind(a_, *b_) || b_->sizes() != a_.sizes())) ||
         !gamma.is_contiguous() || !beta.is_contiguous() || !aligned16(gamma) || !aligned16(beta))
         return std::nullopt;
+    if (!ordinary({&a_, &gamma, &beta}) || (b_ && !ordinary({&*b_}))) return std::nullopt;
     const Tensor a = a_.contiguous(), b = b_ ? b_->contiguous() : Tensor();
     if (!aligned16(a) || (b.defined() && !aligned16(b))) return std::nullopt;
     if (at::GradMode::is_enabled() && (a.requires_grad() || (b.defined() && b.requires_grad()) || gamma.requires_grad() ||

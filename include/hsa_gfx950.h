@@ -282,6 +282,13 @@ int hsa_build_parents_strided_bwd(const void *dout, const void *qp, const void *
                                   void *dkc, void *dvc, int B, int P, int H, int D,
                                   const int64_t *batch_strides, const int64_t *row_strides, int dtype,
                                   void *stream);
+/* The same with the gradient of the level's rows in two parts, added in fp32: dout (strided as
+ * above) and dout2 [B, P, H, D] dense, or NULL. */
+int hsa_build_parents_level_bwd(const void *dout, const void *dout2, const void *qp, const void *kp,
+                                const void *vp, const void *kc, const void *vc, void *dqp, void *dkp,
+                                void *dvp, void *dkc, void *dvc, int B, int P, int H, int D,
+                                const int64_t *batch_strides, const int64_t *row_strides, int dtype,
+                                void *stream);
 
 /*
  * Backward of the span attention for the canonical tables.
@@ -413,6 +420,28 @@ size_t hsa_add_layer_norm_bwd_workspace_bytes(long rows, int C);
 int hsa_add_layer_norm_bwd(const void *dnorm, const void *dsum, const void *s, const float *stats,
                            const void *gamma, void *dx, void *dgamma, void *dbeta, void *workspace,
                            size_t workspace_bytes, long rows, int C, int dtype, void *stream);
+
+/*
+ * Weight gradient of linear projections, dw[o, i] = sum over segments and rows of dy[r, o] * x[r, i],
+ * and with one segment the bias gradient dbias[o] = sum over rows of dy[r, o]: what the reference's
+ * nn.Linear layers (hierarchical_attention/modules/attention.py:22-37) leave to autograd's matrix
+ * products.  Sums in fp32; several segments may add to the same rows of dw, rows that none covers
+ * become zero.
+ *   dy [rows, O], x [rows, I]  16-bit, row strides ld_dy, ld_x in elements, rows 16-byte aligned
+ *   o_first                    first row of dw the segment adds to
+ *   dw [O, I] dense, dbias [O] of out_dtype: HSA_F32 or the operands' type; dbias may be NULL
+ *   workspace                  hsa_weight_grad_workspace_bytes bytes (0: sizes not handled; O and I
+ *                              have to be multiples of 8), written before read
+ */
+#define HSA_WEIGHT_GRAD_MAX_SEGMENTS 3
+typedef struct {
+    const void *dy, *x;
+    int64_t ld_dy, ld_x, rows;
+    int O, o_first;
+} hsa_weight_grad_segment;
+size_t hsa_weight_grad_workspace_bytes(int nseg, const hsa_weight_grad_segment *seg, int I, int with_bias);
+int hsa_weight_grad(int nseg, const hsa_weight_grad_segment *seg, int O, int I, void *dw, void *dbias,
+                    int out_dtype, void *workspace, size_t workspace_bytes, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

@@ -53,7 +53,8 @@ struct BwdStrides {
 
 template <typename T, int VEC, int CH>
 __global__ void __launch_bounds__(256)
-build_parents_bwd_kernel(const typename T::storage *__restrict__ dO, const typename T::storage *__restrict__ Qp,
+build_parents_bwd_kernel(const typename T::storage *__restrict__ dO, const typename T::storage *__restrict__ dO2,
+                         const typename T::storage *__restrict__ Qp,
                          const typename T::storage *__restrict__ Kp, const typename T::storage *__restrict__ Vp,
                          const typename T::storage *__restrict__ Kc, const typename T::storage *__restrict__ Vc,
                          typename T::storage *__restrict__ dQ, typename T::storage *__restrict__ dKp,
@@ -71,6 +72,7 @@ build_parents_bwd_kernel(const typename T::storage *__restrict__ dO, const typen
     const int b = (int)(u / ((long)H * P));
     // element offset of this (batch, row, head) in operand o; children: rows 2i and 2i+1
     auto at = [&](int o, int row) { return (size_t)b * sd.bs[o] + (size_t)row * sd.rs[o] + (size_t)h * D; };
+    if (dO2) dO2 += (((size_t)b * P + i) * H + h) * D;
     dO += at(0, i); Qp += at(1, i); Kp += at(2, i); Vp += at(3, i);
     dQ += at(6, i); dKp += at(7, i); dVp += at(8, i);
     const typename T::storage *Kc1 = Kc + at(4, 2 * i + 1), *Vc1 = Vc + at(5, 2 * i + 1);
@@ -91,6 +93,12 @@ build_parents_bwd_kernel(const typename T::storage *__restrict__ dO, const typen
             bload<T, VEC>(Vc + d, v0[c]);
             bload<T, VEC>(Vc1 + d, v1[c]);
             bload<T, VEC>(dO + d, g[c]);
+            if (dO2) {
+                float g2[VEC];
+                bload<T, VEC>(dO2 + d, g2);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) g[c][e] += g2[e];
+            }
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 s0 = fmaf(q[c][e], kp[c][e], s0);
@@ -143,12 +151,12 @@ build_parents_bwd_kernel(const typename T::storage *__restrict__ dO, const typen
 }
 
 template <typename T>
-static int build_parents_bwd_typed(const void *dout, const void *qp, const void *kp, const void *vp, const void *kc,
+static int build_parents_bwd_typed(const void *dout, const void *dout2, const void *qp, const void *kp, const void *vp, const void *kc,
                                    const void *vc, void *dqp, void *dkp, void *dvp, void *dkc, void *dvc, int B,
                                    int P, int H, int D, const BwdStrides &sd, hipStream_t st) {
     using S = typename T::storage;
     constexpr int VEC16 = 16 / (int)sizeof(S);
-    const uintptr_t al = (uintptr_t)dout | (uintptr_t)qp | (uintptr_t)kp | (uintptr_t)vp | (uintptr_t)kc |
+    const uintptr_t al = (uintptr_t)dout | (uintptr_t)dout2 | (uintptr_t)qp | (uintptr_t)kp | (uintptr_t)vp | (uintptr_t)kc |
                          (uintptr_t)vc | (uintptr_t)dqp | (uintptr_t)dkp | (uintptr_t)dvp | (uintptr_t)dkc |
                          (uintptr_t)dvc;
     int64_t strides = 0;
@@ -165,7 +173,7 @@ static int build_parents_bwd_typed(const void *dout, const void *qp, const void 
     const float scale = 1.0f / sqrtf((float)D);
 #define HSA_BWD(VECN, CHN)                                                                                  \
     build_parents_bwd_kernel<T, VECN, CHN><<<(unsigned)blocks, 256, 0, st>>>(                               \
-        (const S *)dout, (const S *)qp, (const S *)kp, (const S *)vp, (const S *)kc, (const S *)vc, (S *)dqp, \
+        (const S *)dout, (const S *)dout2, (const S *)qp, (const S *)kp, (const S *)vp, (const S *)kc, (const S *)vc, (S *)dqp, \
         (S *)dkp, (S *)dvp, (S *)dkc, (S *)dvc, B, P, H, D, G, sd, scale)
     if (vec_ok) {
         if (CH == 1) HSA_BWD(VEC16, 1);
@@ -823,7 +831,7 @@ static int attn_bwd_fused_typed(const void *q, const void *k, const void *v, con
 
 extern "C" {
 
-static int build_parents_bwd_any(const void *dout, const void *qp, const void *kp, const void *vp, const void *kc,
+static int build_parents_bwd_any(const void *dout, const void *dout2, const void *qp, const void *kp, const void *vp, const void *kc,
                                  const void *vc, void *dqp, void *dkp, void *dvp, void *dkc, void *dvc, int B, int P,
                                  int H, int D, const int64_t *batch_strides, const int64_t *row_strides, int dtype,
                                  void *stream) {
@@ -839,9 +847,9 @@ static int build_parents_bwd_any(const void *dout, const void *qp, const void *k
     }
     hipStream_t st = (hipStream_t)stream;
     switch (dtype) {
-        case HSA_F32: return hsa::build_parents_bwd_typed<hsa::F32>(dout, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
-        case HSA_F16: return hsa::build_parents_bwd_typed<hsa::F16>(dout, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
-        case HSA_BF16: return hsa::build_parents_bwd_typed<hsa::BF16>(dout, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
+        case HSA_F32: return hsa::build_parents_bwd_typed<hsa::F32>(dout, dout2, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
+        case HSA_F16: return hsa::build_parents_bwd_typed<hsa::F16>(dout, dout2, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
+        case HSA_BF16: return hsa::build_parents_bwd_typed<hsa::BF16>(dout, dout2, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, sd, st);
     }
     return hsa::fail(HSA_ERR_INVALID, "unknown dtype %d", dtype);
 }
@@ -849,7 +857,7 @@ static int build_parents_bwd_any(const void *dout, const void *qp, const void *k
 int hsa_build_parents_bwd(const void *dout, const void *qp, const void *kp, const void *vp, const void *kc,
                           const void *vc, void *dqp, void *dkp, void *dvp, void *dkc, void *dvc, int B, int P,
                           int H, int D, int dtype, void *stream) {
-    return build_parents_bwd_any(dout, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, nullptr, nullptr,
+    return build_parents_bwd_any(dout, nullptr, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, nullptr, nullptr,
                                  dtype, stream);
 }
 
@@ -857,7 +865,15 @@ int hsa_build_parents_strided_bwd(const void *dout, const void *qp, const void *
                                   const void *vc, void *dqp, void *dkp, void *dvp, void *dkc, void *dvc, int B,
                                   int P, int H, int D, const int64_t *batch_strides, const int64_t *row_strides,
                                   int dtype, void *stream) {
-    return build_parents_bwd_any(dout, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, batch_strides,
+    return build_parents_bwd_any(dout, nullptr, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, batch_strides,
+                                 row_strides, dtype, stream);
+}
+
+int hsa_build_parents_level_bwd(const void *dout, const void *dout2, const void *qp, const void *kp, const void *vp,
+                                const void *kc, const void *vc, void *dqp, void *dkp, void *dvp, void *dkc, void *dvc,
+                                int B, int P, int H, int D, const int64_t *batch_strides, const int64_t *row_strides,
+                                int dtype, void *stream) {
+    return build_parents_bwd_any(dout, dout2, qp, kp, vp, kc, vc, dqp, dkp, dvp, dkc, dvc, B, P, H, D, batch_strides,
                                  row_strides, dtype, stream);
 }
 

@@ -15,6 +15,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
@@ -269,10 +270,104 @@ std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const 
     return add_norm_plain(a, b, gamma, beta, eps, Tensor());
 }
 
+// ------------------------------------------------------------------ linear projections in training
+bool rows_ok(const Tensor &t) {
+    return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && aligned16(t);
+}
+
+using Segments = std::vector<std::tuple<Tensor, Tensor, int64_t>>;  // dY [rows, O], X [rows, I], first row of dW
+
+// (dW [O, I], db [O] or undefined) of the sum over the segments of dY^T X, in `type`; nullopt where the
+// kernel does not take the operands
+std::optional<std::pair<Tensor, Tensor>> weight_grad(const Segments &segs, int64_t O, at::ScalarType type, bool bias) {
+    if (segs.empty() || segs.size() > HSA_WEIGHT_GRAD_MAX_SEGMENTS || (bias && segs.size() != 1)) return std::nullopt;
+    const Tensor &like = std::get<1>(segs[0]);
+    if (!like.is_cuda() || (like.scalar_type() != at::kHalf && like.scalar_type() != at::kBFloat16) ||
+        (type != at::kFloat && type != like.scalar_type()))
+        return std::nullopt;
+    const int64_t I = like.size(-1);
+    hsa_weight_grad_segment seg[HSA_WEIGHT_GRAD_MAX_SEGMENTS];
+    int n = 0;
+    for (const auto &[dy, x, first] : segs) {
+        if (!same_kind(like, dy) || !same_kind(like, x) || !rows_ok(dy) || !rows_ok(x) || x.size(1) != I ||
+            x.size(0) != dy.size(0))
+            return std::nullopt;
+        if (x.size(0) == 0) continue;
+        seg[n++] = {dy.data_ptr(), x.data_ptr(), dy.stride(0), x.stride(0), x.size(0), (int)dy.size(1), (int)first};
+    }
+    const size_t bytes = n ? hsa_weight_grad_workspace_bytes(n, seg, (int)I, bias) : 0;
+    if (bytes == 0) return std::nullopt;
+    Tensor ws = workspace(like, bytes);
+    Tensor dw = at::empty({O, I}, like.options().dtype(type)), db = bias ? at::empty({O}, dw.options()) : Tensor();
+    c10::DeviceGuard guard(like.device());
+    check(hsa_weight_grad(n, seg, (int)O, (int)I, dw.data_ptr(), bias ? db.data_ptr() : nullptr, type_code(dw),
+                          ws.data_ptr(), ws.nbytes(), type_code(like), stream_of(like)),
+          "hsa_weight_grad");
+    return std::make_pair(dw, db);
+}
+
+// y = x w^T + b by the library's product; backward: the input's gradient by the library, the weight's
+// and the bias's by the split-rows kernel, straight into the parameters' type.  `w`, `b` are the
+// parameters in x's type (the casts that autocast makes), without their graph.
+struct Linear : public torch::autograd::Function<Linear> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias,
+                          const Tensor &w, const std::optional<Tensor> &b) {
+        ctx->save_for_backward({x, w, weight});
+        ctx->saved_data["bias"] = bias.has_value();
+        return at::linear(x, w, b);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &w = saved[1], &weight = saved[2];
+        const bool bias = ctx->saved_data["bias"].toBool();
+        const Tensor &g = grads[0];
+        Tensor dx, dw, db;
+        if (!g.defined()) return {dx, dw, db, Tensor(), Tensor()};
+        const Tensor g2 = g.reshape({-1, g.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
+        // a backward that is itself differentiated goes through the parameter, not its detached cast
+        const bool again = at::GradMode::is_enabled();
+        if (ctx->needs_input_grad(0)) dx = at::matmul(g, again ? weight.to(x.scalar_type()) : w);
+        const bool need_w = ctx->needs_input_grad(1), need_b = bias && ctx->needs_input_grad(2);
+        if (need_w && !again) {
+            if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), weight.scalar_type(), need_b)) {
+                dw = r->first;
+                db = r->second;
+            }
+        }
+        if (need_w && !dw.defined()) dw = at::mm(g2.t(), x2).to(weight.scalar_type());
+        if (need_b && !db.defined()) db = g2.sum(0).to(weight.scalar_type());
+        return {dx, dw, db, Tensor(), Tensor()};
+    }
+};
+
+// F.linear(x, weight, bias) under the current autocast state; nullopt where nothing is to be gained
+// (no gradient of the weight, types other than the 16-bit ones, a result large enough to fill the chip
+// by itself) or where the call is not a plain one
+std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias) {
+    if (!at::GradMode::is_enabled() || !weight.requires_grad() || !x.is_cuda() || x.dim() < 2 || weight.dim() != 2 ||
+        x.numel() == 0 || x.size(-1) != weight.size(1) || x.device() != weight.device() || !weight.is_contiguous())
+        return std::nullopt;
+    const int64_t O = weight.size(0), I = weight.size(1);
+    if (O % 8 || I % 8 || ((O + 127) / 128) * ((I + 127) / 128) > 256) return std::nullopt;
+    if (bias && (bias->dim() != 1 || bias->size(0) != O || !same_kind(weight, *bias))) return std::nullopt;
+    if (!ordinary({&x, &weight}) || (bias && !ordinary({&*bias}))) return std::nullopt;
+    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    const at::ScalarType type = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
+    if (type != at::kHalf && type != at::kBFloat16) return std::nullopt;
+    if (!cast && weight.scalar_type() != type) return std::nullopt;
+    if (cast && ((weight.scalar_type() != at::kFloat && weight.scalar_type() != type) || type_code(x) < 0)) return std::nullopt;
+    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t; };
+    const Tensor w = as(weight).detach();
+    const std::optional<Tensor> b = bias ? std::optional<Tensor>(as(*bias).detach()) : std::nullopt;
+    return Linear::apply(as(x), weight, bias, w, b);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_hsa_torch, m) {
     m.def("span_attention", &span_attention);
     m.def("build_tree", &build_tree);
     m.def("add_layer_norm", &add_layer_norm);
+    m.def("linear", &linear);
+    m.def("weight_grad", &weight_grad);
 }

@@ -17,6 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
+from ..ops.linear import linear
 from ..ops.topology import build_tree_topology
 
 
@@ -233,8 +234,8 @@ class HierarchicalAttention(nn.Module):
     def _span_levels_backward(self, dy: torch.Tensor, kept: dict):
         """Gradients of `_span_levels` with respect to x, y_in and the stacked q|k|v weights:
         per level one kernel (the three weights are recomputed, every gradient row written once
-        into the fused layouts) and two GEMMs (input gradient and weight gradient of the fused
-        key/value projection).  Returns (dx, dy_in, dW_qkv [3D, D] fp32)."""
+        into the fused layouts) and one GEMM (gradient of the level's input); the weight gradients
+        of all levels are one contraction at the end.  Returns (dx, dy_in, dW_qkv [3D, D])."""
         x, y_in, qkv, blocks = kept["x"], kept["y_in"], kept["qkv"], kept["blocks"]
         kvs, masks, w_qkv, w_kv = kept["kvs"], kept["masks"], kept["w_qkv"], kept["w_kv"]
         B, N, D = x.shape
@@ -242,37 +243,41 @@ class HierarchicalAttention(nn.Module):
         cdt, es = x.dtype, x.element_size()
         dy = dy.to(cdt).contiguous()
         dqkv = torch.empty_like(qkv)
-        dw_kv = torch.zeros((2 * D, D), dtype=torch.float32, device=x.device)
+        # level-major like `blocks`: the children of level 1 (the leaves), then those of the levels above
+        dkv = torch.empty((B * (2 * N - 2), 2 * D), dtype=cdt, device=x.device)
         A = ctypes.c_int64 * 11
-        bwd, code, stream = _lib.lib().hsa_build_parents_strided_bwd, _lib.dtype_code(x), _lib.stream_of(x)
+        bwd, code, stream = _lib.lib().hsa_build_parents_level_bwd, _lib.dtype_code(x), _lib.stream_of(x)
         rs = A(D, 3 * D, 3 * D, 3 * D, 2 * D, 2 * D, 3 * D, 3 * D, 3 * D, 2 * D, 2 * D)
         T3 = (N - 1) * 3 * D
-        d_above, dx = None, None
+        d_above = None
         with _lib.on_device(x):
             for lvl in range(len(self.sizes) - 1, -1, -1):
                 P, off = self.sizes[lvl], self.offsets[lvl]
-                g = dy[:, off:off + P]
-                g = (g + d_above) if d_above is not None else g.contiguous()
                 kv = kvs[lvl]
-                dkv = torch.empty_like(kv)
+                row = 0 if lvl == 0 else B * (N + self.offsets[lvl - 1])
+                dkv_l = dkv[row:row + 2 * B * P]
                 par, dpar = qkv.data_ptr() + off * 3 * D * es, dqkv.data_ptr() + off * 3 * D * es
-                kv_p, dkv_p = kv.data_ptr(), dkv.data_ptr()
-                rc = bwd(g.data_ptr(), par, par + D * es, par + 2 * D * es, kv_p, kv_p + D * es,
+                kv_p, dkv_p = kv.data_ptr(), dkv_l.data_ptr()
+                rc = bwd(dy.data_ptr() + off * D * es, None if d_above is None else d_above.data_ptr(),
+                         par, par + D * es, par + 2 * D * es, kv_p, kv_p + D * es,
                          dpar, dpar + D * es, dpar + 2 * D * es, dkv_p, dkv_p + D * es, B, P, H, Dh,
-                         A(P * D, T3, T3, T3, 4 * P * D, 4 * P * D, T3, T3, T3, 4 * P * D, 4 * P * D), rs, code, stream)
-                _lib.check(rc, "hsa_build_parents_strided_bwd")
+                         A((N - 1) * D, T3, T3, T3, 4 * P * D, 4 * P * D, T3, T3, T3, 4 * P * D, 4 * P * D), rs, code,
+                         stream)
+                _lib.check(rc, "hsa_build_parents_level_bwd")
                 if masks:
-                    dkv[:, :, D:].mul_(masks[lvl]).mul_(kept["scales"][lvl])
-                src = x if lvl == 0 else blocks[B * self.offsets[lvl - 1] * D:B * off * D].view(B, 2 * P, D)
-                dw_kv += torch.matmul(dkv.reshape(-1, 2 * D).t(), src.reshape(-1, D)).float()
-                d_src = torch.matmul(dkv, w_kv)  # [B, 2P, D]
-                if lvl == 0:
-                    dx = d_src
-                else:
-                    d_above = d_src
+                    dkv_l.view(B, 2 * P, 2 * D)[:, :, D:].mul_(masks[lvl]).mul_(kept["scales"][lvl])
+                d_above = torch.matmul(dkv_l, w_kv)  # [B * 2P, D]
+        dx = d_above.view(B, N, D)
         dy_in = torch.matmul(dqkv, w_qkv)
-        dw_qkv = torch.matmul(dqkv.reshape(-1, 3 * D).t(), y_in.reshape(-1, D)).float()
-        dw_qkv[D:] += dw_kv
+        inner = B * (N - 2)  # rows of all children above the leaves
+        pairs = [(dqkv.view(-1, 3 * D), y_in.view(-1, D), 0), (dkv[:B * N], x.view(-1, D), D),
+                 (dkv[B * N:], blocks[:inner * D].view(inner, D), D)]
+        res = _lib.ext().weight_grad(pairs, 3 * D, torch.float32, False)
+        if res is not None:
+            return dx, dy_in, res[0]
+        dw_qkv = torch.matmul(pairs[0][0].t(), pairs[0][1]).float()
+        for g, src, _ in pairs[1:]:
+            dw_qkv[D:] += torch.matmul(g.t(), src).float()
         return dx, dy_in, dw_qkv
 
     # -- bottom-up: leaves -> span nodes ----------------------------------------
@@ -291,7 +296,7 @@ class HierarchicalAttention(nn.Module):
         if self.fused_training and x.is_cuda and N >= 2:
             # the same fused level loop as one differentiable function
             y_new = _SpanLevels.apply(self, drop_p, x, y_in, self.Wq_y.weight, self.Wk_y.weight, self.Wv_y.weight)
-            return self.out_proj_y(y_new)
+            return linear(self.out_proj_y, y_new)
 
         q_lv = torch.split(self._heads(self.Wq_y(y_in)), self.sizes, dim=1)
         k_lv = torch.split(self._heads(self.Wk_y(y_in)), self.sizes, dim=1)
@@ -311,7 +316,7 @@ class HierarchicalAttention(nn.Module):
                         mask: Optional[torch.Tensor] = None) -> torch.Tensor:
         B, N, D = x.shape
         assert y is not None, "y (parents) cannot be None during top-down update"
-        q = self._heads(self.Wq_x(x))
+        q = self._heads(linear(self.Wq_x, x))
         grad = self._needs_autograd((x, y), (self.Wq_x, self.Wk_x, self.Wv_x))
         if (not grad and not (self.training and self.dropout.p > 0) and y.size(1) == N - 1
                 and B * N * D >= self._DIRECT_PROJECTION_MIN_ELEMENTS):
@@ -333,13 +338,13 @@ class HierarchicalAttention(nn.Module):
             k, v = self._heads(k), self._heads(v)
         else:
             xy = torch.cat([x, y], dim=1)
-            k = self._heads(self.Wk_x(xy))
-            v = self.dropout(self._heads(self.Wv_x(xy)))
+            k = self._heads(linear(self.Wk_x, xy))
+            v = self.dropout(self._heads(linear(self.Wv_x, xy)))
         is_causal = mask is not None  # only the presence of a mask is looked at
         t = self._get_lookup_table(N, is_causal, x.device)
         heads = hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"],
                                        t["forward_mask"] if is_causal else None, self.window_size)
-        return self.out_proj_x(heads.view(B, N, D))
+        return linear(self.out_proj_x, heads.view(B, N, D))
 
     def _standard_attention(self, Q, K, V, mask):
         scores = torch.matmul(Q, K.transpose(-1, -2)) / math.sqrt(Q.size(-1))

@@ -1,0 +1,27 @@
+"""`linear(layer, x)`: an nn.Linear whose weight and bias gradients run on this package's kernel."""
+from __future__ import annotations
+
+import torch
+import torch.nn as nn
+from torch.nn.modules import module as _module
+
+from .. import _lib
+
+
+def _plain(layer) -> bool:
+    """An nn.Linear that nobody hooks into, so that its forward may be bypassed."""
+    return (type(layer) is nn.Linear and "forward" not in layer.__dict__
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+            and not (_module._global_forward_hooks or _module._global_forward_pre_hooks
+                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+
+
+def linear(layer, x: torch.Tensor) -> torch.Tensor:
+    """layer(x).  In training on the GPU with 16-bit activations (or under autocast to such a type) the
+    backward computes the weight's and the bias's gradient in one contraction over the tokens
+    (csrc/hsa_weight_grad.hip), directly in the parameters' type; everything else is the layer itself."""
+    if x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(layer):
+        y = _lib.ext().linear(x, layer.weight, layer.bias)
+        if y is not None:
+            return y
+    return layer(x)

@@ -18,6 +18,7 @@ import torch.nn.functional as F
 from . import _lib
 from .modules import HierarchicalAttention
 from .ops import generate_span_input_Y
+from .ops.linear import linear
 
 
 def _plain_norm(m) -> bool:
@@ -55,7 +56,7 @@ class PositionwiseFeedForward(nn.Module):
         self.activation = {"relu": F.relu, "gelu": F.gelu}[activation]
 
     def forward(self, x):
-        return self.fc2(self.dropout(self.activation(self.fc1(x))))
+        return linear(self.fc2, self.dropout(self.activation(linear(self.fc1, x))))
 
 
 class PositionalEncoding(nn.Module):

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import sparseattention_amd as sa
+from sparseattention_amd.ops.linear import linear
 from sparseattention_amd.transformer import layer_norm
 
 pytestmark = pytest.mark.gpu
@@ -29,10 +30,11 @@ def test_saved_tensors_with_another_layout():
     mk = lambda n: torch.randn(B, n, H, D, device=DEV, dtype=torch.bfloat16, requires_grad=True)
     q, k, v = mk(N), mk(2 * N - 1), mk(2 * N - 1)
     norm = torch.nn.LayerNorm(D).to(DEV).to(torch.bfloat16)
+    lin = torch.nn.Linear(D, D).to(DEV).to(torch.bfloat16)
 
     def grads():
         o = sa.hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 4)
-        return torch.autograd.grad(layer_norm(o, norm).float().square().sum(), [q, k, v, norm.weight, norm.bias])
+        return torch.autograd.grad(linear(lin, layer_norm(o, norm)).float().square().sum(), [q, k, v, lin.weight, lin.bias])
 
     want = grads()
     turn = lambda s: s.transpose(0, -1).contiguous().transpose(0, -1)

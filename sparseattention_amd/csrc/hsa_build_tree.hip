@@ -37,7 +37,8 @@ struct TreeArgs {
     void *out, *out2;
     unsigned *counters;  // this launch's slice: counters_per_batch per batch element, all zero
     int N, H, D, L;
-    int lgG, lgH;        // lanes per head row, heads (both powers of two)
+    int groups, pieces;  // head groups per batch element; 16-byte pieces of a head row
+    int lgG, lgH;        // lanes per head row, heads per group (both powers of two)
     int lgS;             // subtrees per workgroup (phase B finishes lgS levels)
     int lg_nsub;         // subtrees per (batch, head) = N >> TL
     int gcap;            // most levels one phase-C stage takes
@@ -145,13 +146,15 @@ __device__ __forceinline__ void scores3(const VPack<T, VEC> &q, const VPack<T, V
     }
 }
 
-// one parent from its q/k/v row pieces and its two children's pieces (children are both key and value)
+// one parent from its q/k/v row pieces and its two children's pieces (children are both key and value);
+// a lane behind the head's last piece (live false) adds nothing to the scores
 template <typename T, int VEC>
 __device__ __forceinline__ VPack<T, VEC> combine(const VPack<T, VEC> &q, const VPack<T, VEC> &k,
                                                   const VPack<T, VEC> &v, const VPack<T, VEC> &c0,
-                                                  const VPack<T, VEC> &c1, int G, float scale) {
+                                                  const VPack<T, VEC> &c1, int G, float scale, bool live) {
     float s0, s1, s2;
     scores3<T, VEC>(q, k, c0, c1, s0, s1, s2);
+    if (!live) s0 = s1 = s2 = 0.f;
     s0 = group_sum(s0, G);
     s1 = group_sum(s1, G);
     s2 = group_sum(s2, G);
@@ -167,9 +170,14 @@ __device__ __forceinline__ VPack<T, VEC> combine(const VPack<T, VEC> &q, const V
 // LGG / LGH: log2 of the lanes per head row and of the head count when known at compile time
 // (-1: taken from the arguments).  With both fixed, the subtrees per workgroup, every slot
 // index and the cross-lane sums become constants: about half the instructions per level.
+// PART: a head row may fill fewer lanes than its group has (heads of 40, 48, 80, 96 ... channels): the
+// lanes behind it repeat its last piece on load, add nothing and store nothing.
+// GROUPED: heads are independent, so a head count that is no power of two is split into groups of its largest
+// power-of-two divisor; a group is to the rest of the kernel a batch element of its own whose rows
+// happen to lie a full row apart.
 struct VPackBits { uint32_t x, y, z, w; };
 
-template <typename T, int VEC, int TL, int THREADS, int LGG, int LGH>
+template <typename T, int VEC, int TL, int THREADS, int LGG, int LGH, bool PART, bool GROUPED>
 __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
     using S = typename T::storage;
     using P = VPack<T, VEC>;
@@ -197,10 +205,13 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
     const int p_local = u_local >> lgH;                 // subtree inside the workgroup
     const int lg_wpb = a.lg_nsub - lgS;                 // workgroups per batch element (log2)
     const int wg = (int)blockIdx.x & ((1 << lg_wpb) - 1);
-    const int b = (int)blockIdx.x >> lg_wpb;
+    const int vb = (int)blockIdx.x >> lg_wpb;           // (batch element, head group)
+    const int b = GROUPED ? vb / a.groups : vb;
+    const int h0 = GROUPED ? (vb - b * a.groups) << lgH : 0;  // first head of the group
+    const bool live = !PART || gl < a.pieces;
     const int sub = (wg << lgS) + p_local;
-    const size_t rs = (size_t)H * D;
-    const size_t hd = (size_t)h * D + (size_t)gl * VEC;
+    const size_t rs = (size_t)(GROUPED ? a.H : H) * D;
+    const size_t hd = (size_t)(h0 + h) * D + (size_t)(live ? gl : a.pieces - 1) * VEC;
     const S *Qp = (const S *)a.qp + (size_t)b * a.qp_bs + hd;
     const S *Kp = (const S *)a.kp + (size_t)b * a.kp_bs + hd;
     const S *Vp = (const S *)a.vp + (size_t)b * a.vp_bs + hd;
@@ -274,18 +285,25 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
     {
         const int first_lvl = TL + lgS + 1;
         const long rows_top = (long)(N >> (first_lvl - 1)) - 1;   // nodes of levels first_lvl .. root
-        const long ppr = (long)(rs / VEC);                        // 16-byte pieces per row
-        const long n_pieces = rows_top > 0 ? 3 * rows_top * ppr : 1;
+        const int lgP = lgH + lgG;                                // pieces of a row of this head group
+        const long per = rows_top > 0 ? rows_top << lgP : 1;
+        const long n_pieces = 3 * per;
         long t = (long)wg * THREADS + (long)threadIdx.x;
         if (t >= n_pieces) t = n_pieces - 1;
-        const long per = rows_top > 0 ? rows_top * ppr : 1;
         const int which = (int)(t / per);
         const long rem = t - (long)which * per;
         const S *base = which == 0 ? (const S *)a.qp + (size_t)b * a.qp_bs
                       : which == 1 ? (const S *)a.kp + (size_t)b * a.kp_bs
                                    : (const S *)a.vp + (size_t)b * a.vp_bs;
         const size_t first_row = rows_top > 0 ? (size_t)(level_offset(N, first_lvl) - N) : 0;
-        touch = *reinterpret_cast<const P *>(base + first_row * rs + (size_t)rem * VEC);
+        size_t at;
+        if constexpr (PART || GROUPED) {
+            const int slot = (int)(rem & ((1 << lgP) - 1)), pc = slot & (G - 1);
+            at = (size_t)(rem >> lgP) * rs + (h0 + (slot >> lgG)) * D + (!PART || pc < a.pieces ? pc : a.pieces - 1) * VEC;
+        } else {
+            at = (size_t)rem * VEC;
+        }
+        touch = *reinterpret_cast<const P *>(base + first_row * rs + at);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -298,6 +316,7 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
         for (int i = 0; i < NC / 2; ++i) {
             float s0, s1, s2;
             scores3<T, VEC>(rq[i], rk[i], rck[2 * i], rck[2 * i + 1], s0, s1, s2);
+            if (!live) s0 = s1 = s2 = 0.f;
             s0 = group_sum(s0, G);
             s1 = group_sum(s1, G);
             s2 = group_sum(s2, G);
@@ -308,7 +327,7 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
             for (int e = 0; e < VEC; ++e)
                 o[e] = w0 * to_float<T>(rv[i].e[e]) + w1 * to_float<T>(rcv[2 * i].e[e]) + w2 * to_float<T>(rcv[2 * i + 1].e[e]);
             keep[i] = pack_piece<T, VEC>(o);
-            store_node<STREAM>(Out + node_row(1, sub * (NC / 2) + i), keep[i]);
+            if (live) store_node<STREAM>(Out + node_row(1, sub * (NC / 2) + i), keep[i]);
         }
         // levels 2..TL
 #pragma unroll
@@ -320,9 +339,10 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
             for (int i = 0; i < NC / 4; ++i) {
                 if (i < np) {
                     const P r = combine<T, VEC>(rq[base + i], rk[base + i], rv[base + i], keep[cbase + 2 * i],
-                                                keep[cbase + 2 * i + 1], G, a.scale);
+                                                keep[cbase + 2 * i + 1], G, a.scale, live);
                     keep[base + i] = r;
                     const size_t row = node_row(j, sub * np + i);
+                    if (!live) continue;
                     if (j == TL && lgS == 0 && lg_wpb > 0) publish_piece(Out + row, r);  // the workgroup's node
                     else store_node<STREAM>(Out + row, r);
                 }
@@ -355,7 +375,7 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
     // deferring `out` as well loses again: the closing workgroups then work inside twice the
     // write traffic).  A closing workgroup writes its own after its last stage.
     auto second_copy = [&]() {
-        if (!Out2) return;
+        if (!Out2 || !live) return;
 #pragma unroll
         for (int j = 1; j <= TL; ++j) {
             const int np = NC >> j;
@@ -373,7 +393,7 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
     int level = TL + lgS;        // after the run this workgroup holds node `idx` of that level (all heads)
     int idx = wg;
     int lg_width = lg_wpb;       // nodes of that level per batch element (log2)
-    unsigned *cnt = a.counters + (size_t)b * a.counters_per_batch;
+    unsigned *cnt = a.counters + (size_t)vb * a.counters_per_batch;
     const int upb = THREADS >> lgG;  // (node, head) slots one pass of the workgroup covers
     asm volatile("" : "+s"(n_lds));  // one copy of the loop for every run: nothing specialised for the first
     if (n_lds > 0) lds_barrier();
@@ -390,11 +410,13 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
                 const size_t c_off = ((size_t)(((2 * p_local) << lgH) + h) << lgG) + gl;
                 const P c0 = *reinterpret_cast<const P *>(src + c_off * PB);
                 const P c1 = *reinterpret_cast<const P *>(src + (c_off + ((size_t)1 << (lgH + lgG))) * PB);
-                const P r = combine<T, VEC>(q, k, v, c0, c1, G, a.scale);
+                const P r = combine<T, VEC>(q, k, v, c0, c1, G, a.scale, live);
                 const size_t row = node_row(lvl_base + jj, (idx_base >> jj) + p_local);
-                if (jj == n_lds && more) publish_piece(Out + row, r);  // read by the stage that follows
-                else store_node<STREAM>(Out + row, r);
-                if (Out2) store_node<STREAM>(Out2 + row, r);
+                if (live) {
+                    if (jj == n_lds && more) publish_piece(Out + row, r);  // read by the stage that follows
+                    else store_node<STREAM>(Out + row, r);
+                    if (Out2) store_node<STREAM>(Out2 + row, r);
+                }
                 if (jj < n_lds) *reinterpret_cast<P *>(dst + (size_t)threadIdx.x * PB) = r;
             }
             if (jj < n_lds) lds_barrier();
@@ -487,11 +509,13 @@ __global__ void __launch_bounds__(THREADS) build_tree_fused_kernel(TreeArgs a) {
                 const int u = u_local + pass * upb;
                 const int p = u >> lgH;
                 if (p < (1 << (g - 1))) {
-                    const P r = combine<T, VEC>(cq[pass], ckk[pass], cvv[pass], ch0[pass], ch1[pass], G, a.scale);
+                    const P r = combine<T, VEC>(cq[pass], ckk[pass], cvv[pass], ch0[pass], ch1[pass], G, a.scale, live);
                     const size_t row = node_row(level + 1, (grp << (g - 1)) + p);
-                    if (g == 1 && lg_width > g) publish_piece(Out + row, r);  // read by the next stage
-                    else store_node<STREAM>(Out + row, r);
-                    if (Out2) store_node<STREAM>(Out2 + row, r);
+                    if (live) {
+                        if (g == 1 && lg_width > g) publish_piece(Out + row, r);  // read by the next stage
+                        else store_node<STREAM>(Out + row, r);
+                        if (Out2) store_node<STREAM>(Out2 + row, r);
+                    }
                     if (g > 1) *reinterpret_cast<P *>(bufX + (((size_t)u << lgG) + gl) * PB) = r;
                 }
             }
@@ -611,8 +635,14 @@ static int build_tree_fused_typed(const void *qp, const void *kp, const void *vp
                             (uintptr_t)out | (uintptr_t)out2;
     const int64_t strides = qp_bs | kp_bs | vp_bs | kleaf_bs | vleaf_bs | out_bs | out2_bs;
     if (D % VEC != 0 || (align & 15) != 0 || (strides % VEC) != 0) return HSA_ERR_UNSUPPORTED;
-    const int lgG = ilog2_pow2(D / VEC), lgH = ilog2_pow2(H), L = ilog2_exact(N);
-    if (lgG < 0 || lgG > 6 || lgH < 0 || L < TL) return HSA_ERR_UNSUPPORTED;
+    const int pieces = D / VEC, L = ilog2_exact(N);
+    int lgG = 0, lgH = 0;
+    while ((1 << lgG) < pieces) ++lgG;
+    if (lgG > 6 || L < TL) return HSA_ERR_UNSUPPORTED;
+    const bool part = pieces != 1 << lgG;
+    while ((H >> lgH & 1) == 0 && lgG + lgH < 9) ++lgH;  // heads per group
+    const int groups = H >> lgH;
+    const long VB = (long)B * groups;                    // to the kernel: batch elements
     const int lg_nsub = L - TL;
     // workgroup size: the preferred one, shrunk until a workgroup stays inside one batch element
     // and finishes at most TREE_NLMAX levels; it must hold whole (subtree, all heads) slots
@@ -622,11 +652,15 @@ static int build_tree_fused_typed(const void *qp, const void *kp, const void *vp
         // automatic: one resident round of workgroups is where the single launch pays (its
         // arrival step costs every workgroup a memory round trip, which only a kernel whose
         // workgroups all run at once does not feel): 512 threads when that fills the chip,
-        // 256 when it would leave half the compute units idle, the multi-launch path beyond
-        const long wg512 = ((long)B << lg_nsub) >> (9 - lg_slot);  // subtrees of all batch elements / subtrees per workgroup
+        // 256 when it would leave half the compute units idle, the multi-launch path beyond.
+        // us, several launches -> one: B5 N1024 H12 D64 18.2 -> 15.1, B4 N4096 H5 D64 31.1 -> 22.9, B3 N2048
+        // H8 D96 33.5 -> 21.0; past one round B8 N2048 H12 D64 38.6 -> 40.6.  Heads that fill part of
+        // their lanes have no kernel for the top levels in the other path (three launches and more):
+        // one launch up to two rounds (B4 N2048 H11 D80 40.9 -> 35.2, B4 N4096 H8 D96 51.1 -> 44.7).
+        const long wg512 = (VB << lg_nsub) >> (9 - lg_slot);  // subtrees of all batch elements / subtrees per workgroup
         const int cus = device_compute_units();
-        if (!force && wg512 > cus) return HSA_ERR_UNSUPPORTED;
-        threads_pref = wg512 * 2 <= cus ? 256 : 512;
+        if (!force && wg512 > (part ? 2 * cus : cus)) return HSA_ERR_UNSUPPORTED;
+        threads_pref = wg512 * 2 <= cus || (part && wg512 > cus) ? 256 : 512;
     }
     int lgT = ilog2_pow2(threads_pref);
     if (lgT < 0) return HSA_ERR_UNSUPPORTED;
@@ -638,11 +672,11 @@ static int build_tree_fused_typed(const void *qp, const void *kp, const void *vp
     const int threads = 1 << lgT;
     const int lgS = ilog2_pow2(threads >> (lgG + lgH));
     const int lg_wpb = lg_nsub - lgS;
-    const long blocks = (long)B << lg_wpb;
+    const long blocks = VB << lg_wpb;
     if (blocks > 0x7fffffffL) return HSA_ERR_UNSUPPORTED;
     TreeArgs a;
     a.qp = qp; a.kp = kp; a.vp = vp; a.kleaf = k_leaf; a.vleaf = v_leaf; a.out = out; a.out2 = out2;
-    a.N = N; a.H = H; a.D = D; a.L = L; a.lgG = lgG; a.lgH = lgH; a.lgS = lgS; a.lg_nsub = lg_nsub;
+    a.N = N; a.H = H; a.D = D; a.L = L; a.groups = groups; a.pieces = pieces; a.lgG = lgG; a.lgH = lgH; a.lgS = lgS; a.lg_nsub = lg_nsub;
     a.gcap = lgS + 2 < TREE_GCAP_MAX ? lgS + 2 : TREE_GCAP_MAX;
     a.qp_bs = qp_bs; a.kp_bs = kp_bs; a.vp_bs = vp_bs; a.kleaf_bs = kleaf_bs; a.vleaf_bs = vleaf_bs;
     a.out_bs = out_bs; a.out2_bs = out2_bs;
@@ -656,30 +690,35 @@ static int build_tree_fused_typed(const void *qp, const void *kp, const void *vp
     a.counters_per_batch = (int)per_batch;
     a.counters = nullptr;
     if (per_batch > 0) {
-        if (per_batch * B > TREE_SLICE_COUNTERS) return HSA_ERR_UNSUPPORTED;
+        if (per_batch * VB > TREE_SLICE_COUNTERS) return HSA_ERR_UNSUPPORTED;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
             (void)hipGetLastError();
             return HSA_ERR_UNSUPPORTED;
         }
-        a.counters = cap != hipStreamCaptureStatusNone ? tree_counters_for_capture(per_batch * B) : tree_counter_slice(st);
+        a.counters = cap != hipStreamCaptureStatusNone ? tree_counters_for_capture(per_batch * VB) : tree_counter_slice(st);
         if (!a.counters) return HSA_ERR_UNSUPPORTED;
     }
-#define HSA_TREE_LAUNCH(THR, GG, HH) \
-    build_tree_fused_kernel<T, VEC, TL, THR, GG, HH><<<(unsigned)blocks, THR, 0, st>>>(a)
+#define HSA_TREE_LAUNCH(THR, GG, HH, PT, GR) \
+    build_tree_fused_kernel<T, VEC, TL, THR, GG, HH, PT, GR><<<(unsigned)blocks, THR, 0, st>>>(a)
     // the common head layouts get their own instantiation at the two larger workgroup sizes
-    const int key = lgG * 16 + lgH;
-    if (threads == 512 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(512, 3, 3);        // 8 heads, 8 lanes per row
-    else if (threads == 512 && key == 4 * 16 + 4) HSA_TREE_LAUNCH(512, 4, 4);   // 16 heads, 16 lanes per row
-    else if (threads == 512 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(512, 4, 3);   // 8 heads, 16 lanes per row
-    else if (threads == 512 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(512, 3, 4);   // 16 heads, 8 lanes per row
-    else if (threads == 256 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(256, 3, 3);
-    else if (threads == 256 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(256, 4, 3);
-    else if (threads == 256 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(256, 3, 4);
-    else if (threads == 512) HSA_TREE_LAUNCH(512, -1, -1);
-    else if (threads == 256) HSA_TREE_LAUNCH(256, -1, -1);
-    else if (threads == 128) HSA_TREE_LAUNCH(128, -1, -1);
-    else HSA_TREE_LAUNCH(64, -1, -1);
+    const int key = part || groups > 1 ? -1 : lgG * 16 + lgH;
+    const bool heads12 = !part && lgG == 3 && lgH == 2, part8 = part && groups == 1 && lgG == 4 && lgH == 3;
+    if (threads == 512 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(512, 3, 3, false, false);        // 8 heads, 8 lanes per row
+    else if (threads == 512 && key == 4 * 16 + 4) HSA_TREE_LAUNCH(512, 4, 4, false, false);   // 16 heads, 16 lanes per row
+    else if (threads == 512 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(512, 4, 3, false, false);   // 8 heads, 16 lanes per row
+    else if (threads == 512 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(512, 3, 4, false, false);   // 16 heads, 8 lanes per row
+    else if (threads == 512 && heads12) HSA_TREE_LAUNCH(512, 3, 2, false, true);              // 4 or 12 heads, 8 lanes per row
+    else if (threads == 512 && part8) HSA_TREE_LAUNCH(512, 4, 3, true, false);                // 8 heads of 72 .. 120 channels
+    else if (threads == 256 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(256, 3, 3, false, false);
+    else if (threads == 256 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(256, 4, 3, false, false);
+    else if (threads == 256 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(256, 3, 4, false, false);
+    else if (threads == 256 && heads12) HSA_TREE_LAUNCH(256, 3, 2, false, true);
+    else if (threads == 256 && part8) HSA_TREE_LAUNCH(256, 4, 3, true, false);
+    else if (threads == 512) HSA_TREE_LAUNCH(512, -1, -1, true, true);
+    else if (threads == 256) HSA_TREE_LAUNCH(256, -1, -1, true, true);
+    else if (threads == 128) HSA_TREE_LAUNCH(128, -1, -1, true, true);
+    else HSA_TREE_LAUNCH(64, -1, -1, true, true);
 #undef HSA_TREE_LAUNCH
     return check_launch("build_tree_fused_kernel");
 }

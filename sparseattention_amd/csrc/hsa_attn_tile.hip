@@ -67,6 +67,56 @@ bool attn_tile_eligible(int N, int M, int H, int D, int L, int R, int dtype, boo
     return nbw <= TILE_MAX_NBW || nbw <= TILE_MAX_NBW_WIDE;
 }
 
+// Strip length (query blocks per wavefront) and wavefronts per workgroup.
+//
+// A CU takes one workgroup of up to eight wavefronts at a time (four at 128 channels: one wavefront per
+// SIMD), so what counts is how many query blocks the busiest CU walks, sb * wpb * ceil(workgroups /
+// 256), and whether they fit one resident round: every further round repeats the first loads' latency,
+// which a longer strip spreads over more blocks (measured per block against one round of strips of four:
+// 1.7 for single blocks, 1.2 to 1.45 for two, 1.15 for four, 1.1 for eight).  Among equals more
+// wavefronts win in one round (more loads in flight), longer strips in several.  Without the causal mask
+// strips of eight lose (three leaf blocks per query block in 256 registers: B8 H8 N8192 D64 84.3 -> 89.8
+// us).
+//
+// Against the longest strip that filled every wavefront slot (us, bf16, causal unless noted): B5 N1024
+// H12 D64 16.2 -> 10.3, not causal 18.5 -> 10.8; B12 N512 H8 D64 11.7 -> 9.1; B4 N2048 H6 D64 11.7 ->
+// 9.2; B3 N2048 H12 D64 15.6 -> 13.0; B12 N1024 H8 D64 18.4 -> 15.7, B6 N2048 H8 not causal 20.3 -> 16.1;
+// B2 N8192 H10 D64 25.2 -> 22.7; B3 N4096 H6 D128 26.1 -> 23.0; B3 N2048 H8 D96 18.4 -> 15.3.  B8 N2048
+// H8 D64 (strips of four), B16 N512 H8 D64 (two) and the long sequences (eight) stay as they were.
+//
+// Wavefronts per workgroup: all the variant allows, or a divisor of the head count at least half as
+// large, so that a workgroup's wavefronts are heads of one strip and read whole contiguous token rows;
+// four in one round where that leaves fewer blocks to the busiest CU.
+struct StripChoice {
+    int sb, wpb;
+};
+StripChoice choose_strip(long blocks, int H, int max_wpb, int most, bool eight, int forced_sb, int forced_wpb) {
+    int full = max_wpb;
+    if (H % max_wpb != 0)
+        for (int d = max_wpb - 1; d >= max_wpb / 2; --d)
+            if (H % d == 0) { full = d; break; }
+    const int first = forced_wpb ? forced_wpb : full;
+    StripChoice best = {1, first};
+    long least = -1;
+    const int longest = forced_sb ? forced_sb : (eight ? 8 : most);
+    for (int wpb : {first, 4}) {
+        if (wpb != first && (forced_wpb || wpb > max_wpb || (H % wpb != 0 && H % full == 0))) continue;
+        for (int sb = forced_sb ? forced_sb : 1; sb <= longest; sb *= 2) {
+            const long wgs = (blocks / sb + wpb - 1) / wpb, rounds = (wgs + 255) / 256;
+            if (wpb != first && rounds > 1) continue;
+            const long one[] = {120, 100, 100, 100}, several[] = {170, 145, 115, 110};
+            const int lg = sb == 1 ? 0 : sb == 2 ? 1 : sb == 4 ? 2 : 3;
+            // in units of 1/1600 block; ties: more wavefronts in one round, longer strips in several
+            const long cost = rounds * sb * wpb * (rounds > 1 ? several : one)[lg] * 16 + (rounds > 1 ? 8 / sb : sb);
+            if (least < 0 || cost < least) {
+                least = cost;
+                best = {sb, wpb};
+            }
+        }
+    }
+    return best;
+}
+
 int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, float *weights, float *lse, int B,
                        int N, int M, int H, int D, int L, int R, int causal, int dtype, hipStream_t st) {
     if ((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) != 0)
@@ -79,36 +129,21 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
     p.B = B; p.N = N; p.M = M; p.H = H; p.L = L; p.R = R;
     const int NB = N / TILE_Q;
     TileKnobs &knobs = tile_knobs();
-    // strip length: long enough to amortise the halo and to prefetch, short enough to fill every
-    // wavefront slot of the 256 CUs once (two per SIMD up to 64 channels, one at 128: there a
-    // second round of shorter strips loses to one round of longer ones, B1 H16 N4096 D128 R32
-    // 26.1 -> 24.0 us)
-    const long block_units = (long)B * H * NB;
+    const int nbw = (R + TILE_Q - 1) / TILE_Q;
     const bool part = tile_head_is_part(D);
-    const long slots = D > 64 ? 1024 : 2048;
-    int sb = block_units >= 4 * slots ? 4 : (block_units >= 2 * slots ? 2 : 1);
-    // long sequences with the causal mask: a wavefront walks two runs of four blocks, the window's
-    // neighbouring leaf blocks are then fetched once per eight blocks.  From eight blocks per
-    // wavefront slot on (us, strips of 4 -> 8): B1 H16 N65536 D128 R32 302 -> 286, N16384 80.0 ->
-    // 73.5, N8192 42.6 -> 39.1; B8 H8 N4096 D64 R16 40.2 -> 38.2, B1 H16 N65536 D64 156 -> 146; the
-    // headline shape (four blocks per slot) 20.4 -> 23.8, so not there.  Without the mask (three
-    // leaf blocks per query block in 256 registers) it loses: B8 H8 N8192 D64 84.3 -> 89.8.  Four
-    // runs gain nothing more at 64 channels and at 128 their code no longer fits the instruction
-    // cache (1465 us).
-    int runs = (causal && block_units >= 8 * slots) ? 2 : 1;
-    if (const int forced = knobs.sb) {
-        sb = forced > 4 ? 4 : forced;
-        runs = forced > 4 ? forced / 4 : 1;
-    }
-    // four or five leaf blocks per query block: shorter strips keep the operands in registers
-    if ((R + TILE_Q - 1) / TILE_Q >= (causal ? 3 : 2) && sb > 2) sb = 2;
-    if ((R + TILE_Q - 1) / TILE_Q >= 4 && !knobs.sb) sb = 1;  // longer strips spill at five leaf blocks + halo
-    if (!causal && (R + TILE_Q - 1) / TILE_Q > TILE_MAX_NBW) sb = 1;  // seven or nine leaf blocks: one block per wavefront
-    while (sb > NB) sb >>= 1;  // NB is a power of two
-    // runs: strips of four blocks, one or two blocks of neighbours to either side (two: causal), no weights output
-    const int nbw_ = (R + TILE_Q - 1) / TILE_Q;
-    if (sb != 4 || weights || part || nbw_ < 1 || nbw_ > (causal ? 2 : 1)) runs = 1;
-    while (sb * runs > NB) runs >>= 1;
+    // longest strip the variant takes: four blocks, with four or five leaf blocks per query block two
+    // (shorter strips keep the operands in registers), with more one
+    int most = 4;
+    if (nbw >= (causal ? 3 : 2)) most = 2;
+    if (nbw >= 4 && !knobs.sb) most = 1;        // longer strips spill at five leaf blocks + halo
+    if (!causal && nbw > TILE_MAX_NBW) most = 1;  // seven or nine leaf blocks: one block per wavefront
+    if (weights) most = 1;
+    while (most > NB) most >>= 1;               // NB is a power of two
+    // two runs of four blocks: the window's neighbouring leaf blocks are fetched once per eight blocks
+    const bool runs_built = most == 4 && !weights && !part && nbw >= 1 && nbw <= (causal ? 2 : 1) && NB >= 8;
+    const StripChoice c = choose_strip((long)B * H * NB, H, D > 64 ? 4 : 8, most, runs_built && causal, knobs.sb, knobs.wpb);
+    int sb = c.sb > 4 ? 4 : c.sb, runs = c.sb > 4 && runs_built ? 2 : 1;
+    if (sb > most) sb = most;
     p.runs = runs;
     p.NS = NB / (sb * runs);
     sb *= runs;  // the launchers switch on the strip length
@@ -119,19 +154,7 @@ int attn_tile_dispatch(const void *q, const void *k, const void *v, void *out, f
     p.alternate = knobs.alternate;
     p.dh = D;
     p.scale_log2e = 1.4426950408889634f / sqrtf((float)D);
-    // wavefronts per workgroup: as many as the variant allows, but a divisor of the head count
-    // where one at least half that large exists, so that a workgroup's wavefronts are heads of one
-    // strip and read whole contiguous token rows together (12 heads: 6 per workgroup, 35 -> 32 us
-    // at B8 N2048 D64)
-    int wpb = knobs.wpb;
-    if (wpb == 0) {
-        const int maxw = D > 64 ? 4 : 8;
-        wpb = maxw;
-        if (H % maxw != 0)
-            for (int d = maxw - 1; d >= maxw / 2; --d)
-                if (H % d == 0) { wpb = d; break; }
-    }
-    const int nbw = (R + TILE_Q - 1) / TILE_Q;
+    const int wpb = c.wpb;
     if (weights) {
         // one query block per wavefront
         p.NS = NB;

@@ -786,20 +786,41 @@ static int bwd_fused_launch_sb(const BwdFusedParams &q, int sb, hipStream_t st) 
     }
 }
 
+// Blocks per strip (4, 8, 16, 32).  One wavefront runs per SIMD, so the launch is rounds of 1024
+// wavefronts; longer strips fetch fewer halo blocks and finish more tree levels themselves, but quantise
+// coarser.  A round takes at least what one wavefront needs for its strip, and a full one what the
+// memory system needs for all of them; the rule takes the least of max(rounds x the former, wavefronts /
+// 1024 x the latter), both measured (us, bf16).  Measured for strips of 4 / 8 / 16 / 32: B6 N2048 H7 D64
+// 43.3 / 38.7 / 63 / 116, B12 N1024 H8 D64 43.9 / 39.7 / 64 / 116, B2 N8192 H10 D64 67.1 / 71.0 / 67.0 /
+// 117, B3 N2048 H8 D96 52.1 / 49.1 / 73.8 / 139, B3 N4096 H6 D128 71.8 / 78.7 / 80.7 / 133, B8 N2048 H8 D64
+// 51.0 / 44.7 / 65 / 116, B16 N512 H8 D64 27.1 / 37.6; strips of 8 / 16 / 32: B8 H8 N4096 D64 93 / 88 / 119,
+// B8 H8 N8192 D64 180 / 173 / 166, B1 H16 N65536 D64 348 / 327 / 317, B1 H16 N65536 D128 R32 734 / 679 / 657.
+// With 32 channels strips of four win throughout (B2 N4096 H9 22.7 / 26.2 / 42).
+inline int bwd_fused_strip(long waves1, int NB, int D) {
+    const int knob = bwd_fused_strip_knob();
+    const double alone[2][4] = {{22.5, 37, 63, 114}, {25, 44, 77, 132}};  // up to 64 channels, above
+    const double full[2][4] = {{26, 44.7, 88, 166}, {27, 45.9, 85, 164}};
+    int best = 4;
+    double least = 0;
+    for (int i = 0, sb = 4; i < 4 && NB % sb == 0; ++i, sb *= 2) {
+        if (knob ? sb > knob : (D < 64 && sb > 4)) break;
+        const double waves = (double)(waves1 / sb) / 1024, rounds = (double)((waves1 / sb + 1023) / 1024);
+        const double by_wave = rounds * alone[D > 64][i], by_memory = waves * full[D > 64][i];
+        const double us = by_wave > by_memory ? by_wave : by_memory;
+        if (i == 0 || knob || us < least) {
+            best = sb;
+            least = us;
+        }
+    }
+    return best;
+}
+
 // both launches of the one-pass backward on the layout of D channels
 template <typename T, int D, bool PART>
 static int bwd_fused_launch(const BwdFusedParams &fp, bool causal, hipStream_t st) {
     BwdFusedParams q = fp;
     const int NB = fp.t.N / TILE_Q, dh = PART ? fp.t.dh : D;
-    // the longest strips (8, 16, 32 blocks) whose wavefronts still fill the chip once (one per SIMD
-    // on 256 CUs): fewer halo blocks, more tree levels final inside the strip.  Measured (us, strips
-    // of 8 / 16 / 32): B8 H8 N4096 D64 93 / 88 / 119, B8 H8 N8192 D64 180 / 173 / 166, B1 H16 N65536
-    // D64 348 / 327 / 317, B1 H16 N65536 D128 R32 734 / 679 / 657, B1 H16 N16384 D64 92.6 / 94.2 / 120
-    const long waves8 = (long)(fp.t.n_units / 8) * (D > 64 ? 2 : 1);
-    const int knob = bwd_fused_strip_knob();
-    int sb = (NB % 8 == 0 && knob != 4 && (knob >= 8 || (D >= 64 && waves8 >= 1024))) ? 8 : 4;
-    if (sb == 8 && NB % 16 == 0 && (knob >= 16 || (knob == 0 && waves8 >= 2 * 1024))) sb = 16;
-    if (sb == 16 && NB % 32 == 0 && (knob >= 32 || (knob == 0 && waves8 >= 4 * 1024))) sb = 32;
+    const int sb = bwd_fused_strip((long)fp.t.n_units * (D > 64 ? 2 : 1), NB, D);
     const int nbw = fp.t.R > TILE_Q ? 2 : 1;
     if (nbw == 2 && !causal) return fail(HSA_ERR_UNSUPPORTED, "one-pass backward: window radius above 16 needs the causal mask");
     q.t.n_units = fp.t.n_units / sb;

@@ -453,7 +453,10 @@ int attn_tile_f32_dispatch(const void *q, const void *k, const void *v, void *ou
     const int NB = N / TQ;
     const int nbw = (R + TQ - 1) / TQ;
     const long block_units = (long)B * H * NB;
-    int sb = block_units >= 4 * 2048 ? 4 : (block_units >= 2 * 2048 ? 2 : 1);
+    // strips of two from three quarters of the wavefront slots on, of four where they fill all of them (us,
+    // strips of 1 / 2 / 4, D64 R16 causal: B3 N1024 H8 14.1 / 13.8 / 20.0, B4 N2048 H6 24.8 / 21.5 / 21.9, B5
+    // N1024 H12 26.6 / 23.0 / 23.6, B8 N2048 H8 54.0 / 46.3 / 40.8; B2 N256 H4 D32 5.1 / 7.0)
+    int sb = block_units >= 4 * 2048 ? 4 : (block_units >= 1536 ? 2 : 1);
     int forced_sb = 0, swizzle = 1;
     attn_tile_knobs_sb_swizzle(&forced_sb, &swizzle);
     if (forced_sb) sb = forced_sb;

@@ -291,6 +291,26 @@ int hsa_build_parents_level_bwd(const void *dout, const void *dout2, const void 
                                 void *stream);
 
 /*
+ * Backward of the last levels of HierarchicalAttention.cross_update_Y, from C children rows per batch
+ * element up to the root, one launch per level: the gradient that a level's rows get from the key /
+ * value projections of the level above and the level's parent backward together
+ * (hierarchical_attention/modules/attention.py:119-157; autograd there).  16-bit types, Dh 32 / 64 / 128.
+ *   dy     gradient of the parents' rows, pointing at the first level's first parent; the C-1 parents
+ *          follow level after level, root last
+ *   qkv    the parents' q | k | v rows, numbered alike; dqkv their gradients
+ *   kv     [B, 2C-2, 2*H*Dh] dense: the children's keys | values, the first level's C rows, then C/2, ..., 2;
+ *          dkv their gradients, same layout
+ *   w_kv   the stacked key and value weights W [2*H*Dh, H*Dh] (row = output feature) in the kernel's
+ *          operand order: element e of lane 16 g + r, contraction step s, column tile t of head h is
+ *          W[32 s + 8 g + e][h*Dh + 16 t + r], stored as [h][t][s][g][r][e]
+ *   *_bs, *_rs  batch / row strides in elements
+ */
+int hsa_span_levels_bwd(const void *dy, const void *qkv, const void *kv, const void *w_kv, void *dqkv,
+                        void *dkv, int B, int C, int H, int Dh, int64_t dy_bs, int64_t dy_rs,
+                        int64_t qkv_bs, int64_t qkv_rs, int64_t dqkv_bs, int64_t dqkv_rs, int dtype,
+                        void *stream);
+
+/*
  * Backward of the span attention for the canonical tables.
  * Replaces HierarchicalAttentionFunc.backward and its five kernels
  * (hierarchical_attention/ops/functional.py:171-264,
@@ -433,7 +453,7 @@ int hsa_add_layer_norm_bwd(const void *dnorm, const void *dsum, const void *s, c
  *   workspace                  hsa_weight_grad_workspace_bytes bytes (0: sizes not handled; O and I
  *                              have to be multiples of 8), written before read
  */
-#define HSA_WEIGHT_GRAD_MAX_SEGMENTS 3
+#define HSA_WEIGHT_GRAD_MAX_SEGMENTS 4
 typedef struct {
     const void *dy, *x;
     int64_t ld_dy, ld_x, rows;

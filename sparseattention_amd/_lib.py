@@ -74,6 +74,8 @@ def _declare(lib):
     lib.hsa_build_parents_strided_bwd.restype = I
     lib.hsa_build_parents_level_bwd.argtypes = [P] * 12 + [I] * 4 + [P, P, I, P]
     lib.hsa_build_parents_level_bwd.restype = I
+    lib.hsa_span_levels_bwd.argtypes = [P] * 6 + [I] * 4 + [I64] * 6 + [I, P]
+    lib.hsa_span_levels_bwd.restype = I
     lib.hsa_attn_fwd_lse.argtypes = [P] * 5 + [I] * 9 + [P]
     lib.hsa_attn_fwd_lse.restype = I
     lib.hsa_attn_bwd_saved_workspace_bytes.argtypes = [I] * 9

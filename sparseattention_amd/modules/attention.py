@@ -43,8 +43,8 @@ class _SpanLevels(torch.autograd.Function):
         # giving wrong gradients, and saved-tensor hooks (checkpointing, offloading) see them
         nl = len(kept["kvs"])
         ctx.save_for_backward(kept["x"], kept["y_in"], kept["qkv"], kept["blocks"], kept["w_qkv"], kept["w_kv"],
-                              *kept["kvs"], *kept["masks"])
-        ctx.module, ctx.levels, ctx.scales = module, nl, kept["scales"]
+                              *kept["kvs"], *kept["masks"], *kept["chain"])
+        ctx.module, ctx.levels, ctx.scales, ctx.masks = module, nl, kept["scales"], len(kept["masks"])
         ctx.in_dtypes = (x.dtype, y_in.dtype, wq.dtype)
         return y_new
 
@@ -53,7 +53,8 @@ class _SpanLevels(torch.autograd.Function):
         saved = ctx.saved_tensors  # raises autograd's own error if they were freed or modified
         nl = ctx.levels
         kept = dict(zip(("x", "y_in", "qkv", "blocks", "w_qkv", "w_kv"), saved[:6]))
-        kept["kvs"], kept["masks"], kept["scales"] = list(saved[6:6 + nl]), list(saved[6 + nl:]), ctx.scales
+        kept["kvs"], kept["masks"], kept["scales"] = list(saved[6:6 + nl]), list(saved[6 + nl:6 + nl + ctx.masks]), ctx.scales
+        kept["chain"] = saved[6 + nl + ctx.masks:]
         dx, dy_in, dw = ctx.module._span_levels_backward(dy, kept)
         xd, yd, wd = ctx.in_dtypes
         D = dx.shape[-1]
@@ -105,6 +106,10 @@ class HierarchicalAttention(nn.Module):
         return sizes, offsets
 
     _DIRECT_PROJECTION_MIN_ELEMENTS = 1 << 20
+    # training: levels of at most this many children over the batch run as fused chains, forward and backward
+    # (no chain / 1024 / 4096, us forward and backward of one module, fp16: B8 N2048 d768 2034 / 1996 / 1967, B2
+    # N512 d512 1503 / 1096 / 1102, B4 N64 d768 1330 / 1084 / 1089, B1 N4096 d1024 1649 / 1232 / 1159)
+    _TRAINING_CHAIN_ROWS = 4096
 
     def _heads(self, t: torch.Tensor) -> torch.Tensor:
         return t.view(t.shape[0], -1, self.num_heads, self.head_dim)
@@ -187,8 +192,12 @@ class HierarchicalAttention(nn.Module):
         qkv_p, blk_p, out_p = qkv.data_ptr(), blocks.data_ptr(), y_new.data_ptr()
         # child rows the fused upper levels take (0: shape not handled)
         # (y_new's rows are 16-byte aligned: the fused upper levels may run as a launch per level)
-        top_rows = 0 if keep or not self.fuse_top_levels else _lib.lib().hsa_cross_update_level_rows(B, H, Dh, code)
-        kvs, masks, scales = [], [], []
+        top_rows = 0
+        if self.fuse_top_levels and not (keep and drop_p > 0):
+            top_rows = _lib.lib().hsa_cross_update_level_rows(B, H, Dh, code)
+            if keep:  # (the projected rows are needed again: only where launches are what counts)
+                top_rows = min(top_rows, self._TRAINING_CHAIN_ROWS // B)
+        kvs, masks, scales, chain = [], [], [], ()
         src, off = x, 0
         with _lib.on_device(x):
             for lvl, P in enumerate(self.sizes):
@@ -200,6 +209,10 @@ class HierarchicalAttention(nn.Module):
                         src.data_ptr(), qkv_p + off * 3 * D * es, w_top.data_ptr(), out_p + off * D * es,
                         B, 2 * P, H, Dh, 0, (N - 1) * 3 * D, 3 * D, (N - 1) * D, D, code, stream)
                     _lib.check(rc, "hsa_cross_update_top_fwd")
+                    if keep:
+                        # the backward's keys and values of these levels' children, one GEMM for all
+                        rows = torch.cat([src, y_new[:, off:N - 2]], dim=1)  # [B, 4P-2, D]
+                        chain = (rows, F.linear(rows, w_kv))
                     break
                 kv = F.linear(src, w_kv)  # [B, 2P, 2D]
                 assert kv.dtype == cdt and kv.is_contiguous(), "projection result has an unexpected layout"
@@ -229,32 +242,50 @@ class HierarchicalAttention(nn.Module):
         if not keep:
             return y_new
         return y_new, {"x": x, "y_in": y_in, "qkv": qkv, "blocks": blocks, "kvs": kvs, "masks": masks,
-                       "scales": scales, "w_qkv": w_qkv, "w_kv": w_kv}
+                       "scales": scales, "w_qkv": w_qkv, "w_kv": w_kv, "chain": chain}
 
     def _span_levels_backward(self, dy: torch.Tensor, kept: dict):
         """Gradients of `_span_levels` with respect to x, y_in and the stacked q|k|v weights:
         per level one kernel (the three weights are recomputed, every gradient row written once
         into the fused layouts) and one GEMM (gradient of the level's input); the weight gradients
-        of all levels are one contraction at the end.  Returns (dx, dy_in, dW_qkv [3D, D])."""
+        of all levels are one contraction at the end.  The last levels, where the forward ran them as
+        a chain, are one launch each.  Returns (dx, dy_in, dW_qkv [3D, D])."""
         x, y_in, qkv, blocks = kept["x"], kept["y_in"], kept["qkv"], kept["blocks"]
         kvs, masks, w_qkv, w_kv = kept["kvs"], kept["masks"], kept["w_qkv"], kept["w_kv"]
         B, N, D = x.shape
         H, Dh = self.num_heads, self.head_dim
         cdt, es = x.dtype, x.element_size()
+        sizes, offsets = self._build_level_info(N)
         dy = dy.to(cdt).contiguous()
+        if dy.data_ptr() % 16:  # the chain's kernels move row pieces
+            dy = dy.clone()
         dqkv = torch.empty_like(qkv)
         # level-major like `blocks`: the children of level 1 (the leaves), then those of the levels above
-        dkv = torch.empty((B * (2 * N - 2), 2 * D), dtype=cdt, device=x.device)
+        inner = B * offsets[len(kvs) - 1] if kvs else 0  # rows of all children above the leaves
+        dkv = torch.empty((B * N + inner if kvs else 0, 2 * D), dtype=cdt, device=x.device)
         A = ctypes.c_int64 * 11
         bwd, code, stream = _lib.lib().hsa_build_parents_level_bwd, _lib.dtype_code(x), _lib.stream_of(x)
         rs = A(D, 3 * D, 3 * D, 3 * D, 2 * D, 2 * D, 3 * D, 3 * D, 3 * D, 2 * D, 2 * D)
         T3 = (N - 1) * 3 * D
         d_above = None
+        pairs = [(dqkv.view(-1, 3 * D), y_in.view(-1, D), 0)]
         with _lib.on_device(x):
-            for lvl in range(len(self.sizes) - 1, -1, -1):
-                P, off = self.sizes[lvl], self.offsets[lvl]
+            if kept["chain"]:
+                rows, kv = kept["chain"]
+                dkv_up, C, off = torch.empty_like(kv), 2 * sizes[len(kvs)], offsets[len(kvs)]
+                # the weights in the order the kernel multiplies them: [head][16-column tile][step][4][16][8]
+                w_ops = w_kv.view(2 * D // 32, 4, 8, H, Dh // 16, 16).permute(3, 4, 0, 1, 5, 2).contiguous()
+                rc = _lib.lib().hsa_span_levels_bwd(
+                    dy.data_ptr() + off * D * es, qkv.data_ptr() + off * 3 * D * es, kv.data_ptr(), w_ops.data_ptr(),
+                    dqkv.data_ptr() + off * 3 * D * es, dkv_up.data_ptr(), B, C, H, Dh, (N - 1) * D, D, T3, 3 * D, T3,
+                    3 * D, code, stream)
+                _lib.check(rc, "hsa_span_levels_bwd")
+                d_above = torch.mm(dkv_up[:, :C].reshape(-1, 2 * D), w_kv)  # [B * C, D]
+                pairs.append((dkv_up.view(-1, 2 * D), rows.view(-1, D), D))
+            for lvl in range(len(kvs) - 1, -1, -1):
+                P, off = sizes[lvl], offsets[lvl]
                 kv = kvs[lvl]
-                row = 0 if lvl == 0 else B * (N + self.offsets[lvl - 1])
+                row = 0 if lvl == 0 else B * (N + offsets[lvl - 1])
                 dkv_l = dkv[row:row + 2 * B * P]
                 par, dpar = qkv.data_ptr() + off * 3 * D * es, dqkv.data_ptr() + off * 3 * D * es
                 kv_p, dkv_p = kv.data_ptr(), dkv_l.data_ptr()
@@ -269,9 +300,10 @@ class HierarchicalAttention(nn.Module):
                 d_above = torch.matmul(dkv_l, w_kv)  # [B * 2P, D]
         dx = d_above.view(B, N, D)
         dy_in = torch.matmul(dqkv, w_qkv)
-        inner = B * (N - 2)  # rows of all children above the leaves
-        pairs = [(dqkv.view(-1, 3 * D), y_in.view(-1, D), 0), (dkv[:B * N], x.view(-1, D), D),
-                 (dkv[B * N:], blocks[:inner * D].view(inner, D), D)]
+        if kvs:
+            pairs.append((dkv[:B * N], x.view(-1, D), D))
+        if inner:
+            pairs.append((dkv[B * N:], blocks[:inner * D].view(inner, D), D))
         res = _lib.ext().weight_grad(pairs, 3 * D, torch.float32, False)
         if res is not None:
             return dx, dy_in, res[0]

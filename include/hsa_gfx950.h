@@ -463,6 +463,19 @@ size_t hsa_weight_grad_workspace_bytes(int nseg, const hsa_weight_grad_segment *
 int hsa_weight_grad(int nseg, const hsa_weight_grad_segment *seg, int O, int I, void *dw, void *dbias,
                     int out_dtype, void *workspace, size_t workspace_bytes, int dtype, void *stream);
 
+/*
+ * Leaf rows x [B, N, C] and span-node rows y [B, M, C], each of its own type (HSA_F32 or `dtype`), as
+ * one matrix out [B, N + M, C] of the 16-bit `dtype`: the cat([x, y]) of update_X_from_Y
+ * (hierarchical_attention/modules/attention.py:178-195) and its conversion.  C a multiple of 8, all
+ * tensors dense and 16-byte aligned.
+ * hsa_add_split_rows is its backward for two projections: a + b (both [B, N + M, C] of `dtype`, added
+ * in fp32) as dx and dy of their own types; either of the two may be NULL.
+ */
+int hsa_pack_rows(const void *x, const void *y, void *out, int B, int N, int M, int C, int x_dtype,
+                  int y_dtype, int dtype, void *stream);
+int hsa_add_split_rows(const void *a, const void *b, void *dx, void *dy, int B, int N, int M, int C,
+                       int x_dtype, int y_dtype, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

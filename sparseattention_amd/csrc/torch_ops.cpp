@@ -362,6 +362,90 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     return Linear::apply(as(x), weight, bias, w, b);
 }
 
+// ------------------------------------------------------------------ keys and values of leaves and nodes
+// k = cat([x, y]) wk^T, v = cat([x, y]) wv^T in the type of `wk`, `wv` (the parameters in the type that
+// autocast computes in, without their graph).  The rows are converted once into one matrix; the
+// backward adds the two input gradients in fp32 and hands x and y theirs in their own types.
+struct KeyValueRows : public torch::autograd::Function<KeyValueRows> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &y, const Tensor &weight_k,
+                                 const Tensor &weight_v, const Tensor &wk, const Tensor &wv) {
+        const int B = (int)x.size(0), N = (int)x.size(1), M = (int)y.size(1), C = (int)x.size(2);
+        Tensor xy = at::empty({B, N + M, C}, wk.options());
+        c10::DeviceGuard guard(x.device());
+        check(hsa_pack_rows(x.data_ptr(), y.data_ptr(), xy.data_ptr(), B, N, M, C, type_code(x), type_code(y),
+                            type_code(xy), stream_of(x)),
+              "hsa_pack_rows");
+        ctx->set_materialize_grads(false);
+        ctx->save_for_backward({x, y, xy, wk, wv, weight_k, weight_v});
+        return {at::linear(xy, wk), at::linear(xy, wv)};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &y = saved[1], &xy = saved[2], &wk = saved[3], &wv = saved[4];
+        const Tensor *weight[2] = {&saved[5], &saved[6]};
+        const int64_t B = x.size(0), N = x.size(1), M = y.size(1), C = x.size(2);
+        const bool again = at::GradMode::is_enabled();
+        const at::ScalarType type = xy.scalar_type();
+        Tensor dx, dy, dw[2], d[2];
+        const bool need_in = ctx->needs_input_grad(0) || ctx->needs_input_grad(1);
+        const Tensor rows = again ? at::cat({x.to(type), y.to(type)}, 1) : xy.contiguous();
+        for (int i = 0; i < 2; ++i) {
+            const Tensor &g = grads[i];
+            if (!g.defined()) continue;
+            const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = rows.reshape({-1, C});
+            if (need_in) d[i] = at::mm(g2, again ? weight[i]->to(type) : i == 0 ? wk : wv);
+            if (!ctx->needs_input_grad(2 + i)) continue;
+            if (!again)
+                if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), weight[i]->scalar_type(), false)) dw[i] = r->first;
+            if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(weight[i]->scalar_type());
+        }
+        if (need_in && (d[0].defined() || d[1].defined())) {
+            if (!again && d[0].defined() && d[1].defined()) {
+                if (ctx->needs_input_grad(0)) dx = at::empty({B, N, C}, x.options());
+                if (ctx->needs_input_grad(1)) dy = at::empty({B, M, C}, y.options());
+                c10::DeviceGuard guard(x.device());
+                check(hsa_add_split_rows(d[0].data_ptr(), d[1].data_ptr(), dx.defined() ? dx.data_ptr() : nullptr,
+                                         dy.defined() ? dy.data_ptr() : nullptr, (int)B, (int)N, (int)M, (int)C,
+                                         type_code(x), type_code(y), type_code(xy), stream_of(x)),
+                      "hsa_add_split_rows");
+            } else {
+                Tensor t = d[0].defined() && d[1].defined() ? d[0].to(at::kFloat) + d[1].to(at::kFloat)
+                                                            : (d[0].defined() ? d[0] : d[1]);
+                t = t.view({B, N + M, C});
+                dx = t.narrow(1, 0, N).to(x.scalar_type());
+                dy = t.narrow(1, N, M).to(y.scalar_type());
+            }
+        }
+        return {dx, dy, dw[0], dw[1], Tensor(), Tensor()};
+    }
+};
+
+// (keys, values) of the rows of x [B, N, C] and y [B, M, C] under the current autocast state; nullopt where
+// the call is not a plain one in training on 16-bit types
+std::optional<std::pair<Tensor, Tensor>> key_value_rows(const Tensor &x, const Tensor &y, const Tensor &weight_k,
+                                                        const Tensor &weight_v) {
+    if (!at::GradMode::is_enabled() || !x.is_cuda() || x.dim() != 3 || y.dim() != 3 || x.numel() == 0 || y.numel() == 0 ||
+        x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || !same_kind(weight_k, weight_v) ||
+        weight_k.device() != x.device() || weight_k.dim() != 2 || weight_k.sizes() != weight_v.sizes() ||
+        weight_k.size(1) != x.size(2) || !weight_k.is_contiguous() || !weight_v.is_contiguous() ||
+        !weight_k.requires_grad() || !weight_v.requires_grad())
+        return std::nullopt;
+    const int64_t O = weight_k.size(0), C = weight_k.size(1);
+    if (O % 8 || C % 8 || ((O + 127) / 128) * ((C + 127) / 128) > 256 || x.numel() + y.numel() > (int64_t)1 << 40 ||
+        x.size(1) + y.size(1) > (1 << 30) || !ordinary({&x, &y, &weight_k, &weight_v}))
+        return std::nullopt;
+    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    const at::ScalarType type = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
+    if (type != at::kHalf && type != at::kBFloat16) return std::nullopt;
+    for (const Tensor *t : {&x, &y, &weight_k})
+        if (t->scalar_type() != type && !(cast && t->scalar_type() == at::kFloat)) return std::nullopt;
+    const Tensor xc = x.contiguous(), yc = y.contiguous();
+    if (!aligned16(xc) || !aligned16(yc)) return std::nullopt;
+    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA).detach() : t.detach(); };
+    variable_list r = KeyValueRows::apply(xc, yc, weight_k, weight_v, as(weight_k), as(weight_v));
+    return std::make_pair(r[0], r[1]);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_hsa_torch, m) {
@@ -370,4 +454,5 @@ PYBIND11_MODULE(_hsa_torch, m) {
     m.def("add_layer_norm", &add_layer_norm);
     m.def("linear", &linear);
     m.def("weight_grad", &weight_grad);
+    m.def("key_value_rows", &key_value_rows);
 }

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import linear
+from ..ops.linear import key_value_rows, linear
 from ..ops.topology import build_tree_topology
 
 
@@ -369,9 +369,11 @@ class HierarchicalAttention(nn.Module):
                 torch.bmm(yc, wt, out=dst[:, N:])
             k, v = self._heads(k), self._heads(v)
         else:
-            xy = torch.cat([x, y], dim=1)
-            k = self._heads(linear(self.Wk_x, xy))
-            v = self.dropout(self._heads(linear(self.Wv_x, xy)))
+            kv = key_value_rows(self.Wk_x, self.Wv_x, x, y)
+            if kv is None:
+                xy = torch.cat([x, y], dim=1)
+                kv = linear(self.Wk_x, xy), linear(self.Wv_x, xy)
+            k, v = self._heads(kv[0]), self.dropout(self._heads(kv[1]))
         is_causal = mask is not None  # only the presence of a mask is looked at
         t = self._get_lookup_table(N, is_causal, x.device)
         heads = hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"],

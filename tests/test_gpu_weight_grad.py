@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from sparseattention_amd import _lib
-from sparseattention_amd.ops.linear import linear
+from sparseattention_amd.ops.linear import key_value_rows, linear
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -153,3 +153,52 @@ def test_linear_differentiated_twice():
 
     for a, b in zip(second(lambda t: linear(layer, t)), second(layer)):
         assert torch.equal(a, b)
+
+
+# ---------------------------------------------------------------- keys and values of leaves and nodes
+@pytest.mark.parametrize("shape", [(1, 1, 1, 8), (2, 64, 63, 96), (3, 5, 9, 264), (1, 2000, 1999, 64)])
+@pytest.mark.parametrize("types", [(None, torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32, torch.float16),
+                                   (torch.bfloat16, torch.float32, torch.float32), (torch.float16, torch.float16, torch.float32)])
+def test_key_value_rows(shape, types):
+    B, N, M, C = shape
+    amp, xt, yt = types
+    low = amp or xt
+    wt = torch.float32 if amp else low
+    g = torch.Generator().manual_seed(C)
+    mk = lambda *s: torch.randn(*s, generator=g).to(low)
+    x, y, gk, gv = mk(B, N, C).to(xt), mk(B, M, C).to(yt), mk(B, N + M, C), mk(B, N + M, C)
+    lk, lv = (torch.nn.Linear(C, C, bias=False).to(DEV).to(wt) for _ in range(2))
+    xd, yd = x.to(DEV).requires_grad_(True), y.to(DEV).requires_grad_(True)
+    with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+        k, v = key_value_rows(lk, lv, xd, yd)
+        xy = torch.cat([xd.detach().to(low), yd.detach().to(low)], dim=1)
+        assert k.dtype == low and torch.equal(k, lk(xy)) and torch.equal(v, lv(xy))
+    torch.autograd.backward([k, v], [gk.to(DEV), gv.to(DEV)])
+    # what the library's products give, added in fp32 and rounded to the inputs' types
+    d = gk.to(DEV).view(-1, C).mm(lk.weight.detach().to(low)).float() + gv.to(DEV).view(-1, C).mm(lv.weight.detach().to(low)).float()
+    d = d.view(B, N + M, C)
+    assert torch.equal(xd.grad, d[:, :N].to(xt)) and torch.equal(yd.grad, d[:, N:].to(yt))
+    half = 0.0 if amp else {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11}[low]
+    for layer, go in ((lk, gk), (lv, gv)):
+        want = go.double().view(-1, C).t() @ xy.double().cpu().view(-1, C)
+        _close(layer.weight.grad, want, B * (N + M), half, "dw")
+
+
+def test_key_value_rows_partial_use():
+    """Only one result used, only one input needing a gradient, layers with hooks or biases left alone."""
+    lk, lv = (torch.nn.Linear(64, 64, bias=False).to(DEV).to(torch.bfloat16) for _ in range(2))
+    x = torch.randn(2, 8, 64, device=DEV, dtype=torch.bfloat16)
+    y = torch.randn(2, 7, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    k, v = key_value_rows(lk, lv, x, y)
+    v.sum().backward()
+    assert lk.weight.grad is None and lv.weight.grad is not None
+    want = torch.ones_like(v.detach()).matmul(lv.weight.detach())[:, 8:]
+    assert torch.equal(y.grad, want)
+    y.grad = None
+    k, v = key_value_rows(lk, lv, x, y)
+    (k + v).sum().backward()
+    assert y.grad is not None and x.grad is None
+    with torch.no_grad():
+        assert key_value_rows(lk, lv, x, y) is None
+    assert key_value_rows(torch.nn.Linear(64, 64).to(DEV).to(torch.bfloat16), lv, x, y) is None
+    assert key_value_rows(lk, lv, x.float(), y.float()) is None

@@ -8,8 +8,8 @@
 // part in its own type.
 //
 // Bound: HBM; eight elements per thread, every row read and written once.  B8 N2048 C768, x fp32, y fp16:
-// 22 us forward (126 MB, 5.6 TB/s), 29 us backward (176 MB); the copies, conversions and additions they
-// replace took 230 us of a module's training step.
+// 22 us forward (126 MB, 5.6 TB/s), 29 us backward (176 MB); with them the module's
+// training step takes 1805 us instead of 1961.
 #include "hsa_common.h"
 
 namespace hsa {

@@ -468,13 +468,15 @@ int hsa_weight_grad(int nseg, const hsa_weight_grad_segment *seg, int O, int I, 
  * one matrix out [B, N + M, C] of the 16-bit `dtype`: the cat([x, y]) of update_X_from_Y
  * (hierarchical_attention/modules/attention.py:178-195) and its conversion.  C a multiple of 8, all
  * tensors dense and 16-byte aligned.
- * hsa_add_split_rows is its backward for two projections: a + b (both [B, N + M, C] of `dtype`, added
- * in fp32) as dx and dy of their own types; either of the two may be NULL.
+ * out_x [B, N, C], unless NULL, receives x's converted rows once more by themselves.
+ * hsa_add_split_rows is its backward for two projections of the matrix and one of x's rows: a + b (both
+ * [B, N + M, C] of `dtype`) and, on x's rows, c ([B, N, C], or NULL), added in fp32, as dx and dy of
+ * their own types; either of these two may be NULL.
  */
-int hsa_pack_rows(const void *x, const void *y, void *out, int B, int N, int M, int C, int x_dtype,
-                  int y_dtype, int dtype, void *stream);
-int hsa_add_split_rows(const void *a, const void *b, void *dx, void *dy, int B, int N, int M, int C,
-                       int x_dtype, int y_dtype, int dtype, void *stream);
+int hsa_pack_rows(const void *x, const void *y, void *out, void *out_x, int B, int N, int M, int C,
+                  int x_dtype, int y_dtype, int dtype, void *stream);
+int hsa_add_split_rows(const void *a, const void *b, const void *c, void *dx, void *dy, int B, int N,
+                       int M, int C, int x_dtype, int y_dtype, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

@@ -3,13 +3,13 @@
 // HierarchicalAttention.update_X_from_Y (reference hierarchical_attention/modules/attention.py:178-195)
 // projects cat([x, y]) to keys and values.  Under autocast x and y come in fp32 and 16 bits: the
 // concatenation is made in fp32, converted once per projection, and in the backward two fp32 copies of the
-// gradients are added, cut apart and converted again.  Here the rows are converted on the way into
-// one [B, N + M, C] matrix; the backward adds the two projections' input gradients in fp32 and writes each
-// part in its own type.
+// gradients are added, cut apart, converted again and added to the query projection's.  Here the rows are
+// converted on the way into one [B, N + M, C] matrix (x's also by themselves, for the queries); the
+// backward adds the projections' input gradients in fp32 and writes each part in its own type.
 //
 // Bound: HBM; eight elements per thread, every row read and written once.  B8 N2048 C768, x fp32, y fp16:
-// 22 us forward (126 MB, 5.6 TB/s), 29 us backward (176 MB); with them the module's
-// training step takes 1805 us instead of 1961.
+// 22 us forward (126 MB, 5.6 TB/s), 29 us backward (176 MB) without the queries' part; with them the
+// module's training step takes 1744 us instead of 1961.
 #include "hsa_common.h"
 
 namespace hsa {
@@ -46,7 +46,8 @@ template <typename T> __device__ __forceinline__ void rows_store(void *p, long a
 
 struct RowsArgs {
     const void *a, *b;  // pack: x, y; unpack: the two gradients
-    void *o, *o2;       // pack: the matrix; unpack: dx, dy (either may be null)
+    const void *c;      // unpack: a third gradient, of the rows of x alone (or null)
+    void *o, *o2;       // pack: the matrix, x's rows once more by themselves (or null); unpack: dx, dy (either may be null)
     int N, M, C;
     long pieces;        // of the whole matrix
 };
@@ -68,9 +69,11 @@ __global__ void __launch_bounds__(256) pack_rows_kernel(RowsArgs p) {
     for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < p.pieces; i += (long)gridDim.x * 256) {
         long at, part;
         float f[8];
-        if (rows_at(p, i, at, part)) rows_load<X>(p.a, part, f);
+        const bool from_x = rows_at(p, i, at, part);
+        if (from_x) rows_load<X>(p.a, part, f);
         else rows_load<Y>(p.b, part, f);
         rows_store<T>(p.o, at, f);
+        if (from_x && p.o2) rows_store<T>(p.o2, part, f);
     }
 }
 
@@ -85,6 +88,11 @@ __global__ void __launch_bounds__(256) add_split_rows_kernel(RowsArgs p) {
         rows_load<T>(p.b, at, g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) f[e] += g[e];
+        if (from_x && p.c) {
+            rows_load<T>(p.c, part, g);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] += g[e];
+        }
         if (from_x) rows_store<X>(p.o, part, f);
         else rows_store<Y>(p.o2, part, f);
     }
@@ -110,7 +118,7 @@ int rows_checked(RowsArgs &p, bool pack, int B, int N, int M, int C, int x_dtype
     HSA_REQUIRE(dtype == HSA_F16 || dtype == HSA_BF16, "rows of a 16-bit type only (dtype %d)", dtype);
     HSA_REQUIRE((x_dtype == HSA_F32 || x_dtype == dtype) && (y_dtype == HSA_F32 || y_dtype == dtype), "bad part types %d, %d",
                 x_dtype, y_dtype);
-    HSA_REQUIRE((((uintptr_t)p.a | (uintptr_t)p.b | (uintptr_t)p.o | (uintptr_t)p.o2) & 15) == 0, "rows need 16-byte aligned tensors");
+    HSA_REQUIRE((((uintptr_t)p.a | (uintptr_t)p.b | (uintptr_t)p.c | (uintptr_t)p.o | (uintptr_t)p.o2) & 15) == 0, "rows need 16-byte aligned tensors");
     p.N = N; p.M = M; p.C = C;
     p.pieces = (long)B * (N + M) * C / 8;
     return dtype == HSA_F16 ? rows_launch<F16>(p, pack, x_dtype == HSA_F32, y_dtype == HSA_F32, st)
@@ -123,17 +131,17 @@ int rows_checked(RowsArgs &p, bool pack, int B, int N, int M, int C, int x_dtype
 
 extern "C" {
 
-int hsa_pack_rows(const void *x, const void *y, void *out, int B, int N, int M, int C, int x_dtype, int y_dtype,
+int hsa_pack_rows(const void *x, const void *y, void *out, void *out_x, int B, int N, int M, int C, int x_dtype, int y_dtype,
                   int dtype, void *stream) {
     HSA_REQUIRE(x && y && out, "null pointer");
-    hsa::RowsArgs p = {x, y, out, nullptr, 0, 0, 0, 0};
+    hsa::RowsArgs p = {x, y, nullptr, out, out_x, 0, 0, 0, 0};
     return hsa::rows_checked(p, true, B, N, M, C, x_dtype, y_dtype, dtype, (hipStream_t)stream);
 }
 
-int hsa_add_split_rows(const void *a, const void *b, void *dx, void *dy, int B, int N, int M, int C, int x_dtype,
+int hsa_add_split_rows(const void *a, const void *b, const void *c, void *dx, void *dy, int B, int N, int M, int C, int x_dtype,
                        int y_dtype, int dtype, void *stream) {
     HSA_REQUIRE(a && b && (dx || dy), "null pointer");
-    hsa::RowsArgs p = {a, b, dx, dy, 0, 0, 0, 0};
+    hsa::RowsArgs p = {a, b, c, dx, dy, 0, 0, 0, 0};
     return hsa::rows_checked(p, false, B, N, M, C, x_dtype, y_dtype, dtype, (hipStream_t)stream);
 }
 

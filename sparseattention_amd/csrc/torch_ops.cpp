@@ -362,77 +362,86 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     return Linear::apply(as(x), weight, bias, w, b);
 }
 
-// ------------------------------------------------------------------ keys and values of leaves and nodes
-// k = cat([x, y]) wk^T, v = cat([x, y]) wv^T in the type of `wk`, `wv` (the parameters in the type that
-// autocast computes in, without their graph).  The rows are converted once into one matrix; the
-// backward adds the two input gradients in fp32 and hands x and y theirs in their own types.
-struct KeyValueRows : public torch::autograd::Function<KeyValueRows> {
-    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &y, const Tensor &weight_k,
-                                 const Tensor &weight_v, const Tensor &wk, const Tensor &wv) {
+// ------------------------------------------------------- queries, keys and values of leaves and nodes
+// q = x wq^T, k = cat([x, y]) wk^T, v = cat([x, y]) wv^T in the type of `w` (the parameters in the type
+// that autocast computes in, without their graph).  The rows are converted once; the backward adds the
+// three input gradients in fp32 and hands x and y theirs in their own types.
+struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &y, const Tensor &weight_q,
+                                 const Tensor &weight_k, const Tensor &weight_v, const Tensor &wq, const Tensor &wk,
+                                 const Tensor &wv) {
         const int B = (int)x.size(0), N = (int)x.size(1), M = (int)y.size(1), C = (int)x.size(2);
         Tensor xy = at::empty({B, N + M, C}, wk.options());
+        // rows of x by themselves: x itself where it has the type already
+        Tensor xs = x.scalar_type() == xy.scalar_type() ? x : at::empty({B, N, C}, wk.options());
         c10::DeviceGuard guard(x.device());
-        check(hsa_pack_rows(x.data_ptr(), y.data_ptr(), xy.data_ptr(), B, N, M, C, type_code(x), type_code(y),
-                            type_code(xy), stream_of(x)),
+        check(hsa_pack_rows(x.data_ptr(), y.data_ptr(), xy.data_ptr(), xs.is_same(x) ? nullptr : xs.data_ptr(), B, N, M, C,
+                            type_code(x), type_code(y), type_code(xy), stream_of(x)),
               "hsa_pack_rows");
         ctx->set_materialize_grads(false);
-        ctx->save_for_backward({x, y, xy, wk, wv, weight_k, weight_v});
-        return {at::linear(xy, wk), at::linear(xy, wv)};
+        ctx->save_for_backward({x, y, xs, xy, wq, wk, wv, weight_q, weight_k, weight_v});
+        return {at::linear(xs, wq), at::linear(xy, wk), at::linear(xy, wv)};
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &y = saved[1], &xy = saved[2], &wk = saved[3], &wv = saved[4];
-        const Tensor *weight[2] = {&saved[5], &saved[6]};
+        const Tensor &x = saved[0], &y = saved[1], *w = &saved[4], *weight = &saved[7];
         const int64_t B = x.size(0), N = x.size(1), M = y.size(1), C = x.size(2);
+        const at::ScalarType type = saved[3].scalar_type();
+        // a backward that is itself differentiated goes through the inputs and the parameters
         const bool again = at::GradMode::is_enabled();
-        const at::ScalarType type = xy.scalar_type();
-        Tensor dx, dy, dw[2], d[2];
-        const bool need_in = ctx->needs_input_grad(0) || ctx->needs_input_grad(1);
-        const Tensor rows = again ? at::cat({x.to(type), y.to(type)}, 1) : xy.contiguous();
-        for (int i = 0; i < 2; ++i) {
+        const Tensor xs = again ? x.to(type) : saved[2].contiguous();
+        const Tensor xy = again ? at::cat({xs, y.to(type)}, 1) : saved[3].contiguous();
+        const bool need_x = ctx->needs_input_grad(0), need_y = ctx->needs_input_grad(1);
+        Tensor dx, dy, dw[3], d[3];  // d: input gradients of the three projections
+        for (int i = 0; i < 3; ++i) {
             const Tensor &g = grads[i];
             if (!g.defined()) continue;
-            const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = rows.reshape({-1, C});
-            if (need_in) d[i] = at::mm(g2, again ? weight[i]->to(type) : i == 0 ? wk : wv);
+            const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = (i == 0 ? xs : xy).reshape({-1, C});
+            if (i == 0 ? need_x : need_x || need_y) d[i] = at::mm(g2, again ? weight[i].to(type) : w[i]);
             if (!ctx->needs_input_grad(2 + i)) continue;
             if (!again)
-                if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), weight[i]->scalar_type(), false)) dw[i] = r->first;
-            if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(weight[i]->scalar_type());
+                if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), weight[i].scalar_type(), false)) dw[i] = r->first;
+            if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(weight[i].scalar_type());
         }
-        if (need_in && (d[0].defined() || d[1].defined())) {
-            if (!again && d[0].defined() && d[1].defined()) {
-                if (ctx->needs_input_grad(0)) dx = at::empty({B, N, C}, x.options());
-                if (ctx->needs_input_grad(1)) dy = at::empty({B, M, C}, y.options());
-                c10::DeviceGuard guard(x.device());
-                check(hsa_add_split_rows(d[0].data_ptr(), d[1].data_ptr(), dx.defined() ? dx.data_ptr() : nullptr,
-                                         dy.defined() ? dy.data_ptr() : nullptr, (int)B, (int)N, (int)M, (int)C,
-                                         type_code(x), type_code(y), type_code(xy), stream_of(x)),
-                      "hsa_add_split_rows");
-            } else {
-                Tensor t = d[0].defined() && d[1].defined() ? d[0].to(at::kFloat) + d[1].to(at::kFloat)
-                                                            : (d[0].defined() ? d[0] : d[1]);
+        if (!again && d[1].defined() && d[2].defined()) {
+            if (need_x) dx = at::empty({B, N, C}, x.options());
+            if (need_y) dy = at::empty({B, M, C}, y.options());
+            c10::DeviceGuard guard(x.device());
+            check(hsa_add_split_rows(d[1].data_ptr(), d[2].data_ptr(), d[0].defined() ? d[0].data_ptr() : nullptr,
+                                     need_x ? dx.data_ptr() : nullptr, need_y ? dy.data_ptr() : nullptr, (int)B, (int)N,
+                                     (int)M, (int)C, type_code(x), type_code(y), type_code(saved[3]), stream_of(x)),
+                  "hsa_add_split_rows");
+        } else {
+            Tensor t;  // in fp32
+            for (int i = 1; i < 3; ++i)
+                if (d[i].defined()) t = t.defined() ? t + d[i].to(at::kFloat) : d[i].to(at::kFloat);
+            if (t.defined()) {
                 t = t.view({B, N + M, C});
-                dx = t.narrow(1, 0, N).to(x.scalar_type());
+                dx = t.narrow(1, 0, N);
                 dy = t.narrow(1, N, M).to(y.scalar_type());
             }
+            if (d[0].defined()) dx = dx.defined() ? dx + d[0].view({B, N, C}).to(at::kFloat) : d[0].view({B, N, C});
+            if (dx.defined()) dx = dx.to(x.scalar_type());
         }
-        return {dx, dy, dw[0], dw[1], Tensor(), Tensor()};
+        return {dx, dy, dw[0], dw[1], dw[2], Tensor(), Tensor(), Tensor()};
     }
 };
 
-// (keys, values) of the rows of x [B, N, C] and y [B, M, C] under the current autocast state; nullopt where
-// the call is not a plain one in training on 16-bit types
-std::optional<std::pair<Tensor, Tensor>> key_value_rows(const Tensor &x, const Tensor &y, const Tensor &weight_k,
-                                                        const Tensor &weight_v) {
+// (queries of the rows of x [B, N, C]; keys, values of those and of y [B, M, C]) under the current autocast
+// state; nullopt where the call is not a plain one in training on 16-bit types
+std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Tensor &x, const Tensor &y,
+                                                                       const Tensor &weight_q, const Tensor &weight_k,
+                                                                       const Tensor &weight_v) {
     if (!at::GradMode::is_enabled() || !x.is_cuda() || x.dim() != 3 || y.dim() != 3 || x.numel() == 0 || y.numel() == 0 ||
-        x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || !same_kind(weight_k, weight_v) ||
-        weight_k.device() != x.device() || weight_k.dim() != 2 || weight_k.sizes() != weight_v.sizes() ||
-        weight_k.size(1) != x.size(2) || !weight_k.is_contiguous() || !weight_v.is_contiguous() ||
-        !weight_k.requires_grad() || !weight_v.requires_grad())
+        x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || weight_k.device() != x.device() ||
+        weight_k.dim() != 2 || weight_k.size(1) != x.size(2))
         return std::nullopt;
+    for (const Tensor *t : {&weight_q, &weight_k, &weight_v})
+        if (!same_kind(weight_k, *t) || t->sizes() != weight_k.sizes() || !t->is_contiguous() || !t->requires_grad())
+            return std::nullopt;
     const int64_t O = weight_k.size(0), C = weight_k.size(1);
     if (O % 8 || C % 8 || ((O + 127) / 128) * ((C + 127) / 128) > 256 || x.numel() + y.numel() > (int64_t)1 << 40 ||
-        x.size(1) + y.size(1) > (1 << 30) || !ordinary({&x, &y, &weight_k, &weight_v}))
+        x.size(1) + y.size(1) > (1 << 30) || !ordinary({&x, &y, &weight_q, &weight_k, &weight_v}))
         return std::nullopt;
     const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
     const at::ScalarType type = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
@@ -442,8 +451,8 @@ std::optional<std::pair<Tensor, Tensor>> key_value_rows(const Tensor &x, const T
     const Tensor xc = x.contiguous(), yc = y.contiguous();
     if (!aligned16(xc) || !aligned16(yc)) return std::nullopt;
     auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA).detach() : t.detach(); };
-    variable_list r = KeyValueRows::apply(xc, yc, weight_k, weight_v, as(weight_k), as(weight_v));
-    return std::make_pair(r[0], r[1]);
+    variable_list r = QueryKeyValueRows::apply(xc, yc, weight_q, weight_k, weight_v, as(weight_q), as(weight_k), as(weight_v));
+    return std::make_tuple(r[0], r[1], r[2]);
 }
 
 }  // namespace
@@ -454,5 +463,5 @@ PYBIND11_MODULE(_hsa_torch, m) {
     m.def("add_layer_norm", &add_layer_norm);
     m.def("linear", &linear);
     m.def("weight_grad", &weight_grad);
-    m.def("key_value_rows", &key_value_rows);
+    m.def("query_key_value_rows", &query_key_value_rows);
 }

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import key_value_rows, linear
+from ..ops.linear import linear, query_key_value_rows
 from ..ops.topology import build_tree_topology
 
 
@@ -348,8 +348,9 @@ class HierarchicalAttention(nn.Module):
                         mask: Optional[torch.Tensor] = None) -> torch.Tensor:
         B, N, D = x.shape
         assert y is not None, "y (parents) cannot be None during top-down update"
-        q = self._heads(linear(self.Wq_x, x))
         grad = self._needs_autograd((x, y), (self.Wq_x, self.Wk_x, self.Wv_x))
+        qkv = query_key_value_rows(self.Wq_x, self.Wk_x, self.Wv_x, x, y) if grad else None
+        q = self._heads(linear(self.Wq_x, x) if qkv is None else qkv[0])
         if (not grad and not (self.training and self.dropout.p > 0) and y.size(1) == N - 1
                 and B * N * D >= self._DIRECT_PROJECTION_MIN_ELEMENTS):
             # leaves and span nodes are projected straight into their rows of the [B, 2N-1, D]
@@ -369,11 +370,12 @@ class HierarchicalAttention(nn.Module):
                 torch.bmm(yc, wt, out=dst[:, N:])
             k, v = self._heads(k), self._heads(v)
         else:
-            kv = key_value_rows(self.Wk_x, self.Wv_x, x, y)
-            if kv is None:
+            if qkv is None:
                 xy = torch.cat([x, y], dim=1)
-                kv = linear(self.Wk_x, xy), linear(self.Wv_x, xy)
-            k, v = self._heads(kv[0]), self.dropout(self._heads(kv[1]))
+                k, v = linear(self.Wk_x, xy), linear(self.Wv_x, xy)
+            else:
+                k, v = qkv[1:]
+            k, v = self._heads(k), self.dropout(self._heads(v))
         is_causal = mask is not None  # only the presence of a mask is looked at
         t = self._get_lookup_table(N, is_causal, x.device)
         heads = hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"],

@@ -27,11 +27,12 @@ def linear(layer, x: torch.Tensor) -> torch.Tensor:
     return layer(x)
 
 
-def key_value_rows(layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
-    """layer_k and layer_v of cat([x, y], dim=1) in training on 16-bit types (or under autocast to one):
-    the rows are converted and joined in one pass, their gradients added and cut apart in one
-    (csrc/hsa_rows.hip).  None where that does not apply."""
-    if (x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(layer_k) and _plain(layer_v)
-            and layer_k.bias is None and layer_v.bias is None):
-        return _lib.ext().key_value_rows(x, y, layer_k.weight, layer_v.weight)
+def query_key_value_rows(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
+    """(layer_q of x; layer_k, layer_v of cat([x, y], dim=1)) in training on 16-bit types (or under
+    autocast to one): the rows are converted and joined in one pass, their gradients added and cut apart
+    in one (csrc/hsa_rows.hip).  None where that does not apply."""
+    layers = (layer_q, layer_k, layer_v)
+    if (x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and all(_plain(m) and m.bias is None for m in layers)):
+        return _lib.ext().query_key_value_rows(x, y, *(m.weight for m in layers))
     return None

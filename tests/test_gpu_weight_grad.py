@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from sparseattention_amd import _lib
-from sparseattention_amd.ops.linear import key_value_rows, linear
+from sparseattention_amd.ops.linear import linear, query_key_value_rows
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -155,50 +155,71 @@ def test_linear_differentiated_twice():
         assert torch.equal(a, b)
 
 
-# ---------------------------------------------------------------- keys and values of leaves and nodes
+# ------------------------------------------------------- queries, keys and values of leaves and nodes
 @pytest.mark.parametrize("shape", [(1, 1, 1, 8), (2, 64, 63, 96), (3, 5, 9, 264), (1, 2000, 1999, 64)])
 @pytest.mark.parametrize("types", [(None, torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32, torch.float16),
                                    (torch.bfloat16, torch.float32, torch.float32), (torch.float16, torch.float16, torch.float32)])
-def test_key_value_rows(shape, types):
+def test_query_key_value_rows(shape, types):
     B, N, M, C = shape
     amp, xt, yt = types
     low = amp or xt
     wt = torch.float32 if amp else low
     g = torch.Generator().manual_seed(C)
     mk = lambda *s: torch.randn(*s, generator=g).to(low)
-    x, y, gk, gv = mk(B, N, C).to(xt), mk(B, M, C).to(yt), mk(B, N + M, C), mk(B, N + M, C)
-    lk, lv = (torch.nn.Linear(C, C, bias=False).to(DEV).to(wt) for _ in range(2))
+    x, y, gq, gk, gv = mk(B, N, C).to(xt), mk(B, M, C).to(yt), mk(B, N, C), mk(B, N + M, C), mk(B, N + M, C)
+    lq, lk, lv = (torch.nn.Linear(C, C, bias=False).to(DEV).to(wt) for _ in range(3))
     xd, yd = x.to(DEV).requires_grad_(True), y.to(DEV).requires_grad_(True)
     with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
-        k, v = key_value_rows(lk, lv, xd, yd)
-        xy = torch.cat([xd.detach().to(low), yd.detach().to(low)], dim=1)
-        assert k.dtype == low and torch.equal(k, lk(xy)) and torch.equal(v, lv(xy))
-    torch.autograd.backward([k, v], [gk.to(DEV), gv.to(DEV)])
+        q, k, v = query_key_value_rows(lq, lk, lv, xd, yd)
+        xs = xd.detach().to(low)
+        xy = torch.cat([xs, yd.detach().to(low)], dim=1)
+        assert k.dtype == low and torch.equal(q, lq(xs)) and torch.equal(k, lk(xy)) and torch.equal(v, lv(xy))
+    torch.autograd.backward([q, k, v], [gq.to(DEV), gk.to(DEV), gv.to(DEV)])
     # what the library's products give, added in fp32 and rounded to the inputs' types
-    d = gk.to(DEV).view(-1, C).mm(lk.weight.detach().to(low)).float() + gv.to(DEV).view(-1, C).mm(lv.weight.detach().to(low)).float()
-    d = d.view(B, N + M, C)
-    assert torch.equal(xd.grad, d[:, :N].to(xt)) and torch.equal(yd.grad, d[:, N:].to(yt))
+    back = lambda go, layer: go.to(DEV).view(-1, C).mm(layer.weight.detach().to(low)).float().view(B, -1, C)
+    d = back(gk, lk) + back(gv, lv)
+    assert torch.equal(xd.grad, (d[:, :N] + back(gq, lq)).to(xt)) and torch.equal(yd.grad, d[:, N:].to(yt))
     half = 0.0 if amp else {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11}[low]
-    for layer, go in ((lk, gk), (lv, gv)):
-        want = go.double().view(-1, C).t() @ xy.double().cpu().view(-1, C)
+    for layer, go, rows in ((lq, gq, xs), (lk, gk, xy), (lv, gv, xy)):
+        want = go.double().view(-1, C).t() @ rows.double().cpu().reshape(-1, C)
         _close(layer.weight.grad, want, B * (N + M), half, "dw")
 
 
-def test_key_value_rows_partial_use():
-    """Only one result used, only one input needing a gradient, layers with hooks or biases left alone."""
-    lk, lv = (torch.nn.Linear(64, 64, bias=False).to(DEV).to(torch.bfloat16) for _ in range(2))
+def test_query_key_value_rows_partial_use():
+    """Some results unused, only one input needing a gradient, layers with hooks or biases left alone."""
+    lq, lk, lv = (torch.nn.Linear(64, 64, bias=False).to(DEV).to(torch.bfloat16) for _ in range(3))
     x = torch.randn(2, 8, 64, device=DEV, dtype=torch.bfloat16)
     y = torch.randn(2, 7, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True)
-    k, v = key_value_rows(lk, lv, x, y)
+    q, k, v = query_key_value_rows(lq, lk, lv, x, y)
     v.sum().backward()
-    assert lk.weight.grad is None and lv.weight.grad is not None
-    want = torch.ones_like(v.detach()).matmul(lv.weight.detach())[:, 8:]
-    assert torch.equal(y.grad, want)
+    assert lk.weight.grad is None and lq.weight.grad is None and lv.weight.grad is not None
+    assert torch.equal(y.grad, torch.ones_like(v.detach()).matmul(lv.weight.detach())[:, 8:])
     y.grad = None
-    k, v = key_value_rows(lk, lv, x, y)
-    (k + v).sum().backward()
-    assert y.grad is not None and x.grad is None
+    q, k, v = query_key_value_rows(lq, lk, lv, x, y)
+    ((k + v).sum() + q.sum()).backward()
+    assert y.grad is not None and x.grad is None and lq.weight.grad is not None
+    x.requires_grad_(True)
+    query_key_value_rows(lq, lk, lv, x, y)[0].sum().backward()
+    assert torch.equal(x.grad, torch.ones_like(x).matmul(lq.weight.detach()))
     with torch.no_grad():
-        assert key_value_rows(lk, lv, x, y) is None
-    assert key_value_rows(torch.nn.Linear(64, 64).to(DEV).to(torch.bfloat16), lv, x, y) is None
-    assert key_value_rows(lk, lv, x.float(), y.float()) is None
+        assert query_key_value_rows(lq, lk, lv, x, y) is None
+    assert query_key_value_rows(lq, torch.nn.Linear(64, 64).to(DEV).to(torch.bfloat16), lv, x, y) is None
+    assert query_key_value_rows(lq, lk, lv, x.float(), y.float()) is None
+
+
+def test_query_key_value_rows_differentiated_twice():
+    lq, lk, lv = (torch.nn.Linear(32, 32, bias=False).to(DEV).to(torch.bfloat16) for _ in range(3))
+    x, y = (torch.randn(2, n, 32, device=DEV, dtype=torch.bfloat16, requires_grad=True) for n in (8, 7))
+
+    def second(f):
+        q, k, v = f()
+        gx, gw = torch.autograd.grad(q.float().square().sum() + (k * v).float().sum(), [x, lk.weight], create_graph=True)
+        return torch.autograd.grad(gx.float().square().sum() + gw.float().square().sum(), [x, y, lq.weight, lv.weight])
+
+    def plain():
+        xy = torch.cat([x, y], dim=1)
+        return lq(x), lk(xy), lv(xy)
+
+    for a, b in zip(second(lambda: query_key_value_rows(lq, lk, lv, x, y)), second(plain)):
+        # bf16 through two backward passes, summed in other orders: a few units of 2^-8 of the norm
+        assert (a.float() - b.float()).norm() <= 2e-2 * b.float().norm()

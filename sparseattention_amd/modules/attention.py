@@ -50,7 +50,9 @@ class _SpanLevels(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        saved = ctx.saved_tensors  # raises autograd's own error if they were freed or modified
+        # raises autograd's own error if they were freed or modified; saved-tensor hooks may give back
+        # another layout, the kernels read them as dense
+        saved = [t.contiguous() for t in ctx.saved_tensors]
         nl = ctx.levels
         kept = dict(zip(("x", "y_in", "qkv", "blocks", "w_qkv", "w_kv"), saved[:6]))
         kept["kvs"], kept["masks"], kept["scales"] = list(saved[6:6 + nl]), list(saved[6 + nl:6 + nl + ctx.masks]), ctx.scales

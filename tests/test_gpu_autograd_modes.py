@@ -42,3 +42,20 @@ def test_saved_tensors_with_another_layout():
         got = grads()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_span_levels_saved_with_another_layout():
+    """The same for the span-node update, chains of small levels included."""
+    net = sa.HierarchicalAttention(128, 2, dropout=0.0).to(DEV).to(torch.bfloat16)
+    net._TRAINING_CHAIN_ROWS = 64
+    x, y = (torch.randn(2, n, 128, device=DEV, dtype=torch.bfloat16, requires_grad=True) for n in (128, 127))
+
+    def grads():
+        return torch.autograd.grad(net.cross_update_Y(x, y).float().square().sum(), [x, y, net.Wk_y.weight, net.Wq_y.weight])
+
+    want = grads()
+    turn = lambda s: s.transpose(0, -1).contiguous().transpose(0, -1)
+    with torch.autograd.graph.saved_tensors_hooks(turn, lambda s: s):
+        got = grads()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -67,7 +67,8 @@ const char *hsa_last_error(void);
  *   dtype       HSA_F32 / HSA_F16 / HSA_BF16
  *   algo        HSA_ATTN_*.  The MFMA tile kernels take canonical tables (idx == NULL),
  *               16 <= N <= 2^22, R <= 32 (16-bit types: R <= 64), head sizes 32 / 64 / 128 (16-bit types:
- *               also every other multiple of 8 up to 128, R <= 32, without `weights`), and
+ *               also every other multiple of 8 up to 128, R <= 32, without `weights`; those keep the
+ *               softmax weights in fp32, which the other sizes round to the element type), and
  *               write weights only for the 16-bit types; everything else runs on the gather
  *               kernel
  */
@@ -320,7 +321,7 @@ int hsa_span_levels_bwd(const void *dy, const void *qkv, const void *kv, const v
  *   q, dout, dq  [B, N, H, D];  k, v, dk, dv  [B, M, H, D], M >= 2N-1
  *   workspace    device memory of at least hsa_attn_bwd_workspace_bytes(...) bytes, provided by
  *                the caller (scratch only: nothing in it has to survive the call)
- *   algo         HSA_ATTN_AUTO: MFMA tile kernels when eligible (head size 32, 64 or 128, 16-bit types also other multiples of 8 up to 128 with R <= 32; 16-bit:
+ *   algo         HSA_ATTN_AUTO: MFMA tile kernels when eligible (head size 32, 64 or 128, 16-bit types also other multiples of 8 up to 128 with R <= 32 (weights and score gradients in fp32 there); 16-bit:
  *                R <= 64; fp32: R <= 32: a query-stationary pass and a key-stationary pass that
  *                also sums the first pass's fp32 partial rows for the upper tree levels), else the
  *                gather kernels; both are deterministic (no atomics).

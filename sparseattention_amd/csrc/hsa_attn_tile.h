@@ -37,8 +37,12 @@
 // head's last piece again (the same cache line, no extra traffic), the query operand's missing
 // channels are set to zero once they are in operand form (so whatever the other operand holds
 // there contributes nothing), and nothing is stored behind the head.  The traffic is that of the
-// real head size; only the instruction count is that of the layout.  B3 H8 N2048 D96 R16 causal:
-// 451 us on the gather kernel, 19.3 us here; forward and backward 2089 us -> 119 us a call.
+// real head size; only the instruction count is that of the layout.  The weights keep all their fp32
+// bits in the second product (SplitWeights: two or three 16-bit numbers each), as on the gather kernel,
+// where other layouts round them once.  B3 H8 N2048 D96 R16 causal: 451 us on the gather kernel, 16.9 us
+// here in bf16 and 15.7 in fp16 (15.5 with rounded weights; 20.5 with the product on the fp32 matrix
+// instruction).  Error against fp64: the gather kernel's to four digits (with rounded weights 1.2
+// to 1.4 times as large).
 #pragma once
 
 #include "hsa_common.h"
@@ -460,7 +464,10 @@ attn_tile_kernel(TileParams p) {
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
 
         float den = 0.f;
-        u32x2_t P[NKL + 2];
+        // the weights (at most 1): rounded to the element type once; for part heads all their bits
+        // (SplitWeights, fp16: times 2^14, so that small ones keep theirs)
+        constexpr float kUp = PART && std::is_same<T, F16>::value ? 16384.f : 1.f;
+        typename std::conditional<PART, SplitWeights<T>, RoundedWeights<T>>::type P[NKL + 2];
         float ew[WT ? NKL + 2 : 1][4];
 #pragma unroll
         for (int c = 0; c < NKL + 2; ++c) {
@@ -470,12 +477,13 @@ attn_tile_kernel(TileParams p) {
                 e[i] = __builtin_amdgcn_exp2f(sc[c][i] - mx);
                 den += e[i];
                 if constexpr (WT) ew[c][i] = e[i];
+                e[i] *= kUp;
             }
-            P[c] = u32x2_t{M_::pack(e[0], e[1]), M_::pack(e[2], e[3])};
+            P[c].set(e);
         }
         den += __shfl_xor(den, 16, 64);
         den += __shfl_xor(den, 32, 64);
-        const float inv = 1.0f / den;
+        const float inv = 1.0f / (kUp * den);
         // what a backward pass needs to rebuild this query's weights without its whole row:
         // P = exp2(logit * log2(e) / sqrt(D) + bias - lse)
         // (a variant of its own: as a run-time branch it cost the widest variants their last
@@ -533,9 +541,9 @@ attn_tile_kernel(TileParams p) {
                 const int j = 2 * ks + jj;
                 f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int c = 0; c < NKL; ++c) o = M_::k16(Vl[c][j], P[c], o);
-                o = M_::k16(Vt[j], P[NKL], o);
-                o = M_::k16(Vu[j], P[NKL + 1], o);
+                for (int c = 0; c < NKL; ++c) o = P[c].product(Vl[c][j], o);
+                o = P[NKL].product(Vt[j], o);
+                o = P[NKL + 1].product(Vu[j], o);
                 w[2 * jj] = M_::pack(o[0] * inv, o[1] * inv);
                 w[2 * jj + 1] = M_::pack(o[2] * inv, o[3] * inv);
             }

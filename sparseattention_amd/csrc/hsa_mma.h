@@ -61,4 +61,73 @@ template <> struct Mma<F16> {
     static __device__ __forceinline__ uint32_t pack_exact(float a, float b) { return pack(a, b); }
 };
 
+// k16 with the B operand in fp32 (b[i]: row 4g + i of column r): products and sums in fp32, on four
+// v_mfma_f32_16x16x4_f32 whose steps take the same element of every lane's four (any order of the
+// contraction will do).  Eight times the matrix-core cycles of k16.
+template <typename T>
+__device__ __forceinline__ f32x4 k16_f32(u32x2_t a, const float (&b)[4], f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float<T>((uint16_t)(a[i >> 1] >> (16 * (i & 1)))), b[i], c, 0, 0, 0);
+    return c;
+}
+
+// weights as the B operand of k16, rounded to the element type
+template <typename T> struct RoundedWeights {
+    u32x2_t h;
+    __device__ __forceinline__ void set(const float (&b)[4]) { h = u32x2_t{Mma<T>::pack(b[0], b[1]), Mma<T>::pack(b[2], b[3])}; }
+    __device__ __forceinline__ f32x4 product(u32x2_t a, f32x4 c) const { return Mma<T>::k16(a, h, c); }
+};
+
+// in fp32
+template <typename T> struct Fp32Weights {
+    float f[4];
+    __device__ __forceinline__ void set(const float (&b)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = b[i];
+    }
+    __device__ __forceinline__ f32x4 product(u32x2_t a, f32x4 c) const { return k16_f32<T>(a, f, c); }
+};
+
+// The same bits on the 16-bit matrix instructions: b as a sum of 16-bit numbers, each the rounded rest of the ones
+// before it (the rests are exact in fp32).  bf16: three numbers, all 24 bits of b.  fp16: two, an error of at
+// most 2^-23 |b| for 2^-2 <= |b| <= 2^15, of at most 2^-25 below.  The first two go into one 32-deep
+// product against the A operand taken twice; the third takes a 32-deep product as well, because a k16
+// result as the very next k32's accumulator gave wrong sums here: one shape per chain of products.
+template <typename T> struct SplitWeights;
+template <> struct SplitWeights<BF16> {
+    u32x4_t hm, lo;
+    __device__ __forceinline__ void set(const float (&b)[4]) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const uint32_t h = Mma<BF16>::pack(b[2 * p], b[2 * p + 1]);
+            const float r0 = b[2 * p] - __uint_as_float(h << 16), r1 = b[2 * p + 1] - __uint_as_float(h & 0xffff0000u);
+            const uint32_t m = Mma<BF16>::pack(r0, r1);
+            hm[p] = h;
+            hm[2 + p] = m;
+            lo[2 + p] = 0;
+            lo[p] = Mma<BF16>::pack(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
+        }
+    }
+    __device__ __forceinline__ f32x4 product(u32x2_t a, f32x4 c) const {
+        const u32x4_t twice = {a[0], a[1], a[0], a[1]};
+        return Mma<BF16>::k32(twice, hm, Mma<BF16>::k32(twice, lo, c));
+    }
+};
+template <> struct SplitWeights<F16> {
+    u32x4_t hm;
+    __device__ __forceinline__ void set(const float (&b)[4]) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const uint32_t h = Mma<F16>::pack(b[2 * p], b[2 * p + 1]);
+            const f16x2_t f = __builtin_bit_cast(f16x2_t, h);
+            hm[p] = h;
+            hm[2 + p] = Mma<F16>::pack(b[2 * p] - (float)f[0], b[2 * p + 1] - (float)f[1]);
+        }
+    }
+    __device__ __forceinline__ f32x4 product(u32x2_t a, f32x4 c) const {
+        return Mma<F16>::k32(u32x4_t{a[0], a[1], a[0], a[1]}, hm, c);
+    }
+};
+
 }  // namespace hsa

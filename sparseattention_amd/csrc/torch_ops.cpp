@@ -96,13 +96,14 @@ Tensor attention_plain(const Tensor &Q, const Tensor &K, const Tensor &V, bool c
 // log-sum-exp per (query, head) (the reference keeps its Weights tensor,
 // hierarchical_attention/ops/functional.py:116-264).
 struct SpanAttention : public torch::autograd::Function<SpanAttention> {
+    // one_pass: whether the one-pass backward is wanted where it is built for the head size
     static Tensor forward(AutogradContext *ctx, const Tensor &Qi, const Tensor &Ki, const Tensor &Vi, bool causal,
-                          int64_t R) {
+                          int64_t R, bool one_pass) {
         const Tensor Q = Qi.contiguous(), K = Ki.contiguous(), V = Vi.contiguous();
         const Shape s = shape_of(Q, K);
         ctx->saved_data["causal"] = causal;
         ctx->saved_data["R"] = R;
-        if (hsa_attn_bwd_saved_workspace_bytes(s.B, s.N, s.M, s.H, s.D, s.L, (int)R, causal, s.dtype) > 0 &&
+        if (one_pass && hsa_attn_bwd_saved_workspace_bytes(s.B, s.N, s.M, s.H, s.D, s.L, (int)R, causal, s.dtype) > 0 &&
             aligned16(Q) && aligned16(K) && aligned16(V)) {
             Tensor out = at::empty_like(Q);
             Tensor lse = at::empty({s.B, s.N, s.H}, Q.options().dtype(at::kFloat));
@@ -148,19 +149,23 @@ struct SpanAttention : public torch::autograd::Function<SpanAttention> {
                                s.dtype, algo, stream_of(Q)),
                   "hsa_attn_bwd");
         }
-        return {dq, dk, dv, Tensor(), Tensor()};
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
     }
 };
 
-// The tables are known to be build_tree_topology's for N = Q's rows with this causal flag.
-std::optional<Tensor> span_attention(const Tensor &Q, const Tensor &K, const Tensor &V, bool causal, int64_t R) {
+// The tables are known to be build_tree_topology's for N = Q's rows with this causal flag.  part_one_pass:
+// the one-pass backward for head sizes other than 32 / 64 / 128 channels too.
+std::optional<Tensor> span_attention(const Tensor &Q, const Tensor &K, const Tensor &V, bool causal, int64_t R,
+                                     bool part_one_pass) {
     if (!Q.is_cuda() || Q.dim() != 4 || K.dim() != 4 || !same_kind(Q, K) || !same_kind(Q, V) || type_code(Q) < 0 ||
         K.sizes() != V.sizes() || K.size(0) != Q.size(0) || K.size(2) != Q.size(2) || K.size(3) != Q.size(3) ||
         K.size(1) < 2 * Q.size(1) - 1 || Q.numel() == 0 || log2_exact(Q.size(1)) < 0 || R < 0 || R > (1 << 20) ||
         !ordinary({&Q, &K, &V}))
         return std::nullopt;
-    if (at::GradMode::is_enabled() && (Q.requires_grad() || K.requires_grad() || V.requires_grad()))
-        return SpanAttention::apply(Q, K, V, causal, R);
+    if (at::GradMode::is_enabled() && (Q.requires_grad() || K.requires_grad() || V.requires_grad())) {
+        const int64_t D = Q.size(3);
+        return SpanAttention::apply(Q, K, V, causal, R, part_one_pass || D == 32 || D == 64 || D == 128);
+    }
     return attention_plain(Q.contiguous(), K.contiguous(), V.contiguous(), causal, (int)R);
 }
 

@@ -425,17 +425,19 @@ class BuildParentNodesFunc(torch.autograd.Function):
 # with the causal mask).  The one pass moves less (0.76 of the two passes' HBM
 # traffic at B8 H8 N2048 D64) and measured faster on every shape tried (50.8 against 56.4 us there,
 # 29.6 against 34.7 us at B16 H8 N512, 64.0 against 68.9 us at B2 H16 N8192 D32, 53.8 against 58.7 us
-# at B8 H8 N2048 without the causal mask).
-#   None (default): the one pass wherever it is built
-#   True / False:   the same / never
+# at B8 H8 N2048 without the causal mask).  It rounds the weights and the scores' gradients to 16 bits and
+# takes delta from the rounded output.  Head sizes other than 32 / 64 / 128 channels keep all three in fp32 and
+# therefore use the two passes unless it is asked for.
+#   None (default): the one pass wherever it is built for 32, 64 or 128 channels
+#   True / False:   wherever it is built / never
 # Process-wide; read when the forward runs.
 one_pass_backward = None
 
 
 def _use_one_pass(Q, K, window_size, causal) -> bool:
-    if one_pass_backward is False or not saved_state_backward_available(Q, K, window_size, causal):
+    if one_pass_backward is False or (one_pass_backward is None and Q.shape[3] not in (32, 64, 128)):
         return False
-    return True
+    return saved_state_backward_available(Q, K, window_size, causal)
 
 
 class HierarchicalAttentionFunc(torch.autograd.Function):
@@ -507,7 +509,7 @@ def hierarchical_attention(Q, K, V, idx_table, gather_table, mask_table=None, wi
     if one_pass_backward is not False and isinstance(window_size, int):
         canon = _is_canonical(idx_table, mask_table, Q.shape[1])
         if canon is not None:
-            out = _lib.ext().span_attention(Q, K, V, canon, window_size)
+            out = _lib.ext().span_attention(Q, K, V, canon, window_size, one_pass_backward is True)
             if out is not None:
                 return out
     return HierarchicalAttentionFunc.apply(Q, K, V, idx_table, gather_table, mask_table, window_size)

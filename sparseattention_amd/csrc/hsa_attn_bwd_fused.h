@@ -103,7 +103,7 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
     const int half = SPLIT == 2 ? wave : 0;
     if (unit >= p.n_units) return;
     BT bt;
-    bt.init(smem + wave * LDS_SLOTS * BT::BLK_BYTES);
+    bt.init(smem + wave * LDS_SLOTS * BT::BLK_BYTES, threadIdx.x & 63);
     const int r16 = bt.r16, g = bt.g, lrow = bt.lrow, lchk = bt.lchk;
     float *carry = carry_mem + wave * 2 * HD;
     float *delta_lds = delta_mem + wave * TILE_Q;
@@ -393,6 +393,10 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
             bt.put(1, rVh[c]);
             bt.get(0, Kc[c]);
             bt.get(1, Vc[c]);
+            if constexpr (PART) {
+                bt.clear_behind(Kc[c], dw);
+                bt.clear_behind(Vc[c], dw);
+            }
         }
     }
     if constexpr (!CAUSAL) {
@@ -419,6 +423,10 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
             bt.put(1, rVu);
             bt.get(0, Kc[NKL + 1]);
             bt.get(1, Vc[NKL + 1]);
+            if constexpr (PART) {
+                bt.clear_behind(Kc[NKL + 1], dw);
+                bt.clear_behind(Vc[NKL + 1], dw);
+            }
             far_biases(q0);
             // a later run of the strip goes on summing the levels whose nodes it shares with the
             // runs before: slot r16 (level 6 + r16) starts over every 4 << r16 blocks
@@ -445,6 +453,11 @@ attn_bwd_tile_fused_kernel(BwdFusedParams fp) {
         if constexpr (PART) {
             bt.clear_behind(Qf, dw);
             bt.clear_behind(Gf, dw);
+#pragma unroll
+            for (int c = NKL - 1; c <= NKL; ++c) {
+                bt.clear_behind(Kc[c], dw);
+                bt.clear_behind(Vc[c], dw);
+            }
         }
         // the operands are in registers: the area takes the next block's rows, after the last
         // block the neighbour's query blocks (three staged blocks each, in the halves of the area)

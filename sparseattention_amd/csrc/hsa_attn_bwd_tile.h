@@ -72,8 +72,9 @@ constexpr int bwd_query_waves(int D, int nkl, int sb) {
 }
 
 // DC > 0: part heads (hsa_attn_tile.h), DC channels of the layout's D in the contractions.  B3 H8 N2048 D96 R16
-// causal, both passes: 46.6 us in bf16 and 60.5 in fp16 (1640 on the gather kernels; 42.2 with weights and
-// score gradients rounded to 16 bits; the one pass 48.6)
+// causal, both passes: 48.1 us in bf16 and 61.4 in fp16 (1640 on the gather kernels; 42.2 with weights and
+// score gradients rounded to 16 bits; the one pass 49; with rows looked at one by one instead of a second
+// form of the code 53.4 in bf16)
 template <typename T, int D, int DC = 0>
 struct BwdTile {
     using M_ = Mma<T>;
@@ -87,8 +88,8 @@ struct BwdTile {
     unsigned char *lds;
     u32x4_t Pi[2];
 
-    __device__ __forceinline__ void init(unsigned char *wave_lds) {
-        lane = threadIdx.x & 63;
+    __device__ __forceinline__ void init(unsigned char *wave_lds, int lane_) {
+        lane = lane_;
         r16 = lane & 15;
         g = lane >> 4;
         lrow = lane / CPR;
@@ -122,11 +123,38 @@ struct BwdTile {
     // be sure to hold, so those products run on the fp32 matrix instruction.
     using W = typename std::conditional<DC == 0, RoundedWeights<T>,
                                         typename std::conditional<std::is_same<T, BF16>::value, SplitWeights<BF16>, Fp32Weights<T>>::type>::type;
-    // sets the channels behind a part head to zero (query-side operands: Q and dO)
+    // sets the channels behind a part head to zero: of the operands on both sides, since 0 times a repeated
+    // infinity is NaN
     __device__ __forceinline__ void clear_behind(u32x4_t (&x)[KS], int dh) const {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             if (8 * (4 * ks + g) >= dh) x[ks] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    // rows of a block with an infinity or a NaN, one bit each (the same value in every lane)
+    __device__ __forceinline__ uint32_t odd_rows(const u32x4_t (&x)[KS]) const {
+        LargestBits m;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) m.add(x[ks]);
+        const uint64_t lanes = __ballot(!m.template finite<T>());
+        const uint32_t two = (uint32_t)(lanes | (lanes >> 32));
+        return (two | (two >> 16)) & 0xffffu;
+    }
+    // the same rows set to zero in a block in transposed form
+    __device__ __forceinline__ void clear_rows(u32x2_t (&x)[NJ], uint32_t rows) const {
+        const uint32_t mine = rows >> (4 * g);
+        u32x2_t keep;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+            keep[p] = ((mine >> (2 * p)) & 1 ? 0u : 0xffffu) | ((mine >> (2 * p + 1)) & 1 ? 0u : 0xffff0000u);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) x[j] &= keep;
+    }
+    // weight and score gradient of query 4g + i: nothing for a dead slot whatever the operands hold; where the
+    // query's dO row has been cleared, NaN instead of the weight
+    __device__ __forceinline__ void settle(bool dead, uint32_t odd_g, int i, float &weight, float &grad) const {
+        if (dead) weight = grad = 0.f;
+        if ((odd_g >> (4 * g + i)) & 1)
+            if (weight != 0.f) weight = __builtin_nanf("");
     }
     // operand rows -> "lane = channel, regs = rows" form
     __device__ __forceinline__ void transpose(const u32x4_t (&op)[KS], u32x2_t (&dst)[NJ]) const {
@@ -166,31 +194,31 @@ struct BwdTile {
 // as well would cost the second wavefront per SIMD (more than 256 registers at D = 64), and two
 // wavefronts that cover each other's waits are worth more than the prefetch.
 //
+// Part heads do with infinities and NaN what the gather kernels do: they reach the rows that have to do with
+// theirs and no others.  A strip that meets one walks again in a second form of the code, in which dead
+// slots are selected away instead of biased away, the channels behind the head are zero on both sides, and
+// a row with such an element counts as zero in the products that carry it to other rows (a query that
+// attends to it has its NaN through the weights).  The same in the key pass.
+//
 // Partial rows (fp32): level 5 per query block when SB == 1, entry 1 of [2][B][N/16][H][2][D]
 // (dK then dV; entry 0 and, for longer strips, the whole area stay unused); levels >= 6 per
 // strip, [2][B][N/16/SB][H][L-6][D], right behind.
-template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
-__global__ void __launch_bounds__(BWD_WPB * 64)
-__attribute__((amdgpu_waves_per_eu(bwd_query_waves(D, CAUSAL ? NBW + 1 : 2 * NBW + 1, SB))))
-attn_bwd_tile_query_kernel(BwdTileParams p) {
+// Returns whether the strip has met an infinity or a NaN and has to be walked again with ODD.
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC, bool ODD>
+__device__ __forceinline__ bool bwd_query_strip(const BwdTileParams &p, int unit, unsigned char *lds, float *carry) {
     using BT = BwdTile<T, D, DC>;
     constexpr bool PART = DC > 0;
     using M_ = Mma<T>;
     constexpr int KS = BT::KS, NJ = BT::NJ, RPI = BT::RPI, NLD = BT::NLD;
     constexpr int NKL = CAUSAL ? NBW + 1 : 2 * NBW + 1;
     constexpr int NKB = NKL + 2;  // leaf blocks, near tree block, far tree block
-    constexpr int LDS_SLOTS = 4;
-    __shared__ __align__(16) unsigned char smem[BWD_WPB * LDS_SLOTS * BT::BLK_BYTES];
-    // level-5 rows (dK, dV) of an even block, kept until the odd block of the pair adds its own
-    __shared__ __align__(16) float carry_mem[SB > 1 ? BWD_WPB * 2 * D : 4];
-
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int unit = bwd_xcd_remap((int)blockIdx.x, (int)gridDim.x) * BWD_WPB + wave;
-    if (unit >= p.n_units) return;
+    float odd_scores = 0.f;       // part heads: NaN once a score or a product with dO is not finite
+    int lane = threadIdx.x & 63;
+    // the first walk's rows are written before they are again, and none of its values are kept for the second
+    if constexpr (ODD) asm volatile("s_waitcnt vmcnt(0)" : "+v"(lane), "+s"(unit)::"memory");
     BT bt;
-    bt.init(smem + wave * LDS_SLOTS * BT::BLK_BYTES);
+    bt.init(lds, lane);
     const int r16 = bt.r16, g = bt.g, lrow = bt.lrow, lchk = bt.lchk;
-    float *carry = carry_mem + (SB > 1 ? wave * 2 * D : 0);
 
     const int N = p.N, L = p.L, R = p.R, H = p.H;
     const int NB = N / TILE_Q, NS = NB / SB;
@@ -273,6 +301,14 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
 
     // everything the first block needs is requested before anything is consumed
     u32x4_t Kc[NKB][KS], Vc[NKB][KS];
+    uint32_t odd_keys[ODD ? NKB : 1];
+    auto key_rows = [&](int c) {
+        if constexpr (ODD) {
+            bt.clear_behind(Kc[c], dh);
+            bt.clear_behind(Vc[c], dh);
+            odd_keys[c] = bt.odd_rows(Kc[c]);
+        }
+    };
     Stage sg;
     {
         u32x4_t rKu[NLD], rVu[NLD], rKh[NKL][NLD], rVh[NKL][NLD];
@@ -291,12 +327,14 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         bt.put(3, rVu);
         bt.get(2, Kc[NKL + 1]);
         bt.get(3, Vc[NKL + 1]);
+        key_rows(NKL + 1);
 #pragma unroll
         for (int c = 0; c + 1 < NKL; ++c) {
             bt.put(2, rKh[c]);
             bt.put(3, rVh[c]);
             bt.get(2, Kc[c]);
             bt.get(3, Vc[c]);
+            key_rows(c);
         }
     }
     // partial rows of the far block, summed over the strip
@@ -317,16 +355,23 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         bt.put(3, sg.v);
         bt.get(0, Qf);
         bt.get(1, Gf);
+        uint32_t odd_q = 0, odd_g = 0;
         if constexpr (PART) {
             bt.clear_behind(Qf, dh);
             bt.clear_behind(Gf, dh);
         }
+        if constexpr (ODD) {
+            odd_q = bt.odd_rows(Qf);
+            odd_g = bt.odd_rows(Gf);
+        }
         bt.get(2, Kc[NKL - 1]);
         bt.get(3, Vc[NKL - 1]);
+        key_rows(NKL - 1);
         bt.put(2, sg.kt);
         bt.put(3, sg.vt);
         bt.get(2, Kc[NKL]);
         bt.get(3, Vc[NKL]);
+        key_rows(NKL);
 
         // liveness of the near block and of the leaf blocks for this query block
         int t_row[NLD];
@@ -384,11 +429,18 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
                 const float bias = c < NKL ? biasL[c < NKL ? c : 0][i] : (c == NKL ? b1T[i] : b1U[i]);
                 sc[c][i] = fmaf(a[i], p.scale_log2e, bias);
                 dp[c][i] = d[i];
+                if constexpr (PART && !ODD) odd_scores = fmaf(a[i], 0.f, fmaf(d[i], 0.f, odd_scores));
+                if (ODD && bias == NEG_INF) {
+                    sc[c][i] = NEG_INF;
+                    dp[c][i] = 0.f;
+                }
                 mx = fmaxf(mx, sc[c][i]);
             }
         }
+        if constexpr (PART && !ODD) asm volatile("" : "+v"(odd_scores));  // summed here, not when registers are short
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if constexpr (ODD) mx = fmaxf(mx, -3.0e38f);  // every key -inf: weights of zero
         float den = 0.f;
 #pragma unroll
         for (int c = 0; c < NKB; ++c)
@@ -399,6 +451,7 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
             }
         den += __shfl_xor(den, 16, 64);
         den += __shfl_xor(den, 32, 64);
+        if constexpr (ODD) den = fmaxf(den, 1.0e-5f);  // (also where it is NaN)
         const float inv = 1.0f / den;
         float delta = 0.f;
 #pragma unroll
@@ -426,6 +479,8 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
             for (int c = 0; c < NKB; ++c) {
                 u32x2_t KT[NJ];
                 bt.transpose(Kc[c], KT);
+                if constexpr (ODD)
+                    if (odd_keys[c]) bt.clear_rows(KT, odd_keys[c]);
                 float ds[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) ds[i] = sc[c][i] * (dp[c][i] - delta) * p.scale;
@@ -445,6 +500,10 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         u32x2_t QT[NJ], GT[NJ];
         bt.transpose(Qf, QT);
         bt.transpose(Gf, GT);
+        if constexpr (ODD) {
+            if (odd_q) bt.clear_rows(QT, odd_q);
+            if (odd_g) bt.clear_rows(GT, odd_g);
+        }
         float lse4[4], del4[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -466,6 +525,7 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
                 const float bias = t == 0 ? b2T[i] : b2U[i];
                 pp[i] = __builtin_amdgcn_exp2f(fmaf(a[i], p.scale_log2e, bias) - lse4[i]);
                 ds[i] = pp[i] * (d[i] - del4[i]) * p.scale;
+                if (ODD) bt.settle(bias == NEG_INF, odd_g, i, pp[i], ds[i]);
             }
             typename BT::W pk, dk;
             pk.set(pp);
@@ -537,6 +597,7 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
         for (int c = 0; c + 1 < NKL; ++c) {
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) { Kc[c][ks] = Kc[c + 1][ks]; Vc[c][ks] = Vc[c + 1][ks]; }
+            if constexpr (ODD) odd_keys[c] = odd_keys[c + 1];
         }
     }
 
@@ -558,6 +619,26 @@ attn_bwd_tile_query_kernel(BwdTileParams p) {
             }
         }
     }
+    return PART && !ODD && __any(odd_scores != 0.f);
+}
+
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
+__global__ void __launch_bounds__(BWD_WPB * 64)
+__attribute__((amdgpu_waves_per_eu(bwd_query_waves(D, CAUSAL ? NBW + 1 : 2 * NBW + 1, SB))))
+attn_bwd_tile_query_kernel(BwdTileParams p) {
+    constexpr int LDS_SLOTS = 4, BLK_BYTES = BwdTile<T, D, DC>::BLK_BYTES;
+    __shared__ __align__(16) unsigned char smem[BWD_WPB * LDS_SLOTS * BLK_BYTES];
+    // level-5 rows (dK, dV) of an even block, kept until the odd block of the pair adds its own
+    __shared__ __align__(16) float carry_mem[SB > 1 ? BWD_WPB * 2 * D : 4];
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int unit = bwd_xcd_remap((int)blockIdx.x, (int)gridDim.x) * BWD_WPB + wave;
+    if (unit >= p.n_units) return;
+    unsigned char *lds = smem + wave * LDS_SLOTS * BLK_BYTES;
+    float *carry = carry_mem + (SB > 1 ? wave * 2 * D : 0);
+    const bool odd = bwd_query_strip<T, D, NBW, CAUSAL, SB, DC, false>(p, unit, lds, carry);
+    if constexpr (DC > 0)
+        if (odd) bwd_query_strip<T, D, NBW, CAUSAL, SB, DC, true>(p, unit, lds, carry);
 }
 
 template <typename T, int SPLIT = 1>
@@ -571,12 +652,8 @@ __device__ __forceinline__ void bwd_reduce_rows(const float *__restrict__ partia
 // A wavefront walks SB consecutive key blocks; the query blocks whose window reaches a key block
 // (NQB of them) slide along in registers in operand form, so each query / dO row is fetched once
 // per strip instead of once per key block it touches.
-// The last red_wgs workgroups of the grid do not take key blocks: they sum the query pass's
-// partial rows into the upper tree levels' dK / dV rows (independent of the leaf rows this pass
-// writes), which fills the chip while the key blocks' last loads and stores drain.
-template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
-__global__ void __launch_bounds__(BWD_WPB * 64)
-attn_bwd_tile_key_kernel(BwdTileParams p) {
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC, bool ODD>
+__device__ __forceinline__ bool bwd_key_strip(const BwdTileParams &p, int unit, unsigned char *lds) {
     using BT = BwdTile<T, D, DC>;
     constexpr bool PART = DC > 0;
     const int dh = PART ? p.dh : D;
@@ -584,22 +661,11 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
     constexpr int KS = BT::KS, NJ = BT::NJ, RPI = BT::RPI, NLD = BT::NLD;
     constexpr int NQB = CAUSAL ? NBW + 1 : 2 * NBW + 1;  // query blocks that reach a key block
     constexpr int QOFF = CAUSAL ? 0 : -NBW;              // first of them, relative to the key block
-    constexpr int LDS_SLOTS = 4;
-    __shared__ __align__(16) unsigned char smem[BWD_WPB * LDS_SLOTS * BT::BLK_BYTES];
-
-    const int key_wgs = (int)gridDim.x - p.red_wgs;
-    if ((int)blockIdx.x >= key_wgs) {
-        using S = typename T::storage;
-        bwd_reduce_rows<T>(p.partial, reinterpret_cast<S *>(p.dk), reinterpret_cast<S *>(p.dv), p.B, p.N, p.M, p.H, dh,
-                           p.L, p.causal, p.red_first_row, p.red_lg_sb,
-                           (size_t)((int)blockIdx.x - key_wgs) * (BWD_WPB * 64) + threadIdx.x);
-        return;
-    }
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int unit = bwd_xcd_remap((int)blockIdx.x, key_wgs) * BWD_WPB + wave;
-    if (unit >= p.n_units) return;
+    float odd_scores = 0.f;
+    int lane = threadIdx.x & 63;
+    if constexpr (ODD) asm volatile("s_waitcnt vmcnt(0)" : "+v"(lane), "+s"(unit)::"memory");  // as in bwd_query_strip
     BT bt;
-    bt.init(smem + wave * LDS_SLOTS * BT::BLK_BYTES);
+    bt.init(lds, lane);
     const int r16 = bt.r16, g = bt.g, lrow = bt.lrow, lchk = bt.lchk;
 
     const int N = p.N, R = p.R, H = p.H;
@@ -627,6 +693,7 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
         u32x4_t Qf[KS], Gf[KS];
         u32x2_t QT[NJ], GT[NJ];
         float lse4[4], del4[4];
+        uint32_t odd_g;  // rows of dO with an infinity or a NaN
     };
     struct Stage {
         u32x4_t k[NLD], v[NLD], q[NLD], g[NLD];
@@ -657,8 +724,18 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
         }
         bt.transpose(qq.Qf, qq.QT);
         bt.transpose(qq.Gf, qq.GT);
+        if constexpr (ODD) {
+            qq.odd_g = bt.odd_rows(qq.Gf);
+            if (const uint32_t odd_q = bt.odd_rows(qq.Qf)) bt.clear_rows(qq.QT, odd_q);
+            if (qq.odd_g) bt.clear_rows(qq.GT, qq.odd_g);
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { qq.lse4[i] = l4[i]; qq.del4[i] = d4[i]; }
+        for (int i = 0; i < 4; ++i) {
+            qq.lse4[i] = l4[i];
+            qq.del4[i] = d4[i];
+            // (a query of this block may have met an infinity in another strip)
+            if constexpr (PART && !ODD) odd_scores = fmaf(l4[i], 0.f, fmaf(d4[i], 0.f, odd_scores));
+        }
     };
 
     QBlock qblk[NQB];
@@ -694,6 +771,10 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
         bt.put(1, sg.v);
         bt.get(0, Kf);
         bt.get(1, Vf);
+        if constexpr (ODD) {
+            bt.clear_behind(Kf, dh);
+            bt.clear_behind(Vf, dh);
+        }
         absorb(qblk[NQB - 1], sg.q, sg.g, sg.lse4, sg.del4);
         if (it + 1 < SB) request(st[it + 1 < SB ? it + 1 : it], kb + 1);
 
@@ -722,7 +803,10 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
                 const float bias = (!inside || cnt == 0) ? NEG_INF : (cnt == 2 ? 1.0f : 0.0f);
                 pp[i] = __builtin_amdgcn_exp2f(fmaf(a[i], p.scale_log2e, bias) - qq.lse4[i]);
                 ds[i] = pp[i] * (d[i] - qq.del4[i]) * p.scale;
+                if constexpr (PART && !ODD) odd_scores = fmaf(a[i], 0.f, fmaf(d[i], 0.f, odd_scores));
+                if (ODD) bt.settle(bias == NEG_INF, qq.odd_g, i, pp[i], ds[i]);
             }
+            if constexpr (PART && !ODD) asm volatile("" : "+v"(odd_scores));
             typename BT::W pk, dk;
             pk.set(pp);
             dk.set(ds);
@@ -746,6 +830,33 @@ attn_bwd_tile_key_kernel(BwdTileParams p) {
 #pragma unroll
         for (int c = 0; c + 1 < NQB; ++c) qblk[c] = qblk[c + 1];
     }
+    return PART && !ODD && __any(odd_scores != 0.f);
+}
+
+// The last red_wgs workgroups of the grid do not take key blocks: they sum the query pass's
+// partial rows into the upper tree levels' dK / dV rows (independent of the leaf rows this pass
+// writes), which fills the chip while the key blocks' last loads and stores drain.
+template <typename T, int D, int NBW, bool CAUSAL, int SB, int DC = 0>
+__global__ void __launch_bounds__(BWD_WPB * 64)
+attn_bwd_tile_key_kernel(BwdTileParams p) {
+    constexpr int LDS_SLOTS = 4, BLK_BYTES = BwdTile<T, D, DC>::BLK_BYTES;
+    __shared__ __align__(16) unsigned char smem[BWD_WPB * LDS_SLOTS * BLK_BYTES];
+
+    const int key_wgs = (int)gridDim.x - p.red_wgs;
+    if ((int)blockIdx.x >= key_wgs) {
+        using S = typename T::storage;
+        bwd_reduce_rows<T>(p.partial, reinterpret_cast<S *>(p.dk), reinterpret_cast<S *>(p.dv), p.B, p.N, p.M, p.H,
+                           DC > 0 ? p.dh : D, p.L, p.causal, p.red_first_row, p.red_lg_sb,
+                           (size_t)((int)blockIdx.x - key_wgs) * (BWD_WPB * 64) + threadIdx.x);
+        return;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int unit = bwd_xcd_remap((int)blockIdx.x, key_wgs) * BWD_WPB + wave;
+    if (unit >= p.n_units) return;
+    unsigned char *lds = smem + wave * LDS_SLOTS * BLK_BYTES;
+    const bool odd = bwd_key_strip<T, D, NBW, CAUSAL, SB, DC, false>(p, unit, lds);
+    if constexpr (DC > 0)
+        if (odd) bwd_key_strip<T, D, NBW, CAUSAL, SB, DC, true>(p, unit, lds);
 }
 
 // Rows from first_row on (a level the query pass left unfinished, up to anything above row 2N-2):

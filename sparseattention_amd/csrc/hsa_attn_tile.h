@@ -35,16 +35,18 @@
 // are laid out for the next of 32 / 64 / 128 channels, of which DC (a multiple of 32) take part in
 // the contractions and dh exist.  A lane whose 16-byte piece lies behind the head fetches the
 // head's last piece again (the same cache line, no extra traffic), the query operand's missing
-// channels are set to zero once they are in operand form (so whatever the other operand holds
-// there contributes nothing), and nothing is stored behind the head.  The traffic is that of the
+// channels are set to zero once they are in operand form (so finite values of the other operand
+// contribute nothing there), and nothing is stored behind the head.  The traffic is that of the
 // real head size; only the instruction count is that of the layout.  The weights keep all their fp32
 // bits in the second product (SplitWeights: two or three 16-bit numbers each), as on the gather kernel,
-// where other layouts round them once.  B3 H8 N2048 D96 R16 causal: 451 us on the gather kernel, 16.9 us
-// here in bf16 and 15.7 in fp16 (15.5 with rounded weights; 20.5 with the product on the fp32 matrix
-// instruction).  Error against fp64: the gather kernel's to four digits (with rounded weights 1.2
-// to 1.4 times as large).
+// where other layouts round them once.  B3 H8 N2048 D96 R16 causal: 451 us on the gather kernel, 17.3 us
+// here in bf16 and 16.3 in fp16 (15.5 with rounded weights; 20.5 with the product on the fp32 matrix
+// instruction; the look for infinities below is 0.5).  Error against fp64: the gather kernel's to four digits (with rounded weights 1.2
+// to 1.4 times as large).  A strip that meets an infinity or a NaN is computed again row by row
+// (gather_query): the whole blocks' products would hand it to queries that do not attend to its row.
 #pragma once
 
+#include "hsa_attn_gather_query.h"
 #include "hsa_common.h"
 #include "hsa_mma.h"
 
@@ -327,6 +329,7 @@ attn_tile_kernel(TileParams p) {
     // the second fetch hits in L2 instead of going back to memory.
     // Kl[c] / Vl[c] hold leaf block (blk - NBW + c) of the query block being processed; the
     // block that enters per step is the top one walking upwards, the bottom one downwards.
+    bool odd = false;  // part heads: the strip has met an infinity or a NaN
     auto run = [&](auto rev_tag) {
     constexpr bool REV = decltype(rev_tag)::value;
     constexpr int NEWI = REV ? 0 : NKL - 1;
@@ -365,6 +368,10 @@ attn_tile_kernel(TileParams p) {
 #pragma unroll
     for (int i = 0; i < AHEAD && i < SB; ++i) request(st[i], seq(i));
 
+    // part heads: NaN once a score is not finite; the value blocks' largest elements
+    float odd_scores = 0.f;
+    LargestBits values;
+
     u32x4_t Ku[KS];
     u32x2_t Vu[NJ];
     auto far_operands = [&]() {
@@ -373,6 +380,7 @@ attn_tile_kernel(TileParams p) {
         lds_put(1, far_v);
         lds_get(0, Ku);
         lds_get(1, vop);
+        if constexpr (PART) for (int ks = 0; ks < KS; ++ks) values.add(vop[ks]);
         transpose_v(vop, Vu);
     };
     far_operands();
@@ -386,6 +394,7 @@ attn_tile_kernel(TileParams p) {
         lds_put(3, halo_v[c]);
         lds_get(2, Kl[c]);
         lds_get(3, vop);
+        if constexpr (PART) for (int ks = 0; ks < KS; ++ks) values.add(vop[ks]);
         transpose_v(vop, Vl[c]);
     }
 
@@ -427,6 +436,20 @@ attn_tile_kernel(TileParams p) {
         for (int ks = 0; ks < KS; ++ks) {
             accT = M_::k32(Kt[ks], Qf[ks], accT);
             accU = M_::k32(Ku[ks], Qf[ks], accU);
+        }
+        if constexpr (PART) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int c = 0; c < NKL; ++c) odd_scores = fmaf(accL[c][i], 0.f, odd_scores);
+                odd_scores = fmaf(accU[i], 0.f, fmaf(accT[i], 0.f, odd_scores));
+            }
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                values.add(Vn[ks]);
+                values.add(Vtn[ks]);
+            }
+            asm volatile("" : "+v"(odd_scores), "+v"(values.m));
         }
         // new value blocks into "lane = channel, regs = keys" form
         u32x2_t Vt[NJ];
@@ -604,10 +627,26 @@ attn_tile_kernel(TileParams p) {
             else process(st[it], seq(i), st[it], -1, std::false_type{});
         }
     }
+    if constexpr (PART) odd = __any(odd_scores != 0.f || !values.finite<T>());
     };  // run
 
     if (p.alternate && (s & 1)) run(std::true_type{});
     else run(std::false_type{});
+    if constexpr (PART) {
+        if (odd) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this strip's rows are written before they are again
+            using S = typename T::storage;
+            const size_t kv = ((size_t)b * p.M * p.H + h) * dh;
+            const float scale = p.scale_log2e * 0.6931471805599453f;
+#pragma nounroll
+            for (int n = blk0 * TILE_Q; n < (blk0 + TOT) * TILE_Q; ++n) {
+                const size_t at = ((size_t)b * N + n) * p.H + h;
+                gather_query<T, 2>({nullptr, nullptr, N, L, R, CAUSAL}, n, (const S *)p.q + at * dh, (const S *)p.k + kv,
+                                   (const S *)p.v + kv, rs, dh, scale, dh == 16, (S *)p.out + at * dh, nullptr,
+                                   LSE ? p.lse + at : nullptr);
+            }
+        }
+    }
 }
 
 template <typename T, int D>

@@ -21,10 +21,12 @@ typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+
 template <typename T> struct Mma;
 
 template <> struct Mma<BF16> {
-    static constexpr uint16_t kOne = 0x3f80;
+    static constexpr uint16_t kOne = 0x3f80, kInf = 0x7f80;
     static __device__ __forceinline__ f32x4 k32(u32x4_t a, u32x4_t b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                        __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
@@ -45,7 +47,7 @@ template <> struct Mma<BF16> {
 };
 
 template <> struct Mma<F16> {
-    static constexpr uint16_t kOne = 0x3c00;
+    static constexpr uint16_t kOne = 0x3c00, kInf = 0x7c00;
     static __device__ __forceinline__ f32x4 k32(u32x4_t a, u32x4_t b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
                                                       __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
@@ -59,6 +61,16 @@ template <> struct Mma<F16> {
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
     }
     static __device__ __forceinline__ uint32_t pack_exact(float a, float b) { return pack(a, b); }
+};
+
+// The largest magnitude (as bits) among 16-bit values: infinities and NaN are those from Mma<T>::kInf on.
+struct LargestBits {
+    u16x2_t m = {0, 0};
+    __device__ __forceinline__ void add(u32x4_t v) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, v[w] & 0x7fff7fffu));
+    }
+    template <typename T> __device__ __forceinline__ bool finite() const { return m[0] < Mma<T>::kInf && m[1] < Mma<T>::kInf; }
 };
 
 // k16 with the B operand in fp32 (b[i]: row 4g + i of column r): products and sums in fp32, on four

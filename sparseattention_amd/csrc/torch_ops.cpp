@@ -228,7 +228,7 @@ struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
         auto [sum, norm] = add_norm_plain(a, b, gamma, beta, eps, stats);
         ctx->set_materialize_grads(false);
         ctx->saved_data["add"] = b.defined();
-        ctx->save_for_backward({b.defined() ? sum : a, stats, gamma});
+        ctx->save_for_backward({b.defined() ? sum : a, stats, gamma, beta});
         if (b.defined()) return {sum, norm};
         return {norm};
     }
@@ -238,6 +238,19 @@ struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
         if (!grads.back().defined() || (add && !grads[1].defined()))  // the norm was not used
             return {dsum, dsum, Tensor(), Tensor(), Tensor()};
         Tensor dnorm = grads.back().contiguous();
+        // a backward that is itself differentiated: torch's norm backward, which has a derivative
+        if (at::GradMode::is_enabled()) {
+            const variable_list saved = ctx->get_saved_variables();
+            const Tensor &x = saved[0];
+            std::vector<int64_t> row = x.sizes().vec();
+            row.back() = 1;
+            const Tensor st = saved[1].detach().t().contiguous();  // means, then reciprocal deviations
+            auto [dx, dgamma, dbeta] = at::native_layer_norm_backward(dnorm, x, {x.size(-1)}, st[0].view(row),
+                                                                      st[1].view(row), saved[2], saved[3],
+                                                                      {true, true, true});
+            if (dsum.defined()) dx = dx + dsum;
+            return {dx, add ? dx : Tensor(), dgamma, dbeta, Tensor()};
+        }
         auto aligned = [](const Tensor &t) { return !t.defined() || aligned16(t) ? t : t.clone(); };
         variable_list saved = ctx->get_saved_variables();
         for (Tensor &t : saved) t = aligned(t.contiguous());  // (saved-tensor hooks may give back another layout)

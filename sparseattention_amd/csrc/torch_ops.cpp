@@ -11,6 +11,7 @@
 // one type, shapes consistent): the Python layer then goes through its own checks, which raise the
 // errors and handle the rest.
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
@@ -148,6 +149,16 @@ struct SpanAttention : public torch::autograd::Function<SpanAttention> {
                                dv.data_ptr(), ws.data_ptr(), ws.nbytes(), s.B, s.N, s.M, s.H, s.D, s.L, R, causal,
                                s.dtype, algo, stream_of(Q)),
                   "hsa_attn_bwd");
+        }
+        if (at::GradMode::is_enabled()) {
+            // the kernels have no derivative: differentiating these gradients again raises instead of leaving
+            // the attention's terms out
+            variable_list once;
+            for (const Tensor &t : {dq, dk, dv}) once.push_back(t.detach().set_requires_grad(true));
+            const auto error = std::make_shared<torch::autograd::DelayedError>(
+                "the span attention cannot be differentiated twice", (int64_t)once.size());
+            once = (*error)(std::move(once));
+            return {once[0], once[1], once[2], Tensor(), Tensor(), Tensor()};
         }
         return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
     }

@@ -475,6 +475,7 @@ class HierarchicalAttentionFunc(torch.autograd.Function):
         return out
 
     @staticmethod
+    @torch.autograd.function.once_differentiable
     def backward(ctx, grad_output):
         if ctx.canonical is None:
             if len(ctx.saved_tensors) < 5:

@@ -41,3 +41,25 @@ def test_layer_norm_differentiated_twice(add, dtype):
     for x, y in zip(second(ours), second(plain)):
         # bf16: two backward passes of single roundings, in other orders: a few units of 2^-8 of the norm
         assert (x.float() - y.float()).norm() <= (1e-5 if dtype == torch.float32 else 3e-2) * y.float().norm()
+
+
+@pytest.mark.parametrize("one_pass", [None, False])
+def test_attention_differentiated_twice_says_so(one_pass):
+    """The span attention has no second derivative: its first one is there with create_graph, and what needs the
+    second raises instead of leaving its terms out."""
+    B, N, H, D = 1, 64, 2, 32
+    t = sa.build_tree_topology(N, True, device=DEV)
+    q, k, v = (torch.randn(B, n, H, D, device=DEV, dtype=torch.bfloat16, requires_grad=True) for n in (N, 2 * N - 1, 2 * N - 1))
+    w = torch.randn(D, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    old, fn.one_pass_backward = fn.one_pass_backward, one_pass
+    try:
+        run = lambda: (sa.hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 4) * w).sum()
+        want = torch.autograd.grad(run(), [q, k, v, w])
+        got = torch.autograd.grad(run(), [q, k, v, w], create_graph=True)
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
+        # the part of the graph in front of the attention is differentiated as before
+        assert torch.equal(torch.autograd.grad(got[3].sum(), q, retain_graph=True)[0].isfinite().all(), torch.tensor(True, device=DEV))
+        with pytest.raises(RuntimeError, match="differentiat"):
+            torch.autograd.grad(got[0].float().sum(), [k])
+    finally:
+        fn.one_pass_backward = old

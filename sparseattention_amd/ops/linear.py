@@ -8,12 +8,19 @@ from torch.nn.modules import module as _module
 from .. import _lib
 
 
-def _plain(layer) -> bool:
-    """An nn.Linear that nobody hooks into, so that its forward may be bypassed."""
-    return (type(layer) is nn.Linear and "forward" not in layer.__dict__
-            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+def plain_module(module, cls) -> bool:
+    """Whether calling `module` runs nothing but `cls`'s own forward, so that the call may be bypassed: no
+    subclass, no forward set on the instance, no hooks on it or on all modules."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks)
             and not (_module._global_forward_hooks or _module._global_forward_pre_hooks
                      or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+
+
+def _plain(layer) -> bool:
+    """An nn.Linear that may be bypassed."""
+    return plain_module(layer, nn.Linear)
 
 
 def linear(layer, x: torch.Tensor) -> torch.Tensor:

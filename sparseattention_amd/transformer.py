@@ -18,13 +18,13 @@ import torch.nn.functional as F
 from . import _lib
 from .modules import HierarchicalAttention
 from .ops import generate_span_input_Y
-from .ops.linear import linear
+from .ops.linear import linear, plain_module
 
 
 def _plain_norm(m) -> bool:
-    """An nn.LayerNorm over the last dimension with weight and bias that nobody hooks into."""
-    return (type(m) is nn.LayerNorm and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None
-            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+    """An nn.LayerNorm over the last dimension with weight and bias that may be bypassed."""
+    return (plain_module(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None
+            and m.bias is not None)
 
 
 def layer_norm(x, norm):
@@ -112,9 +112,8 @@ class DecoderLayer(nn.Module):
         return x, y, nx, ny
 
     def _may_chain(self) -> bool:
-        """Whether `_chained` may stand in for calling the layer: a plain DecoderLayer without hooks."""
-        return type(self) is DecoderLayer and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
-                                                   or self._backward_pre_hooks)
+        """Whether `_chained` may stand in for calling the layer."""
+        return plain_module(self, DecoderLayer)
 
 
 class TransformerLM(nn.Module):

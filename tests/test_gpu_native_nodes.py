@@ -63,3 +63,47 @@ def test_attention_differentiated_twice_says_so(one_pass):
             torch.autograd.grad(got[0].float().sum(), [k])
     finally:
         fn.one_pass_backward = old
+
+
+# ------------------------------------------------------------------------- replaced and watched modules
+def _small_lm():
+    torch.manual_seed(0)
+    return sa.TransformerLM(50, 64, 2, 128, 2, dropout=0.0, window_size=4, max_len=32).to(DEV).to(torch.bfloat16)
+
+
+def test_a_replaced_forward_runs():
+    """A forward set on the instance (what checkpointing and offloading helpers do) is called, of layers and norms."""
+    net = _small_lm()
+    tok = torch.randint(0, 50, (1, 32), device=DEV)
+    want = net(tok)
+    for module in (net.layers[1], net.layers[0].norm1, net.layers[1].norm2, net.layers[1].norm_y, net.layers[1].feed_forward.fc1):
+        seen, inner = [], module.forward
+
+        def forward(*args, **kwargs):
+            seen.append(1)
+            return inner(*args, **kwargs)
+
+        module.forward = forward
+        got = net(tok)
+        del module.forward
+        assert seen, type(module)
+        # the layer's own code path in place of the chained one: single roundings
+        assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()
+    assert torch.equal(net(tok), want)
+
+
+@pytest.mark.parametrize("register", [torch.nn.modules.module.register_module_forward_hook,
+                                      torch.nn.modules.module.register_module_forward_pre_hook,
+                                      torch.nn.modules.module.register_module_full_backward_hook])
+def test_global_module_hooks_see_every_module(register):
+    net = _small_lm()
+    tok = torch.randint(0, 50, (1, 32), device=DEV)
+    seen = []
+    handle = register(lambda m, *args: seen.append(m))
+    try:
+        net(tok).float().sum().backward()
+    finally:
+        handle.remove()
+    for layer in net.layers:
+        for m in (layer, layer.norm1, layer.norm2, layer.norm_y, layer.feed_forward.fc1):
+            assert any(m is s for s in seen), type(m)

@@ -12,6 +12,7 @@
 // errors and handle the rest.
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
@@ -29,14 +30,15 @@ using at::Tensor;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-int type_code(const Tensor &t) {
-    switch (t.scalar_type()) {
+int type_code(at::ScalarType type) {
+    switch (type) {
         case at::kFloat: return HSA_F32;
         case at::kHalf: return HSA_F16;
         case at::kBFloat16: return HSA_BF16;
         default: return -1;
     }
 }
+int type_code(const Tensor &t) { return type_code(t.scalar_type()); }
 
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
@@ -335,36 +337,44 @@ std::optional<std::pair<Tensor, Tensor>> weight_grad(const Segments &segs, int64
     return std::make_pair(dw, db);
 }
 
+// A tensor that a node keeps for its backward without an edge of its own to it.
+struct Kept {
+    Tensor t;
+};
+
 // y = x w^T + b by the library's product; backward: the input's gradient by the library, the weight's
 // and the bias's by the split-rows kernel, straight into the parameters' type.  `w`, `b` are the
-// parameters in x's type (the casts that autocast makes), without their graph.
+// parameters in x's type (the casts that autocast makes); `w` keeps its graph, which a backward that is itself
+// differentiated goes through.  The parameter is not saved: under autocast it may be written to before the
+// backward.
 struct Linear : public torch::autograd::Function<Linear> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias,
-                          const Tensor &w, const std::optional<Tensor> &b) {
-        ctx->save_for_backward({x, w, weight});
+                          const Kept &w, const std::optional<Tensor> &b) {
+        ctx->save_for_backward({x, w.t});
         ctx->saved_data["bias"] = bias.has_value();
-        return at::linear(x, w, b);
+        ctx->saved_data["type"] = (int64_t)weight.scalar_type();
+        return at::linear(x, w.t, b);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &w = saved[1], &weight = saved[2];
+        const Tensor &x = saved[0], &w = saved[1];
         const bool bias = ctx->saved_data["bias"].toBool();
+        const auto type = (at::ScalarType)ctx->saved_data["type"].toInt();  // the parameters'
         const Tensor &g = grads[0];
         Tensor dx, dw, db;
         if (!g.defined()) return {dx, dw, db, Tensor(), Tensor()};
         const Tensor g2 = g.reshape({-1, g.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
-        // a backward that is itself differentiated goes through the parameter, not its detached cast
         const bool again = at::GradMode::is_enabled();
-        if (ctx->needs_input_grad(0)) dx = at::matmul(g, again ? weight.to(x.scalar_type()) : w);
+        if (ctx->needs_input_grad(0)) dx = at::matmul(g, w);
         const bool need_w = ctx->needs_input_grad(1), need_b = bias && ctx->needs_input_grad(2);
         if (need_w && !again) {
-            if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), weight.scalar_type(), need_b)) {
+            if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), type, need_b)) {
                 dw = r->first;
                 db = r->second;
             }
         }
-        if (need_w && !dw.defined()) dw = at::mm(g2.t(), x2).to(weight.scalar_type());
-        if (need_b && !db.defined()) db = g2.sum(0).to(weight.scalar_type());
+        if (need_w && !dw.defined()) dw = at::mm(g2.t(), x2).to(type);
+        if (need_b && !db.defined()) db = g2.sum(0).to(type);
         return {dx, dw, db, Tensor(), Tensor()};
     }
 };
@@ -386,19 +396,37 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     if (!cast && weight.scalar_type() != type) return std::nullopt;
     if (cast && ((weight.scalar_type() != at::kFloat && weight.scalar_type() != type) || type_code(x) < 0)) return std::nullopt;
     auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t; };
-    const Tensor w = as(weight).detach();
+    const Kept w{as(weight)};
     const std::optional<Tensor> b = bias ? std::optional<Tensor>(as(*bias).detach()) : std::nullopt;
     return Linear::apply(as(x), weight, bias, w, b);
 }
 
 // ------------------------------------------------------- queries, keys and values of leaves and nodes
+// The rows of x and y [B, N / M, C] converted and joined, as a node: what stands between the joined rows and their
+// originals when a backward is itself differentiated.
+struct JoinedRows : public torch::autograd::Node {
+    int64_t N = 0;
+    at::ScalarType x_type = at::kFloat, y_type = at::kFloat;
+    variable_list apply(variable_list &&grads) override {
+        const Tensor &g = grads[0];
+        if (!g.defined()) return {Tensor(), Tensor()};
+        return {g.narrow(1, 0, N).to(x_type), g.narrow(1, N, g.size(1) - N).to(y_type)};
+    }
+};
+// where the gradients of x and y go, kept without their data
+struct RowEdges : public torch::CustomClassHolder {
+    torch::autograd::Edge x, y;
+};
+
 // q = x wq^T, k = cat([x, y]) wk^T, v = cat([x, y]) wv^T in the type of `w` (the parameters in the type
-// that autocast computes in, without their graph).  The rows are converted once; the backward adds the
-// three input gradients in fp32 and hands x and y theirs in their own types.
+// that autocast computes in, with their graph).  The rows are converted once; the backward adds the
+// three input gradients in fp32 and hands x and y theirs in their own types.  Only the converted rows are
+// saved: the originals may be written to or freed.
 struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
     static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &y, const Tensor &weight_q,
-                                 const Tensor &weight_k, const Tensor &weight_v, const Tensor &wq, const Tensor &wk,
-                                 const Tensor &wv) {
+                                 const Tensor &weight_k, const Tensor &weight_v, const Kept &q, const Kept &k,
+                                 const Kept &v) {
+        const Tensor &wq = q.t, &wk = k.t, &wv = v.t;
         const int B = (int)x.size(0), N = (int)x.size(1), M = (int)y.size(1), C = (int)x.size(2);
         Tensor xy = at::empty({B, N + M, C}, wk.options());
         // rows of x by themselves: x itself where it has the type already
@@ -408,37 +436,56 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
                             type_code(x), type_code(y), type_code(xy), stream_of(x)),
               "hsa_pack_rows");
         ctx->set_materialize_grads(false);
-        ctx->save_for_backward({x, y, xs, xy, wq, wk, wv, weight_q, weight_k, weight_v});
+        ctx->save_for_backward({xs, xy, wq, wk, wv});
+        auto edges = c10::make_intrusive<RowEdges>();
+        if (x.requires_grad()) edges->x = torch::autograd::impl::gradient_edge(x);
+        if (y.requires_grad()) edges->y = torch::autograd::impl::gradient_edge(y);
+        ctx->saved_data["edges"] = c10::IValue::make_capsule(std::move(edges));
+        ctx->saved_data["N"] = (int64_t)N;
+        ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)x.scalar_type(), (int64_t)y.scalar_type(), (int64_t)weight_k.scalar_type()};
         return {at::linear(xs, wq), at::linear(xy, wk), at::linear(xy, wv)};
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &y = saved[1], *w = &saved[4], *weight = &saved[7];
-        const int64_t B = x.size(0), N = x.size(1), M = y.size(1), C = x.size(2);
-        const at::ScalarType type = saved[3].scalar_type();
-        // a backward that is itself differentiated goes through the inputs and the parameters
+        const Tensor *w = &saved[2];
+        Tensor xs = saved[0].contiguous(), xy = saved[1].contiguous();
+        const int64_t N = ctx->saved_data["N"].toInt(), B = xy.size(0), M = xy.size(1) - N, C = xy.size(2);
+        const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
+        const auto x_type = (at::ScalarType)types[0], y_type = (at::ScalarType)types[1], w_type = (at::ScalarType)types[2];
+        // a backward that is itself differentiated: the rows' graph leads to x and y
         const bool again = at::GradMode::is_enabled();
-        const Tensor xs = again ? x.to(type) : saved[2].contiguous();
-        const Tensor xy = again ? at::cat({xs, y.to(type)}, 1) : saved[3].contiguous();
+        if (again) {
+            const auto edges = c10::static_intrusive_pointer_cast<RowEdges>(ctx->saved_data["edges"].toCapsule());
+            xy = xy.detach();
+            if (edges->x.is_valid() || edges->y.is_valid()) {
+                auto join = std::shared_ptr<JoinedRows>(new JoinedRows(), torch::autograd::deleteNode);
+                join->N = N;
+                join->x_type = x_type;
+                join->y_type = y_type;
+                join->set_next_edges({edges->x, edges->y});
+                torch::autograd::set_history(xy, join);
+            }
+            xs = xy.narrow(1, 0, N);
+        }
         const bool need_x = ctx->needs_input_grad(0), need_y = ctx->needs_input_grad(1);
         Tensor dx, dy, dw[3], d[3];  // d: input gradients of the three projections
         for (int i = 0; i < 3; ++i) {
             const Tensor &g = grads[i];
             if (!g.defined()) continue;
             const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = (i == 0 ? xs : xy).reshape({-1, C});
-            if (i == 0 ? need_x : need_x || need_y) d[i] = at::mm(g2, again ? weight[i].to(type) : w[i]);
+            if (i == 0 ? need_x : need_x || need_y) d[i] = at::mm(g2, w[i]);
             if (!ctx->needs_input_grad(2 + i)) continue;
             if (!again)
-                if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), weight[i].scalar_type(), false)) dw[i] = r->first;
-            if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(weight[i].scalar_type());
+                if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), w_type, false)) dw[i] = r->first;
+            if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(w_type);
         }
         if (!again && d[1].defined() && d[2].defined()) {
-            if (need_x) dx = at::empty({B, N, C}, x.options());
-            if (need_y) dy = at::empty({B, M, C}, y.options());
-            c10::DeviceGuard guard(x.device());
+            if (need_x) dx = at::empty({B, N, C}, xy.options().dtype(x_type));
+            if (need_y) dy = at::empty({B, M, C}, xy.options().dtype(y_type));
+            c10::DeviceGuard guard(xy.device());
             check(hsa_add_split_rows(d[1].data_ptr(), d[2].data_ptr(), d[0].defined() ? d[0].data_ptr() : nullptr,
                                      need_x ? dx.data_ptr() : nullptr, need_y ? dy.data_ptr() : nullptr, (int)B, (int)N,
-                                     (int)M, (int)C, type_code(x), type_code(y), type_code(saved[3]), stream_of(x)),
+                                     (int)M, (int)C, type_code(x_type), type_code(y_type), type_code(xy), stream_of(xy)),
                   "hsa_add_split_rows");
         } else {
             Tensor t;  // in fp32
@@ -447,10 +494,10 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
             if (t.defined()) {
                 t = t.view({B, N + M, C});
                 dx = t.narrow(1, 0, N);
-                dy = t.narrow(1, N, M).to(y.scalar_type());
+                dy = t.narrow(1, N, M).to(y_type);
             }
             if (d[0].defined()) dx = dx.defined() ? dx + d[0].view({B, N, C}).to(at::kFloat) : d[0].view({B, N, C});
-            if (dx.defined()) dx = dx.to(x.scalar_type());
+            if (dx.defined()) dx = dx.to(x_type);
         }
         return {dx, dy, dw[0], dw[1], dw[2], Tensor(), Tensor(), Tensor()};
     }
@@ -479,7 +526,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Ten
         if (t->scalar_type() != type && !(cast && t->scalar_type() == at::kFloat)) return std::nullopt;
     const Tensor xc = x.contiguous(), yc = y.contiguous();
     if (!aligned16(xc) || !aligned16(yc)) return std::nullopt;
-    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA).detach() : t.detach(); };
+    auto as = [&](const Tensor &t) { return Kept{cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t}; };
     variable_list r = QueryKeyValueRows::apply(xc, yc, weight_q, weight_k, weight_v, as(weight_q), as(weight_k), as(weight_v));
     return std::make_tuple(r[0], r[1], r[2]);
 }

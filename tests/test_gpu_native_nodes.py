@@ -107,3 +107,79 @@ def test_global_module_hooks_see_every_module(register):
     for layer in net.layers:
         for m in (layer, layer.norm1, layer.norm2, layer.norm_y, layer.feed_forward.fc1):
             assert any(m is s for s in seen), type(m)
+
+
+# ------------------------------------------------------------------------- what a backward needs
+@pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16])
+def test_autocast_backward_after_an_update(amp):
+    """Under autocast the backward works from 16-bit copies: the fp32 parameters and activations may be written
+    to in between (an in-place residual sum, an optimizer step between two backwards)."""
+    lq, lk, lv = (torch.nn.Linear(64, 64, bias=False).to(DEV) for _ in range(3))
+    lin = torch.nn.Linear(64, 96).to(DEV)
+    x0, y0 = torch.randn(2, 8, 64, device=DEV), torch.randn(2, 7, 64, device=DEV)
+    params = [lq.weight, lk.weight, lv.weight, lin.weight, lin.bias]
+
+    def run(update):
+        leaves = [x0.clone().requires_grad_(True), y0.clone().requires_grad_(True)]
+        x, y = leaves[0] * 1.0, leaves[1] * 1.0
+        with torch.autocast("cuda", dtype=amp):
+            q, k, v = query_key_value_rows(lq, lk, lv, x, y)
+            z = linear(lin, x)
+        loss = sum((t.float() ** 2).sum() for t in (q, k, v, z))
+        if update:
+            with torch.no_grad():
+                x.add_(1.0)
+                y.add_(1.0)
+                for p in params:
+                    p.add_(1.0)
+        grads = torch.autograd.grad(loss, leaves + params)
+        if update:
+            with torch.no_grad():
+                for p in params:
+                    p.sub_(1.0)
+        return grads
+
+    want = run(False)
+    kept = [p.detach().clone() for p in params]
+    got = run(True)
+    with torch.no_grad():
+        for p, old in zip(params, kept):
+            p.copy_(old)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+def test_autocast_keeps_no_fp32_activations():
+    """The rows' fp32 originals are free once their 16-bit copies are made."""
+    lq, lk, lv = (torch.nn.Linear(64, 64, bias=False).to(DEV) for _ in range(3))
+    leaf = torch.randn(4, 4096, 64, device=DEV, requires_grad=True)
+    y = torch.randn(4, 4095, 64, device=DEV, dtype=torch.float16)
+    x = leaf * 1.0
+    bytes_x = x.numel() * 4
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = query_key_value_rows(lq, lk, lv, x, y)
+    before = torch.cuda.memory_allocated()
+    del x
+    assert before - torch.cuda.memory_allocated() >= bytes_x
+    sum(t.float().sum() for t in out).backward()
+    assert leaf.grad is not None
+
+
+def test_autocast_backward_differentiated_twice():
+    """The saved 16-bit copies lead back to the fp32 activations and parameters."""
+    lq, lk, lv, lin = (torch.nn.Linear(64, 64, bias=False).to(DEV) for _ in range(4))
+    x, y = (torch.randn(2, n, 64, device=DEV, requires_grad=True) for n in (8, 7))
+
+    def second(f):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            q, k, v, z = f()
+        first = torch.autograd.grad(sum((t.float() ** 3).sum() for t in (q, k, v, z)), [x, y, lk.weight], create_graph=True)
+        leaves = [x, y, lq.weight, lk.weight, lv.weight, lin.weight]
+        return torch.autograd.grad(sum((g ** 2).sum() for g in first), leaves, allow_unused=True)
+
+    def plain():
+        xy = torch.cat([x, y], dim=1)
+        return lq(x), lk(xy), lv(xy), lin(x)
+
+    for a, b in zip(second(lambda: (*query_key_value_rows(lq, lk, lv, x, y), linear(lin, x))), second(plain)):
+        # bf16 through two backward passes, summed in other orders: a few units of 2^-8 of the norm
+        assert a.dtype == b.dtype and (a - b).norm() <= 2e-2 * b.norm()

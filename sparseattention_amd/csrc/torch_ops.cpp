@@ -54,13 +54,23 @@ bool same_kind(const Tensor &a, const Tensor &b) {
 // or functional transform, no forward-mode tangent.  Such calls go the general way, which either
 // supports them or says that it does not.
 bool ordinary(std::initializer_list<const Tensor *> ts) {
-    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
-                                           c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize});
+    constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::Batched,
+                                           c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                           c10::DispatchKey::Functionalize});
     if (at::tracer::impl::is_dispatch_enabled() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python))
         return false;
     for (const Tensor *t : ts)
         if (t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
     return true;
+}
+
+// Whether a backward computes with torch's operations instead of the kernels: it is itself differentiated,
+// or a transform watches the gradients (a batch of them under vmap).
+bool composed(const variable_list &grads) {
+    if (at::GradMode::is_enabled()) return true;
+    for (const Tensor &g : grads)
+        if (g.defined() && !ordinary({&g})) return true;
+    return false;
 }
 
 bool aligned16(const Tensor &t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
@@ -251,8 +261,7 @@ struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
         if (!grads.back().defined() || (add && !grads[1].defined()))  // the norm was not used
             return {dsum, dsum, Tensor(), Tensor(), Tensor()};
         Tensor dnorm = grads.back().contiguous();
-        // a backward that is itself differentiated: torch's norm backward, which has a derivative
-        if (at::GradMode::is_enabled()) {
+        if (composed(grads)) {  // torch's norm backward, which has a derivative and a batched form
             const variable_list saved = ctx->get_saved_variables();
             const Tensor &x = saved[0];
             std::vector<int64_t> row = x.sizes().vec();
@@ -364,10 +373,9 @@ struct Linear : public torch::autograd::Function<Linear> {
         Tensor dx, dw, db;
         if (!g.defined()) return {dx, dw, db, Tensor(), Tensor()};
         const Tensor g2 = g.reshape({-1, g.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
-        const bool again = at::GradMode::is_enabled();
         if (ctx->needs_input_grad(0)) dx = at::matmul(g, w);
         const bool need_w = ctx->needs_input_grad(1), need_b = bias && ctx->needs_input_grad(2);
-        if (need_w && !again) {
+        if (need_w && !composed(grads)) {
             if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), type, need_b)) {
                 dw = r->first;
                 db = r->second;
@@ -452,9 +460,8 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
         const int64_t N = ctx->saved_data["N"].toInt(), B = xy.size(0), M = xy.size(1) - N, C = xy.size(2);
         const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
         const auto x_type = (at::ScalarType)types[0], y_type = (at::ScalarType)types[1], w_type = (at::ScalarType)types[2];
-        // a backward that is itself differentiated: the rows' graph leads to x and y
-        const bool again = at::GradMode::is_enabled();
-        if (again) {
+        const bool by_torch = composed(grads);
+        if (at::GradMode::is_enabled()) {  // itself differentiated: the rows' graph leads to x and y
             const auto edges = c10::static_intrusive_pointer_cast<RowEdges>(ctx->saved_data["edges"].toCapsule());
             xy = xy.detach();
             if (edges->x.is_valid() || edges->y.is_valid()) {
@@ -475,11 +482,11 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
             const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = (i == 0 ? xs : xy).reshape({-1, C});
             if (i == 0 ? need_x : need_x || need_y) d[i] = at::mm(g2, w[i]);
             if (!ctx->needs_input_grad(2 + i)) continue;
-            if (!again)
+            if (!by_torch)
                 if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), w_type, false)) dw[i] = r->first;
             if (!dw[i].defined()) dw[i] = at::mm(g2.t(), r2).to(w_type);
         }
-        if (!again && d[1].defined() && d[2].defined()) {
+        if (!by_torch && d[1].defined() && d[2].defined()) {
             if (need_x) dx = at::empty({B, N, C}, xy.options().dtype(x_type));
             if (need_y) dy = at::empty({B, M, C}, xy.options().dtype(y_type));
             c10::DeviceGuard guard(xy.device());
@@ -492,11 +499,11 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
             for (int i = 1; i < 3; ++i)
                 if (d[i].defined()) t = t.defined() ? t + d[i].to(at::kFloat) : d[i].to(at::kFloat);
             if (t.defined()) {
-                t = t.view({B, N + M, C});
+                t = t.reshape({B, N + M, C});
                 dx = t.narrow(1, 0, N);
                 dy = t.narrow(1, N, M).to(y_type);
             }
-            if (d[0].defined()) dx = dx.defined() ? dx + d[0].view({B, N, C}).to(at::kFloat) : d[0].view({B, N, C});
+            if (d[0].defined()) dx = dx.defined() ? dx + d[0].reshape({B, N, C}).to(at::kFloat) : d[0].reshape({B, N, C});
             if (dx.defined()) dx = dx.to(x_type);
         }
         return {dx, dy, dw[0], dw[1], dw[2], Tensor(), Tensor(), Tensor()};

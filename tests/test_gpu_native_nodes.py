@@ -183,3 +183,25 @@ def test_autocast_backward_differentiated_twice():
     for a, b in zip(second(lambda: (*query_key_value_rows(lq, lk, lv, x, y), linear(lin, x))), second(plain)):
         # bf16 through two backward passes, summed in other orders: a few units of 2^-8 of the norm
         assert a.dtype == b.dtype and (a - b).norm() <= 2e-2 * b.norm()
+
+
+# ------------------------------------------------------------------------- batched gradients, wrapped parameters
+def test_batched_gradients():
+    """vmap over the gradients of the outputs (is_grads_batched) through the norm and the linear layers."""
+    B, C, n = 2, 64, 3
+    lq, lk, lv = (torch.nn.Linear(C, C, bias=False).to(DEV).to(torch.bfloat16) for _ in range(3))
+    lin, norm = (m.to(DEV).to(torch.bfloat16) for m in (torch.nn.Linear(C, 96), torch.nn.LayerNorm(C)))
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    x, y, b = (mk(B, m, C).requires_grad_(True) for m in (8, 7, 8))
+    calls = {"linear": (lambda: [linear(lin, x)], [x, lin.weight, lin.bias]),
+             "norm": (lambda: [layer_norm(x, norm)], [x, norm.weight, norm.bias]),
+             "sum and norm": (lambda: list(add_layer_norm(x, b, norm)), [x, b, norm.weight, norm.bias]),
+             "rows": (lambda: list(query_key_value_rows(lq, lk, lv, x, y)), [x, y, lq.weight, lk.weight, lv.weight])}
+    for name, (call, leaves) in calls.items():
+        outs = call()
+        gs = [mk(n, *o.shape) for o in outs]
+        got = torch.autograd.grad(outs, leaves, gs, is_grads_batched=True, retain_graph=True)
+        for i in range(n):
+            for a, w in zip(got, torch.autograd.grad(call(), leaves, [g[i] for g in gs])):
+                # bf16: a few roundings of 2^-9 more or less
+                assert (a[i].float() - w.float()).norm() <= 2e-2 * w.float().norm(), name

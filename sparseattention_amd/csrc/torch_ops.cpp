@@ -294,12 +294,13 @@ struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
 // (a + b, layer_norm(a + b)), or (None, layer_norm(a)) without b; None where the kernel does not take it
 std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const std::optional<Tensor> &b_,
                                                         const Tensor &gamma, const Tensor &beta, double eps) {
+    // (before anything is asked for its data pointer)
+    if (!ordinary({&a_, &gamma, &beta}) || (b_ && !ordinary({&*b_}))) return std::nullopt;
     if (!a_.is_cuda() || a_.numel() == 0 || !same_kind(a_, gamma) || !same_kind(a_, beta) || gamma.dim() != 1 ||
         gamma.size(0) != a_.size(-1) || beta.sizes() != gamma.sizes() || type_code(a_) < 0 ||
         !hsa_add_layer_norm_ok((int)a_.size(-1), type_code(a_)) || (b_ && (!same_kind(a_, *b_) || b_->sizes() != a_.sizes())) ||
         !gamma.is_contiguous() || !beta.is_contiguous() || !aligned16(gamma) || !aligned16(beta))
         return std::nullopt;
-    if (!ordinary({&a_, &gamma, &beta}) || (b_ && !ordinary({&*b_}))) return std::nullopt;
     const Tensor a = a_.contiguous(), b = b_ ? b_->contiguous() : Tensor();
     if (!aligned16(a) || (b.defined() && !aligned16(b))) return std::nullopt;
     if (at::GradMode::is_enabled() && (a.requires_grad() || (b.defined() && b.requires_grad()) || gamma.requires_grad() ||

@@ -205,3 +205,26 @@ def test_batched_gradients():
             for a, w in zip(got, torch.autograd.grad(call(), leaves, [g[i] for g in gs])):
                 # bf16: a few roundings of 2^-9 more or less
                 assert (a[i].float() - w.float()).norm() <= 2e-2 * w.float().norm(), name
+
+
+class _Normed(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.norm = torch.nn.LayerNorm(64)
+
+    def forward(self, x, b):
+        return add_layer_norm(x, b, self.norm)[1] + layer_norm(x, self.norm)
+
+
+def test_norm_with_wrapped_parameters():
+    """A functional transform over the norm's parameters (an ensemble of weights) goes through torch's own norm."""
+    net = _Normed().to(DEV)
+    x, b = torch.randn(5, 64, device=DEV), torch.randn(5, 64, device=DEV)
+    ws, bs = torch.randn(3, 64, device=DEV), torch.randn(3, 64, device=DEV)
+    one = lambda w, c: torch.func.functional_call(net, {"norm.weight": w, "norm.bias": c}, (x, b))
+    got = torch.func.vmap(one)(ws, bs)
+    for i in range(3):
+        assert (got[i] - one(ws[i], bs[i])).abs().max() < 1e-4
+    g = torch.func.grad(lambda w: one(w, bs[0]).square().sum())(ws[0])
+    w = ws[0].clone().requires_grad_(True)
+    assert (g - torch.autograd.grad(one(w, bs[0]).square().sum(), w)[0]).abs().max() < 1e-3

@@ -228,3 +228,17 @@ def test_norm_with_wrapped_parameters():
     g = torch.func.grad(lambda w: one(w, bs[0]).square().sum())(ws[0])
     w = ws[0].clone().requires_grad_(True)
     assert (g - torch.autograd.grad(one(w, bs[0]).square().sum(), w)[0]).abs().max() < 1e-3
+
+
+# ------------------------------------------------------------------------- refusals
+@pytest.mark.parametrize("dtype,grad", [(torch.bfloat16, False), (torch.float32, False), (torch.float32, True)])
+def test_tables_on_the_host_are_refused(dtype, grad):
+    """(The one-pass training forward takes them: it never looked at the tables' place.)"""
+    B, N, H, D = 1, 64, 2, 32
+    q, k, v = (torch.randn(B, n, H, D, device=DEV, dtype=dtype, requires_grad=grad) for n in (N, 2 * N - 1, 2 * N - 1))
+    gpu, cpu = sa.build_tree_topology(N, True, device=DEV), sa.build_tree_topology(N, True, device="cpu")
+    for idx, mask in ((cpu, cpu), (cpu, gpu), (gpu, cpu)):
+        with pytest.raises(_lib.HsaError):
+            sa.hierarchical_attention(q, k, v, idx["forward_idx"], gpu["backward_gather"], mask["forward_mask"], 4)
+    with pytest.raises(_lib.HsaError):
+        sa.hierarchical_attention(q, k, v, cpu["forward_idx"], gpu["backward_gather"], None, 4)

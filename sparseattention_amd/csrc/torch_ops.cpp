@@ -42,8 +42,12 @@ int type_code(const Tensor &t) { return type_code(t.scalar_type()); }
 
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
+// what the library refuses: _lib.HsaError in Python
+struct LibraryError : public std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
 void check(int rc, const char *what) {
-    TORCH_CHECK(rc == HSA_OK, what, " failed (", rc, "): ", hsa_last_error());
+    if (rc != HSA_OK) throw LibraryError(c10::str(what, " failed (", rc, "): ", hsa_last_error()));
 }
 
 bool same_kind(const Tensor &a, const Tensor &b) {
@@ -542,6 +546,13 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Ten
 }  // namespace
 
 PYBIND11_MODULE(_hsa_torch, m) {
+    py::register_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (const LibraryError &e) {
+            PyErr_SetString(py::module_::import("sparseattention_amd._lib").attr("HsaError").ptr(), e.what());
+        }
+    });
     m.def("span_attention", &span_attention);
     m.def("build_tree", &build_tree);
     m.def("add_layer_norm", &add_layer_norm);

@@ -508,7 +508,7 @@ def hierarchical_attention(Q, K, V, idx_table, gather_table, mask_table=None, wi
     `mask_table is None` selects the non-causal mode; `gather_table` is unused by the
     forward pass."""
     # (tables on the host, like other unusual arguments, go on to the checks below)
-    if (one_pass_backward is not False and isinstance(window_size, int) and idx_table.is_cuda
+    if (one_pass_backward is not False and isinstance(window_size, int) and Q.dim() == 4 and idx_table.is_cuda
             and (mask_table is None or mask_table.is_cuda)):
         canon = _is_canonical(idx_table, mask_table, Q.shape[1])
         if canon is not None:

@@ -242,3 +242,16 @@ def test_tables_on_the_host_are_refused(dtype, grad):
             sa.hierarchical_attention(q, k, v, idx["forward_idx"], gpu["backward_gather"], mask["forward_mask"], 4)
     with pytest.raises(_lib.HsaError):
         sa.hierarchical_attention(q, k, v, cpu["forward_idx"], gpu["backward_gather"], None, 4)
+
+
+def test_errors_of_the_library_keep_their_type():
+    """What the library itself refuses is an HsaError on the native route too."""
+    B, N, H, D = 1, 64, 1, 32
+    t = sa.build_tree_topology(N, True, device=DEV)
+    q, k, v = (torch.randn(B, n, H, D, device=DEV, dtype=torch.bfloat16) for n in (N, 2 * N - 1, 2 * N - 1))
+    for grad in (False, True):
+        q.requires_grad_(grad)
+        with pytest.raises(_lib.HsaError, match="slots"):  # 2R+1+L beyond the gather kernel's 256 slots
+            sa.hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 200)
+    with pytest.raises(AssertionError):
+        sa.hierarchical_attention(q.detach()[0, :, 0, 0], k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 4)

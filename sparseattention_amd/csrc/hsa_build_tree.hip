@@ -701,24 +701,36 @@ static int build_tree_fused_typed(const void *qp, const void *kp, const void *vp
     }
 #define HSA_TREE_LAUNCH(THR, GG, HH, PT, GR) \
     build_tree_fused_kernel<T, VEC, TL, THR, GG, HH, PT, GR><<<(unsigned)blocks, THR, 0, st>>>(a)
-    // the common head layouts get their own instantiation at the two larger workgroup sizes
-    const int key = part || groups > 1 ? -1 : lgG * 16 + lgH;
-    const bool heads12 = !part && lgG == 3 && lgH == 2, part8 = part && groups == 1 && lgG == 4 && lgH == 3;
-    if (threads == 512 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(512, 3, 3, false, false);        // 8 heads, 8 lanes per row
-    else if (threads == 512 && key == 4 * 16 + 4) HSA_TREE_LAUNCH(512, 4, 4, false, false);   // 16 heads, 16 lanes per row
-    else if (threads == 512 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(512, 4, 3, false, false);   // 8 heads, 16 lanes per row
-    else if (threads == 512 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(512, 3, 4, false, false);   // 16 heads, 8 lanes per row
-    else if (threads == 512 && heads12) HSA_TREE_LAUNCH(512, 3, 2, false, true);              // 4 or 12 heads, 8 lanes per row
-    else if (threads == 512 && part8) HSA_TREE_LAUNCH(512, 4, 3, true, false);                // 8 heads of 72 .. 120 channels
-    else if (threads == 256 && key == 3 * 16 + 3) HSA_TREE_LAUNCH(256, 3, 3, false, false);
-    else if (threads == 256 && key == 4 * 16 + 3) HSA_TREE_LAUNCH(256, 4, 3, false, false);
-    else if (threads == 256 && key == 3 * 16 + 4) HSA_TREE_LAUNCH(256, 3, 4, false, false);
-    else if (threads == 256 && heads12) HSA_TREE_LAUNCH(256, 3, 2, false, true);
-    else if (threads == 256 && part8) HSA_TREE_LAUNCH(256, 4, 3, true, false);
-    else if (threads == 512) HSA_TREE_LAUNCH(512, -1, -1, true, true);
-    else if (threads == 256) HSA_TREE_LAUNCH(256, -1, -1, true, true);
-    else if (threads == 128) HSA_TREE_LAUNCH(128, -1, -1, true, true);
-    else HSA_TREE_LAUNCH(64, -1, -1, true, true);
+    // Instantiations of the two larger workgroup sizes.  With the lanes per row fixed at compile time (8 or 16: 64
+    // and 128 channels of a 16-bit type, 32 and 64 in fp32) the cross-lane sums become constants, with the head
+    // count as well every slot index.  us, nothing fixed / lanes / both: B5 N1024 H12 D64 17.8 / 15.2 / 15.0, B4
+    // N2048 H4 D64 16.2 / 12.9 / 12.6, B3 N2048 H8 D96 24.9 / 21.6 / 21.0, B4 N1024 H8 D80 17.9 / 15.0 / 14.2; nothing
+    // fixed / lanes: B4 N2048 H6 D64 16.9 / 14.0, B2 N2048 H10 D64 16.3 / 13.3, B2 N2048 H12 D128 25.4 / 21.9, B4
+    // N1024 H6 D48 14.5 / 11.9, fp32 B2 N1024 H12 D64 19.3 / 16.2, B4 N4096 H5 D64 22.8 / 22.7.  So both for 8 and
+    // 16 heads, the lanes alone for every other head count.
+    const int key = groups > 1 ? -1 : lgG * 16 + lgH;
+    const bool wide = threads == 512;
+#define HSA_TREE_BOTH(GG, HH, PT, GR)                      \
+    if (wide) HSA_TREE_LAUNCH(512, GG, HH, PT, GR);        \
+    else HSA_TREE_LAUNCH(256, GG, HH, PT, GR)
+    if (threads < 256) {
+        if (threads == 128) HSA_TREE_LAUNCH(128, -1, -1, true, true);
+        else HSA_TREE_LAUNCH(64, -1, -1, true, true);
+    } else if (part) {
+        if (key == 4 * 16 + 3) { HSA_TREE_BOTH(4, 3, true, false); }            // 8 heads of 72 .. 120 channels
+        else if (lgG == 3) { HSA_TREE_BOTH(3, -1, true, true); }
+        else if (lgG == 4) { HSA_TREE_BOTH(4, -1, true, true); }
+        else { HSA_TREE_BOTH(-1, -1, true, true); }
+    } else {
+        if (key == 3 * 16 + 3) { HSA_TREE_BOTH(3, 3, false, false); }           // 8 heads, 8 lanes per row
+        else if (key == 4 * 16 + 3) { HSA_TREE_BOTH(4, 3, false, false); }      // 8 heads, 16 lanes per row
+        else if (key == 3 * 16 + 4) { HSA_TREE_BOTH(3, 4, false, false); }      // 16 heads, 8 lanes per row
+        else if (wide && key == 4 * 16 + 4) HSA_TREE_LAUNCH(512, 4, 4, false, false);  // 16 heads, 16 lanes per row
+        else if (lgG == 3) { HSA_TREE_BOTH(3, -1, false, true); }
+        else if (lgG == 4) { HSA_TREE_BOTH(4, -1, false, true); }
+        else { HSA_TREE_BOTH(-1, -1, true, true); }
+    }
+#undef HSA_TREE_BOTH
 #undef HSA_TREE_LAUNCH
     return check_launch("build_tree_fused_kernel");
 }

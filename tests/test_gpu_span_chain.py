@@ -53,3 +53,34 @@ def test_span_levels_bwd_refuses():
     assert lib.hsa_span_levels_bwd(*args(48, 2)) == -95 and lib.hsa_span_levels_bwd(*args(64, 0)) == -95
     assert lib.hsa_span_levels_bwd(*args(64, 2, p + 2)) == -22
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [(2, 8, 3, 64), (1, 1, 2, 40), (3, 33, 1, 128)])
+def test_strided_parent_backward(dtype, case):
+    """hsa_build_parents_strided_bwd, and hsa_build_parents_level_bwd without a second gradient, on column
+    slices of fused projections: the bits of the dense entry point, nothing written beside the slices."""
+    import ctypes
+    lib = _lib.lib()
+    B, P, H, D = case
+    Dm = H * D
+    g = torch.Generator(device=DEV).manual_seed(P)
+    mk = lambda rows, cols: torch.randn(B, rows, cols, generator=g, device=DEV).to(dtype)
+    dout, qkv, kv = mk(P, Dm), mk(P, 3 * Dm), mk(2 * P, 2 * Dm)
+    heads = lambda t: t.reshape(B, t.shape[1], H, D).contiguous()
+    parts = [heads(dout)] + [heads(t) for t in qkv.split(Dm, dim=2)] + [heads(t) for t in kv.split(Dm, dim=2)]
+    want = [torch.empty_like(parts[i]) for i in (1, 2, 3, 4, 5)]
+    code, stream = _lib.dtype_code(dout), _lib.stream_of(dout)
+    assert lib.hsa_build_parents_bwd(*(_lib.ptr(t) for t in parts + want), B, P, H, D, code, stream) == 0
+    es = dout.element_size()
+    A = ctypes.c_int64 * 11
+    bs = A(P * Dm, *[3 * P * Dm] * 3, *[4 * P * Dm] * 2, *[3 * P * Dm] * 3, *[4 * P * Dm] * 2)
+    rs = A(Dm, *[3 * Dm] * 3, *[2 * Dm] * 2, *[3 * Dm] * 3, *[2 * Dm] * 2)
+    for name in ("hsa_build_parents_strided_bwd", "hsa_build_parents_level_bwd"):
+        dqkv, dkv = torch.full_like(qkv, 7.0), torch.full_like(kv, 7.0)
+        cols = lambda t, n: [t.data_ptr() + i * Dm * es for i in range(n)]
+        first = [dout.data_ptr()] + ([None] if "level" in name else [])
+        assert getattr(lib, name)(*first, *cols(qkv, 3), *cols(kv, 2), *cols(dqkv, 3), *cols(dkv, 2), B, P, H, D, bs, rs,
+                                  code, stream) == 0
+        got = [heads(t) for t in dqkv.split(Dm, dim=2)] + [heads(t) for t in dkv.split(Dm, dim=2)]
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), name

@@ -804,11 +804,11 @@ static int bwd_fused_launch_sb(const BwdFusedParams &q, int sb, hipStream_t st) 
 // coarser.  A round takes at least what one wavefront needs for its strip, and a full one what the
 // memory system needs for all of them; the rule takes the least of max(rounds x the former, wavefronts /
 // 1024 x the latter), both measured (us, bf16).  Measured for strips of 4 / 8 / 16 / 32: B6 N2048 H7 D64
-// 43.3 / 38.7 / 63 / 116, B12 N1024 H8 D64 43.9 / 39.7 / 64 / 116, B2 N8192 H10 D64 67.1 / 71.0 / 67.0 /
-// 117, B3 N2048 H8 D96 52.1 / 49.1 / 73.8 / 139, B3 N4096 H6 D128 71.8 / 78.7 / 80.7 / 133, B8 N2048 H8 D64
-// 51.0 / 44.7 / 65 / 116, B16 N512 H8 D64 27.1 / 37.6; strips of 8 / 16 / 32: B8 H8 N4096 D64 93 / 88 / 119,
+// 43.4 / 38.7 / 63 / 116, B12 N1024 H8 D64 44.6 / 40.3 / 64 / 116, B2 N8192 H10 D64 67.4 / 70.9 / 66.1 /
+// 116, B3 N4096 H6 D128 70.5 / 78.5 / 79.1 / 132, B8 N2048 H8 D64 49.0 / 44.3 / 65 / 117, B16 N512 H8 D64
+// 27.1 / 37.3; strips of 8 / 16 / 32: B8 H8 N4096 D64 93 / 88 / 119,
 // B8 H8 N8192 D64 180 / 173 / 166, B1 H16 N65536 D64 348 / 327 / 317, B1 H16 N65536 D128 R32 734 / 679 / 657.
-// With 32 channels strips of four win throughout (B2 N4096 H9 22.7 / 26.2 / 42).
+// With 32 channels strips of four win throughout (B2 N4096 H9 22.9 / 26.4 / 42).
 inline int bwd_fused_strip(long waves1, int NB, int D) {
     const int knob = bwd_fused_strip_knob();
     const double alone[2][4] = {{22.5, 37, 63, 114}, {25, 44, 77, 132}};  // up to 64 channels, above

@@ -79,9 +79,9 @@ bool attn_tile_eligible(int N, int M, int H, int D, int L, int R, int dtype, boo
 // us).
 //
 // Against the longest strip that filled every wavefront slot (us, bf16, causal unless noted): B5 N1024
-// H12 D64 16.2 -> 10.3, not causal 18.5 -> 10.8; B12 N512 H8 D64 11.7 -> 9.1; B4 N2048 H6 D64 11.7 ->
-// 9.2; B3 N2048 H12 D64 15.6 -> 13.0; B12 N1024 H8 D64 18.4 -> 15.7, B6 N2048 H8 not causal 20.3 -> 16.1;
-// B2 N8192 H10 D64 25.2 -> 22.7; B3 N4096 H6 D128 26.1 -> 23.0; B3 N2048 H8 D96 18.4 -> 15.3.  B8 N2048
+// H12 D64 16.0 -> 10.5, not causal 18.1 -> 10.7; B12 N512 H8 D64 11.7 -> 9.1; B4 N2048 H6 D64 11.5 ->
+// 9.2; B3 N2048 H12 D64 15.6 -> 13.1; B12 N1024 H8 D64 17.9 -> 15.3, B6 N2048 H8 not causal 20.1 -> 16.4;
+// B2 N8192 H10 D64 24.9 -> 22.7; B3 N4096 H6 D128 26.1 -> 22.9; B3 N2048 H8 D96 19.8 -> 17.0.  B8 N2048
 // H8 D64 (strips of four), B16 N512 H8 D64 (two) and the long sequences (eight) stay as they were.
 //
 // Wavefronts per workgroup: all the variant allows, or a divisor of the head count at least half as

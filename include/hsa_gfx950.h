@@ -479,6 +479,28 @@ int hsa_pack_rows(const void *x, const void *y, void *out, void *out_x, int B, i
 int hsa_add_split_rows(const void *a, const void *b, const void *c, void *dx, void *dy, int B, int N,
                        int M, int C, int x_dtype, int y_dtype, int dtype, void *stream);
 
+/*
+ * Linear projections of one contraction length K, all in one launch: for every segment and batch element
+ *   out[r, n] = sum over k of x[r, k] * w[n, k] + bias[n]     (nn.Linear), or, with w_rows_contract,
+ *   out[r, n] = sum over k of x[r, k] * w[k, n] + bias[n]     (its input gradient),
+ * `dtype` HSA_F16 or HSA_BF16 throughout, fp32 sums, one rounding.  ld_*: elements between rows; batch_*: elements
+ * between the batch elements' first rows; bias [cols] or NULL.  The results may not overlap the operands.
+ * tile: 0, 1, 2 for tiles of 256 x 256, 256 x 192, 128 x 128 (results at least that large, K a multiple of
+ * 64 from 128 on, cols a multiple of 8); 3 for few rows (any number of rows, K a multiple of 32, cols of 4,
+ * not with w_rows_contract); 4 as 0 for results whose rows and columns are of any number and begin at any element
+ * (not with w_rows_contract).  Strides multiples of 8, addresses 16-byte aligned (bias: 2-byte).
+ * hsa_linear_tile: the tile to take, or -1 where the sizes are not handled or a library's product is as fast.
+ */
+#define HSA_LINEAR_MAX_SEGMENTS 5
+typedef struct {
+    const void *x, *w, *bias;
+    void *out;
+    int64_t ld_x, ld_w, ld_out, batch_x, batch_out;
+    int batches, rows, cols;
+} hsa_linear_segment;
+int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int dtype);
+int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,639 @@
+// Linear projections: out[r, n] = sum over k of X[r, k] * W[n, k] (+ bias[n]), and with the weight read the other
+// way round, sum over k of X[r, k] * W[k, n] (the input gradient of a projection).  16-bit operands, fp32 sums.
+// Several projections of one contraction length (the queries, keys and values of leaves and nodes) go into one
+// launch, each with row blocks that lie apart in memory on either side (the leaves' and the nodes' rows of
+// the joined key buffer).
+//
+// Why not the library's product: the contraction is short (256 to 1024), so a tile is 8 steps of 64 and then 128 KB
+// of results; the library starts a workgroup per tile, which pays for its first rows and its last stores each
+// time.  Here a workgroup stays on its CU and walks tiles: the rows of the next tile's first two steps are
+// requested before the results of the last one are stored.
+//
+// Tile 256 x 256 (or 256 x 192 where that leaves fewer CUs idle in the last round), eight wavefronts of 64 rows by
+// 128 (96) columns.  Two stages of 64 contraction steps, both operands straight into LDS; a row's 16-byte pieces are
+// permuted by its number, on the global side of the transfer, so that operand reads meet no bank twice.  Each step is
+// two halves of 32: while one is multiplied, the operands of the next are read (the X side into a second set
+// of registers, the W side in place, a fragment after its last use).  The last tiles of a row or column
+// range lie flush with its end and compute what they share with their neighbour twice, to the same bits:
+// no partial tiles.  The products are taken as (columns of the result) x (rows), so that a lane holds four
+// consecutive columns; two exchanges between lanes make 128-byte lines of eight rows out of them
+// (16 x 64 bytes: 1930 us at 32768 x 50304 x 512, lines 1890, lines stored past the caches 1550).
+//
+// Results whose rows begin at any element (a vocabulary of odd size): a line that two tiles share costs more
+// than the line.  With rows enough, a tile takes every 64th row: their results lie alike in their lines, so the
+// tiles' columns can begin where the lines do (32768 x 50257 x 512: 1865 us; the library 2200).  Else the rows go
+// through the LDS and are stored as 16-byte pieces where they lie (4096 x 50257 x 512: 283 us; 330 as they come,
+// the library 349).
+//
+// Bound: the matrix cores (1.4 PFLOP/s in the steps) and, not overlapped with them, the stores of the results
+// at the rate of the memory (32768 x 2048 x 512: 66 us, 50 without stores).  Slower: two workgroups of 128 x 256 on
+// a CU, whose stores would overlap (82 us); four wavefronts for the transfers alone, so that none waits for
+// its stores (72); starts spread over a tile's time (66).
+#include "hsa_lds_dma.h"
+
+#include <cmath>
+#include <type_traits>
+
+namespace hsa {
+
+namespace {
+
+constexpr int LN_STEP = 64;
+
+struct LnSeg {
+    const char *x, *w;
+    const uint16_t *bias;
+    char *out;
+    long ld_x, ld_w, ld_out, batch_x, batch_out;  // bytes
+    int rows, cols;                                // per batch element
+    int row_tiles, col_tiles;                      // row_tiles: per batch element
+    int all_row_tiles, first;                      // over the batch; first tile
+    int period;                                    // ANY: tiles hold every period-th row, whose results lie alike in lines
+};
+struct LnArgs {
+    LnSeg seg[HSA_LINEAR_MAX_SEGMENTS];
+    int nseg, K, tiles, group;
+};
+
+// Q transfers of 1 KiB, the rows of each `step` bytes behind those of the one before, to consecutive LDS addresses
+template <int Q>
+__device__ __forceinline__ void lds_dma16_rows(const char *base, long step, const uint32_t (&off)[Q], uint32_t lds) {
+    static_assert(Q == 3 || Q == 4);
+    uint32_t keep;
+    const char *b1 = base + step, *b2 = b1 + step, *b3 = b2 + step;
+    if constexpr (Q == 4)
+        asm volatile(
+            "s_mov_b32 %0, m0\n\t"
+            "s_mov_b32 m0, %9\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %1, %5\n\t"
+            "s_add_u32 m0, m0, 0x400\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %2, %6\n\t"
+            "s_add_u32 m0, m0, 0x400\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %3, %7\n\t"
+            "s_add_u32 m0, m0, 0x400\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %4, %8\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(keep)
+            : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(b1), "s"(b2), "s"(b3), "s"(lds)
+            : "memory", "scc");
+    else
+        asm volatile(
+            "s_mov_b32 %0, m0\n\t"
+            "s_mov_b32 m0, %7\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %1, %4\n\t"
+            "s_add_u32 m0, m0, 0x400\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %2, %5\n\t"
+            "s_add_u32 m0, m0, 0x400\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %3, %6\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(keep)
+            : "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(base), "s"(b1), "s"(b2), "s"(lds)
+            : "memory", "scc");
+}
+
+// lane l's 2 bytes, as the low half of LDS[lds_base + 4 l]
+__device__ __forceinline__ void lds_dma2(const void *g, uint32_t lds_base) {
+    uint32_t keep;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_ushort %1, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(g), "s"(lds_base)
+        : "memory");
+}
+
+__device__ const uint16_t ln_no_bias[256] = {};
+
+typedef u32x4_t LnLoosePiece __attribute__((aligned(2)));
+
+typedef short ln_s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2_t ln_read_tr(const char *p) {
+    return __builtin_bit_cast(
+        u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ln_s16x4 *)p));
+}
+
+// BM, BN: rows and columns of a tile; TW: W is [K, N] instead of [N, K]; PAST: results stored past the caches;
+// ANY: rows of the result begin at any element (2: tiles of rows that lie alike in lines)
+template <typename T, int BM, int BN, bool TW, bool PAST, int ANY = 0>
+__global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
+    constexpr int XB = BM * LN_STEP * 2, STAGE = XB + BN * LN_STEP * 2;  // bytes of a stage
+    constexpr int NJ = BN / 32, NP = NJ / 2, QW = BN * 4 / BM;
+    constexpr int PITCH = 2 * BN;  // of a row of W in the LDS, TW
+    __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
+    __shared__ __attribute__((aligned(16))) uint32_t lds_bias[2][BN];
+    constexpr int OUT_PITCH = BN + 16;  // bytes: a wavefront's columns of a row, and 16 so that rows lie in other banks
+    __shared__ __attribute__((aligned(16))) char lds_out[ANY == 1 ? BM / 32 * 8 * OUT_PITCH : 16];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, r = lane & 15, wm = w >> 1, wn = w & 1;
+    const uint32_t lds0 = lds_address(lds);
+    // consecutive tiles on one XCD: they share rows of X and W in its L2
+    const int per = p.tiles >> 3, rest = p.tiles & 7, xcd = blockIdx.x & 7;
+    const int first = xcd * per + (xcd < rest ? xcd : rest), count = per + (xcd < rest);
+    const int slots = gridDim.x >> 3, slot = blockIdx.x >> 3;
+    if (slot >= count) return;
+    struct Tile {
+        int seg, b, m0, n0;
+    };
+    auto tile_of = [&](int t) {  // `group` row tiles, column by column, then the next
+        Tile c;
+        t += first;
+        c.seg = 0;
+        while (c.seg + 1 < p.nseg && t >= p.seg[c.seg + 1].first) ++c.seg;
+        const LnSeg &s = p.seg[c.seg];
+        t -= s.first;
+        const int per_group = p.group * s.col_tiles, grp = t / per_group, in = t - grp * per_group;
+        const int left = s.all_row_tiles - grp * p.group, rows = left < p.group ? left : p.group;
+        const int ct = in / rows, rt = grp * p.group + in - ct * rows;
+        c.b = rt / s.row_tiles;
+        c.m0 = (rt - c.b * s.row_tiles) * BM;
+        c.n0 = ct * BN;
+        if constexpr (ANY == 2) {
+            const int each = s.row_tiles / s.period, in_batch = rt - c.b * s.row_tiles, rho = in_batch / each;
+            const int rows = (s.rows - rho + s.period - 1) / s.period - BM, at = (in_batch - rho * each) * BM;
+            c.m0 = rho + s.period * (at < rows ? at : rows);
+            // whole lines: all but the first and the last columns' tiles begin where a line does
+            if (ct) c.n0 -= (int)(((uintptr_t)s.out + c.b * s.batch_out + c.m0 * s.ld_out) & 127) / 2;
+        } else {
+            c.m0 = c.m0 < s.rows - BM ? c.m0 : s.rows - BM;
+        }
+        c.n0 = c.n0 < s.cols - BN ? c.n0 : s.cols - BN;
+        return c;
+    };
+
+    // ---- transfers.  X: rows 32 w + 8 q + lane / 8, piece lane & 7 of 8.  W likewise (8 QW w + ..), or, TW,
+    // rows of the contraction: pieces (w QW + q) 64 + lane of rows of BN / 8.
+    const int lrow = lane >> 3, lslot = lane & 7;
+    uint32_t off_x[4], off_w[QW];
+    long ld_x = 0, ld_w = 0;
+    const char *load_x = nullptr, *load_w = nullptr;
+    int lt = slot, lk = 0, lbuf = 0;
+    auto aim = [&]() {
+        const Tile c = tile_of(lt);
+        const LnSeg &s = p.seg[c.seg];
+        ld_x = ANY == 2 ? s.period * s.ld_x : s.ld_x;
+        ld_w = s.ld_w;
+        load_x = s.x + c.b * s.batch_x + c.m0 * s.ld_x + w * 32 * ld_x;
+        load_w = TW ? s.w + 2l * c.n0 : s.w + (long)(c.n0 + w * 8 * QW) * ld_w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            off_x[q] = (uint32_t)lrow * (uint32_t)ld_x + 16 * (lslot ^ ((lrow >> 1) | ((q & 1) << 2)));
+#pragma unroll
+        for (int q = 0; q < QW; ++q) {
+            if constexpr (TW) {
+                const int at = (w * QW + q) * 64 + lane, row = at / (BN / 8), piece = at - row * (BN / 8);
+                const int key = BN != 192 ? (row & 3) | ((row & 8) >> 1) : ((row >> 1) & 1) | ((row >> 2) & 2);
+                off_w[q] = (uint32_t)row * (uint32_t)ld_w + 16 * (((piece >> 1) ^ key) << 1 | (piece & 1));
+            } else {
+                off_w[q] = (uint32_t)lrow * (uint32_t)ld_w + 16 * (lslot ^ ((lrow >> 1) | (((w * QW + q) & 1) << 2)));
+            }
+        }
+    };
+    auto load = [&]() {
+        if (lt >= count) return;
+        const uint32_t to = lds0 + lbuf * STAGE;
+        lds_dma16_rows<4>(load_x + 2l * lk, 8 * ld_x, off_x, to + w * 4096);
+        lds_dma16_rows<QW>(TW ? load_w + lk * ld_w : load_w + 2l * lk, TW ? 0 : 8 * ld_w, off_w, to + XB + w * (QW * 1024));
+        lk += LN_STEP;
+        lbuf ^= 1;
+        if (lk >= p.K) {
+            lk = 0;
+            lt += slots;
+            if (lt < count) aim();
+        }
+    };
+
+    // ---- operands: lane (g, r) holds row r of X's 16, column r of W's, contraction 8 g .. of 32
+    int rd_x[2], rd_w[TW ? NJ : 2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) rd_x[h] = (wm * 64 + r) * 128 + 16 * ((4 * h + g) ^ (r >> 1));
+    if constexpr (TW) {
+        // a group of 16 lanes reads 4 rows by 16 columns, lane i the i & 3-th four columns of row i >> 2
+        const int key = BN != 192 ? (r >> 2) | ((g & 1) << 2) : ((r >> 3) & 1) | ((g & 1) << 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            rd_w[j] = XB + (8 * g + (r >> 2)) * PITCH + 32 * ((wn * NJ + j) ^ key) + 8 * (r & 3);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) rd_w[h] = XB + (wn * (BN / 2) + r) * 128 + 16 * ((4 * h + g) ^ (r >> 1));
+    }
+    u32x4_t ox[2][4], ow[NJ];
+    auto fetch_x = [&](int buf, int h, u32x4_t (&o)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = *(const u32x4_t *)(lds + buf * STAGE + rd_x[h] + i * 2048);
+    };
+    auto fetch_w = [&](int buf, int h, int j) {
+        if constexpr (TW) {
+            const char *q = lds + buf * STAGE + rd_w[j] + h * 32 * PITCH;
+            const u32x2_t a = ln_read_tr(q), b = ln_read_tr(q + 4 * PITCH);
+            ow[j] = u32x4_t{a[0], a[1], b[0], b[1]};
+        } else {
+            ow[j] = *(const u32x4_t *)(lds + buf * STAGE + rd_w[h] + j * 2048);
+        }
+    };
+    f32x4 acc[4][NJ];  // [16 rows][16 columns]: lane (g, r) holds row r, columns 4 g ..
+    // the products of 32 contraction steps while the next operands (half h of `buf`) take the places of those used up
+    auto products = [&](const u32x4_t (&x)[4], int buf, int h, u32x4_t (&next)[4]) {
+        fetch_x(buf, h, next);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i][j] = Mma<T>::k32(ow[j], x[i], acc[i][j]);
+            fetch_w(buf, h, j);
+        }
+        // (the order written here is the order issued)
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, TW ? 2 : 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // the bias of a tile's columns, one per thread
+    auto load_bias = [&](const Tile &c, int to) {
+        const uint16_t *b = p.seg[c.seg].bias;
+        const int at = (int)threadIdx.x;
+        if (at < BN) lds_dma2(b ? b + c.n0 + at : ln_no_bias + at, lds_address(lds_bias[to]) + 256 * w);
+    };
+    Tile c = tile_of(slot);
+    int which = 0;
+    load_bias(c, 0);
+    aim();
+    load();
+    load();
+    int buf = 0;
+    wait_vmem_all_but<4 + QW>();  // (K >= 2 stages)
+    lds_only_barrier();
+    fetch_x(0, 0, ox[0]);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) fetch_w(0, 0, j);
+    bool stored = false;
+    for (int t = slot; t < count; t += slots) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < p.K; k += LN_STEP) {
+            products(ox[0], buf, 1, ox[1]);
+            // The next stage and the bias are there (the results of the last tile, stored after they were
+            // requested, need not be), and, behind the barrier, everybody has read this stage: its place
+            // takes the one after next.
+            if (stored) wait_vmem_all_but<4 * NP>();
+            else wait_vmem_all_but<0>();
+            stored = false;
+            lds_only_barrier();
+            load();
+            __builtin_amdgcn_sched_barrier(0);
+            buf ^= 1;
+            products(ox[1], buf, 0, ox[0]);  // (behind the last stage: operands that nothing uses)
+        }
+        // ---- results
+        const LnSeg &s = p.seg[c.seg];
+        const int col = 16 * (g & 1) + 8 * (g >> 1);  // of a lane's eight columns in 32, after the exchange
+        const long ld_out = ANY == 2 ? s.period * s.ld_out : s.ld_out;
+        char *out = s.out + c.b * s.batch_out + c.m0 * s.ld_out + wm * 64 * ld_out + 2 * (c.n0 + wn * (BN / 2) + col);
+        if (t + slots < count) {
+            c = tile_of(t + slots);
+            load_bias(c, which ^ 1);
+        }
+        auto store = [&](char *q, u32x4_t v) {
+            // (2: the first and last columns' tiles begin at any element)
+            using piece_t = std::conditional_t<ANY == 2, LnLoosePiece, u32x4_t>;
+            if constexpr (PAST) __builtin_nontemporal_store(v, (piece_t *)q);
+            else *(piece_t *)q = v;
+        };
+        auto eight = [&](int i, int jp) {
+            u32x2_t d[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int j = 2 * jp + h;
+                const u32x4_t b = *(const u32x4_t *)(lds_bias[which] + wn * (BN / 2) + 16 * j + 4 * g);
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + to_float<T>((uint16_t)b[e]);
+                d[h] = u32x2_t{Mma<T>::pack(v[0], v[1]), Mma<T>::pack(v[2], v[3])};
+            }
+            // groups 1 and 3 of the first 16 columns against groups 0 and 2 of the second
+            const auto lo = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
+            return u32x4_t{lo[0], hi[0], lo[1], hi[1]};
+        };
+        // the sixteen columns of jp and jp + 1, lanes of rows r and r + 8 exchanging halves: lane (g, r) then holds, in
+        // a of row r & 7 and in b of row 8 + (r & 7), eight columns at 32 (r / 8) + col
+        auto lines = [&](int i, int jp, u32x4_t &a, u32x4_t &b) {
+            const u32x4_t v0 = eight(i, jp), v1 = eight(i, jp + 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t give = r < 8 ? v1[e] : v0[e];
+                const uint32_t got = __builtin_amdgcn_update_dpp(0, give, 0x128, 0xF, 0xF, true);  // row_ror:8
+                a[e] = r < 8 ? v0[e] : got;
+                b[e] = r < 8 ? got : v1[e];
+            }
+        };
+        if constexpr (ANY == 1) {
+            // Eight rows at a time through the LDS, from where they are read 16 bytes at a time as they lie in
+            // memory; the elements before the first and behind the last such piece, eight a row, one by one.
+            char *mine = lds_out + w * 8 * OUT_PITCH;
+            char *rows = out - 2 * col;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                u32x4_t v[2][2];  // [rows 0 .. 7, 8 .. 15][columns 0 .. 63, 64 .. 127]
+                lines(i, 0, v[0][0], v[1][0]);
+                lines(i, 2, v[0][1], v[1][1]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        *(u32x4_t *)(mine + (r & 7) * OUT_PITCH + 128 * q + (r & 8) * 8 + 2 * col) = v[h][q];
+                    char *eight_rows = rows + (long)(16 * i + 8 * h) * ld_out;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const int row = 4 * u + (lane >> 4), piece = lane & 15;
+                        char *to = eight_rows + row * ld_out;
+                        const int before = (int)(-(intptr_t)to & 15);  // bytes up to the first whole piece
+                        u32x4_t d;
+                        __builtin_memcpy(&d, __builtin_assume_aligned(mine + row * OUT_PITCH + before + 16 * piece, 2), 16);
+                        if (piece < 15 || before == 0) store(to + before + 16 * piece, d);
+                    }
+                    const int row = lane >> 3, e = lane & 7;
+                    char *to = eight_rows + row * ld_out;
+                    const int before = (int)(-(intptr_t)to & 15) / 2, at = e < before ? e : 120 + e;
+                    const uint16_t one = *(const uint16_t *)(mine + row * OUT_PITCH + 2 * at);
+                    if (before != 0) *(uint16_t *)(to + 2 * at) = one;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int jp = 0; jp + 1 < NP; jp += 2)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {  // a store covers eight rows by 128 bytes
+                    u32x4_t a, b;
+                    lines(i, jp, a, b);
+                    char *q = out + (long)(16 * i + (r & 7)) * ld_out + 64 * jp + (r & 8) * 8;
+                    store(q, a);
+                    store(q + 8 * ld_out, b);
+                }
+            if constexpr (NP & 1)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) store(out + (long)(16 * i + r) * ld_out + 64 * (NP - 1), eight(i, NP - 1));
+        }
+        stored = true;
+        which ^= 1;
+    }
+}
+
+// ---- few rows.  256 x 512 x 512 is a prompt's projection: 0.13 GFLOP, nothing but latency.  A workgroup owns 32 x 32
+// results and its wavefronts a quarter of the contraction each, taken in groups of 128 whose operands are all
+// requested before the first is multiplied, straight into registers in operand order; the partial tiles meet
+// in the LDS.  One trip to memory, four products deep, one exchange.
+constexpr int LS_TILE = 32, LS_WAVES = 4, LS_DEPTH = 4;  // LS_DEPTH: steps of 32 requested together
+
+template <typename T>
+__global__ void __launch_bounds__(64 * LS_WAVES) linear_few_rows_kernel(LnArgs p) {
+    __shared__ float part[LS_WAVES][LS_TILE][LS_TILE + 4];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, r = lane & 15;
+    int t = blockIdx.x, seg = 0;
+    while (seg + 1 < p.nseg && t >= p.seg[seg + 1].first) ++seg;
+    const LnSeg &q = p.seg[seg];
+    t -= q.first;
+    const int rt = t / q.col_tiles, n0 = (t - rt * q.col_tiles) * LS_TILE, batch = rt / q.row_tiles;
+    const int m0 = (rt - batch * q.row_tiles) * LS_TILE;
+    const int steps = p.K / 32, s0 = steps * w / LS_WAVES, s1 = steps * (w + 1) / LS_WAVES;
+    const char *px[2], *pw[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        // rows and columns behind the end: the last one's, not stored
+        const int m = m0 + 16 * i + r < q.rows ? m0 + 16 * i + r : q.rows - 1;
+        const int n = n0 + 16 * i + r < q.cols ? n0 + 16 * i + r : q.cols - 1;
+        px[i] = q.x + batch * q.batch_x + m * q.ld_x + 64 * s0 + 16 * g;
+        pw[i] = q.w + n * q.ld_w + 64 * s0 + 16 * g;
+    }
+    f32x4 acc[2][2];  // [rows][columns]: lane (g, r) holds row r, columns 4 g ..
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Ops {
+        u32x4_t x[2], w[2];
+    };
+    auto request = [&](int s, Ops &o) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            o.x[i] = *(const u32x4_t *)(px[i] + 64 * s);
+            o.w[i] = *(const u32x4_t *)(pw[i] + 64 * s);
+        }
+    };
+    auto products = [&](const Ops &o) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = Mma<T>::k32(o.w[j], o.x[i], acc[i][j]);
+    };
+    const int n = s1 - s0;
+    Ops o[LS_DEPTH];
+    int s = 0;
+    if (n >= LS_DEPTH) {
+#pragma unroll
+        for (int u = 0; u < LS_DEPTH; ++u) request(u, o[u]);
+        for (s = LS_DEPTH; s + LS_DEPTH <= n; s += LS_DEPTH)
+#pragma unroll
+            for (int u = 0; u < LS_DEPTH; ++u) {
+                products(o[u]);
+                request(s + u, o[u]);
+            }
+#pragma unroll
+        for (int u = 0; u < LS_DEPTH; ++u) products(o[u]);
+    }
+    for (; s < n; ++s) {
+        request(s, o[0]);
+        products(o[0]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *(f32x4 *)&part[w][16 * i + r][16 * j + 4 * g] = acc[i][j];
+    __syncthreads();
+    const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
+    if (m0 + row >= q.rows || n0 + c >= q.cols) return;  // (cols is a multiple of 4)
+    f32x4 sum = *(const f32x4 *)&part[0][row][c];
+#pragma unroll
+    for (int u = 1; u < LS_WAVES; ++u) sum += *(const f32x4 *)&part[u][row][c];
+    if (q.bias)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += to_float<T>(q.bias[n0 + c + e]);
+    *(u32x2_t *)(q.out + batch * q.batch_out + (m0 + row) * q.ld_out + 2 * (n0 + c)) =
+        u32x2_t{Mma<T>::pack(sum[0], sum[1]), Mma<T>::pack(sum[2], sum[3])};
+}
+
+// tiles, rows by columns; the fourth is the few-row kernel's, the last for results whose rows begin at any element
+struct LnTile {
+    int rows, cols;
+};
+constexpr LnTile LN_TILES[5] = {{256, 256}, {256, 192}, {128, 128}, {LS_TILE, LS_TILE}, {256, 256}};
+
+template <typename T, bool TW>
+void launch(int tile, bool past, const LnArgs &p, hipStream_t st) {
+    auto go = [&](auto kernel, int bm) { kernel<<<256 * 256 / bm, 2 * bm, 0, st>>>(p); };
+    if (tile == 0) past ? go(linear_kernel<T, 256, 256, TW, true>, 256) : go(linear_kernel<T, 256, 256, TW, false>, 256);
+    else if (tile == 1) past ? go(linear_kernel<T, 256, 192, TW, true>, 256) : go(linear_kernel<T, 256, 192, TW, false>, 256);
+    else if (tile == 2) go(linear_kernel<T, 128, 128, TW, false>, 128);
+    else if constexpr (!TW) {
+        if (p.seg[0].period > 1) past ? go(linear_kernel<T, 256, 256, false, true, 2>, 256) : go(linear_kernel<T, 256, 256, false, false, 2>, 256);
+        else go(linear_kernel<T, 256, 256, false, false, 1>, 256);
+    }
+}
+
+long tiles_of(const hsa_linear_segment &s, LnTile t) {
+    return (long)s.batches * ((s.rows + t.rows - 1) / t.rows) * ((s.cols + t.cols - 1) / t.cols);
+}
+
+// what the kernel of a tile takes
+bool takes(int tile, int nseg, const hsa_linear_segment *seg, int K, bool w_rows_contract) {
+    if (nseg < 1 || nseg > HSA_LINEAR_MAX_SEGMENTS || !seg || K > (1 << 20)) return false;
+    const bool few = tile == 3, any = tile == 4;
+    if (any && w_rows_contract) return false;
+    if (few ? K < 32 || K % 32 || w_rows_contract : K < 2 * LN_STEP || K % LN_STEP) return false;
+    for (int i = 0; i < nseg; ++i) {
+        const hsa_linear_segment &s = seg[i];
+        if (s.batches < 1 || s.rows < (few ? 1 : LN_TILES[tile].rows) || s.cols < (few ? 4 : LN_TILES[tile].cols) ||
+            s.cols % (any ? 1 : few ? 4 : 8) || s.batches > (1 << 24) || s.rows > (1 << 28) || s.cols > (1 << 24) || s.ld_x < K ||
+            s.ld_w < (w_rows_contract ? s.cols : K) || s.ld_out < s.cols || s.ld_x > (1 << 21) || s.ld_w > (1 << 21))
+            return false;
+        const int64_t strides = s.ld_x | s.ld_w | (any ? 0 : s.ld_out) | (s.batches > 1 ? s.batch_x | (any ? 0 : s.batch_out) : 0);
+        const uintptr_t bits = (uintptr_t)s.x | (uintptr_t)s.w | (any ? 8 : 1) * (uintptr_t)s.out | 8 * (uintptr_t)s.bias;
+        if (strides % 8 || bits % 16) return false;
+    }
+    return true;
+}
+
+double all_tiles(int tile, int nseg, const hsa_linear_segment *seg) {
+    double n = 0;
+    for (int i = 0; i < nseg; ++i) n += (double)tiles_of(seg[i], LN_TILES[tile]);
+    return n;
+}
+
+}  // namespace
+
+}  // namespace hsa
+
+extern "C" {
+
+int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int dtype) {
+    using namespace hsa;
+    if (dtype != HSA_F16 && dtype != HSA_BF16) return -1;
+    double results = 0;
+    if (nseg < 1 || nseg > HSA_LINEAR_MAX_SEGMENTS || !seg) return -1;
+    for (int i = 0; i < nseg; ++i) results += (double)seg[i].batches * seg[i].rows * seg[i].cols;
+    // Few rows (us, library / here; the library's call also takes 15 us more of host time): 64 x 512 x 512 5.6 / 4.0,
+    // 256 x 512 x 512 5.0 / 4.0, 256 x 2048 x 512 5.9 / 6.0, 256 x 1024 x 1024 5.5 / 5.9, 512 x 672 x 672 7.2 / 5.6; beyond: 512
+    // x 2048 x 512 6.4 / 9.7, 256 x 512 x 2048 6.3 / 9.3.  Several projections are several library calls.
+    if (K <= 1024 && results * K <= (double)(1 << 27) * (nseg + 1) && takes(3, nseg, seg, K, w_rows_contract)) return 3;
+    // Tiles: rounds of the chip times the time of a tile, 256 x 256 as 1 (256 x 192 0.8, two of 128 x 128 on one CU 0.74).
+    // The library has the better inner loop from contractions of about 1000 on and with its widest tiles at
+    // 768; at 512 and below this kernel is the faster one unless it leaves a good part of the chip idle
+    // (rows x cols x K, us, library / here): 8192 x 1536 x 512 27.9 / 18.9, 16384 x 1536 x 512 40.7 / 32.4, 32768 x 2048
+    // x 512 75 / 68, 4096 x 2048 x 512 15.6 / 15.1, 16384 x 768 x 768 24.2 / 23.7, 32752 x 768 x 768 46.5 / 38.4; not taken:
+    // 4096 x 512 x 512 8.0 / 8.9, 8192 x 768 x 768 15.2 / 17.5, 16384 x 3072 x 768 69 / 76, 16384 x 1024 x 1024 30.5 / 35,
+    // 32768 x 512 x 2048 51 / 56.  Rows that begin anywhere (a vocabulary of 50257): 256 x 50257 x 512 31 / 23,
+    // 4096 349 / 283, 32768 2200 / 1865; 8192 x 50257 x 768 593 / 722.
+    int best = -1;
+    double least = 0;
+    for (int t = 0; t < 3; ++t) {
+        if (!takes(t, nseg, seg, K, w_rows_contract)) continue;
+        const double n = all_tiles(t, nseg, seg);
+        const double us = t == 0 ? ceil(n / 256) : t == 1 ? 0.8 * ceil(n / 256) : n <= 256 ? 0.42 : 0.74 * ceil(n / 512);
+        if (best < 0 || us <= least) {
+            best = t;
+            least = us;
+        }
+    }
+    if (best < 0 && takes(4, nseg, seg, K, w_rows_contract)) {
+        best = 4;
+        least = ceil(all_tiles(4, nseg, seg) / 256);
+    }
+    if (best < 0) return -1;
+    const double used = results / (65536.0 * 256.0) / least;
+    if (K > 768 || used < (K > 512 ? 0.9 : 0.6) || (K > 512 && best != 1)) return -1;
+    return best;
+}
+
+int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int dtype, void *stream) {
+    using namespace hsa;
+    HSA_REQUIRE(dtype == HSA_F16 || dtype == HSA_BF16, "projections of 16-bit operands only (dtype %d)", dtype);
+    HSA_REQUIRE(tile >= 0 && tile < 5, "bad tile %d", tile);
+    if (!takes(tile, nseg, seg, K, w_rows_contract != 0))
+        return fail(HSA_ERR_UNSUPPORTED, "projection: sizes or alignment not handled by tile %d (K=%d)", tile, K);
+    const double all = all_tiles(tile, nseg, seg);
+    if (all >= (double)(1 << 30)) return fail(HSA_ERR_UNSUPPORTED, "projection: too many tiles");
+    LnArgs p = {};
+    p.nseg = nseg;
+    p.K = K;
+    p.group = 2048 / LN_TILES[tile].rows;
+    double bytes = 0;
+    for (int i = 0; i < nseg; ++i) {
+        const hsa_linear_segment &s = seg[i];
+        HSA_REQUIRE(s.x && s.w && s.out, "null pointer");
+        LnSeg &t = p.seg[i];
+        t.x = (const char *)s.x;
+        t.w = (const char *)s.w;
+        t.bias = (const uint16_t *)s.bias;
+        t.out = (char *)s.out;
+        t.ld_x = 2 * s.ld_x;
+        t.ld_w = 2 * s.ld_w;
+        t.ld_out = 2 * s.ld_out;
+        t.batch_x = 2 * s.batch_x;
+        t.batch_out = 2 * s.batch_out;
+        t.rows = s.rows;
+        t.cols = s.cols;
+        t.row_tiles = (s.rows + LN_TILES[tile].rows - 1) / LN_TILES[tile].rows;
+        t.period = 1;
+        if (tile == 4) {
+            // rows after which the results lie in their lines of 64 elements as before
+            long a = s.ld_out & 63, line = 64;
+            while (a) {
+                const long rest = line % a;
+                line = a;
+                a = rest;
+            }
+            const int period = (int)(64 / line);
+            if (nseg == 1 && period > 1 && s.rows / period >= LN_TILES[tile].rows) {
+                t.period = period;
+                t.row_tiles = period * (((s.rows + period - 1) / period + LN_TILES[tile].rows - 1) / LN_TILES[tile].rows);
+                t.col_tiles = (s.cols + 63 + LN_TILES[tile].cols - 1) / LN_TILES[tile].cols;
+            }
+        }
+        t.col_tiles = (s.cols + LN_TILES[tile].cols - 1) / LN_TILES[tile].cols;
+        t.all_row_tiles = s.batches * t.row_tiles;
+        t.first = p.tiles;
+        p.tiles += t.all_row_tiles * t.col_tiles;
+        bytes += 2.0 * s.batches * s.rows * s.cols;
+    }
+    // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 8 / 32: 2180
+    // / 2200 / 2550 us at 32768 x 50257 x 512)
+    if (tile == 4 && p.seg[0].period == 1) p.group = 2;
+    // results that the memory-side cache could not hold for the next kernel anyway go past the caches
+    const bool past = bytes > (double)(1 << 28);
+    const hipStream_t st = (hipStream_t)stream;
+    if (tile == 3) {
+        if (dtype == HSA_F16) linear_few_rows_kernel<F16><<<p.tiles, 64 * LS_WAVES, 0, st>>>(p);
+        else linear_few_rows_kernel<BF16><<<p.tiles, 64 * LS_WAVES, 0, st>>>(p);
+        return check_launch("linear_few_rows_kernel");
+    }
+    if (dtype == HSA_F16) w_rows_contract ? launch<F16, true>(tile, past, p, st) : launch<F16, false>(tile, past, p, st);
+    else w_rows_contract ? launch<BF16, true>(tile, past, p, st) : launch<BF16, false>(tile, past, p, st);
+    return check_launch("linear_kernel");
+}
+
+}  // extern "C"

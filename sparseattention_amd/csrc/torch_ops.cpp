@@ -315,6 +315,65 @@ std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const 
     return add_norm_plain(a, b, gamma, beta, eps, Tensor());
 }
 
+// ------------------------------------------------------------------------------- linear projections
+// x [.., K] dense, w [N, K] (contract: [K, N]) with dense rows, of one 16-bit type; out: rows of N with the strides
+// it has.  batches: x and out are [B, R, ..] whose batch elements lie apart.
+bool projectable(const Tensor &x, const Tensor &w, const Tensor &b, bool contract) {
+    return x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) && x.numel() > 0 &&
+           x.dim() >= 2 && x.is_contiguous() && same_kind(x, w) && w.dim() == 2 && w.is_contiguous() && w.numel() > 0 &&
+           x.size(-1) == w.size(contract ? 0 : 1) &&
+           (!b.defined() || (same_kind(x, b) && b.dim() == 1 && b.is_contiguous() && b.size(0) == w.size(contract ? 1 : 0)));
+}
+hsa_linear_segment flat_rows(const Tensor &x, const Tensor &w, const Tensor &b, const Tensor &out) {
+    const int64_t K = x.size(-1), N = out.size(-1), rows = x.numel() / K;
+    hsa_linear_segment s = {x.data_ptr(), w.data_ptr(), b.defined() ? b.data_ptr() : nullptr, out.data_ptr(), K,
+                            w.size(1), N, 0, 0, 1, 0, (int)N};
+    s.rows = rows < INT32_MAX ? (int)rows : 0;  // (0: refused)
+    return s;
+}
+// Whether the segments' products were launched.  few: also on the kernel for few rows, which adds in another order
+// than the library (the others add in the same, bit for bit).
+bool projected(const std::vector<hsa_linear_segment> &segs, const Tensor &like, int64_t K, bool contract, bool few) {
+    if (K > (1 << 20)) return false;
+    const int tile = hsa_linear_tile((int)segs.size(), segs.data(), (int)K, contract, type_code(like));
+    if (tile < 0 || (tile == 3 && !few)) return false;
+    c10::DeviceGuard guard(like.device());
+    check(hsa_linear((int)segs.size(), segs.data(), (int)K, contract, tile, type_code(like), stream_of(like)), "hsa_linear");
+    return true;
+}
+
+// x w^T + b, or x w with `contract`, without autograd: on this library's kernels where they are the faster
+// ones, else by torch
+Tensor project(const Tensor &x, const Tensor &w, const std::optional<Tensor> &b_, bool contract, bool few) {
+    const Tensor b = b_ ? *b_ : Tensor();
+    if (projectable(x, w, b, contract)) {
+        std::vector<int64_t> size = x.sizes().vec();
+        size.back() = w.size(contract ? 1 : 0);
+        Tensor out = at::empty(size, x.options());
+        if (projected({flat_rows(x, w, b, out)}, x, x.size(-1), contract, few)) return out;
+    }
+    return contract ? at::matmul(x, w) : at::linear(x, w, b_);
+}
+
+// The same of several (x, w), all without bias, in one launch where that pays.
+variable_list project_all(const std::vector<std::pair<Tensor, Tensor>> &parts, bool contract) {
+    std::vector<hsa_linear_segment> segs;
+    variable_list out;
+    for (const auto &[x, w] : parts) {
+        if (parts.size() > HSA_LINEAR_MAX_SEGMENTS || !projectable(x, w, Tensor(), contract) || x.size(-1) != parts[0].first.size(-1) ||
+            !same_kind(x, parts[0].first))
+            break;
+        std::vector<int64_t> size = x.sizes().vec();
+        size.back() = w.size(contract ? 1 : 0);
+        out.push_back(at::empty(size, x.options()));
+        segs.push_back(flat_rows(x, w, Tensor(), out.back()));
+    }
+    if (segs.size() == parts.size() && projected(segs, parts[0].first, parts[0].first.size(-1), contract, false)) return out;
+    out.clear();
+    for (const auto &[x, w] : parts) out.push_back(project(x, w, std::nullopt, contract, false));
+    return out;
+}
+
 // ------------------------------------------------------------------ linear projections in training
 bool rows_ok(const Tensor &t) {
     return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && aligned16(t);
@@ -356,8 +415,7 @@ struct Kept {
     Tensor t;
 };
 
-// y = x w^T + b by the library's product; backward: the input's gradient by the library, the weight's
-// and the bias's by the split-rows kernel, straight into the parameters' type.  `w`, `b` are the
+// y = x w^T + b; backward: the weight's and the bias's gradients by the split-rows kernel, straight into the parameters' type.  `w`, `b` are the
 // parameters in x's type (the casts that autocast makes); `w` keeps its graph, which a backward that is itself
 // differentiated goes through.  The parameter is not saved: under autocast it may be written to before the
 // backward.
@@ -367,7 +425,7 @@ struct Linear : public torch::autograd::Function<Linear> {
         ctx->save_for_backward({x, w.t});
         ctx->saved_data["bias"] = bias.has_value();
         ctx->saved_data["type"] = (int64_t)weight.scalar_type();
-        return at::linear(x, w.t, b);
+        return project(x, w.t, b, false, false);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
@@ -378,7 +436,7 @@ struct Linear : public torch::autograd::Function<Linear> {
         Tensor dx, dw, db;
         if (!g.defined()) return {dx, dw, db, Tensor(), Tensor()};
         const Tensor g2 = g.reshape({-1, g.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
-        if (ctx->needs_input_grad(0)) dx = at::matmul(g, w);
+        if (ctx->needs_input_grad(0)) dx = composed(grads) ? at::matmul(g, w) : project(g.contiguous(), w, std::nullopt, true, false);
         const bool need_w = ctx->needs_input_grad(1), need_b = bias && ctx->needs_input_grad(2);
         if (need_w && !composed(grads)) {
             if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), type, need_b)) {
@@ -393,14 +451,15 @@ struct Linear : public torch::autograd::Function<Linear> {
 };
 
 // F.linear(x, weight, bias) under the current autocast state; nullopt where nothing is to be gained
-// (no gradient of the weight, types other than the 16-bit ones, a result large enough to fill the chip
-// by itself) or where the call is not a plain one
+// (types other than the 16-bit ones; in training no gradient of the weight or a result large enough to fill
+// the chip by itself) or where the call is not a plain one
 std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias) {
-    if (!at::GradMode::is_enabled() || !weight.requires_grad() || !x.is_cuda() || x.dim() < 2 || weight.dim() != 2 ||
-        x.numel() == 0 || x.size(-1) != weight.size(1) || x.device() != weight.device() || !weight.is_contiguous())
+    if (!x.is_cuda() || x.dim() < 2 || weight.dim() != 2 || x.numel() == 0 || x.size(-1) != weight.size(1) ||
+        x.device() != weight.device() || !weight.is_contiguous())
         return std::nullopt;
+    const bool train = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
     const int64_t O = weight.size(0), I = weight.size(1);
-    if (O % 8 || I % 8 || ((O + 127) / 128) * ((I + 127) / 128) > 256) return std::nullopt;
+    if (train && (!weight.requires_grad() || O % 8 || I % 8 || ((O + 127) / 128) * ((I + 127) / 128) > 256)) return std::nullopt;
     if (bias && (bias->dim() != 1 || bias->size(0) != O || !same_kind(weight, *bias))) return std::nullopt;
     if (!ordinary({&x, &weight}) || (bias && !ordinary({&*bias}))) return std::nullopt;
     const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
@@ -410,6 +469,7 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     if (cast && ((weight.scalar_type() != at::kFloat && weight.scalar_type() != type) || type_code(x) < 0)) return std::nullopt;
     auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t; };
     const Kept w{as(weight)};
+    if (!train) return project(as(x), w.t, bias ? std::optional<Tensor>(as(*bias)) : std::nullopt, false, true);
     const std::optional<Tensor> b = bias ? std::optional<Tensor>(as(*bias).detach()) : std::nullopt;
     return Linear::apply(as(x), weight, bias, w, b);
 }
@@ -456,7 +516,7 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
         ctx->saved_data["edges"] = c10::IValue::make_capsule(std::move(edges));
         ctx->saved_data["N"] = (int64_t)N;
         ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)x.scalar_type(), (int64_t)y.scalar_type(), (int64_t)weight_k.scalar_type()};
-        return {at::linear(xs, wq), at::linear(xy, wk), at::linear(xy, wv)};
+        return project_all({{xs, wq}, {xy, wk}, {xy, wv}}, false);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
@@ -481,11 +541,16 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
         }
         const bool need_x = ctx->needs_input_grad(0), need_y = ctx->needs_input_grad(1);
         Tensor dx, dy, dw[3], d[3];  // d: input gradients of the three projections
+        if (!by_torch && need_x && grads[0].defined() && grads[1].defined() && grads[2].defined()) {
+            const auto rows = [](const Tensor &g) { return g.reshape({-1, g.size(-1)}).contiguous(); };
+            const variable_list r = project_all({{rows(grads[0]), w[0]}, {rows(grads[1]), w[1]}, {rows(grads[2]), w[2]}}, true);
+            for (int i = 0; i < 3; ++i) d[i] = r[i];
+        }
         for (int i = 0; i < 3; ++i) {
             const Tensor &g = grads[i];
             if (!g.defined()) continue;
             const Tensor g2 = g.reshape({-1, g.size(-1)}), r2 = (i == 0 ? xs : xy).reshape({-1, C});
-            if (i == 0 ? need_x : need_x || need_y) d[i] = at::mm(g2, w[i]);
+            if (!d[i].defined() && (i == 0 ? need_x : need_x || need_y)) d[i] = at::mm(g2, w[i]);
             if (!ctx->needs_input_grad(2 + i)) continue;
             if (!by_torch)
                 if (auto r = weight_grad({{g2, r2, 0}}, g2.size(1), w_type, false)) dw[i] = r->first;
@@ -515,18 +580,15 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
     }
 };
 
-// (queries of the rows of x [B, N, C]; keys, values of those and of y [B, M, C]) under the current autocast
-// state; nullopt where the call is not a plain one in training on 16-bit types
-std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Tensor &x, const Tensor &y,
-                                                                       const Tensor &weight_q, const Tensor &weight_k,
-                                                                       const Tensor &weight_v) {
-    if (!at::GradMode::is_enabled() || !x.is_cuda() || x.dim() != 3 || y.dim() != 3 || x.numel() == 0 || y.numel() == 0 ||
-        x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || weight_k.device() != x.device() ||
+// The element type in which the three projections of the rows of x [B, N, C] and y [B, M, C] compute under the current
+// autocast state; nullopt where the call is not a plain one on 16-bit types.
+std::optional<at::ScalarType> rows_type(const Tensor &x, const Tensor &y, const Tensor &weight_q, const Tensor &weight_k,
+                                        const Tensor &weight_v) {
+    if (x.dim() != 3 || y.dim() != 3 || x.numel() == 0 || y.numel() == 0 || x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || weight_k.device() != x.device() ||
         weight_k.dim() != 2 || weight_k.size(1) != x.size(2))
         return std::nullopt;
     for (const Tensor *t : {&weight_q, &weight_k, &weight_v})
-        if (!same_kind(weight_k, *t) || t->sizes() != weight_k.sizes() || !t->is_contiguous() || !t->requires_grad())
-            return std::nullopt;
+        if (!same_kind(weight_k, *t) || t->sizes() != weight_k.sizes() || !t->is_contiguous()) return std::nullopt;
     const int64_t O = weight_k.size(0), C = weight_k.size(1);
     if (O % 8 || C % 8 || ((O + 127) / 128) * ((C + 127) / 128) > 256 || x.numel() + y.numel() > (int64_t)1 << 40 ||
         x.size(1) + y.size(1) > (1 << 30) || !ordinary({&x, &y, &weight_q, &weight_k, &weight_v}))
@@ -536,11 +598,59 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Ten
     if (type != at::kHalf && type != at::kBFloat16) return std::nullopt;
     for (const Tensor *t : {&x, &y, &weight_k})
         if (t->scalar_type() != type && !(cast && t->scalar_type() == at::kFloat)) return std::nullopt;
+    return type;
+}
+
+// (queries of the rows of x [B, N, C]; keys, values of those and of y [B, M, C]) under the current autocast
+// state; nullopt where the call is not a plain one in training on 16-bit types
+std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Tensor &x, const Tensor &y,
+                                                                       const Tensor &weight_q, const Tensor &weight_k,
+                                                                       const Tensor &weight_v) {
+    if (!at::GradMode::is_enabled() || !x.is_cuda()) return std::nullopt;
+    for (const Tensor *t : {&weight_q, &weight_k, &weight_v})
+        if (!t->requires_grad()) return std::nullopt;
+    const std::optional<at::ScalarType> type = rows_type(x, y, weight_q, weight_k, weight_v);
+    if (!type) return std::nullopt;
     const Tensor xc = x.contiguous(), yc = y.contiguous();
     if (!aligned16(xc) || !aligned16(yc)) return std::nullopt;
-    auto as = [&](const Tensor &t) { return Kept{cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t}; };
+    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    auto as = [&](const Tensor &t) { return Kept{cast ? at::autocast::cached_cast(*type, t, at::kCUDA) : t}; };
     variable_list r = QueryKeyValueRows::apply(xc, yc, weight_q, weight_k, weight_v, as(weight_q), as(weight_k), as(weight_v));
     return std::make_tuple(r[0], r[1], r[2]);
+}
+
+// The same without autograd: the rows stay where they are, every projection writes its part of the results, in one
+// launch.  nullopt where that does not pay.
+std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value(const Tensor &x_, const Tensor &y_, const Tensor &weight_q,
+                                                                  const Tensor &weight_k, const Tensor &weight_v) {
+    if (!x_.is_cuda()) return std::nullopt;
+    if (at::GradMode::is_enabled())
+        for (const Tensor *t : {&x_, &y_, &weight_q, &weight_k, &weight_v})
+            if (t->requires_grad()) return std::nullopt;
+    const std::optional<at::ScalarType> type = rows_type(x_, y_, weight_q, weight_k, weight_v);
+    if (!type) return std::nullopt;
+    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(*type, t, at::kCUDA) : t; };
+    const Tensor x = x_.to(*type).contiguous(), y = y_.to(*type).contiguous();
+    const Tensor wq = as(weight_q), wk = as(weight_k), wv = as(weight_v);
+    if (!projectable(x, wq, Tensor(), false) || !projectable(x, wk, Tensor(), false) || !projectable(x, wv, Tensor(), false) ||
+        !projectable(y, wk, Tensor(), false))
+        return std::nullopt;
+    const int64_t B = x.size(0), N = x.size(1), M = y.size(1), O = wk.size(0);
+    if (N + M > (1 << 28) || B > (1 << 24)) return std::nullopt;
+    Tensor q = at::empty({B, N, O}, x.options()), k = at::empty({B, N + M, O}, x.options()), v = at::empty_like(k);
+    const auto rows = [&](const Tensor &in, const Tensor &w, const Tensor &out, int64_t first) {
+        hsa_linear_segment s = flat_rows(in, w, Tensor(), out);
+        s.out = (char *)s.out + first * O * out.element_size();
+        s.batches = (int)B;
+        s.rows = (int)in.size(1);
+        s.batch_x = in.stride(0);
+        s.batch_out = out.stride(0);
+        return s;
+    };
+    if (!projected({rows(x, wq, q, 0), rows(x, wk, k, 0), rows(x, wv, v, 0), rows(y, wk, k, N), rows(y, wv, v, N)}, x, x.size(2), false, true))
+        return std::nullopt;
+    return std::make_tuple(q, k, v);
 }
 
 }  // namespace
@@ -557,6 +667,8 @@ PYBIND11_MODULE(_hsa_torch, m) {
     m.def("build_tree", &build_tree);
     m.def("add_layer_norm", &add_layer_norm);
     m.def("linear", &linear);
+    m.def("project", &project);
     m.def("weight_grad", &weight_grad);
     m.def("query_key_value_rows", &query_key_value_rows);
+    m.def("query_key_value", &query_key_value);
 }

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import linear, query_key_value_rows
+from ..ops.linear import linear, query_key_value, query_key_value_rows
 from ..ops.topology import build_tree_topology
 
 
@@ -179,7 +179,8 @@ class HierarchicalAttention(nn.Module):
         cdt = self._compute_dtype(x)
         x, y_in = x.to(cdt).contiguous(), y_in.to(cdt).contiguous()
         w_qkv = self._fused_weight("qkv_y", (self.Wq_y, self.Wk_y, self.Wv_y), cdt)
-        qkv = F.linear(y_in, w_qkv)  # [B, N-1, 3D]
+        project = _lib.ext().project
+        qkv = project(y_in, w_qkv, None, False, not keep)  # [B, N-1, 3D]
         w_kv = self._fused_weight("kv_y", (self.Wk_y, self.Wv_y), cdt)
         # every buffer the kernels address by raw pointer has the one element type
         assert qkv.dtype == cdt and qkv.is_contiguous(), "projection result has an unexpected layout"
@@ -214,9 +215,9 @@ class HierarchicalAttention(nn.Module):
                     if keep:
                         # the backward's keys and values of these levels' children, one GEMM for all
                         rows = torch.cat([src, y_new[:, off:N - 2]], dim=1)  # [B, 4P-2, D]
-                        chain = (rows, F.linear(rows, w_kv))
+                        chain = (rows, project(rows, w_kv, None, False, False))
                     break
-                kv = F.linear(src, w_kv)  # [B, 2P, 2D]
+                kv = project(src, w_kv, None, False, not keep)  # [B, 2P, 2D]
                 assert kv.dtype == cdt and kv.is_contiguous(), "projection result has an unexpected layout"
                 if drop_p > 0:
                     # dropout on the value half: a saved boolean keep-mask (drawn in fp32) and one
@@ -282,7 +283,7 @@ class HierarchicalAttention(nn.Module):
                     dqkv.data_ptr() + off * 3 * D * es, dkv_up.data_ptr(), B, C, H, Dh, (N - 1) * D, D, T3, 3 * D, T3,
                     3 * D, code, stream)
                 _lib.check(rc, "hsa_span_levels_bwd")
-                d_above = torch.mm(dkv_up[:, :C].reshape(-1, 2 * D), w_kv)  # [B * C, D]
+                d_above = _lib.ext().project(dkv_up[:, :C].reshape(-1, 2 * D), w_kv, None, True, False)  # [B * C, D]
                 pairs.append((dkv_up.view(-1, 2 * D), rows.view(-1, D), D))
             for lvl in range(len(kvs) - 1, -1, -1):
                 P, off = sizes[lvl], offsets[lvl]
@@ -299,9 +300,9 @@ class HierarchicalAttention(nn.Module):
                 _lib.check(rc, "hsa_build_parents_level_bwd")
                 if masks:
                     dkv_l.view(B, 2 * P, 2 * D)[:, :, D:].mul_(masks[lvl]).mul_(kept["scales"][lvl])
-                d_above = torch.matmul(dkv_l, w_kv)  # [B * 2P, D]
+                d_above = _lib.ext().project(dkv_l, w_kv, None, True, False)  # [B * 2P, D]
         dx = d_above.view(B, N, D)
-        dy_in = torch.matmul(dqkv, w_qkv)
+        dy_in = _lib.ext().project(dqkv, w_qkv, None, True, False)
         if kvs:
             pairs.append((dkv[:B * N], x.view(-1, D), D))
         if inner:
@@ -326,7 +327,7 @@ class HierarchicalAttention(nn.Module):
         grad = self._needs_autograd((x, y_in), (self.Wq_y, self.Wk_y, self.Wv_y))
         drop_p = self.dropout.p if self.training else 0.0
         if not grad and drop_p == 0:
-            return self.out_proj_y(self._span_levels(x, y_in))
+            return linear(self.out_proj_y, self._span_levels(x, y_in))
         if self.fused_training and x.is_cuda and N >= 2:
             # the same fused level loop as one differentiable function
             y_new = _SpanLevels.apply(self, drop_p, x, y_in, self.Wq_y.weight, self.Wk_y.weight, self.Wv_y.weight)
@@ -351,9 +352,11 @@ class HierarchicalAttention(nn.Module):
         B, N, D = x.shape
         assert y is not None, "y (parents) cannot be None during top-down update"
         grad = self._needs_autograd((x, y), (self.Wq_x, self.Wk_x, self.Wv_x))
-        qkv = query_key_value_rows(self.Wq_x, self.Wk_x, self.Wv_x, x, y) if grad else None
+        dropped = self.training and self.dropout.p > 0
+        join = query_key_value_rows if grad else query_key_value
+        qkv = join(self.Wq_x, self.Wk_x, self.Wv_x, x, y)
         q = self._heads(linear(self.Wq_x, x) if qkv is None else qkv[0])
-        if (not grad and not (self.training and self.dropout.p > 0) and y.size(1) == N - 1
+        if (qkv is None and not grad and not dropped and y.size(1) == N - 1
                 and B * N * D >= self._DIRECT_PROJECTION_MIN_ELEMENTS):
             # leaves and span nodes are projected straight into their rows of the [B, 2N-1, D]
             # key / value buffers (batched GEMMs with a strided output): no concatenated input.

@@ -1,4 +1,4 @@
-"""`linear(layer, x)`: an nn.Linear whose weight and bias gradients run on this package's kernel."""
+"""`linear(layer, x)`: an nn.Linear on this package's kernels, forward and backward."""
 from __future__ import annotations
 
 import torch
@@ -24,10 +24,11 @@ def _plain(layer) -> bool:
 
 
 def linear(layer, x: torch.Tensor) -> torch.Tensor:
-    """layer(x).  In training on the GPU with 16-bit activations (or under autocast to such a type) the
-    backward computes the weight's and the bias's gradient in one contraction over the tokens
-    (csrc/hsa_weight_grad.hip), directly in the parameters' type; everything else is the layer itself."""
-    if x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(layer):
+    """layer(x).  On the GPU with 16-bit activations (or under autocast to such a type) the product runs on this
+    package's kernels where they are the faster ones (csrc/hsa_linear.hip), and in training the backward
+    computes the weight's and the bias's gradient in one contraction over the tokens (csrc/hsa_weight_grad.hip),
+    directly in the parameters' type; everything else is the layer itself."""
+    if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer):
         y = _lib.ext().linear(x, layer.weight, layer.bias)
         if y is not None:
             return y
@@ -42,4 +43,13 @@ def query_key_value_rows(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Te
     if (x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling()
             and all(_plain(m) and m.bias is None for m in layers)):
         return _lib.ext().query_key_value_rows(x, y, *(m.weight for m in layers))
+    return None
+
+
+def query_key_value(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
+    """The same without autograd: the rows stay where they are and the five products write into the joined
+    results in one launch (csrc/hsa_linear.hip).  None where that does not apply."""
+    layers = (layer_q, layer_k, layer_v)
+    if x.is_cuda and not torch.compiler.is_compiling() and all(_plain(m) and m.bias is None for m in layers):
+        return _lib.ext().query_key_value(x, y, *(m.weight for m in layers))
     return None

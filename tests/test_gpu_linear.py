@@ -1,0 +1,171 @@
+"""The projection kernels (csrc/hsa_linear.hip) against fp64 at the edges of their tiles, and the routes to them."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from sparseattention_amd import _lib
+from sparseattention_amd.ops.linear import linear, query_key_value
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+class Segment(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "w", "bias", "out")]
+                + [(n, ctypes.c_int64) for n in ("ld_x", "ld_w", "ld_out", "batch_x", "batch_out")]
+                + [(n, ctypes.c_int) for n in ("batches", "rows", "cols")])
+
+
+def _segment(x, w, bias, out):
+    return Segment(x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), x.stride(1),
+                   w.stride(0), out.stride(1), x.stride(0), out.stride(0), x.shape[0], x.shape[1], out.shape[2])
+
+
+def _call(segs, K, contract, tile, dtype):
+    arr = (Segment * len(segs))(*segs)
+    rc = _lib.lib().hsa_linear(len(segs), arr, K, int(contract), tile, 1 if dtype == torch.float16 else 2,
+                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    _lib.check(rc, "hsa_linear")
+
+
+def _bound(x, w, ref, dtype):
+    """One rounding of the result (half a unit in the last place, half the smallest subnormal below) and K fp32
+    additions and products, each off by at most 2^-24 of the sum of magnitudes."""
+    half = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8  # 10 and 7 stored bits
+    sums = x.double().abs() @ w.double().abs()
+    return half * ref.abs() * 1.01 + 2.0 ** -25 + x.shape[-1] * 2.0 ** -23 * (sums + 1)
+
+
+def _check(dtype, contract, tile, B, R, N, K, pad, first):
+    """Two projections of one launch, one with a bias and one without, into the middle of larger buffers."""
+    g = torch.Generator(DEV).manual_seed(B + R + N + K)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
+    x, w, bias = mk(B, R, K), mk(K, N) if contract else mk(N, K), mk(N + 1)[1:]
+    ld = N + pad
+    bufs = [torch.full((B * (R + 1) * ld + 64,), 7.0, device=DEV, dtype=dtype) for _ in range(2)]
+    outs = [b.as_strided((B, R, N), ((R + 1) * ld, ld, 1), first) for b in bufs]
+    _call([_segment(x, w, bias, outs[0]), _segment(x, w, None, outs[1])][:1 if tile == 4 else 2], K, contract, tile, dtype)
+    wt = w if contract else w.t()
+    ref = x.double() @ wt.double()
+    for i, want in enumerate((ref + bias.double(), ref)[:1 if tile == 4 else 2]):
+        err = (outs[i].double() - want).abs()
+        assert bool((err <= _bound(x, wt, want, dtype)).all()), (i, float(err.max()))
+        rest = bufs[i].clone()
+        rest.as_strided((B, R, N), ((R + 1) * ld, ld, 1), first).fill_(7.0)
+        assert bool((rest == 7).all()), "written outside the result"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("contract", [False, True])
+@pytest.mark.parametrize("tile,B,R,N,K", [
+    (0, 1, 256, 256, 128), (0, 3, 257, 264, 192), (0, 2, 511, 512, 320), (0, 1, 8448, 520, 128),
+    (1, 1, 256, 192, 128), (1, 2, 300, 200, 512), (1, 5, 257, 392, 192),
+    (2, 1, 128, 128, 128), (2, 3, 130, 136, 192), (2, 1, 4099, 768, 128)])
+def test_tiles_against_fp64(dtype, contract, tile, B, R, N, K):
+    _check(dtype, contract, tile, B, R, N, K, 8, 16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,R,N,K", [(1, 1, 4, 32), (2, 17, 36, 64), (1, 33, 32, 96), (3, 31, 100, 672), (1, 256, 512, 2080)])
+def test_few_rows_against_fp64(dtype, B, R, N, K):
+    _check(dtype, False, 3, B, R, N, K, (8 - N % 8) % 8 + 8, 16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,R,N,K,pad,first", [
+    (1, 256, 256, 128, 0, 0), (2, 257, 257, 192, 0, 3), (1, 300, 511, 512, 2, 1), (1, 512, 1000, 128, 3, 7),
+    (1, 16384, 257, 128, 0, 0), (1, 16447, 513, 192, 2, 5), (1, 8300, 320, 128, 2, 1)])
+def test_results_that_begin_anywhere(dtype, B, R, N, K, pad, first):
+    """Rows through the LDS; from 256 rows per line period on (16384 for odd strides, 8192 for twice an odd one)
+    tiles of rows that lie alike."""
+    _check(dtype, False, 4, B, R, N, K, pad, first)
+
+
+def test_refused_sizes():
+    x, w = torch.zeros(1, 256, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(256, 128, device=DEV, dtype=torch.bfloat16)
+    out = torch.empty(1, 256, 256, device=DEV, dtype=torch.bfloat16)
+    ok = _segment(x, w, None, out)
+    tile = _lib.lib().hsa_linear_tile
+    assert tile(1, ctypes.byref(ok), 128, 0, 0) == -1  # fp32
+    assert tile(0, ctypes.byref(ok), 128, 0, 2) == -1
+    for kind, K, name, value in ((0, 96, None, 0), (0, 128, "rows", 255), (0, 128, "cols", 248), (0, 128, "ld_out", 260),
+                                 (0, 128, "ld_x", 120), (3, 33, None, 0), (4, 128, "cols", 255)):
+        s = _segment(x, w, None, out)
+        if name:
+            setattr(s, name, value)
+        with pytest.raises(_lib.HsaError):
+            _call([s], K, False, kind, torch.bfloat16)
+    with pytest.raises(_lib.HsaError):
+        _call([ok], 128, True, 3, torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,cols,K,bias", [(8192, 1536, 512, False), (256, 512, 512, True), (4096, 10001, 256, True),
+                                              (64, 40, 96, True)])
+def test_linear_without_autograd(rows, cols, K, bias):
+    """Each route, chosen by the sizes: tiles, few rows, results that begin anywhere."""
+    torch.manual_seed(0)
+    layer = nn.Linear(K, cols, bias=bias).to(DEV, torch.bfloat16)
+    x = torch.randn(2, rows // 2, K, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        got = linear(layer, x)
+        strided = x.transpose(0, 1).contiguous().transpose(0, 1)  # rows that lie apart: the layer itself
+        assert torch.equal(linear(layer, strided), layer(strided))
+    wt = layer.weight.detach().t()
+    want = x.double() @ wt.double() + (layer.bias.detach().double() if bias else 0)
+    assert got.shape == want.shape and got.dtype == torch.bfloat16 and not got.requires_grad
+    assert bool(((got.double() - want).abs() <= _bound(x, wt, want, torch.bfloat16)).all())
+
+
+@pytest.mark.parametrize("amp", [None, torch.float16])
+@pytest.mark.parametrize("B,N,C", [(1, 64, 64), (2, 256, 256), (4, 1024, 512)])
+def test_query_key_value(amp, B, N, C):
+    torch.manual_seed(0)
+    dtype = torch.float32 if amp else torch.bfloat16
+    layers = [nn.Linear(C, C, bias=False).to(DEV, dtype) for _ in range(3)]
+    x, y = torch.randn(B, N, C, device=DEV).to(dtype), torch.randn(B, N - 1, C, device=DEV).to(dtype)
+    with torch.no_grad(), torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+        got = query_key_value(*layers, x, y)
+    low = amp or dtype
+    assert got is not None
+    for i, (t, layer) in enumerate(zip(got, layers)):
+        rows = (x if i == 0 else torch.cat([x, y], dim=1)).to(low)
+        wt = layer.weight.detach().to(low).t()
+        want = rows.double() @ wt.double()
+        assert t.dtype == low and t.is_contiguous() and t.shape == want.shape
+        assert bool(((t.double() - want).abs() <= _bound(rows, wt, want, low)).all())
+    x.requires_grad_(True)
+    assert query_key_value(*layers, x, y) is None  # not with autograd
+
+
+def test_input_gradient_on_tiles():
+    """The input gradient of a projection that is large enough for the kernel, against fp64."""
+    torch.manual_seed(0)
+    layer = nn.Linear(512, 512).to(DEV, torch.bfloat16)
+    x = torch.randn(16384, 512, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(16384, 512, device=DEV, dtype=torch.bfloat16)
+    linear(layer, x).backward(dy)
+    w = layer.weight.detach()
+    want = dy.double() @ w.double()
+    assert bool(((x.grad.double() - want).abs() <= _bound(dy, w, want, torch.bfloat16)).all())
+
+
+def test_replays_of_a_graph_with_projections():
+    torch.manual_seed(0)
+    layer = nn.Linear(256, 1024).to(DEV, torch.bfloat16)
+    small, large = (torch.randn(n, 256, device=DEV, dtype=torch.bfloat16) for n in (64, 8192))
+    with torch.no_grad():
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            linear(layer, small), linear(layer, large)
+        torch.cuda.current_stream().wait_stream(s)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = linear(layer, small), linear(layer, large)
+        for i in range(3):
+            small.normal_(), large.normal_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(outs[0], linear(layer, small)) and torch.equal(outs[1], linear(layer, large))

@@ -501,6 +501,18 @@ typedef struct {
 int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int dtype);
 int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int dtype, void *stream);
 
+/*
+ * out[r, n] = sum over k of x[r, k] * w[k, n] for a long contraction (the input gradient of a vocabulary projection):
+ * x [M, K] with rows that begin at any element, w [K, N] and out [M, N] with 16-byte aligned rows, M and N from 256
+ * on, N a multiple of 8, `dtype` HSA_F16 or HSA_BF16, fp32 sums.  The contraction is split and the parts' fp32
+ * results are added in a fixed order; workspace: hsa_linear_long_workspace_bytes bytes (0: not handled), 16-byte
+ * aligned, written before read.  hsa_linear_long_pays: whether a library product is the slower one.
+ */
+size_t hsa_linear_long_workspace_bytes(int M, int N, int K, int dtype);
+int hsa_linear_long_pays(int M, int N, int K, int dtype);
+int hsa_linear_long(const void *x, int64_t ld_x, const void *w, int64_t ld_w, void *out, int64_t ld_out, int M, int N, int K,
+                    void *workspace, size_t workspace_bytes, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -38,6 +38,12 @@ def _declare(lib):
     lib.hsa_linear.restype = I
     lib.hsa_linear_tile.argtypes = [I, P, I, I, I]
     lib.hsa_linear_tile.restype = I
+    lib.hsa_linear_long.argtypes = [P, I64, P, I64, P, I64, I, I, I, P, ctypes.c_size_t, I, P]
+    lib.hsa_linear_long.restype = I
+    lib.hsa_linear_long_workspace_bytes.argtypes = [I] * 4
+    lib.hsa_linear_long_workspace_bytes.restype = ctypes.c_size_t
+    lib.hsa_linear_long_pays.argtypes = [I] * 4
+    lib.hsa_linear_long_pays.restype = I
     lib.hsa_cross_update_level_tune.argtypes = [I, ctypes.c_long]
     lib.hsa_cross_update_level_tune.restype = I
     lib.hsa_attn_bwd_tables.argtypes = [P] * 11 + [ctypes.c_size_t] + [I] * 9 + [P]

@@ -410,66 +410,76 @@ __global__ void __launch_bounds__(64 * LS_WAVES) linear_few_rows_kernel(LnArgs p
     t -= q.first;
     const int rt = t / q.col_tiles, n0 = (t - rt * q.col_tiles) * LS_TILE, batch = rt / q.row_tiles;
     const int m0 = (rt - batch * q.row_tiles) * LS_TILE;
-    const int steps = p.K / 32, s0 = steps * w / LS_WAVES, s1 = steps * (w + 1) / LS_WAVES;
+    const int steps = p.K / 32;
+    const bool whole = steps < 2 * LS_WAVES;  // a short contraction: each wavefront all of it for a quarter of the results
+    const int s0 = whole ? 0 : steps * w / LS_WAVES, n = whole ? steps : steps * (w + 1) / LS_WAVES - s0;
     const char *px[2], *pw[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         // rows and columns behind the end: the last one's, not stored
         const int m = m0 + 16 * i + r < q.rows ? m0 + 16 * i + r : q.rows - 1;
-        const int n = n0 + 16 * i + r < q.cols ? n0 + 16 * i + r : q.cols - 1;
+        const int col = n0 + 16 * i + r < q.cols ? n0 + 16 * i + r : q.cols - 1;
         px[i] = q.x + batch * q.batch_x + m * q.ld_x + 64 * s0 + 16 * g;
-        pw[i] = q.w + n * q.ld_w + 64 * s0 + 16 * g;
+        pw[i] = q.w + col * q.ld_w + 64 * s0 + 16 * g;
     }
-    f32x4 acc[2][2];  // [rows][columns]: lane (g, r) holds row r, columns 4 g ..
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    struct Ops {
-        u32x4_t x[2], w[2];
-    };
-    auto request = [&](int s, Ops &o) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            o.x[i] = *(const u32x4_t *)(px[i] + 64 * s);
-            o.w[i] = *(const u32x4_t *)(pw[i] + 64 * s);
-        }
-    };
-    auto products = [&](const Ops &o) {
+    if (whole) {
+        const char *x = w & 2 ? px[1] : px[0], *wt = w & 1 ? pw[1] : pw[0];
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < n; ++s)
+            acc = Mma<T>::k32(*(const u32x4_t *)(wt + 64 * s), *(const u32x4_t *)(x + 64 * s), acc);
+        *(f32x4 *)&part[0][8 * (w & 2) + r][16 * (w & 1) + 4 * g] = acc;
+    } else {
+        f32x4 acc[2][2];  // [rows][columns]: lane (g, r) holds row r, columns 4 g ..
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = Mma<T>::k32(o.w[j], o.x[i], acc[i][j]);
-    };
-    const int n = s1 - s0;
-    Ops o[LS_DEPTH];
-    int s = 0;
-    if (n >= LS_DEPTH) {
+            for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        struct Ops {
+            u32x4_t x[2], w[2];
+        };
+        auto request = [&](int s, Ops &o) {
 #pragma unroll
-        for (int u = 0; u < LS_DEPTH; ++u) request(u, o[u]);
-        for (s = LS_DEPTH; s + LS_DEPTH <= n; s += LS_DEPTH)
-#pragma unroll
-            for (int u = 0; u < LS_DEPTH; ++u) {
-                products(o[u]);
-                request(s + u, o[u]);
+            for (int i = 0; i < 2; ++i) {
+                o.x[i] = *(const u32x4_t *)(px[i] + 64 * s);
+                o.w[i] = *(const u32x4_t *)(pw[i] + 64 * s);
             }
+        };
+        auto products = [&](const Ops &o) {
 #pragma unroll
-        for (int u = 0; u < LS_DEPTH; ++u) products(o[u]);
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = Mma<T>::k32(o.w[j], o.x[i], acc[i][j]);
+        };
+        Ops o[LS_DEPTH];
+        int s = 0;
+        if (n >= LS_DEPTH) {
+#pragma unroll
+            for (int u = 0; u < LS_DEPTH; ++u) request(u, o[u]);
+            for (s = LS_DEPTH; s + LS_DEPTH <= n; s += LS_DEPTH)
+#pragma unroll
+                for (int u = 0; u < LS_DEPTH; ++u) {
+                    products(o[u]);
+                    request(s + u, o[u]);
+                }
+#pragma unroll
+            for (int u = 0; u < LS_DEPTH; ++u) products(o[u]);
+        }
+        for (; s < n; ++s) {
+            request(s, o[0]);
+            products(o[0]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) *(f32x4 *)&part[w][16 * i + r][16 * j + 4 * g] = acc[i][j];
     }
-    for (; s < n; ++s) {
-        request(s, o[0]);
-        products(o[0]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) *(f32x4 *)&part[w][16 * i + r][16 * j + 4 * g] = acc[i][j];
     __syncthreads();
     const int row = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
     if (m0 + row >= q.rows || n0 + c >= q.cols) return;  // (cols is a multiple of 4)
     f32x4 sum = *(const f32x4 *)&part[0][row][c];
+    if (!whole)
 #pragma unroll
-    for (int u = 1; u < LS_WAVES; ++u) sum += *(const f32x4 *)&part[u][row][c];
+        for (int u = 1; u < LS_WAVES; ++u) sum += *(const f32x4 *)&part[u][row][c];
     if (q.bias)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[e] += to_float<T>(q.bias[n0 + c + e]);

@@ -324,53 +324,79 @@ bool projectable(const Tensor &x, const Tensor &w, const Tensor &b, bool contrac
            x.size(-1) == w.size(contract ? 0 : 1) &&
            (!b.defined() || (same_kind(x, b) && b.dim() == 1 && b.is_contiguous() && b.size(0) == w.size(contract ? 1 : 0)));
 }
-hsa_linear_segment flat_rows(const Tensor &x, const Tensor &w, const Tensor &b, const Tensor &out) {
-    const int64_t K = x.size(-1), N = out.size(-1), rows = x.numel() / K;
+hsa_linear_segment flat_rows(const Tensor &x, const Tensor &w, const Tensor &b, const Tensor &out, int64_t N) {
+    const int64_t K = x.size(-1), rows = x.numel() / K;
     hsa_linear_segment s = {x.data_ptr(), w.data_ptr(), b.defined() ? b.data_ptr() : nullptr, out.data_ptr(), K,
                             w.size(1), N, 0, 0, 1, 0, (int)N};
     s.rows = rows < INT32_MAX ? (int)rows : 0;  // (0: refused)
     return s;
 }
-// Whether the segments' products were launched.  few: also on the kernel for few rows, which adds in another order
-// than the library (the others add in the same, bit for bit).
-bool projected(const std::vector<hsa_linear_segment> &segs, const Tensor &like, int64_t K, bool contract, bool few) {
-    if (K > (1 << 20)) return false;
-    const int tile = hsa_linear_tile((int)segs.size(), segs.data(), (int)K, contract, type_code(like));
-    if (tile < 0 || (tile == 3 && !few)) return false;
+// the tile for the segments' products, or -1
+int tile_for(const std::vector<hsa_linear_segment> &segs, const Tensor &like, int64_t K, bool contract) {
+    return K > (1 << 20) ? -1 : hsa_linear_tile((int)segs.size(), segs.data(), (int)K, contract, type_code(like));
+}
+void launch_products(const std::vector<hsa_linear_segment> &segs, const Tensor &like, int64_t K, bool contract, int tile) {
     c10::DeviceGuard guard(like.device());
     check(hsa_linear((int)segs.size(), segs.data(), (int)K, contract, tile, type_code(like), stream_of(like)), "hsa_linear");
-    return true;
 }
 
 // x w^T + b, or x w with `contract`, without autograd: on this library's kernels where they are the faster
 // ones, else by torch
-Tensor project(const Tensor &x, const Tensor &w, const std::optional<Tensor> &b_, bool contract, bool few) {
+Tensor project(const Tensor &x, const Tensor &w, const std::optional<Tensor> &b_, bool contract) {
     const Tensor b = b_ ? *b_ : Tensor();
     if (projectable(x, w, b, contract)) {
-        std::vector<int64_t> size = x.sizes().vec();
-        size.back() = w.size(contract ? 1 : 0);
-        Tensor out = at::empty(size, x.options());
-        if (projected({flat_rows(x, w, b, out)}, x, x.size(-1), contract, few)) return out;
+        const int64_t K = x.size(-1), N = w.size(contract ? 1 : 0), rows = x.numel() / K;
+        const auto result = [&] {
+            std::vector<int64_t> size = x.sizes().vec();
+            size.back() = N;
+            return at::empty(size, x.options());
+        };
+        // (the choice does not depend on where the result will lie: a tensor of its own begins aligned)
+        std::vector<hsa_linear_segment> segs = {flat_rows(x, w, b, x, N)};
+        const int tile = tile_for(segs, x, K, contract);
+        if (tile >= 0) {
+            Tensor out = result();
+            segs[0].out = out.data_ptr();
+            launch_products(segs, x, K, contract, tile);
+            return out;
+        }
+        if (contract && !b.defined() && K >= 1024 && rows < INT32_MAX && K < INT32_MAX && N < INT32_MAX && N % 8 == 0 &&
+            aligned16(w) && hsa_linear_long_pays((int)rows, (int)N, (int)K, type_code(x))) {
+            Tensor out = result(), ws = workspace(x, hsa_linear_long_workspace_bytes((int)rows, (int)N, (int)K, type_code(x)));
+            c10::DeviceGuard guard(x.device());
+            check(hsa_linear_long(x.data_ptr(), K, w.data_ptr(), N, out.data_ptr(), N, (int)rows, (int)N, (int)K, ws.data_ptr(),
+                                  ws.nbytes(), type_code(x), stream_of(x)),
+                  "hsa_linear_long");
+            return out;
+        }
     }
     return contract ? at::matmul(x, w) : at::linear(x, w, b_);
 }
 
 // The same of several (x, w), all without bias, in one launch where that pays.
 variable_list project_all(const std::vector<std::pair<Tensor, Tensor>> &parts, bool contract) {
+    const Tensor &like = parts[0].first;
+    const int64_t K = like.size(-1);
     std::vector<hsa_linear_segment> segs;
-    variable_list out;
     for (const auto &[x, w] : parts) {
-        if (parts.size() > HSA_LINEAR_MAX_SEGMENTS || !projectable(x, w, Tensor(), contract) || x.size(-1) != parts[0].first.size(-1) ||
-            !same_kind(x, parts[0].first))
+        if (parts.size() > HSA_LINEAR_MAX_SEGMENTS || !projectable(x, w, Tensor(), contract) || x.size(-1) != K || !same_kind(x, like))
             break;
-        std::vector<int64_t> size = x.sizes().vec();
-        size.back() = w.size(contract ? 1 : 0);
-        out.push_back(at::empty(size, x.options()));
-        segs.push_back(flat_rows(x, w, Tensor(), out.back()));
+        segs.push_back(flat_rows(x, w, Tensor(), x, w.size(contract ? 1 : 0)));
     }
-    if (segs.size() == parts.size() && projected(segs, parts[0].first, parts[0].first.size(-1), contract, false)) return out;
-    out.clear();
-    for (const auto &[x, w] : parts) out.push_back(project(x, w, std::nullopt, contract, false));
+    const int tile = segs.size() == parts.size() ? tile_for(segs, like, K, contract) : -1;
+    variable_list out;
+    for (size_t i = 0; i < parts.size(); ++i) {
+        const auto &[x, w] = parts[i];
+        if (tile < 0) {
+            out.push_back(project(x, w, std::nullopt, contract));
+            continue;
+        }
+        std::vector<int64_t> size = x.sizes().vec();
+        size.back() = segs[i].cols;
+        out.push_back(at::empty(size, x.options()));
+        segs[i].out = out.back().data_ptr();
+    }
+    if (tile >= 0) launch_products(segs, like, K, contract, tile);
     return out;
 }
 
@@ -410,6 +436,9 @@ std::optional<std::pair<Tensor, Tensor>> weight_grad(const Segments &segs, int64
     return std::make_pair(dw, db);
 }
 
+// whether a weight's gradient is small enough for the split-rows kernel to be the faster one
+bool small_result(const Tensor &w) { return ((w.size(0) + 127) / 128) * ((w.size(1) + 127) / 128) <= 256; }
+
 // A tensor that a node keeps for its backward without an edge of its own to it.
 struct Kept {
     Tensor t;
@@ -425,7 +454,7 @@ struct Linear : public torch::autograd::Function<Linear> {
         ctx->save_for_backward({x, w.t});
         ctx->saved_data["bias"] = bias.has_value();
         ctx->saved_data["type"] = (int64_t)weight.scalar_type();
-        return project(x, w.t, b, false, false);
+        return project(x, w.t, b, false);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const variable_list saved = ctx->get_saved_variables();
@@ -436,9 +465,9 @@ struct Linear : public torch::autograd::Function<Linear> {
         Tensor dx, dw, db;
         if (!g.defined()) return {dx, dw, db, Tensor(), Tensor()};
         const Tensor g2 = g.reshape({-1, g.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
-        if (ctx->needs_input_grad(0)) dx = composed(grads) ? at::matmul(g, w) : project(g.contiguous(), w, std::nullopt, true, false);
+        if (ctx->needs_input_grad(0)) dx = composed(grads) ? at::matmul(g, w) : project(g.contiguous(), w, std::nullopt, true);
         const bool need_w = ctx->needs_input_grad(1), need_b = bias && ctx->needs_input_grad(2);
-        if (need_w && !composed(grads)) {
+        if (need_w && !composed(grads) && small_result(w)) {
             if (auto r = weight_grad({{g2, x2, 0}}, w.size(0), type, need_b)) {
                 dw = r->first;
                 db = r->second;
@@ -451,15 +480,16 @@ struct Linear : public torch::autograd::Function<Linear> {
 };
 
 // F.linear(x, weight, bias) under the current autocast state; nullopt where nothing is to be gained
-// (types other than the 16-bit ones; in training no gradient of the weight or a result large enough to fill
-// the chip by itself) or where the call is not a plain one
-std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias) {
+// (types other than the 16-bit ones; in training no gradient of the weight or, unless `wide`, a result large
+// enough to fill the chip by itself) or where the call is not a plain one.  wide: a vocabulary projection, whose
+// input gradient is the long contraction.
+std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias, bool wide) {
     if (!x.is_cuda() || x.dim() < 2 || weight.dim() != 2 || x.numel() == 0 || x.size(-1) != weight.size(1) ||
         x.device() != weight.device() || !weight.is_contiguous())
         return std::nullopt;
     const bool train = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || (bias && bias->requires_grad()));
     const int64_t O = weight.size(0), I = weight.size(1);
-    if (train && (!weight.requires_grad() || O % 8 || I % 8 || ((O + 127) / 128) * ((I + 127) / 128) > 256)) return std::nullopt;
+    if (train && (!weight.requires_grad() || (!wide && (O % 8 || I % 8 || !small_result(weight))))) return std::nullopt;
     if (bias && (bias->dim() != 1 || bias->size(0) != O || !same_kind(weight, *bias))) return std::nullopt;
     if (!ordinary({&x, &weight}) || (bias && !ordinary({&*bias}))) return std::nullopt;
     const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
@@ -469,7 +499,7 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     if (cast && ((weight.scalar_type() != at::kFloat && weight.scalar_type() != type) || type_code(x) < 0)) return std::nullopt;
     auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(type, t, at::kCUDA) : t; };
     const Kept w{as(weight)};
-    if (!train) return project(as(x), w.t, bias ? std::optional<Tensor>(as(*bias)) : std::nullopt, false, true);
+    if (!train) return project(as(x), w.t, bias ? std::optional<Tensor>(as(*bias)) : std::nullopt, false);
     const std::optional<Tensor> b = bias ? std::optional<Tensor>(as(*bias).detach()) : std::nullopt;
     return Linear::apply(as(x), weight, bias, w, b);
 }
@@ -640,7 +670,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value(const Tensor &
     if (N + M > (1 << 28) || B > (1 << 24)) return std::nullopt;
     Tensor q = at::empty({B, N, O}, x.options()), k = at::empty({B, N + M, O}, x.options()), v = at::empty_like(k);
     const auto rows = [&](const Tensor &in, const Tensor &w, const Tensor &out, int64_t first) {
-        hsa_linear_segment s = flat_rows(in, w, Tensor(), out);
+        hsa_linear_segment s = flat_rows(in, w, Tensor(), out, O);
         s.out = (char *)s.out + first * O * out.element_size();
         s.batches = (int)B;
         s.rows = (int)in.size(1);
@@ -648,8 +678,11 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value(const Tensor &
         s.batch_out = out.stride(0);
         return s;
     };
-    if (!projected({rows(x, wq, q, 0), rows(x, wk, k, 0), rows(x, wv, v, 0), rows(y, wk, k, N), rows(y, wv, v, N)}, x, x.size(2), false, true))
-        return std::nullopt;
+    const std::vector<hsa_linear_segment> segs = {rows(x, wq, q, 0), rows(x, wk, k, 0), rows(x, wv, v, 0), rows(y, wk, k, N),
+                                                  rows(y, wv, v, N)};
+    const int tile = tile_for(segs, x, x.size(2), false);
+    if (tile < 0) return std::nullopt;
+    launch_products(segs, x, x.size(2), false, tile);
     return std::make_tuple(q, k, v);
 }
 

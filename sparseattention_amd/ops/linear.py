@@ -23,13 +23,14 @@ def _plain(layer) -> bool:
     return plain_module(layer, nn.Linear)
 
 
-def linear(layer, x: torch.Tensor) -> torch.Tensor:
+def linear(layer, x: torch.Tensor, wide: bool = False) -> torch.Tensor:
     """layer(x).  On the GPU with 16-bit activations (or under autocast to such a type) the product runs on this
     package's kernels where they are the faster ones (csrc/hsa_linear.hip), and in training the backward
     computes the weight's and the bias's gradient in one contraction over the tokens (csrc/hsa_weight_grad.hip),
-    directly in the parameters' type; everything else is the layer itself."""
+    directly in the parameters' type; everything else is the layer itself.  wide: a vocabulary projection, whose
+    input gradient is a product with a long contraction (csrc/hsa_linear_long.hip)."""
     if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer):
-        y = _lib.ext().linear(x, layer.weight, layer.bias)
+        y = _lib.ext().linear(x, layer.weight, layer.bias, wide)
         if y is not None:
             return y
     return layer(x)

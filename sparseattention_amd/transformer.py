@@ -151,7 +151,7 @@ class TransformerLM(nn.Module):
             nx, ny = layer_norm(x, layers[0].norm1), layer_norm(y, layers[0].norm_y)
             for layer, following in zip(layers, layers[1:] + [None]):
                 x, y, nx, ny = layer._chained(x, y, nx, ny, mask, following)
-            return linear(self.fc_out, x)
+            return linear(self.fc_out, x, wide=True)
         for layer in layers:
             if return_attention:
                 x, y, _ = layer(x, y, mask=mask, return_attention=True)

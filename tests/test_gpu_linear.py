@@ -169,3 +169,54 @@ def test_replays_of_a_graph_with_projections():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(outs[0], linear(layer, small)) and torch.equal(outs[1], linear(layer, large))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 128), (257, 264, 129), (300, 512, 1001), (511, 1000, 777), (256, 256, 16385)])
+def test_long_contraction_against_fp64(dtype, M, N, K):
+    """Parts of the contraction that end within a step, rows that begin at any element, tiles flush with the end.
+    What lies behind a row's end and behind the weight's last row is not read as a number."""
+    g = torch.Generator(DEV).manual_seed(K)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
+    x, w = mk(M, K + 5), mk(K + 64, N)
+    x[:, 0], x[:, K + 1:] = float("nan"), float("nan")
+    w[K:] = float("inf")
+    x, w = x[:, 1:K + 1], w[:K]
+    lib, code = _lib.lib(), 1 if dtype == torch.float16 else 2
+    ws = torch.empty(lib.hsa_linear_long_workspace_bytes(M, N, K, code) // 4, device=DEV)
+    out = torch.empty(M, N + 8, device=DEV, dtype=dtype)[:, :N]
+    args = (x.data_ptr(), K + 5, w.data_ptr(), N, out.data_ptr(), N + 8, M, N, K, ws.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib.hsa_linear_long(*args, ws.numel() * 4, code, stream), "hsa_linear_long")
+    ref = x.double() @ w.double()
+    assert bool(((out.double() - ref).abs() <= _bound(x, w, ref, dtype)).all())
+    with pytest.raises(_lib.HsaError):
+        _lib.check(lib.hsa_linear_long(*args, ws.numel() * 4 - 4, code, stream), "hsa_linear_long")
+
+
+@pytest.mark.parametrize("vocab", [50257, 5120])
+def test_vocabulary_projection_in_training(vocab):
+    """Forward and all three gradients against fp64, and a second derivative against the layer's own."""
+    torch.manual_seed(0)
+    layer = nn.Linear(256, vocab).to(DEV, torch.bfloat16)
+    x = torch.randn(2, 512, 256, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    y = linear(layer, x, wide=True)
+    w, b = layer.weight.detach(), layer.bias.detach()
+    assert bool(((y.double() - (x.double() @ w.double().t() + b.double())).abs() <= _bound(x.detach(), w.t(), y.detach().double(), torch.bfloat16)).all())
+    dy = torch.randn_like(y)
+    y.backward(dy)
+    g, r = dy.reshape(-1, vocab), x.detach().reshape(-1, 256)
+    want = g.double() @ w.double()
+    assert bool(((x.grad.reshape(-1, 256).double() - want).abs() <= _bound(g, w, want, torch.bfloat16)).all())
+    want = g.double().t() @ r.double()
+    assert bool(((layer.weight.grad.double() - want).abs() <= _bound(g.t(), r, want, torch.bfloat16)).all())
+    want = g.double().sum(0)
+    assert bool(((layer.bias.grad.double() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 1024 * 2.0 ** -23 * g.double().abs().sum(0)).all())
+    second = []
+    for f in (lambda: linear(layer, x, wide=True), lambda: layer(x)):
+        x.grad = None
+        d, = torch.autograd.grad(f().float().square().mean(), x, create_graph=True)
+        d.float().square().mean().backward()
+        second.append(x.grad.float())
+    # bf16 on both sides, two products deep: a hundredth of the norm
+    assert float((second[0] - second[1]).norm()) <= 0.01 * float(second[1].norm()) and float(second[1].norm()) > 0

@@ -650,40 +650,127 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value_rows(const Ten
 }
 
 // The same without autograd: the rows stay where they are, every projection writes its part of the results, in one
-// launch.  nullopt where that does not pay.
-std::optional<std::tuple<Tensor, Tensor, Tensor>> query_key_value(const Tensor &x_, const Tensor &y_, const Tensor &weight_q,
-                                                                  const Tensor &weight_k, const Tensor &weight_v) {
-    if (!x_.is_cuda()) return std::nullopt;
-    if (at::GradMode::is_enabled())
-        for (const Tensor *t : {&x_, &y_, &weight_q, &weight_k, &weight_v})
-            if (t->requires_grad()) return std::nullopt;
-    const std::optional<at::ScalarType> type = rows_type(x_, y_, weight_q, weight_k, weight_v);
-    if (!type) return std::nullopt;
-    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
-    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(*type, t, at::kCUDA) : t; };
-    const Tensor x = x_.to(*type).contiguous(), y = y_.to(*type).contiguous();
-    const Tensor wq = as(weight_q), wk = as(weight_k), wv = as(weight_v);
+// launch.  rows_plan: the products (their results to be filled in) and their tile, -1 where that does not pay; it
+// depends on sizes and strides only.
+using Three = std::optional<std::tuple<Tensor, Tensor, Tensor>>;
+std::pair<std::vector<hsa_linear_segment>, int> rows_plan(const Tensor &x, const Tensor &y, const Tensor &wq, const Tensor &wk,
+                                                          const Tensor &wv) {
     if (!projectable(x, wq, Tensor(), false) || !projectable(x, wk, Tensor(), false) || !projectable(x, wv, Tensor(), false) ||
         !projectable(y, wk, Tensor(), false))
-        return std::nullopt;
+        return {{}, -1};
     const int64_t B = x.size(0), N = x.size(1), M = y.size(1), O = wk.size(0);
-    if (N + M > (1 << 28) || B > (1 << 24)) return std::nullopt;
-    Tensor q = at::empty({B, N, O}, x.options()), k = at::empty({B, N + M, O}, x.options()), v = at::empty_like(k);
-    const auto rows = [&](const Tensor &in, const Tensor &w, const Tensor &out, int64_t first) {
-        hsa_linear_segment s = flat_rows(in, w, Tensor(), out, O);
-        s.out = (char *)s.out + first * O * out.element_size();
+    if (N + M > (1 << 28) || B > (1 << 24)) return {{}, -1};
+    const auto rows = [&](const Tensor &in, const Tensor &w, int64_t out_rows) {
+        hsa_linear_segment s = flat_rows(in, w, Tensor(), in, O);
         s.batches = (int)B;
         s.rows = (int)in.size(1);
         s.batch_x = in.stride(0);
-        s.batch_out = out.stride(0);
+        s.batch_out = out_rows * O;
         return s;
     };
-    const std::vector<hsa_linear_segment> segs = {rows(x, wq, q, 0), rows(x, wk, k, 0), rows(x, wv, v, 0), rows(y, wk, k, N),
-                                                  rows(y, wv, v, N)};
-    const int tile = tile_for(segs, x, x.size(2), false);
+    std::vector<hsa_linear_segment> segs = {rows(x, wq, N), rows(x, wk, N + M), rows(x, wv, N + M), rows(y, wk, N + M), rows(y, wv, N + M)};
+    const int tile = O % 8 ? -1 : tile_for(segs, x, x.size(2), false);
+    return {std::move(segs), tile};
+}
+Three query_key_value_plain(const Tensor &x, const Tensor &y, const Tensor &wq, const Tensor &wk, const Tensor &wv) {
+    auto [segs, tile] = rows_plan(x, y, wq, wk, wv);
     if (tile < 0) return std::nullopt;
+    const int64_t B = x.size(0), N = x.size(1), M = y.size(1), O = wk.size(0);
+    Tensor q = at::empty({B, N, O}, x.options()), k = at::empty({B, N + M, O}, x.options()), v = at::empty_like(k);
+    const int64_t nodes = N * O * q.element_size();
+    segs[0].out = q.data_ptr();
+    segs[1].out = k.data_ptr();
+    segs[2].out = v.data_ptr();
+    segs[3].out = (char *)k.data_ptr() + nodes;
+    segs[4].out = (char *)v.data_ptr() + nodes;
     launch_products(segs, x, x.size(2), false, tile);
     return std::make_tuple(q, k, v);
+}
+
+Three query_key_value(const Tensor &x, const Tensor &y, const Tensor &weight_q, const Tensor &weight_k, const Tensor &weight_v) {
+    if (!x.is_cuda()) return std::nullopt;
+    if (at::GradMode::is_enabled())
+        for (const Tensor *t : {&x, &y, &weight_q, &weight_k, &weight_v})
+            if (t->requires_grad()) return std::nullopt;
+    const std::optional<at::ScalarType> type = rows_type(x, y, weight_q, weight_k, weight_v);
+    if (!type) return std::nullopt;
+    const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    auto as = [&](const Tensor &t) { return cast ? at::autocast::cached_cast(*type, t, at::kCUDA) : t; };
+    return query_key_value_plain(x.to(*type).contiguous(), y.to(*type).contiguous(), as(weight_q), as(weight_k), as(weight_v));
+}
+
+// ------------------------------------------------------------------------------- one layer of the model
+// A decoder layer without autograd, dropout and autocast on 16-bit tensors, launch for launch what the Python
+// layer does: a short sequence's layer is 15 to 25 launches of a few us each, and through Python they take
+// 170 us to enqueue (six layers of B1 N256: 1056 us a forward against 700 us of kernels).
+//   x [B, N, C], y [B, N-1, C], nx = norm1(x), ny = norm_y(y); p: the parameters in the order of LayerParams
+// Returns x, y and, with `following`, the next layer's norms of them; nullopt before anything is launched where
+// the layer is not of this kind.
+enum LayerParams { W_QKV_Y, W_KV_Y_PACKED, OUT_Y_W, OUT_Y_B, Q_X, K_X, V_X, OUT_X_W, OUT_X_B, NORM2_W, NORM2_B, FC1_W, FC1_B,
+                   FC2_W, FC2_B, NORM_Y_W, NORM_Y_B, NORM1_W, NORM1_B };
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> decoder_layer(const Tensor &x, const Tensor &y, const Tensor &nx, const Tensor &ny,
+                                                                        const std::vector<Tensor> &p, const std::vector<double> &eps,
+                                                                        int64_t heads, int64_t window, bool causal, bool gelu,
+                                                                        bool following) {
+    if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || !x.is_cuda() || x.dim() != 3 || x.numel() == 0 ||
+        (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) || p.size() != (following ? NORM1_B + 1 : NORM_Y_W) ||
+        eps.size() != 3 || heads < 1 || window < 0 || window > (1 << 20))
+        return std::nullopt;
+    const int64_t B = x.size(0), N = x.size(1), C = x.size(2);
+    if (B > (1 << 20) || N < 2 || N > (1 << 24) || log2_exact(N) < 0 || C % heads || C > (1 << 16)) return std::nullopt;
+    const int H = (int)heads, Dh = (int)(C / heads), code = type_code(x);
+    // the whole span-node update as one chain of fused levels, the norms on their kernel
+    if (hsa_cross_update_level_rows((int)B, H, Dh, code) < N || !hsa_add_layer_norm_ok((int)C, code)) return std::nullopt;
+    if (!ordinary({&x, &y, &nx, &ny})) return std::nullopt;
+    for (const Tensor *t : {&x, &y, &nx, &ny})
+        if (!same_kind(x, *t) || t->dim() != 3 || !t->is_contiguous() || !aligned16(*t)) return std::nullopt;
+    if (nx.sizes() != x.sizes() || y.size(0) != B || y.size(1) != N - 1 || y.size(2) != C || ny.sizes() != y.sizes()) return std::nullopt;
+    for (const Tensor &t : p)
+        if (!ordinary({&t}) || !same_kind(x, t) || !t.is_contiguous() || !aligned16(t)) return std::nullopt;
+    const int64_t F = p[FC1_W].size(0);
+    const auto matrix = [&](int i, int64_t rows, int64_t cols) { return p[i].dim() == 2 && p[i].size(0) == rows && p[i].size(1) == cols; };
+    const auto row = [&](int i, int64_t n) { return p[i].dim() == 1 && p[i].size(0) == n; };
+    if (!matrix(W_QKV_Y, 3 * C, C) || p[W_KV_Y_PACKED].numel() != 2 * C * C || !matrix(OUT_Y_W, C, C) || !row(OUT_Y_B, C) ||
+        !matrix(Q_X, C, C) || !matrix(K_X, C, C) || !matrix(V_X, C, C) || !matrix(OUT_X_W, C, C) || !row(OUT_X_B, C) ||
+        !row(NORM2_W, C) || !row(NORM2_B, C) || p[FC1_W].dim() != 2 || !matrix(FC1_W, F, C) || !row(FC1_B, F) || !matrix(FC2_W, C, F) ||
+        !row(FC2_B, C))
+        return std::nullopt;
+    for (int i = NORM_Y_W; following && i <= NORM1_B; ++i)
+        if (!row(i, C)) return std::nullopt;
+    // (larger inputs whose rows' products do not go into one launch: the Python layer has a way without the copy)
+    if (B * N * C >= 1 << 20 && rows_plan(nx, y, p[Q_X], p[K_X], p[V_X]).second < 0) return std::nullopt;
+
+    c10::DeviceGuard guard(x.device());
+    // span nodes: the three projections, every level of the tree, the output projection, the residual
+    const Tensor qkv = project(ny, p[W_QKV_Y], std::nullopt, false);
+    Tensor nodes = at::empty({B, N - 1, C}, x.options());
+    check(hsa_cross_update_top_fwd(x.data_ptr(), qkv.data_ptr(), p[W_KV_Y_PACKED].data_ptr(), nodes.data_ptr(), (int)B, (int)N, H, Dh, 0,
+                                   (N - 1) * 3 * C, 3 * C, (N - 1) * C, C, code, stream_of(x)),
+          "hsa_cross_update_top_fwd");
+    const Tensor u = project(nodes, p[OUT_Y_W], p[OUT_Y_B], false);
+    Tensor y2, ny2;
+    if (following) std::tie(y2, ny2) = add_norm_plain(y, u, p[NORM_Y_W], p[NORM_Y_B], eps[1], Tensor());
+    else y2 = at::add(y, u);
+    // leaves: queries, keys and values of leaves and nodes, the attention, the output projection, the residual
+    Tensor q, k, v;
+    if (const Three r = query_key_value_plain(nx, y2, p[Q_X], p[K_X], p[V_X])) {
+        std::tie(q, k, v) = *r;
+    } else {
+        q = project(nx, p[Q_X], std::nullopt, false);
+        const Tensor xy = at::cat({nx, y2}, 1);
+        k = project(xy, p[K_X], std::nullopt, false);
+        v = project(xy, p[V_X], std::nullopt, false);
+    }
+    const auto split = [&](const Tensor &t) { return t.view({B, t.size(1), heads, Dh}); };
+    const Tensor a = attention_plain(split(q), split(k), split(v), causal, (int)window).view({B, N, C});
+    const Tensor o = project(a, p[OUT_X_W], p[OUT_X_B], false);
+    auto [x2, n2] = add_norm_plain(x, o, p[NORM2_W], p[NORM2_B], eps[0], Tensor());
+    // feed-forward
+    const Tensor hidden = project(n2, p[FC1_W], p[FC1_B], false);
+    const Tensor f = project(gelu ? at::gelu(hidden) : at::relu(hidden), p[FC2_W], p[FC2_B], false);
+    if (!following) return std::make_tuple(at::add(x2, f), y2, Tensor(), Tensor());
+    auto [x3, nx3] = add_norm_plain(x2, f, p[NORM1_W], p[NORM1_B], eps[2], Tensor());
+    return std::make_tuple(x3, y2, nx3, ny2);
 }
 
 }  // namespace
@@ -704,4 +791,5 @@ PYBIND11_MODULE(_hsa_torch, m) {
     m.def("weight_grad", &weight_grad);
     m.def("query_key_value_rows", &query_key_value_rows);
     m.def("query_key_value", &query_key_value);
+    m.def("decoder_layer", &decoder_layer);
 }

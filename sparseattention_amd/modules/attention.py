@@ -148,6 +148,20 @@ class HierarchicalAttention(nn.Module):
             self._fused[name] = hit
         return hit[1]
 
+    def _chain_weights(self, x: torch.Tensor):
+        """(q | k | v, packed k / v) weights of the span nodes' update of leaves x as one chain of fused levels in
+        x's type, or None where that does not apply."""
+        if x.dtype not in (torch.float16, torch.bfloat16) or x.dim() != 3:
+            return None
+        layers = [self._modules[n] for n in ("Wq_y", "Wk_y", "Wv_y")]
+        if any(m._parameters["weight"].dtype != x.dtype or m._parameters["weight"].device != x.device for m in layers):
+            return None
+        if _lib.lib().hsa_cross_update_level_rows(x.shape[0], self.num_heads, self.head_dim, _lib.dtype_code(x)) < x.shape[1]:
+            return None
+        with _lib.on_device(x):
+            return (self._fused_weight("qkv_y", layers, x.dtype),
+                    self._fused_weight("kv_y_packed", layers[1:], x.dtype, packed=True))
+
     @staticmethod
     def _compute_dtype(t: torch.Tensor) -> torch.dtype:
         """Element type the projections produce: the autocast type inside `torch.autocast` (the

@@ -18,6 +18,20 @@ def plain_module(module, cls) -> bool:
                      or _module._global_backward_hooks or _module._global_backward_pre_hooks))
 
 
+def all_plain(modules) -> bool:
+    """plain_module(m, cls) for every (m, cls): one look at the global hooks, the modules' attributes straight
+    from their dictionaries."""
+    if (_module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
+            or _module._global_backward_pre_hooks):
+        return False
+    for m, cls in modules:
+        d = m.__dict__
+        if (type(m) is not cls or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                or d["_backward_pre_hooks"]):
+            return False
+    return True
+
+
 def _plain(layer) -> bool:
     """An nn.Linear that may be bypassed."""
     return plain_module(layer, nn.Linear)

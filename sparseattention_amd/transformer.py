@@ -17,8 +17,9 @@ import torch.nn.functional as F
 
 from . import _lib
 from .modules import HierarchicalAttention
+from .modules import attention as _attention
 from .ops import generate_span_input_Y
-from .ops.linear import linear, plain_module
+from .ops.linear import all_plain, linear, plain_module
 
 
 def _plain_norm(m) -> bool:
@@ -45,6 +46,18 @@ def add_layer_norm(x, branch, norm):
             return r
     x = x + branch
     return x, norm(x)
+
+
+# what the native layer stands in for, as it is when this module is loaded
+_STEPS = tuple((n, getattr(HierarchicalAttention, n)) for n in ("forward", "cross_update_Y", "update_X_from_Y", "_span_levels",
+                                                                "_fused_weight"))
+_ATTENTION = _attention.hierarchical_attention
+
+
+def _own_steps(att) -> bool:
+    """Nobody has replaced the attention's steps, on the class, on the instance or in its module."""
+    return (all(getattr(HierarchicalAttention, n) is f and n not in att.__dict__ for n, f in _STEPS)
+            and _attention.hierarchical_attention is _ATTENTION)
 
 
 class PositionwiseFeedForward(nn.Module):
@@ -111,6 +124,44 @@ class DecoderLayer(nn.Module):
         x, nx = (x + f, None) if following is None else add_layer_norm(x, f, following.norm1)
         return x, y, nx, ny
 
+    def _native(self, x, y, nx, ny, mask, following=None):
+        """`_chained` without autograd as one native call (csrc/torch_ops.cpp), launch for launch the same; None
+        where something may watch or replace one of its steps, or where the call does not take the layer."""
+        if torch.is_grad_enabled() or not x.is_cuda or torch.compiler.is_compiling():
+            return None
+        sub = self._modules
+        att, ff = sub["self_attn"], sub["feed_forward"]
+        a, f = att._modules, ff._modules
+        drops = (sub["dropout"], a["dropout"], f["dropout"])
+        norms = [sub["norm2"]]
+        if following is not None:
+            norms += [following._modules["norm_y"], following._modules["norm1"]]
+        linears = [a[n] for n in ("out_proj_y", "Wq_x", "Wk_x", "Wv_x", "out_proj_x")] + [f["fc1"], f["fc2"]]
+        if not all_plain([(att, HierarchicalAttention), (ff, PositionwiseFeedForward)] + [(m, nn.Dropout) for m in drops]
+                         + [(m, nn.LayerNorm) for m in norms] + [(m, nn.Linear) for m in linears]):
+            return None
+        if any(m.training and m.p > 0 for m in drops) or not att.fuse_top_levels or not _own_steps(att):
+            return None
+        if ff.activation is not F.gelu and ff.activation is not F.relu:
+            return None
+        w = [m._parameters["weight"] for m in linears]
+        b = [m._parameters["bias"] for m in linears]
+        n = [p for m in norms for p in (m._parameters["weight"], m._parameters["bias"])]
+        if any(t is None for t in n) or any(len(m.normalized_shape) != 1 for m in norms):
+            return None
+        if any((t is None) != (i in (1, 2, 3)) for i, t in enumerate(b)):
+            return None
+        if any(type(t) is not nn.Parameter for t in w + n) or any(type(a[m]._parameters["weight"]) is not nn.Parameter
+                                                                  for m in ("Wq_y", "Wk_y", "Wv_y")):
+            return None
+        packed, dt = att._chain_weights(x), x.dtype
+        if packed is None or any(t.dtype != dt for t in w + n):
+            return None
+        params = [*packed, w[0], b[0], w[1], w[2], w[3], w[4], b[4], n[0], n[1], w[5], b[5], w[6], b[6], *n[2:]]
+        eps = [m.eps for m in norms] + [0.0] * (3 - len(norms))
+        return _lib.ext().decoder_layer(x, y, nx, ny, params, eps, att.num_heads, att.window_size, mask is not None,
+                                        ff.activation is F.gelu, following is not None)
+
     def _may_chain(self) -> bool:
         """Whether `_chained` may stand in for calling the layer."""
         return plain_module(self, DecoderLayer)
@@ -150,7 +201,8 @@ class TransformerLM(nn.Module):
         if layers and not return_attention and all(type(m) is DecoderLayer and m._may_chain() for m in layers):
             nx, ny = layer_norm(x, layers[0].norm1), layer_norm(y, layers[0].norm_y)
             for layer, following in zip(layers, layers[1:] + [None]):
-                x, y, nx, ny = layer._chained(x, y, nx, ny, mask, following)
+                done = layer._native(x, y, nx, ny, mask, following)
+                x, y, nx, ny = layer._chained(x, y, nx, ny, mask, following) if done is None else done
             return linear(self.fc_out, x, wide=True)
         for layer in layers:
             if return_attention:

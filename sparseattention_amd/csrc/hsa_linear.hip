@@ -21,12 +21,15 @@
 //
 // Results whose rows begin at any element (a vocabulary of odd size): a line that two tiles share costs more
 // than the line.  With rows enough, a tile takes every 64th row: their results lie alike in their lines, so the
-// tiles' columns can begin where the lines do (32768 x 50257 x 512: 1865 us; the library 2200).  Else the rows go
+// tiles' columns can begin where the lines do (32768 x 50257 x 512: 1740 to 1800 us; the library 2200).  Else the rows go
 // through the LDS and are stored as 16-byte pieces where they lie (4096 x 50257 x 512: 283 us; 330 as they come,
 // the library 349).
 //
+// The transfers of a stage are requested one by one between the products of a half step: together, behind the
+// barrier, they hold up all wavefronts at once (32768 x 2048 x 512: 73.3 -> 70.2 us, 16376 x 768 x 2304 55.7 -> 50.0).
+//
 // Bound: the matrix cores (1.4 PFLOP/s in the steps) and, not overlapped with them, the stores of the results
-// at the rate of the memory (32768 x 2048 x 512: 66 us, 50 without stores).  Slower: two workgroups of 128 x 256 on
+// at the rate of the memory (a third of the time at 32768 x 2048 x 512).  Slower: two workgroups of 128 x 256 on
 // a CU, whose stores would overlap (82 us); four wavefronts for the transfers alone, so that none waits for
 // its stores (72); starts spread over a tile's time (66).
 #include "hsa_lds_dma.h"
@@ -55,47 +58,18 @@ struct LnArgs {
     int nseg, K, tiles, group;
 };
 
-// Q transfers of 1 KiB, the rows of each `step` bytes behind those of the one before, to consecutive LDS addresses
-template <int Q>
-__device__ __forceinline__ void lds_dma16_rows(const char *base, long step, const uint32_t (&off)[Q], uint32_t lds) {
-    static_assert(Q == 3 || Q == 4);
+// one transfer of 1 KiB: a scalar base and 32-bit offsets per lane
+__device__ __forceinline__ void lds_dma16_from(const char *base, uint32_t off, uint32_t lds) {
     uint32_t keep;
-    const char *b1 = base + step, *b2 = b1 + step, *b3 = b2 + step;
-    if constexpr (Q == 4)
-        asm volatile(
-            "s_mov_b32 %0, m0\n\t"
-            "s_mov_b32 m0, %9\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %1, %5\n\t"
-            "s_add_u32 m0, m0, 0x400\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %2, %6\n\t"
-            "s_add_u32 m0, m0, 0x400\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %3, %7\n\t"
-            "s_add_u32 m0, m0, 0x400\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %4, %8\n\t"
-            "s_mov_b32 m0, %0"
-            : "=&s"(keep)
-            : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(b1), "s"(b2), "s"(b3), "s"(lds)
-            : "memory", "scc");
-    else
-        asm volatile(
-            "s_mov_b32 %0, m0\n\t"
-            "s_mov_b32 m0, %7\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %1, %4\n\t"
-            "s_add_u32 m0, m0, 0x400\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %2, %5\n\t"
-            "s_add_u32 m0, m0, 0x400\n\t"
-            "s_nop 0\n\t"
-            "global_load_lds_dwordx4 %3, %6\n\t"
-            "s_mov_b32 m0, %0"
-            : "=&s"(keep)
-            : "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(base), "s"(b1), "s"(b2), "s"(lds)
-            : "memory", "scc");
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(off), "s"(base), "s"(lds)
+        : "memory");
 }
 
 // lane l's 2 bytes, as the low half of LDS[lds_base + 4 l]
@@ -172,8 +146,12 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
 
     // ---- transfers.  X: rows 32 w + 8 q + lane / 8, piece lane & 7 of 8.  W likewise (8 QW w + ..), or, TW,
     // rows of the contraction: pieces (w QW + q) 64 + lane of rows of BN / 8.
+    // (offsets per lane that differ otherwise than by whole rows: X and W two each; at TW and 192 columns all three)
+    constexpr int W_OFFSETS = TW && BN == 192 ? 3 : 2;
+    constexpr auto w_kind = [](int q) { return TW && BN == 192 ? q : TW && BN == 128 ? q >> 1 : q & 1; };
+    constexpr auto w_rows = [](int q) { return !TW ? (q & ~1) * 8 : BN == 192 ? 0 : BN == 128 ? (q & 1) * 4 : (q >> 1) * 4; };
     const int lrow = lane >> 3, lslot = lane & 7;
-    uint32_t off_x[4], off_w[QW];
+    uint32_t off_x[2], off_w[W_OFFSETS];
     long ld_x = 0, ld_w = 0;
     const char *load_x = nullptr, *load_w = nullptr;
     int lt = slot, lk = 0, lbuf = 0;
@@ -185,31 +163,43 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
         load_x = s.x + c.b * s.batch_x + c.m0 * s.ld_x + w * 32 * ld_x;
         load_w = TW ? s.w + 2l * c.n0 : s.w + (long)(c.n0 + w * 8 * QW) * ld_w;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            off_x[q] = (uint32_t)lrow * (uint32_t)ld_x + 16 * (lslot ^ ((lrow >> 1) | ((q & 1) << 2)));
+        for (int q = 0; q < 2; ++q) off_x[q] = (uint32_t)(8 * q + lrow) * (uint32_t)ld_x + 16 * (lslot ^ ((lrow >> 1) | (q << 2)));
 #pragma unroll
-        for (int q = 0; q < QW; ++q) {
+        for (int o = 0; o < W_OFFSETS; ++o) {
             if constexpr (TW) {
-                const int at = (w * QW + q) * 64 + lane, row = at / (BN / 8), piece = at - row * (BN / 8);
+                const int q = BN == 128 ? 2 * o : o, at = (w * QW + q) * 64 + lane, row = at / (BN / 8), piece = at - row * (BN / 8);
                 const int key = BN != 192 ? (row & 3) | ((row & 8) >> 1) : ((row >> 1) & 1) | ((row >> 2) & 2);
-                off_w[q] = (uint32_t)row * (uint32_t)ld_w + 16 * (((piece >> 1) ^ key) << 1 | (piece & 1));
+                off_w[o] = (uint32_t)row * (uint32_t)ld_w + 16 * (((piece >> 1) ^ key) << 1 | (piece & 1));
             } else {
-                off_w[q] = (uint32_t)lrow * (uint32_t)ld_w + 16 * (lslot ^ ((lrow >> 1) | (((w * QW + q) & 1) << 2)));
+                off_w[o] = (uint32_t)(8 * o + lrow) * (uint32_t)ld_w + 16 * (lslot ^ ((lrow >> 1) | (((w * QW + o) & 1) << 2)));
             }
         }
     };
-    auto load = [&]() {
-        if (lt >= count) return;
+    // transfer q of the stage that the cursor is at (4 of X's rows, QW of W's)
+    auto load_one = [&](int q) {
         const uint32_t to = lds0 + lbuf * STAGE;
-        lds_dma16_rows<4>(load_x + 2l * lk, 8 * ld_x, off_x, to + w * 4096);
-        lds_dma16_rows<QW>(TW ? load_w + lk * ld_w : load_w + 2l * lk, TW ? 0 : 8 * ld_w, off_w, to + XB + w * (QW * 1024));
-        lk += LN_STEP;
+        if (q < 4) {
+            lds_dma16_from(load_x + 2l * lk + (q & 2) * 8 * ld_x, off_x[q & 1], to + w * 4096 + q * 1024);
+        } else {
+            const int v = q - 4;
+            lds_dma16_from((TW ? load_w + lk * ld_w : load_w + 2l * lk) + w_rows(v) * ld_w, off_w[w_kind(v)],
+                           to + XB + w * (QW * 1024) + v * 1024);
+        }
+    };
+    auto advance = [&]() {  // (behind the last stage: the last one once more, which nothing reads)
         lbuf ^= 1;
-        if (lk >= p.K) {
+        if (lk + LN_STEP < p.K) {
+            lk += LN_STEP;
+        } else if (lt + slots < count) {
             lk = 0;
             lt += slots;
-            if (lt < count) aim();
+            aim();
         }
+    };
+    auto load = [&]() {
+#pragma unroll
+        for (int q = 0; q < 4 + QW; ++q) load_one(q);
+        advance();
     };
 
     // ---- operands: lane (g, r) holds row r of X's 16, column r of W's, contraction 8 g .. of 32
@@ -241,24 +231,40 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
         }
     };
     f32x4 acc[4][NJ];  // [16 rows][16 columns]: lane (g, r) holds row r, columns 4 g ..
-    // the products of 32 contraction steps while the next operands (half h of `buf`) take the places of those used up
-    auto products = [&](const u32x4_t (&x)[4], int buf, int h, u32x4_t (&next)[4]) {
+    // The products of 32 contraction steps while the next operands (half h of `buf`) take the places of those used up
+    // and, LOAD, the transfers of a stage are requested.
+    auto products = [&](auto LOAD, const u32x4_t (&x)[4], int buf, int h, u32x4_t (&next)[4]) {
         fetch_x(buf, h, next);
+        if constexpr (!LOAD) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
+            for (int j = 0; j < NJ; ++j) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i][j] = Mma<T>::k32(ow[j], x[i], acc[i][j]);
-            fetch_w(buf, h, j);
-        }
-        // (the order written here is the order issued)
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                for (int i = 0; i < 4; ++i) acc[i][j] = Mma<T>::k32(ow[j], x[i], acc[i][j]);
+                fetch_w(buf, h, j);
+            }
+            // (the order written here is the order issued)
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, TW ? 2 : 1, 0);
+            for (int j = 0; j < NJ; ++j) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, TW ? 2 : 1, 0);
+            }
+        } else {
+            // a transfer between products: requested together they would hold up all wavefronts at once
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i][j] = Mma<T>::k32(ow[j], x[i], acc[i][j]);
+                fetch_w(buf, h, j);
+#pragma unroll
+                for (int q = j * (4 + QW) / NJ; q < (j + 1) * (4 + QW) / NJ; ++q) load_one(q);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    const std::integral_constant<bool, true> with_loads;
+    const std::integral_constant<bool, false> without;
 
     // the bias of a tile's columns, one per thread
     auto load_bias = [&](const Tile &c, int to) {
@@ -285,7 +291,7 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < p.K; k += LN_STEP) {
-            products(ox[0], buf, 1, ox[1]);
+            products(without, ox[0], buf, 1, ox[1]);
             // The next stage and the bias are there (the results of the last tile, stored after they were
             // requested, need not be), and, behind the barrier, everybody has read this stage: its place
             // takes the one after next.
@@ -293,10 +299,10 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
             else wait_vmem_all_but<0>();
             stored = false;
             lds_only_barrier();
-            load();
             __builtin_amdgcn_sched_barrier(0);
             buf ^= 1;
-            products(ox[1], buf, 0, ox[0]);  // (behind the last stage: operands that nothing uses)
+            products(with_loads, ox[1], buf, 0, ox[0]);  // (behind the last stage: operands that nothing uses)
+            advance();
         }
         // ---- results
         const LnSeg &s = p.seg[c.seg];
@@ -391,6 +397,7 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
         stored = true;
         which ^= 1;
     }
+    wait_vmem_all_but<0>();  // no transfer outlives the workgroup's LDS
 }
 
 // ---- few rows.  256 x 512 x 512 is a prompt's projection: 0.13 GFLOP, nothing but latency.  A workgroup owns 32 x 32
@@ -553,11 +560,12 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     // Tiles: rounds of the chip times the time of a tile, 256 x 256 as 1 (256 x 192 0.8, two of 128 x 128 on one CU 0.74).
     // The library has the better inner loop from contractions of about 1000 on and with its widest tiles at
     // 768; at 512 and below this kernel is the faster one unless it leaves a good part of the chip idle
-    // (rows x cols x K, us, library / here): 8192 x 1536 x 512 27.9 / 18.9, 16384 x 1536 x 512 40.7 / 32.4, 32768 x 2048
-    // x 512 75 / 68, 4096 x 2048 x 512 15.6 / 15.1, 16384 x 768 x 768 24.2 / 23.7, 32752 x 768 x 768 46.5 / 38.4; not taken:
-    // 4096 x 512 x 512 8.0 / 8.9, 8192 x 768 x 768 15.2 / 17.5, 16384 x 3072 x 768 69 / 76, 16384 x 1024 x 1024 30.5 / 35,
-    // 32768 x 512 x 2048 51 / 56.  Rows that begin anywhere (a vocabulary of 50257): 256 x 50257 x 512 31 / 23,
-    // 4096 349 / 283, 32768 2200 / 1865; 8192 x 50257 x 768 593 / 722.
+    // (rows x cols x K, us, library / here): 8192 x 1536 x 512 27.9 / 18.9, 16384 x 1536 x 512 40.7 / 32, 32768 x 2048
+    // x 512 78 / 70, 4096 x 2048 x 512 15.6 / 15.1, 16384 x 768 x 768 24.2 / 22.8, 32752 x 768 x 768 46.5 / 38; not taken:
+    // 4096 x 512 x 512 8.0 / 8.9, 8192 x 768 x 768 15.2 / 17.5, 16384 x 3072 x 768 69 / 72, 16384 x 1024 x 1024 30.5 / 34,
+    // 32768 x 512 x 2048 50 / 56.  With the weight's rows along the contraction the library is slower: 16384 x 768 x 768
+    // 26.3 / 23.2, x 1536 41.1 / 36.6, x 2304 57.7 / 50.0.  Rows that begin anywhere (a vocabulary of 50257): 256 x 50257 x 512 31 / 23,
+    // 4096 349 / 281, 32768 2200 / 1800; 8192 x 50257 x 768 593 / 722.
     int best = -1;
     double least = 0;
     for (int t = 0; t < 3; ++t) {
@@ -575,7 +583,7 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     }
     if (best < 0) return -1;
     const double used = results / (65536.0 * 256.0) / least;
-    if (K > 768 || used < (K > 512 ? 0.9 : 0.6) || (K > 512 && best != 1)) return -1;
+    if (K > (w_rows_contract ? 2304 : 768) || used < (K > 512 ? 0.9 : 0.6) || (K > 512 && best != 1 && !w_rows_contract)) return -1;
     return best;
 }
 

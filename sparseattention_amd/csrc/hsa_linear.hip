@@ -641,8 +641,10 @@ int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contra
     // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 8 / 32: 2180
     // / 2200 / 2550 us at 32768 x 50257 x 512)
     if (tile == 4 && p.seg[0].period == 1) p.group = 2;
-    // results that the memory-side cache could not hold for the next kernel anyway go past the caches
-    const bool past = bytes > (double)(1 << 28);
+    // large results go past the caches: they would push the operands' rows out of the L2s (4 MiB each) before the
+    // next kernel could find them there (everything above 16 MiB against 256 MiB: a six-layer forward of 32768 tokens
+    // 5727 -> 5678 us, a module in training 1650 -> 1628)
+    const bool past = bytes > (double)(1 << 24);
     const hipStream_t st = (hipStream_t)stream;
     if (tile == 3) {
         if (dtype == HSA_F16) linear_few_rows_kernel<F16><<<p.tiles, 64 * LS_WAVES, 0, st>>>(p);

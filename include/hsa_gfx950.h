@@ -173,7 +173,7 @@ int hsa_build_parents_strided_fwd(const void *qp, const void *kp, const void *vp
  *
  * hsa_cross_update_top_rows returns the largest C the single launch holds for this head layout
  * (0 = not handled: fp32, or a head size other than 32 / 64 / 128, or H*Dh not a multiple of
- * 128); hsa_cross_update_top_fwd returns HSA_ERR_UNSUPPORTED for such shapes, and for a larger C
+ * 64); hsa_cross_update_top_fwd returns HSA_ERR_UNSUPPORTED for such shapes, and for a larger C
  * unless `out` allows the launch per level, which takes any power of two.
  * hsa_cross_update_level_rows returns the C from which on a caller with such an `out` should hand
  * the remaining levels to hsa_cross_update_top_fwd instead of running a GEMM and a parent build

@@ -48,9 +48,9 @@ template <typename T> __device__ __forceinline__ float rounded(float x) {
 // the value columns the output, so only Dh accumulator columns are live at a time.  Row tiles
 // reach past the level's last row when it has fewer than 16*RT children: those lanes re-read the
 // last row, and what they compute belongs to no parent and is dropped.
-// PD = weight k-steps in flight (divides Dm / 32).
+// PD = weight k-steps in flight (divides Dm / 32; TAIL: at most Dm / 32, the last round is shorter).
 // `tile0`: first 16-row tile of the level this call covers (RT tiles from there).
-template <typename T, int CT2, int RT, bool TO_LDS, int PD>
+template <typename T, int CT2, int RT, bool TO_LDS, int PD, bool TAIL = false>
 __device__ __forceinline__ void top_level_head(const TopParams &p, int b, int h, int C, int row,
                                                const unsigned char *cur, unsigned char *nxt, int64_t pitch,
                                                int tile0 = 0) {
@@ -126,16 +126,18 @@ __device__ __forceinline__ void top_level_head(const TopParams &p, int b, int h,
 #pragma unroll
                 for (int ct = 0; ct < CT2; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int u = 0; u < PD; ++u) load_b(u, u);  // NK >= PD (Dm is a multiple of 128)
+            for (int u = 0; u < PD; ++u) load_b(u, u);  // NK >= PD
             __builtin_amdgcn_sched_barrier(0);
-            for (int ks0 = 0; ks0 + PD < NK; ks0 += PD) {
+            int ks0 = 0;
+            for (; ks0 + PD < NK; ks0 += PD) {
 #pragma unroll
-                for (int u = 0; u < PD; ++u) step(u, true);
+                for (int u = 0; u < PD; ++u) step(u, !TAIL || ks0 + PD + u < NK);
                 wp += PD * CT2 * 512;
                 aofs += 64 * PD;
             }
 #pragma unroll
-            for (int u = 0; u < PD; ++u) step(u, false);
+            for (int u = 0; u < PD; ++u)
+                if (!TAIL || ks0 + u < NK) step(u, false);
         };
 
         // ---- keys: the three scores and the softmax weights ----
@@ -218,7 +220,10 @@ __device__ __forceinline__ void top_level(const TopParams &p, int b, int C, int 
                                           unsigned char *nxt, int pitch) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int PD = CT2 >= 8 ? 2 : 4;  // eight wavefronts per workgroup: 256 registers each
-    for (int h = wave; h < p.H; h += TOP_WAVES) top_level_head<T, CT2, RT, true, PD>(p, b, h, C, row, cur, nxt, pitch);
+    for (int h = wave; h < p.H; h += TOP_WAVES) {
+        if (p.Dm % 128 == 0) top_level_head<T, CT2, RT, true, PD>(p, b, h, C, row, cur, nxt, pitch);
+        else top_level_head<T, CT2, RT, true, 2>(p, b, h, C, row, cur, nxt, pitch);
+    }
 }
 
 // One level per launch, one wavefront per (batch element, head): the level's rows are read from
@@ -231,13 +236,13 @@ __device__ __forceinline__ void top_level(const TopParams &p, int b, int C, int 
 // again: the tiles run side by side instead of one wavefront multiplying them in turn.
 // RT = 16-row tiles one wavefront multiplies side by side: with two, a level that would start more
 // wavefronts than the chip has SIMDs streams its weights half as often and runs in one round.
-template <typename T, int CT2, int PD, int RT = 1>
+template <typename T, int CT2, int PD, int RT = 1, bool TAIL = false>
 __global__ void __launch_bounds__(64) cross_update_level_kernel(TopParams p, int C, int row, const uint16_t *lsrc,
                                                                 int64_t lsrc_bs, int64_t lsrc_rs) {
     const int b = blockIdx.x, h = blockIdx.y;
-    top_level_head<T, CT2, RT, false, PD>(p, b, h, C, row,
-                                          reinterpret_cast<const unsigned char *>(lsrc + (size_t)b * lsrc_bs), nullptr,
-                                          lsrc_rs * 2, RT * (int)blockIdx.z);
+    top_level_head<T, CT2, RT, false, PD, TAIL>(p, b, h, C, row,
+                                                reinterpret_cast<const unsigned char *>(lsrc + (size_t)b * lsrc_bs), nullptr,
+                                                lsrc_rs * 2, RT * (int)blockIdx.z);
 }
 
 
@@ -643,7 +648,7 @@ int top_row_tiles(int H, int Dh) {
 bool top_shape_ok(int H, int Dh, int dtype) {
     if (dtype != HSA_F16 && dtype != HSA_BF16) return false;
     if (Dh != 32 && Dh != 64 && Dh != 128) return false;
-    if (H < 1 || ((long)H * Dh) % 128 != 0) return false;
+    if (H < 1 || ((long)H * Dh) % 64 != 0) return false;
     return top_row_tiles(H, Dh) >= 1;
 }
 
@@ -699,7 +704,7 @@ static std::atomic<long> &level_rows_limit() {
 // whether the kernel with the head's weights resident in LDS is built for this head layout
 static bool level_pw_capable(int H, int Dh) {
     const long Dm = (long)H * Dh;
-    return Dh <= 64 && 2 * (Dm / 32) * (Dh / 16) * 1024 <= 128 * 1024;
+    return Dh <= 64 && Dm % 128 == 0 && 2 * (Dm / 32) * (Dh / 16) * 1024 <= 128 * 1024;
 }
 
 constexpr int LEVEL_WG_WAVES = 4;
@@ -781,6 +786,12 @@ int launch_level_wg_any(const TopParams &p, int C, int row, const uint16_t *lsrc
         if (taken || rc != HSA_OK) return rc;
     }
     auto wgs = [&](int rt) { return bh * ((tiles + LEVEL_WG_WAVES * rt - 1) / (LEVEL_WG_WAVES * rt)); };
+    if (NK % 4) {  // (Dm a multiple of 64: heads of up to 64 channels) chunks of two k-steps
+        if constexpr (CT2 <= 4) {
+            if (wgs(2) >= 256) return launch_level_wg<T, CT2, 2, 2>(p, C, row, lsrc, lbs, lrs, st);
+            return launch_level_wg<T, CT2, 1, 2>(p, C, row, lsrc, lbs, lrs, st);
+        }
+    }
     if constexpr (CT2 <= 4) {
         if (wgs(2) >= 512) return launch_level_wg<T, CT2, 2, 4, 2>(p, C, row, lsrc, lbs, lrs, st);
         if (NK % 8 == 0) {
@@ -792,7 +803,7 @@ int launch_level_wg_any(const TopParams &p, int C, int row, const uint16_t *lsrc
     return launch_level_wg<T, CT2, 1, 4>(p, C, row, lsrc, lbs, lrs, st);
 }
 
-template <typename T, int CT2, int PD>
+template <typename T, int CT2, int PD, bool TAIL = false>
 int top_launch_levels_pd(const TopParams &p, hipStream_t st) {
     int C = p.C0, row = 0;
     const uint16_t *lsrc = p.src;
@@ -814,10 +825,10 @@ int top_launch_levels_pd(const TopParams &p, hipStream_t st) {
         // (1024 SIMDs; a lone wavefront's registers hold two tiles' operands up to 64 channels)
         if (CT2 <= 4 && tiles % 2 == 0 && (long)p.B * p.H * tiles >= 2048) {
             const dim3 grid((unsigned)p.B, (unsigned)p.H, (unsigned)(tiles / 2));
-            cross_update_level_kernel<T, CT2, PD, 2><<<grid, 64, 0, st>>>(p, C, row, lsrc, lbs, lrs);
+            cross_update_level_kernel<T, CT2, PD, 2, TAIL><<<grid, 64, 0, st>>>(p, C, row, lsrc, lbs, lrs);
         } else {
             const dim3 grid((unsigned)p.B, (unsigned)p.H, (unsigned)tiles);
-            cross_update_level_kernel<T, CT2, PD><<<grid, 64, 0, st>>>(p, C, row, lsrc, lbs, lrs);
+            cross_update_level_kernel<T, CT2, PD, 1, TAIL><<<grid, 64, 0, st>>>(p, C, row, lsrc, lbs, lrs);
         }
         // the next level's children are the rows just written
         lsrc = p.out + (size_t)row * p.out_rs;
@@ -832,7 +843,11 @@ int top_launch_levels_pd(const TopParams &p, hipStream_t st) {
 template <typename T, int CT2>
 int top_launch_levels(const TopParams &p, hipStream_t st) {
     constexpr int DEEP = CT2 >= 8 ? 4 : 8;
-    if ((p.Dm / 32) % DEEP == 0) return top_launch_levels_pd<T, CT2, DEEP>(p, st);
+    const int NK = p.Dm / 32;
+    if (NK % DEEP == 0) return top_launch_levels_pd<T, CT2, DEEP>(p, st);
+    if constexpr (CT2 <= 4) {  // an odd number of 64 channels: rounds of eight k-steps and a shorter last one
+        if (NK % 4) return NK > DEEP ? top_launch_levels_pd<T, CT2, DEEP, true>(p, st) : top_launch_levels_pd<T, CT2, 2>(p, st);
+    }
     return top_launch_levels_pd<T, CT2, DEEP / 2>(p, st);
 }
 

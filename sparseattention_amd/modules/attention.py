@@ -2,8 +2,8 @@
 
 Parameter names, shapes and method signatures follow the reference's
 hierarchical_attention/modules/attention.py:10-270 so that its state dicts load
-unchanged; the dense projections are torch's own `nn.Linear`, the tree build and
-the span attention are the HIP kernels.
+unchanged; the dense projections are `nn.Linear` modules whose products run on this package's kernels where
+they are the faster ones (`ops/linear.py`), the tree build and the span attention are the HIP kernels.
 """
 from __future__ import annotations
 

@@ -36,6 +36,8 @@ def _declare(lib):
     lib.hsa_attn_fwd_timed.restype = I
     lib.hsa_linear.argtypes = [I, P, I, I, I, I, P]
     lib.hsa_linear.restype = I
+    lib.hsa_linear_rectangles.argtypes = [I, P, I, I, I, P, I]
+    lib.hsa_linear_rectangles.restype = I
     lib.hsa_linear_tile.argtypes = [I, P, I, I, I]
     lib.hsa_linear_tile.restype = I
     lib.hsa_linear_long.argtypes = [P, I64, P, I64, P, I64, I, I, I, P, ctypes.c_size_t, I, P]

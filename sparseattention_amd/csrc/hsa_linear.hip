@@ -58,6 +58,37 @@ struct LnArgs {
     int nseg, K, tiles, group;
 };
 
+// Where tile t lies: rows m0, m0 + period .. of batch element b of a segment, columns from n0.  `group` row tiles, column
+// by column, then the next.
+struct LnPlace {
+    int seg, b, m0, n0;
+};
+template <int BM, int BN, int ANY>
+__host__ __device__ __forceinline__ LnPlace place_of(const LnArgs &p, int t) {
+    LnPlace c;
+    c.seg = 0;
+    while (c.seg + 1 < p.nseg && t >= p.seg[c.seg + 1].first) ++c.seg;
+    const LnSeg &s = p.seg[c.seg];
+    t -= s.first;
+    const int per_group = p.group * s.col_tiles, grp = t / per_group, in = t - grp * per_group;
+    const int left = s.all_row_tiles - grp * p.group, rows = left < p.group ? left : p.group;
+    const int ct = in / rows, rt = grp * p.group + in - ct * rows;
+    c.b = rt / s.row_tiles;
+    c.m0 = (rt - c.b * s.row_tiles) * BM;
+    c.n0 = ct * BN;
+    if constexpr (ANY == 2) {
+        const int each = s.row_tiles / s.period, in_batch = rt - c.b * s.row_tiles, rho = in_batch / each;
+        const int rows = (s.rows - rho + s.period - 1) / s.period - BM, at = (in_batch - rho * each) * BM;
+        c.m0 = rho + s.period * (at < rows ? at : rows);
+        // whole lines: all but the first and the last columns' tiles begin where a line does
+        if (ct) c.n0 -= (int)(((uintptr_t)s.out + c.b * s.batch_out + c.m0 * s.ld_out) & 127) / 2;
+    } else {
+        c.m0 = c.m0 < s.rows - BM ? c.m0 : s.rows - BM;
+    }
+    c.n0 = c.n0 < s.cols - BN ? c.n0 : s.cols - BN;
+    return c;
+}
+
 // one transfer of 1 KiB: a scalar base and 32-bit offsets per lane
 __device__ __forceinline__ void lds_dma16_from(const char *base, uint32_t off, uint32_t lds) {
     uint32_t keep;
@@ -115,34 +146,7 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
     const int first = xcd * per + (xcd < rest ? xcd : rest), count = per + (xcd < rest);
     const int slots = gridDim.x >> 3, slot = blockIdx.x >> 3;
     if (slot >= count) return;
-    struct Tile {
-        int seg, b, m0, n0;
-    };
-    auto tile_of = [&](int t) {  // `group` row tiles, column by column, then the next
-        Tile c;
-        t += first;
-        c.seg = 0;
-        while (c.seg + 1 < p.nseg && t >= p.seg[c.seg + 1].first) ++c.seg;
-        const LnSeg &s = p.seg[c.seg];
-        t -= s.first;
-        const int per_group = p.group * s.col_tiles, grp = t / per_group, in = t - grp * per_group;
-        const int left = s.all_row_tiles - grp * p.group, rows = left < p.group ? left : p.group;
-        const int ct = in / rows, rt = grp * p.group + in - ct * rows;
-        c.b = rt / s.row_tiles;
-        c.m0 = (rt - c.b * s.row_tiles) * BM;
-        c.n0 = ct * BN;
-        if constexpr (ANY == 2) {
-            const int each = s.row_tiles / s.period, in_batch = rt - c.b * s.row_tiles, rho = in_batch / each;
-            const int rows = (s.rows - rho + s.period - 1) / s.period - BM, at = (in_batch - rho * each) * BM;
-            c.m0 = rho + s.period * (at < rows ? at : rows);
-            // whole lines: all but the first and the last columns' tiles begin where a line does
-            if (ct) c.n0 -= (int)(((uintptr_t)s.out + c.b * s.batch_out + c.m0 * s.ld_out) & 127) / 2;
-        } else {
-            c.m0 = c.m0 < s.rows - BM ? c.m0 : s.rows - BM;
-        }
-        c.n0 = c.n0 < s.cols - BN ? c.n0 : s.cols - BN;
-        return c;
-    };
+    auto tile_of = [&](int t) { return place_of<BM, BN, ANY>(p, first + t); };
 
     // ---- transfers.  X: rows 32 w + 8 q + lane / 8, piece lane & 7 of 8.  W likewise (8 QW w + ..), or, TW,
     // rows of the contraction: pieces (w QW + q) 64 + lane of rows of BN / 8.
@@ -156,7 +160,7 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
     const char *load_x = nullptr, *load_w = nullptr;
     int lt = slot, lk = 0, lbuf = 0;
     auto aim = [&]() {
-        const Tile c = tile_of(lt);
+        const LnPlace c = tile_of(lt);
         const LnSeg &s = p.seg[c.seg];
         ld_x = ANY == 2 ? s.period * s.ld_x : s.ld_x;
         ld_w = s.ld_w;
@@ -267,12 +271,12 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
     const std::integral_constant<bool, false> without;
 
     // the bias of a tile's columns, one per thread
-    auto load_bias = [&](const Tile &c, int to) {
+    auto load_bias = [&](const LnPlace &c, int to) {
         const uint16_t *b = p.seg[c.seg].bias;
         const int at = (int)threadIdx.x;
         if (at < BN) lds_dma2(b ? b + c.n0 + at : ln_no_bias + at, lds_address(lds_bias[to]) + 256 * w);
     };
-    Tile c = tile_of(slot);
+    LnPlace c = tile_of(slot);
     int which = 0;
     load_bias(c, 0);
     aim();
@@ -541,6 +545,57 @@ double all_tiles(int tile, int nseg, const hsa_linear_segment *seg) {
     return n;
 }
 
+// rows after which results of a row stride lie in their lines of 64 elements as before
+int line_period(int64_t ld_out) {
+    int64_t a = ld_out & 63, line = 64;
+    while (a) {
+        const int64_t rest = line % a;
+        line = a;
+        a = rest;
+    }
+    return (int)(64 / line);
+}
+
+// the tiles of a launch; false: too many
+bool plan(int tile, int nseg, const hsa_linear_segment *seg, int K, LnArgs &p) {
+    const LnTile size = LN_TILES[tile];
+    p.nseg = nseg;
+    p.K = K;
+    p.group = 2048 / size.rows;
+    long tiles = 0;
+    for (int i = 0; i < nseg; ++i) {
+        const hsa_linear_segment &s = seg[i];
+        LnSeg &t = p.seg[i];
+        t.x = (const char *)s.x;
+        t.w = (const char *)s.w;
+        t.bias = (const uint16_t *)s.bias;
+        t.out = (char *)s.out;
+        t.ld_x = 2 * s.ld_x;
+        t.ld_w = 2 * s.ld_w;
+        t.ld_out = 2 * s.ld_out;
+        t.batch_x = 2 * s.batch_x;
+        t.batch_out = 2 * s.batch_out;
+        t.rows = s.rows;
+        t.cols = s.cols;
+        t.period = tile == 4 && nseg == 1 ? line_period(s.ld_out) : 1;
+        if (s.rows / t.period < size.rows) t.period = 1;
+        // (a tile of every period-th row begins up to 63 columns before its place: the last one has to reach the end)
+        const int each = (s.rows + t.period - 1) / t.period, cols = s.cols + (t.period > 1 ? 63 : 0);
+        t.row_tiles = t.period * ((each + size.rows - 1) / size.rows);
+        t.col_tiles = (cols + size.cols - 1) / size.cols;
+        const double n = (double)s.batches * t.row_tiles * t.col_tiles;
+        if (n + tiles >= (double)(1 << 30)) return false;
+        t.all_row_tiles = s.batches * t.row_tiles;
+        t.first = (int)tiles;
+        tiles += (long)n;
+    }
+    p.tiles = (int)tiles;
+    // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 8 / 32: 2180
+    // / 2200 / 2550 us at 32768 x 50257 x 512)
+    if (tile == 4 && p.seg[0].period == 1) p.group = 2;
+    return true;
+}
+
 }  // namespace
 
 }  // namespace hsa
@@ -587,60 +642,34 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     return best;
 }
 
+int hsa_linear_rectangles(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int (*rects)[7], int capacity) {
+    using namespace hsa;
+    HSA_REQUIRE(tile >= 0 && tile < 5 && tile != 3 && capacity >= 0 && (rects || !capacity), "bad tile %d or no room", tile);
+    LnArgs p = {};
+    if (!takes(tile, nseg, seg, K, w_rows_contract != 0) || !plan(tile, nseg, seg, K, p))
+        return fail(HSA_ERR_UNSUPPORTED, "projection: sizes or alignment not handled by tile %d (K=%d)", tile, K);
+    for (int t = 0; t < p.tiles && t < capacity; ++t) {
+        const LnPlace c = tile == 1 ? place_of<256, 192, 0>(p, t) : tile == 2 ? place_of<128, 128, 0>(p, t)
+                          : tile == 4 && p.seg[0].period > 1 ? place_of<256, 256, 2>(p, t) : place_of<256, 256, 0>(p, t);
+        const int rect[7] = {c.seg, c.b, c.m0, p.seg[c.seg].period, LN_TILES[tile].rows, c.n0, LN_TILES[tile].cols};
+        for (int i = 0; i < 7; ++i) rects[t][i] = rect[i];
+    }
+    return p.tiles;
+}
+
 int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int dtype, void *stream) {
     using namespace hsa;
     HSA_REQUIRE(dtype == HSA_F16 || dtype == HSA_BF16, "projections of 16-bit operands only (dtype %d)", dtype);
     HSA_REQUIRE(tile >= 0 && tile < 5, "bad tile %d", tile);
     if (!takes(tile, nseg, seg, K, w_rows_contract != 0))
         return fail(HSA_ERR_UNSUPPORTED, "projection: sizes or alignment not handled by tile %d (K=%d)", tile, K);
-    const double all = all_tiles(tile, nseg, seg);
-    if (all >= (double)(1 << 30)) return fail(HSA_ERR_UNSUPPORTED, "projection: too many tiles");
     LnArgs p = {};
-    p.nseg = nseg;
-    p.K = K;
-    p.group = 2048 / LN_TILES[tile].rows;
+    if (!plan(tile, nseg, seg, K, p)) return fail(HSA_ERR_UNSUPPORTED, "projection: too many tiles");
     double bytes = 0;
     for (int i = 0; i < nseg; ++i) {
-        const hsa_linear_segment &s = seg[i];
-        HSA_REQUIRE(s.x && s.w && s.out, "null pointer");
-        LnSeg &t = p.seg[i];
-        t.x = (const char *)s.x;
-        t.w = (const char *)s.w;
-        t.bias = (const uint16_t *)s.bias;
-        t.out = (char *)s.out;
-        t.ld_x = 2 * s.ld_x;
-        t.ld_w = 2 * s.ld_w;
-        t.ld_out = 2 * s.ld_out;
-        t.batch_x = 2 * s.batch_x;
-        t.batch_out = 2 * s.batch_out;
-        t.rows = s.rows;
-        t.cols = s.cols;
-        t.row_tiles = (s.rows + LN_TILES[tile].rows - 1) / LN_TILES[tile].rows;
-        t.period = 1;
-        if (tile == 4) {
-            // rows after which the results lie in their lines of 64 elements as before
-            long a = s.ld_out & 63, line = 64;
-            while (a) {
-                const long rest = line % a;
-                line = a;
-                a = rest;
-            }
-            const int period = (int)(64 / line);
-            if (nseg == 1 && period > 1 && s.rows / period >= LN_TILES[tile].rows) {
-                t.period = period;
-                t.row_tiles = period * (((s.rows + period - 1) / period + LN_TILES[tile].rows - 1) / LN_TILES[tile].rows);
-                t.col_tiles = (s.cols + 63 + LN_TILES[tile].cols - 1) / LN_TILES[tile].cols;
-            }
-        }
-        t.col_tiles = (s.cols + LN_TILES[tile].cols - 1) / LN_TILES[tile].cols;
-        t.all_row_tiles = s.batches * t.row_tiles;
-        t.first = p.tiles;
-        p.tiles += t.all_row_tiles * t.col_tiles;
-        bytes += 2.0 * s.batches * s.rows * s.cols;
+        HSA_REQUIRE(seg[i].x && seg[i].w && seg[i].out, "null pointer");
+        bytes += 2.0 * seg[i].batches * seg[i].rows * seg[i].cols;
     }
-    // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 8 / 32: 2180
-    // / 2200 / 2550 us at 32768 x 50257 x 512)
-    if (tile == 4 && p.seg[0].period == 1) p.group = 2;
     // large results go past the caches: they would push the operands' rows out of the L2s (4 MiB each) before the
     // next kernel could find them there (everything above 16 MiB against 256 MiB: a six-layer forward of 32768 tokens
     // 5727 -> 5678 us, a module in training 1650 -> 1628)

@@ -6,7 +6,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from sparseattention_amd import _lib
+import sparseattention_amd as sa
+from sparseattention_amd import _lib, transformer
 from sparseattention_amd.ops.linear import linear, query_key_value
 
 pytestmark = pytest.mark.gpu
@@ -77,10 +78,12 @@ def test_few_rows_against_fp64(dtype, B, R, N, K):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,R,N,K,pad,first", [
     (1, 256, 256, 128, 0, 0), (2, 257, 257, 192, 0, 3), (1, 300, 511, 512, 2, 1), (1, 512, 1000, 128, 3, 7),
-    (1, 16384, 257, 128, 0, 0), (1, 16447, 513, 192, 2, 5), (1, 8300, 320, 128, 2, 1)])
+    (1, 16384, 257, 128, 0, 0), (1, 16447, 513, 192, 2, 5), (1, 8300, 320, 128, 2, 1),
+    (1, 16384, 511, 128, 0, 0), (1, 16447, 512, 128, 1, 5), (1, 16384, 450, 192, 1, 63), (1, 8300, 510, 128, 0, 1),
+    (1, 8192, 507, 128, 3, 58), (1, 4100, 508, 128, 0, 0), (1, 4351, 450, 128, 2, 31)])
 def test_results_that_begin_anywhere(dtype, B, R, N, K, pad, first):
-    """Rows through the LDS; from 256 rows per line period on (16384 for odd strides, 8192 for twice an odd one)
-    tiles of rows that lie alike."""
+    """Rows through the LDS; from 256 rows per line period on (16384 for odd strides, 8192 for twice an odd one, 4096
+    for four times one) tiles of rows that lie alike, which begin up to 63 columns before their place."""
     _check(dtype, False, 4, B, R, N, K, pad, first)
 
 
@@ -192,6 +195,37 @@ def test_long_contraction_against_fp64(dtype, M, N, K):
     assert bool(((out.double() - ref).abs() <= _bound(x, w, ref, dtype)).all())
     with pytest.raises(_lib.HsaError):
         _lib.check(lib.hsa_linear_long(*args, ws.numel() * 4 - 4, code, stream), "hsa_linear_long")
+
+
+def test_model_with_a_vocabulary_whose_last_tile_is_nearly_full(monkeypatch):
+    """50428 columns (252 in the last tile of 256) of 4 x 1024 rows: logits and loss, with and without autograd, against
+    the layer's own product; the results' memory held NaN before."""
+    vocab, B, N = 50428, 4, 1024
+    torch.manual_seed(0)
+    net = sa.TransformerLM(vocab, 128, 2, 128, 1, dropout=0.0, window_size=4, max_len=N).to(DEV).to(torch.bfloat16)
+    tok, to = (torch.randint(0, vocab, (B, N), device=DEV) for _ in range(2))
+
+    def run():
+        torch.full((B * N * vocab,), float("nan"), device=DEV, dtype=torch.bfloat16)
+        logits = net(tok)
+        return logits, F.cross_entropy(logits.float().view(-1, vocab), to.view(-1))
+
+    def both():
+        net.zero_grad(set_to_none=True)
+        with torch.no_grad():
+            plain = run()
+        logits, loss = run()
+        loss.backward()
+        return plain + (logits.detach(), loss.detach()), [p.grad.float() for p in net.parameters() if p.grad is not None]
+
+    got, grads = both()
+    with monkeypatch.context() as m:
+        m.setattr(transformer, "linear", lambda layer, x, wide=False: layer(x))
+        want, want_grads = both()
+    for a, b in zip(got, want):  # one rounding to bf16 on either side of sums of 128 products
+        assert bool(((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 1e-4).all())
+    for a, b in zip(grads, want_grads):  # the logits' roundings carried back through a softmax: a hundredth
+        assert float((a - b).norm()) <= 0.01 * float(b.norm()) + 1e-12
 
 
 @pytest.mark.parametrize("vocab", [50257, 5120])

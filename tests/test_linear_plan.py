@@ -1,0 +1,67 @@
+"""The tiles of the projection kernel (csrc/hsa_linear.hip) on the host: every result belongs to one, none reaches outside."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from sparseattention_amd import _lib
+
+
+class Segment(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "w", "bias", "out")]
+                + [(n, ctypes.c_int64) for n in ("ld_x", "ld_w", "ld_out", "batch_x", "batch_out")]
+                + [(n, ctypes.c_int) for n in ("batches", "rows", "cols")])
+
+
+def _segment(B, R, N, K, ld, first=0):
+    """Addresses of nothing: only their alignment counts."""
+    return Segment(1 << 20, 2 << 20, None, (3 << 20) + 2 * first, K, K, ld, R * K, (R + 1) * ld, B, R, N)
+
+
+def _rectangles(tile, K, *segs):
+    arr, room = (Segment * len(segs))(*segs), 1 << 16
+    out = np.zeros((room, 7), dtype=np.int32)
+    n = _lib.lib().hsa_linear_rectangles(len(segs), arr, K, 0, tile, out.ctypes.data, room)
+    assert 0 < n <= room, n
+    return out[:n]
+
+
+def _covered(rects, *segs):
+    for i, s in enumerate(segs):
+        r = rects[rects[:, 0] == i]
+        r = r[np.lexsort((r[:, 5], r[:, 2], r[:, 1]))]
+        step, rows, width = r[0, 3], r[0, 4], r[0, 6]
+        begins = np.ones(len(r), bool)  # of a row block's columns
+        begins[1:] = (r[1:, 1:3] != r[:-1, 1:3]).any(1)
+        ends = np.append(begins[1:], True)
+        assert (r[begins, 5] == 0).all() and (r[ends, 5] + width == s.cols).all()
+        assert (r[1:, 5][~begins[1:]] <= r[:-1, 5][~begins[1:]] + width).all()
+        seen = np.zeros((s.batches, s.rows), bool)
+        blocks = r[begins]
+        at = blocks[:, 2:3] + step * np.arange(rows)[None]
+        assert at.min() >= 0 and at.max() < s.rows and (blocks[:, 1] >= 0).all() and (blocks[:, 1] < s.batches).all()
+        seen[np.broadcast_to(blocks[:, 1:2], at.shape), at] = True
+        assert seen.all()
+
+
+@pytest.mark.parametrize("period", [2, 4, 8, 16, 32, 64])
+def test_rows_that_lie_alike_in_lines(period):
+    """Results whose rows begin anywhere, in tiles of every period-th row: all remainders of the columns, places in a
+    line and row counts around whole tiles."""
+    strided = 0
+    for cols in range(256, 512):
+        ld = next(n for n in range(cols, cols + 129) if 64 // np.gcd(n, 64) == period)
+        for first in (0, 1, 31, 58, 63):
+            for rows in (256 * period, 256 * period + 1, 257 * period + 3):
+                s = _segment(1, rows, cols, 128, ld, first)
+                r = _rectangles(4, 128, s)
+                strided += int(r[0, 3] == period)
+                _covered(r, s)
+    assert strided == 256 * 5 * 3
+
+
+@pytest.mark.parametrize("tile,rows,cols", [(0, 256, 256), (1, 256, 192), (2, 128, 128), (4, 256, 256)])
+def test_consecutive_rows(tile, rows, cols):
+    for B, R, N in ((1, rows, cols), (3, rows + 1, cols + 8), (2, 5 * rows - 1, 3 * cols - 8), (1, 40 * rows + 7, 2 * cols)):
+        segs = [_segment(B, R, N, 192, N + 8, 8), _segment(1, R + 1, N + 8, 192, N + 8)]
+        _covered(_rectangles(tile, 192, *segs), *segs)

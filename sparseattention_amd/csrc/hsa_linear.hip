@@ -21,7 +21,7 @@
 //
 // Results whose rows begin at any element (a vocabulary of odd size): a line that two tiles share costs more
 // than the line.  With rows enough, a tile takes every 64th row: their results lie alike in their lines, so the
-// tiles' columns can begin where the lines do (32768 x 50257 x 512: 1740 to 1800 us; the library 2200).  Else the rows go
+// tiles' columns can begin where the lines do (32768 x 50257 x 512: 1710 us; the library 2160).  Else the rows go
 // through the LDS and are stored as 16-byte pieces where they lie (4096 x 50257 x 512: 283 us; 330 as they come,
 // the library 349).
 //
@@ -577,12 +577,26 @@ bool plan(int tile, int nseg, const hsa_linear_segment *seg, int K, LnArgs &p) {
         t.batch_out = 2 * s.batch_out;
         t.rows = s.rows;
         t.cols = s.cols;
-        t.period = tile == 4 && nseg == 1 ? line_period(s.ld_out) : 1;
-        if (s.rows / t.period < size.rows) t.period = 1;
-        // (a tile of every period-th row begins up to 63 columns before its place: the last one has to reach the end)
-        const int each = (s.rows + t.period - 1) / t.period, cols = s.cols + (t.period > 1 ? 63 : 0);
-        t.row_tiles = t.period * ((each + size.rows - 1) / size.rows);
-        t.col_tiles = (cols + size.cols - 1) / size.cols;
+        t.period = 1;
+        t.row_tiles = (s.rows + size.rows - 1) / size.rows;
+        t.col_tiles = (s.cols + size.cols - 1) / size.cols;
+        // Tiles of rows that lie alike where whole lines pay for it.  They take 0.8 of the time of consecutive rows
+        // through the LDS for the same number of tiles, but a row class that does not fill its tiles makes for more of
+        // them (us, library / alike / through the LDS, in brackets their tiles by the others': 50257 columns, 32768
+        // rows 2163 / 1710 / 2098 (1), 28672 1890 / 1709 / 1840 (1.14), 24576 1618 / 1705 / 1570 (1.33), 20480 1348 / 1730 /
+        // 1303 (1.6); 50260, 4096 rows 340 / 220 / 280 (1), 5120 420 / 430 / 295 (1.6)), and the first and the last columns'
+        // tiles begin at any element all the same (16384 rows of 3001 73 / 70 / 59, 32768 130 / 137 / 112, of 5001 156 /
+        // 145 / 149, of 8001 395 / 310 / 336, of 10001 285 / 246 / 267).
+        const int period = tile == 4 && nseg == 1 ? line_period(s.ld_out) : 1;
+        if (period > 1 && s.rows / period >= size.rows && t.col_tiles >= 32) {
+            const int row_tiles = period * (((s.rows + period - 1) / period + size.rows - 1) / size.rows);
+            if (row_tiles * 20l <= t.row_tiles * 23l) {
+                t.period = period;
+                t.row_tiles = row_tiles;
+                // (a tile begins up to 63 columns before its place: the last one has to reach the end)
+                t.col_tiles = (s.cols + 63 + size.cols - 1) / size.cols;
+            }
+        }
         const double n = (double)s.batches * t.row_tiles * t.col_tiles;
         if (n + tiles >= (double)(1 << 30)) return false;
         t.all_row_tiles = s.batches * t.row_tiles;

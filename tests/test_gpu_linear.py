@@ -79,11 +79,11 @@ def test_few_rows_against_fp64(dtype, B, R, N, K):
 @pytest.mark.parametrize("B,R,N,K,pad,first", [
     (1, 256, 256, 128, 0, 0), (2, 257, 257, 192, 0, 3), (1, 300, 511, 512, 2, 1), (1, 512, 1000, 128, 3, 7),
     (1, 16384, 257, 128, 0, 0), (1, 16447, 513, 192, 2, 5), (1, 8300, 320, 128, 2, 1),
-    (1, 16384, 511, 128, 0, 0), (1, 16447, 512, 128, 1, 5), (1, 16384, 450, 192, 1, 63), (1, 8300, 510, 128, 0, 1),
-    (1, 8192, 507, 128, 3, 58), (1, 4100, 508, 128, 0, 0), (1, 4351, 450, 128, 2, 31)])
+    (1, 16384, 8191, 128, 0, 0), (1, 16384, 8192, 128, 1, 5), (1, 16384, 8130, 192, 1, 63), (1, 8192, 8190, 128, 0, 1),
+    (1, 8192, 8187, 128, 3, 58), (1, 4096, 8188, 128, 0, 0), (1, 28675, 7938, 128, 2, 31), (1, 16384, 8001, 192, 0, 3)])
 def test_results_that_begin_anywhere(dtype, B, R, N, K, pad, first):
-    """Rows through the LDS; from 256 rows per line period on (16384 for odd strides, 8192 for twice an odd one, 4096
-    for four times one) tiles of rows that lie alike, which begin up to 63 columns before their place."""
+    """Rows through the LDS; from 7937 columns and 256 rows per line period on (16384 for odd strides, 8192 for twice an
+    odd one, 4096 for four times one) tiles of rows that lie alike, which begin up to 63 columns before their place."""
     _check(dtype, False, 4, B, R, N, K, pad, first)
 
 

@@ -48,16 +48,26 @@ def _covered(rects, *segs):
 def test_rows_that_lie_alike_in_lines(period):
     """Results whose rows begin anywhere, in tiles of every period-th row: all remainders of the columns, places in a
     line and row counts around whole tiles."""
-    strided = 0
-    for cols in range(256, 512):
+    for cols in range(7937, 7937 + 256):
         ld = next(n for n in range(cols, cols + 129) if 64 // np.gcd(n, 64) == period)
-        for first in (0, 1, 31, 58, 63):
-            for rows in (256 * period, 256 * period + 1, 257 * period + 3):
+        many = cols % 37 == 0
+        for first in (0, 1, 31, 58, 63) if many else (0, 63 - cols % 3):
+            for rows in (256 * period, 1792 * period + 1, 7 * 257 * period + 3) if many else (256 * period,):
                 s = _segment(1, rows, cols, 128, ld, first)
                 r = _rectangles(4, 128, s)
-                strided += int(r[0, 3] == period)
+                assert (r[:, 3] == period).all()
                 _covered(r, s)
-    assert strided == 256 * 5 * 3
+
+
+@pytest.mark.parametrize("rows,cols,period", [
+    (32768, 50257, 64), (28672, 50257, 64), (24576, 50257, 1), (20480, 50257, 1), (16384, 50257, 64), (12288, 50257, 1),
+    (8192, 50258, 32), (10240, 50258, 1), (4096, 50260, 16), (5120, 50260, 1), (7168, 50260, 16), (32768, 3001, 1),
+    (32768, 8001, 64)])
+def test_rows_that_lie_alike_do_not_multiply_the_tiles(rows, cols, period):
+    s = _segment(1, rows, cols, 512, cols)
+    r = _rectangles(4, 512, s)
+    assert (r[:, 3] == period).all() and len(r) <= 1.15 * -(-rows // 256) * -(-cols // 256)
+    _covered(r, s)
 
 
 @pytest.mark.parametrize("tile,rows,cols", [(0, 256, 256), (1, 256, 192), (2, 128, 128), (4, 256, 256)])

@@ -700,6 +700,26 @@ Three query_key_value(const Tensor &x, const Tensor &y, const Tensor &weight_q, 
 }
 
 // ------------------------------------------------------------------------------- one layer of the model
+// the whole span-node update as one chain of fused levels, the norms on their kernel
+bool layer_kind(const Tensor &x, int64_t heads) {
+    if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || !x.is_cuda() || x.dim() != 3 || x.numel() == 0 ||
+        (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) || heads < 1 || heads > (1 << 16))
+        return false;
+    const int64_t B = x.size(0), N = x.size(1), C = x.size(2);
+    return B <= (1 << 20) && N >= 2 && N <= (1 << 24) && log2_exact(N) >= 0 && C % heads == 0 && C <= (1 << 16) &&
+           hsa_cross_update_level_rows((int)B, (int)heads, (int)(C / heads), type_code(x)) >= N && hsa_add_layer_norm_ok((int)C, type_code(x));
+}
+// larger inputs whose rows' products do not go into one launch: the Python layer has a way without the copy
+bool layer_rows(const Tensor &x, const Tensor &y, const Tensor &wq, const Tensor &wk, const Tensor &wv) {
+    return x.numel() < 1 << 20 || rows_plan(x, y, wq, wk, wv).second >= 0;
+}
+// Whether a layer of these sizes is one that decoder_layer takes, asked before its modules are looked at one by one (a
+// forward of B2 N1024, two layers of 4 heads by 128 channels, which it does not take: 905 us when that is found out last,
+// 845 here, 815 without the native layer)
+bool decoder_layer_takes(const Tensor &x, const Tensor &y, const Tensor &w, int64_t heads) {
+    return layer_kind(x, heads) && ordinary({&x, &y, &w}) && y.dim() == 3 && y.numel() > 0 && y.size(0) == x.size(0) && layer_rows(x, y, w, w, w);
+}
+
 // A decoder layer without autograd, dropout and autocast on 16-bit tensors, launch for launch what the Python
 // layer does: a short sequence's layer is 15 to 25 launches of a few us each, and through Python they take
 // 170 us to enqueue (six layers of B1 N256: 1056 us a forward against 700 us of kernels).
@@ -712,15 +732,10 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> decoder_layer(const Te
                                                                         const std::vector<Tensor> &p, const std::vector<double> &eps,
                                                                         int64_t heads, int64_t window, bool causal, bool gelu,
                                                                         bool following) {
-    if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || !x.is_cuda() || x.dim() != 3 || x.numel() == 0 ||
-        (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) || p.size() != (following ? NORM1_B + 1 : NORM_Y_W) ||
-        eps.size() != 3 || heads < 1 || window < 0 || window > (1 << 20))
+    if (!layer_kind(x, heads) || p.size() != (following ? NORM1_B + 1 : NORM_Y_W) || eps.size() != 3 || window < 0 || window > (1 << 20))
         return std::nullopt;
     const int64_t B = x.size(0), N = x.size(1), C = x.size(2);
-    if (B > (1 << 20) || N < 2 || N > (1 << 24) || log2_exact(N) < 0 || C % heads || C > (1 << 16)) return std::nullopt;
     const int H = (int)heads, Dh = (int)(C / heads), code = type_code(x);
-    // the whole span-node update as one chain of fused levels, the norms on their kernel
-    if (hsa_cross_update_level_rows((int)B, H, Dh, code) < N || !hsa_add_layer_norm_ok((int)C, code)) return std::nullopt;
     if (!ordinary({&x, &y, &nx, &ny})) return std::nullopt;
     for (const Tensor *t : {&x, &y, &nx, &ny})
         if (!same_kind(x, *t) || t->dim() != 3 || !t->is_contiguous() || !aligned16(*t)) return std::nullopt;
@@ -737,8 +752,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> decoder_layer(const Te
         return std::nullopt;
     for (int i = NORM_Y_W; following && i <= NORM1_B; ++i)
         if (!row(i, C)) return std::nullopt;
-    // (larger inputs whose rows' products do not go into one launch: the Python layer has a way without the copy)
-    if (B * N * C >= 1 << 20 && rows_plan(nx, y, p[Q_X], p[K_X], p[V_X]).second < 0) return std::nullopt;
+    if (!layer_rows(nx, y, p[Q_X], p[K_X], p[V_X])) return std::nullopt;
 
     c10::DeviceGuard guard(x.device());
     // span nodes: the three projections, every level of the tree, the output projection, the residual
@@ -791,5 +805,6 @@ PYBIND11_MODULE(_hsa_torch, m) {
     m.def("weight_grad", &weight_grad);
     m.def("query_key_value_rows", &query_key_value_rows);
     m.def("query_key_value", &query_key_value);
+    m.def("decoder_layer_takes", &decoder_layer_takes);
     m.def("decoder_layer", &decoder_layer);
 }

@@ -64,7 +64,9 @@ def query_key_value_rows(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Te
 def query_key_value(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
     """The same without autograd: the rows stay where they are and the five products write into the joined
     results in one launch (csrc/hsa_linear.hip).  None where that does not apply."""
-    layers = (layer_q, layer_k, layer_v)
-    if x.is_cuda and not torch.compiler.is_compiling() and all(_plain(m) and m.bias is None for m in layers):
-        return _lib.ext().query_key_value(x, y, *(m.weight for m in layers))
+    if (x.is_cuda and not torch.compiler.is_compiling()
+            and all_plain(((layer_q, nn.Linear), (layer_k, nn.Linear), (layer_v, nn.Linear)))):
+        q, k, v = layer_q._parameters, layer_k._parameters, layer_v._parameters
+        if q.get("bias") is None and k.get("bias") is None and v.get("bias") is None:
+            return _lib.ext().query_key_value(x, y, q["weight"], k["weight"], v["weight"])
     return None

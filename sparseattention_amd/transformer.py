@@ -131,7 +131,12 @@ class DecoderLayer(nn.Module):
             return None
         sub = self._modules
         att, ff = sub["self_attn"], sub["feed_forward"]
+        if type(att) is not HierarchicalAttention or type(ff) is not PositionwiseFeedForward:
+            return None
         a, f = att._modules, ff._modules
+        wq = a["Wq_x"]._parameters.get("weight")
+        if wq is None or not _lib.ext().decoder_layer_takes(x, y, wq, att.num_heads):
+            return None
         drops = (sub["dropout"], a["dropout"], f["dropout"])
         norms = [sub["norm2"]]
         if following is not None:

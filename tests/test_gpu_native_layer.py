@@ -111,6 +111,18 @@ def test_calls_that_stay_with_the_python_layer(monkeypatch):
     assert net(tok).requires_grad and count.native == 0
 
 
+@pytest.mark.parametrize("dim,heads,length", [(768, 12, 1024), (512, 4, 1024), (96, 3, 64)])
+def test_sizes_not_taken_are_not_looked_into(dim, heads, length, monkeypatch):
+    """What is known from the sizes alone costs no look at the layer's modules."""
+    net, tok = _lm(dim, heads, 128, 2, length=length), torch.randint(0, 50, (2, length), device=DEV)
+    looks, inner = [], transformer.all_plain
+    monkeypatch.setattr(transformer, "all_plain", lambda m: (looks.append(1), inner(m))[1])
+    count = _Count(monkeypatch)
+    with torch.no_grad():
+        net(tok)
+    assert count.native == 0 and not looks
+
+
 def test_dropout_goes_the_python_way(monkeypatch):
     net, tok = _lm(dropout=0.5), torch.randint(0, 50, (2, 64), device=DEV)
     count = _Count(monkeypatch)

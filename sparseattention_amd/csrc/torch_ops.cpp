@@ -340,7 +340,7 @@ void launch_products(const std::vector<hsa_linear_segment> &segs, const Tensor &
     check(hsa_linear((int)segs.size(), segs.data(), (int)K, contract, tile, type_code(like), stream_of(like)), "hsa_linear");
 }
 
-// x w^T + b, or x w with `contract`, without autograd: on this library's kernels where they are the faster
+// x w^T + b, or x w + b with `contract`, without autograd: on this library's kernels where they are the faster
 // ones, else by torch
 Tensor project(const Tensor &x, const Tensor &w, const std::optional<Tensor> &b_, bool contract) {
     const Tensor b = b_ ? *b_ : Tensor();
@@ -370,7 +370,8 @@ Tensor project(const Tensor &x, const Tensor &w, const std::optional<Tensor> &b_
             return out;
         }
     }
-    return contract ? at::matmul(x, w) : at::linear(x, w, b_);
+    if (contract) return b.defined() ? at::linear(x, w.t(), b) : at::matmul(x, w);
+    return at::linear(x, w, b_);
 }
 
 // The same of several (x, w), all without bias, in one launch where that pays.

@@ -122,6 +122,18 @@ def test_linear_without_autograd(rows, cols, K, bias):
     assert bool(((got.double() - want).abs() <= _bound(x, wt, want, torch.bfloat16)).all())
 
 
+@pytest.mark.parametrize("rows,K,cols", [(16384, 512, 512), (64, 96, 40)])
+@pytest.mark.parametrize("contract", [False, True])
+def test_products_with_a_bias(rows, K, cols, contract):
+    """Kernel and library, chosen by the sizes: the same sum on either route."""
+    torch.manual_seed(0)
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    x, w, b = mk(rows, K), mk(K, cols) if contract else mk(cols, K), mk(cols)
+    wt = w if contract else w.t()
+    got, want = _lib.ext().project(x, w, b, contract), x.double() @ wt.double() + b.double()
+    assert bool(((got.double() - want).abs() <= _bound(x, wt, want, torch.bfloat16)).all())
+
+
 @pytest.mark.parametrize("amp", [None, torch.float16])
 @pytest.mark.parametrize("B,N,C", [(1, 64, 64), (2, 256, 256), (4, 1024, 512)])
 def test_query_key_value(amp, B, N, C):

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import linear, query_key_value, query_key_value_rows
+from ..ops.linear import FORWARDS, linear, query_key_value, query_key_value_rows
 from ..ops.topology import build_tree_topology
 
 
@@ -423,3 +423,6 @@ class HierarchicalAttention(nn.Module):
         ctx, attn = self._standard_attention(Q, K, V, mask)
         out = self.out_proj_x(ctx.transpose(1, 2).reshape(B, Lq, D))
         return (out, attn) if return_attention else out
+
+
+FORWARDS[HierarchicalAttention] = HierarchicalAttention.forward

@@ -8,14 +8,14 @@ from torch.nn.modules import module as _module
 from .. import _lib
 
 
+# the forwards that calls may be made without, as they are when their classes are defined or this module is loaded
+FORWARDS = {cls: cls.forward for cls in (nn.Linear, nn.LayerNorm, nn.Dropout)}
+
+
 def plain_module(module, cls) -> bool:
     """Whether calling `module` runs nothing but `cls`'s own forward, so that the call may be bypassed: no
-    subclass, no forward set on the instance, no hooks on it or on all modules."""
-    return (type(module) is cls and "forward" not in module.__dict__
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                     or module._backward_pre_hooks)
-            and not (_module._global_forward_hooks or _module._global_forward_pre_hooks
-                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+    subclass, no forward set on the instance or in place of the class's, no hooks on it or on all modules."""
+    return all_plain(((module, cls),))
 
 
 def all_plain(modules) -> bool:
@@ -26,8 +26,8 @@ def all_plain(modules) -> bool:
         return False
     for m, cls in modules:
         d = m.__dict__
-        if (type(m) is not cls or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                or d["_backward_pre_hooks"]):
+        if (type(m) is not cls or cls.forward is not FORWARDS[cls] or "forward" in d or d["_forward_hooks"]
+                or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]):
             return False
     return True
 

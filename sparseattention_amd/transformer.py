@@ -10,6 +10,7 @@ presence is ever looked at (an N x N mask costs 16 MB at N=4096 and is never rea
 from __future__ import annotations
 
 import math
+import sys
 
 import torch
 import torch.nn as nn
@@ -19,7 +20,7 @@ from . import _lib
 from .modules import HierarchicalAttention
 from .modules import attention as _attention
 from .ops import generate_span_input_Y
-from .ops.linear import all_plain, linear, plain_module
+from .ops.linear import FORWARDS, all_plain, linear, plain_module
 
 
 def _plain_norm(m) -> bool:
@@ -48,18 +49,6 @@ def add_layer_norm(x, branch, norm):
     return x, norm(x)
 
 
-# what the native layer stands in for, as it is when this module is loaded
-_STEPS = tuple((n, getattr(HierarchicalAttention, n)) for n in ("forward", "cross_update_Y", "update_X_from_Y", "_span_levels",
-                                                                "_fused_weight"))
-_ATTENTION = _attention.hierarchical_attention
-
-
-def _own_steps(att) -> bool:
-    """Nobody has replaced the attention's steps, on the class, on the instance or in its module."""
-    return (all(getattr(HierarchicalAttention, n) is f and n not in att.__dict__ for n, f in _STEPS)
-            and _attention.hierarchical_attention is _ATTENTION)
-
-
 class PositionwiseFeedForward(nn.Module):
     def __init__(self, d_model: int, d_ff: int, dropout: float = 0.1, activation: str = "relu"):
         super().__init__()
@@ -70,6 +59,9 @@ class PositionwiseFeedForward(nn.Module):
 
     def forward(self, x):
         return linear(self.fc2, self.dropout(self.activation(linear(self.fc1, x))))
+
+
+FORWARDS[PositionwiseFeedForward] = PositionwiseFeedForward.forward
 
 
 class PositionalEncoding(nn.Module):
@@ -145,7 +137,7 @@ class DecoderLayer(nn.Module):
         if not all_plain([(att, HierarchicalAttention), (ff, PositionwiseFeedForward)] + [(m, nn.Dropout) for m in drops]
                          + [(m, nn.LayerNorm) for m in norms] + [(m, nn.Linear) for m in linears]):
             return None
-        if any(m.training and m.p > 0 for m in drops) or not att.fuse_top_levels or not _own_steps(att):
+        if any(m.training and m.p > 0 for m in drops) or not att.fuse_top_levels or not _own_steps(self, att):
             return None
         if ff.activation is not F.gelu and ff.activation is not F.relu:
             return None
@@ -170,6 +162,21 @@ class DecoderLayer(nn.Module):
     def _may_chain(self) -> bool:
         """Whether `_chained` may stand in for calling the layer."""
         return plain_module(self, DecoderLayer)
+
+
+FORWARDS[DecoderLayer] = DecoderLayer.forward
+# what the native layer stands in for besides its modules' forwards, as it is when this module is loaded
+_STEPS = tuple((owner, name, getattr(owner, name)) for owner, names in (
+    (HierarchicalAttention, ("cross_update_Y", "update_X_from_Y", "_span_levels", "_fused_weight", "_chain_weights")),
+    (DecoderLayer, ("_chained",)),
+    (_attention, ("hierarchical_attention", "linear", "query_key_value")),
+    (sys.modules[__name__], ("add_layer_norm", "linear"))) for name in names)
+
+
+def _own_steps(layer, att) -> bool:
+    """Nobody has replaced one of the steps, on its class, on the instance or in its module."""
+    return (all(getattr(owner, name) is f for owner, name, f in _STEPS) and "_chained" not in layer.__dict__
+            and not any(name in att.__dict__ for owner, name, _ in _STEPS if owner is HierarchicalAttention))
 
 
 class TransformerLM(nn.Module):

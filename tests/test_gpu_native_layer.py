@@ -111,6 +111,29 @@ def test_calls_that_stay_with_the_python_layer(monkeypatch):
     assert net(tok).requires_grad and count.native == 0
 
 
+@pytest.mark.parametrize("owner,name,calls", [
+    (transformer.PositionwiseFeedForward, "forward", 2), (transformer.DecoderLayer, "_chained", 2), (transformer.DecoderLayer, "forward", 2),
+    (attention.HierarchicalAttention, "forward", 2), (attention.HierarchicalAttention, "update_X_from_Y", 2), (torch.nn.LayerNorm, "forward", 6),
+    (torch.nn.Linear, "forward", 15), (torch.nn.Dropout, "forward", 11), (transformer, "add_layer_norm", 4), (transformer, "linear", 5),
+    (attention, "linear", 4), (attention, "query_key_value", 2)])
+def test_steps_replaced_on_their_class_or_module(owner, name, calls, monkeypatch):
+    """What stands in a step's place is called, without autograd as in training.  (The results may come from the library's
+    products and torch's norms then: bf16 roundings through two layers.)"""
+    net, tok = _lm(), torch.randint(0, 50, (2, 64), device=DEV)
+    count = _Count(monkeypatch)
+    seen, inner = [], getattr(owner, name)
+    with torch.no_grad():
+        want = net(tok)
+        assert count.native == 2
+        with monkeypatch.context() as m:
+            m.setattr(owner, name, lambda *a, **k: (seen.append(1), inner(*a, **k))[1])
+            got = net(tok)
+        assert count.native == 2 and len(seen) == calls
+        assert float((got.float() - want.float()).norm()) <= 0.03 * float(want.float().norm())
+        net(tok)
+        assert count.native == 4
+
+
 @pytest.mark.parametrize("dim,heads,length", [(768, 12, 1024), (512, 4, 1024), (96, 3, 64)])
 def test_sizes_not_taken_are_not_looked_into(dim, heads, length, monkeypatch):
     """What is known from the sizes alone costs no look at the layer's modules."""

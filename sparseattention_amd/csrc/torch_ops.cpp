@@ -319,7 +319,7 @@ std::optional<std::pair<Tensor, Tensor>> add_layer_norm(const Tensor &a_, const 
 // x [.., K] dense, w [N, K] (contract: [K, N]) with dense rows, of one 16-bit type; out: rows of N with the strides
 // it has.  batches: x and out are [B, R, ..] whose batch elements lie apart.
 bool projectable(const Tensor &x, const Tensor &w, const Tensor &b, bool contract) {
-    return x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) && x.numel() > 0 &&
+    return ordinary({&x, &w}) && x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) && x.numel() > 0 &&
            x.dim() >= 2 && x.is_contiguous() && same_kind(x, w) && w.dim() == 2 && w.is_contiguous() && w.numel() > 0 &&
            x.size(-1) == w.size(contract ? 0 : 1) &&
            (!b.defined() || (same_kind(x, b) && b.dim() == 1 && b.is_contiguous() && b.size(0) == w.size(contract ? 1 : 0)));

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import FORWARDS, linear, query_key_value, query_key_value_rows
+from ..ops.linear import FORWARDS, linear, project, query_key_value, query_key_value_rows
 from ..ops.topology import build_tree_topology
 
 
@@ -193,8 +193,7 @@ class HierarchicalAttention(nn.Module):
         cdt = self._compute_dtype(x)
         x, y_in = x.to(cdt).contiguous(), y_in.to(cdt).contiguous()
         w_qkv = self._fused_weight("qkv_y", (self.Wq_y, self.Wk_y, self.Wv_y), cdt)
-        project = _lib.ext().project
-        qkv = project(y_in, w_qkv, None, False)  # [B, N-1, 3D]
+        qkv = project(y_in, w_qkv)  # [B, N-1, 3D]
         w_kv = self._fused_weight("kv_y", (self.Wk_y, self.Wv_y), cdt)
         # every buffer the kernels address by raw pointer has the one element type
         assert qkv.dtype == cdt and qkv.is_contiguous(), "projection result has an unexpected layout"
@@ -231,9 +230,9 @@ class HierarchicalAttention(nn.Module):
                     if keep:
                         # the backward's keys and values of these levels' children, one GEMM for all
                         rows = torch.cat([src, y_new[:, off:N - 2]], dim=1)  # [B, 4P-2, D]
-                        chain = (rows, project(rows, w_kv, None, False))
+                        chain = (rows, project(rows, w_kv))
                     break
-                kv = project(src, w_kv, None, False)  # [B, 2P, 2D]
+                kv = project(src, w_kv)  # [B, 2P, 2D]
                 assert kv.dtype == cdt and kv.is_contiguous(), "projection result has an unexpected layout"
                 if drop_p > 0:
                     # dropout on the value half: a saved boolean keep-mask (drawn in fp32) and one
@@ -299,7 +298,7 @@ class HierarchicalAttention(nn.Module):
                     dqkv.data_ptr() + off * 3 * D * es, dkv_up.data_ptr(), B, C, H, Dh, (N - 1) * D, D, T3, 3 * D, T3,
                     3 * D, code, stream)
                 _lib.check(rc, "hsa_span_levels_bwd")
-                d_above = _lib.ext().project(dkv_up[:, :C].reshape(-1, 2 * D), w_kv, None, True)  # [B * C, D]
+                d_above = project(dkv_up[:, :C].reshape(-1, 2 * D), w_kv, True)  # [B * C, D]
                 pairs.append((dkv_up.view(-1, 2 * D), rows.view(-1, D), D))
             for lvl in range(len(kvs) - 1, -1, -1):
                 P, off = sizes[lvl], offsets[lvl]
@@ -316,9 +315,9 @@ class HierarchicalAttention(nn.Module):
                 _lib.check(rc, "hsa_build_parents_level_bwd")
                 if masks:
                     dkv_l.view(B, 2 * P, 2 * D)[:, :, D:].mul_(masks[lvl]).mul_(kept["scales"][lvl])
-                d_above = _lib.ext().project(dkv_l, w_kv, None, True)  # [B * 2P, D]
+                d_above = project(dkv_l, w_kv, True)  # [B * 2P, D]
         dx = d_above.view(B, N, D)
-        dy_in = _lib.ext().project(dqkv, w_qkv, None, True)
+        dy_in = project(dqkv, w_qkv, True)
         if kvs:
             pairs.append((dkv[:B * N], x.view(-1, D), D))
         if inner:

@@ -3,7 +3,10 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 from torch.nn.modules import module as _module
+from torch.overrides import _get_current_function_mode_stack, has_torch_function
+from torch.utils._device import DeviceContext
 
 from .. import _lib
 
@@ -32,6 +35,24 @@ def all_plain(modules) -> bool:
     return True
 
 
+def watched(*tensors) -> bool:
+    """Whether something handles torch's own functions on these tensors itself and would miss the calls that the native
+    code makes in their place: a function mode (other than a default device, which only places new tensors) or a
+    tensor subclass."""
+    if not has_torch_function(tensors):
+        return False
+    own = (torch.Tensor, nn.Parameter, type(None))
+    return (any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())
+            or any(type(t) not in own and type(t).__torch_function__ is not torch._C._disabled_torch_function_impl for t in tensors))
+
+
+def project(x: torch.Tensor, w: torch.Tensor, contract: bool = False) -> torch.Tensor:
+    """x w^T, or x w with `contract`, without autograd."""
+    if watched(x, w):
+        return torch.matmul(x, w) if contract else F.linear(x, w)
+    return _lib.ext().project(x, w, None, contract)
+
+
 def _plain(layer) -> bool:
     """An nn.Linear that may be bypassed."""
     return plain_module(layer, nn.Linear)
@@ -43,7 +64,7 @@ def linear(layer, x: torch.Tensor, wide: bool = False) -> torch.Tensor:
     computes the weight's and the bias's gradient in one contraction over the tokens (csrc/hsa_weight_grad.hip),
     directly in the parameters' type; everything else is the layer itself.  wide: a vocabulary projection, whose
     input gradient is a product with a long contraction (csrc/hsa_linear_long.hip)."""
-    if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer):
+    if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer) and not watched(x, layer.weight, layer.bias):
         y = _lib.ext().linear(x, layer.weight, layer.bias, wide)
         if y is not None:
             return y
@@ -56,7 +77,7 @@ def query_key_value_rows(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Te
     in one (csrc/hsa_rows.hip).  None where that does not apply."""
     layers = (layer_q, layer_k, layer_v)
     if (x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling()
-            and all(_plain(m) and m.bias is None for m in layers)):
+            and all(_plain(m) and m.bias is None for m in layers) and not watched(x, y, *(m.weight for m in layers))):
         return _lib.ext().query_key_value_rows(x, y, *(m.weight for m in layers))
     return None
 
@@ -67,6 +88,7 @@ def query_key_value(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor)
     if (x.is_cuda and not torch.compiler.is_compiling()
             and all_plain(((layer_q, nn.Linear), (layer_k, nn.Linear), (layer_v, nn.Linear)))):
         q, k, v = layer_q._parameters, layer_k._parameters, layer_v._parameters
-        if q.get("bias") is None and k.get("bias") is None and v.get("bias") is None:
+        if (q.get("bias") is None and k.get("bias") is None and v.get("bias") is None
+                and not watched(x, y, q["weight"], k["weight"], v["weight"])):
             return _lib.ext().query_key_value(x, y, q["weight"], k["weight"], v["weight"])
     return None

@@ -20,7 +20,7 @@ from . import _lib
 from .modules import HierarchicalAttention
 from .modules import attention as _attention
 from .ops import generate_span_input_Y
-from .ops.linear import FORWARDS, all_plain, linear, plain_module
+from .ops.linear import FORWARDS, all_plain, linear, plain_module, watched
 
 
 def _plain_norm(m) -> bool:
@@ -31,7 +31,7 @@ def _plain_norm(m) -> bool:
 
 def layer_norm(x, norm):
     """norm(x) on this package's kernel where it takes the case."""
-    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda"):
+    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda") and not watched(x, norm.weight, norm.bias):
         r = _lib.ext().add_layer_norm(x, None, norm.weight, norm.bias, norm.eps)
         if r is not None:
             return r[1]
@@ -41,7 +41,8 @@ def layer_norm(x, norm):
 def add_layer_norm(x, branch, norm):
     """(x + branch, norm(x + branch)): one kernel reads both once and writes both results, where it
     takes the case (one GPU, one element type; autocast mixes types and keeps the two steps)."""
-    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda"):
+    if (x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda")
+            and not watched(x, branch, norm.weight, norm.bias)):
         r = _lib.ext().add_layer_norm(x, branch, norm.weight, norm.bias, norm.eps)
         if r is not None:
             return r
@@ -119,7 +120,7 @@ class DecoderLayer(nn.Module):
     def _native(self, x, y, nx, ny, mask, following=None):
         """`_chained` without autograd as one native call (csrc/torch_ops.cpp), launch for launch the same; None
         where something may watch or replace one of its steps, or where the call does not take the layer."""
-        if torch.is_grad_enabled() or not x.is_cuda or torch.compiler.is_compiling():
+        if torch.is_grad_enabled() or not x.is_cuda or torch.compiler.is_compiling() or watched(x, y, nx, ny):
             return None
         sub = self._modules
         att, ff = sub["self_attn"], sub["feed_forward"]
@@ -169,7 +170,7 @@ FORWARDS[DecoderLayer] = DecoderLayer.forward
 _STEPS = tuple((owner, name, getattr(owner, name)) for owner, names in (
     (HierarchicalAttention, ("cross_update_Y", "update_X_from_Y", "_span_levels", "_fused_weight", "_chain_weights")),
     (DecoderLayer, ("_chained",)),
-    (_attention, ("hierarchical_attention", "linear", "query_key_value")),
+    (_attention, ("hierarchical_attention", "linear", "project", "query_key_value")),
     (sys.modules[__name__], ("add_layer_norm", "linear"))) for name in names)
 
 

@@ -6,7 +6,7 @@ import torch
 import sparseattention_amd as sa
 from sparseattention_amd import _lib
 from sparseattention_amd.ops import functional as fn
-from sparseattention_amd.ops.linear import linear, query_key_value_rows
+from sparseattention_amd.ops.linear import linear, query_key_value, query_key_value_rows
 from sparseattention_amd.transformer import add_layer_norm, layer_norm
 
 pytestmark = pytest.mark.gpu
@@ -255,3 +255,66 @@ def test_errors_of_the_library_keep_their_type():
             sa.hierarchical_attention(q, k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 200)
     with pytest.raises(AssertionError):
         sa.hierarchical_attention(q.detach()[0, :, 0, 0], k, v, t["forward_idx"], t["backward_gather"], t["forward_mask"], 4)
+
+
+# ------------------------------------------------------------------------- watched calls
+class _Seen(torch.overrides.TorchFunctionMode):
+    """Counts the functions called under it."""
+
+    def __init__(self):
+        super().__init__()
+        self.calls = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.calls.append(func)
+        return func(*args, **(kwargs or {}))
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+def _small_model():
+    torch.manual_seed(0)
+    return sa.TransformerLM(50, 128, 2, 128, 2, dropout=0.0, window_size=4, max_len=64).to(DEV).to(torch.bfloat16).eval()
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_function_modes_see_the_calls(train):
+    """A mode that handles torch's functions is given the projections and norms, with and without autograd; a default
+    device, which is such a mode too, changes nothing."""
+    net, tok = _small_model(), torch.randint(0, 50, (2, 64), device=DEV)
+    with torch.set_grad_enabled(train):
+        want = net(tok)
+        with _Seen() as seen:
+            got = net(tok)
+        # the last projection and, a layer, seven products besides those that the span nodes share
+        assert seen.calls.count(torch.nn.functional.linear) >= 15
+        assert seen.calls.count(torch.nn.functional.layer_norm) == 6
+        assert (got.float() - want.float()).norm() <= 0.03 * want.float().norm()
+        with torch.device(DEV):
+            assert torch.equal(net(tok), want)
+
+
+def test_subclasses_that_handle_functions_are_kept():
+    """The layer's own call gives back the subclass; so does the native route in its place."""
+    layer, norm = torch.nn.Linear(128, 64).to(DEV, torch.bfloat16), torch.nn.LayerNorm(128).to(DEV, torch.bfloat16)
+    x = torch.randn(2, 32, 128, device=DEV, dtype=torch.bfloat16)
+    t = x.as_subclass(_Tagged)
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            assert type(linear(layer, t)) is _Tagged and type(layer_norm(t, norm)) is _Tagged
+            assert type(linear(layer, x)) is torch.Tensor
+    with torch.no_grad():
+        layers = [torch.nn.Linear(128, 128, bias=False).to(DEV, torch.bfloat16) for _ in range(3)]
+        assert query_key_value(*layers, t, t) is None and query_key_value(*layers, x, x) is not None
+
+
+def test_dispatch_modes_see_the_products():
+    """The products inside the span nodes' update count for a mode that watches dispatched calls."""
+    from torch.utils.flop_counter import FlopCounterMode
+    net, B, N, C = _small_model(), 2, 64, 128
+    x, y = torch.randn(B, N, C, device=DEV, dtype=torch.bfloat16), torch.randn(B, N - 1, C, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad(), FlopCounterMode(display=False) as counter:
+        net.layers[0].self_attn.cross_update_Y(x, y)
+    assert counter.get_total_flops() >= 2 * B * (N - 1) * C * 4 * C  # q, k, v of the nodes and the last projection

@@ -134,17 +134,21 @@ class HierarchicalAttention(nn.Module):
         self._fused.clear()
         return super().train(mode)
 
-    def _fused_weight(self, name: str, layers, dtype: torch.dtype, packed: bool = False) -> torch.Tensor:
+    def _fused_weight(self, name: str, layers, dtype: torch.dtype, packed: bool = False, transposed: bool = False) -> torch.Tensor:
         """Weights of several bias-free projections, cast to `dtype` and stacked along the output
         dimension, so one GEMM computes them all (packed: key / value weights in the operand order
-        of the fused upper levels); rebuilt when any of them has been written to or moved."""
+        of the fused upper levels; transposed: one weight with its rows along the contraction); rebuilt
+        when any of them has been written to or moved."""
         # (the parameter dictionary is read directly: Module.__getattr__ costs a microsecond per use)
         params = [m._parameters["weight"] for m in layers]
         key = tuple((w.data_ptr(), w._version, w.dtype) for w in params) + (dtype,)
         hit = self._fused.get(name)
         if hit is None or hit[0] != key:
             ws = [w.detach().to(dtype) for w in params]
-            hit = (key, pack_kv_weights(ws[0], ws[1], self.num_heads) if packed else torch.cat(ws, dim=0))
+            if packed:
+                hit = (key, pack_kv_weights(ws[0], ws[1], self.num_heads))
+            else:
+                hit = (key, ws[0].t().contiguous() if transposed else torch.cat(ws, dim=0))
             self._fused[name] = hit
         return hit[1]
 
@@ -384,8 +388,11 @@ class HierarchicalAttention(nn.Module):
             xc, yc = x.to(cdt), y.to(cdt)
             k = torch.empty((B, 2 * N - 1, D), dtype=cdt, device=x.device)
             v = torch.empty_like(k)
-            for lin, dst in ((self.Wk_x, k), (self.Wv_x, v)):
-                wt = lin.weight.detach().to(cdt).t().unsqueeze(0).expand(B, D, D)
+            # (bf16: weights laid out along the contraction, since torch's batched bf16 product of a transposed right
+            # operand has faulted on this device; fp16: as they are, 8 x 2048 x 1024 x 1024 33 us against 40)
+            for name, lin, dst in (("k_x_t", self.Wk_x, k), ("v_x_t", self.Wv_x, v)):
+                wt = (self._fused_weight(name, (lin,), cdt, transposed=True) if cdt == torch.bfloat16
+                      else lin.weight.detach().to(cdt).t()).unsqueeze(0).expand(B, D, D)
                 torch.bmm(xc, wt, out=dst[:, :N])
                 torch.bmm(yc, wt, out=dst[:, N:])
             k, v = self._heads(k), self._heads(v)
@@ -402,12 +409,22 @@ class HierarchicalAttention(nn.Module):
                                        t["forward_mask"] if is_causal else None, self.window_size)
         return linear(self.out_proj_x, heads.view(B, N, D))
 
+    def _batched(self, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+        """a @ b over the leading dimensions.  bf16 on the GPU: the same operands in fp32, one rounding, also in
+        the backward (torch's batched bf16 product of a transposed right operand has faulted on this device, and
+        the backward of any makes such a product)."""
+        dtype = self._compute_dtype(a)
+        if not a.is_cuda or dtype != torch.bfloat16:
+            return torch.matmul(a, b)
+        with torch.autocast("cuda", enabled=False):
+            return torch.matmul(a.to(dtype).float(), b.to(dtype).float()).to(dtype)
+
     def _standard_attention(self, Q, K, V, mask):
-        scores = torch.matmul(Q, K.transpose(-1, -2)) / math.sqrt(Q.size(-1))
+        scores = self._batched(Q, K.transpose(-1, -2)) / math.sqrt(Q.size(-1))
         if mask is not None:
             scores = scores.masked_fill(mask == 0, float("-inf"))
         attn = self.dropout(torch.softmax(scores, dim=-1))
-        return torch.matmul(attn, V), attn
+        return self._batched(attn, V), attn
 
     def forward(self, query, key, value, y=None, mask=None, return_attention=False):
         B, Lq, D = query.shape

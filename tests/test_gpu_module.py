@@ -8,6 +8,7 @@ import sys
 import pytest
 import torch
 import torch.nn as nn
+import torch.utils._python_dispatch
 
 import oracle
 from conftest import error_figures, report
@@ -267,6 +268,50 @@ def test_update_x_from_y_direct_projection_matches_concatenation():
             m._DIRECT_PROJECTION_MIN_ELEMENTS = limit
             outs.append(m.update_X_from_Y(x, y, mask=True))
     assert (outs[0].float() - outs[1].float()).abs().max() <= 2e-2
+
+
+class _NoTransposedBatches(torch.utils._python_dispatch.TorchDispatchMode):
+    """Refuses, before it is launched, a batched bf16 product whose right operand is a transposed view: such
+    products have faulted on this device."""
+
+    def __init__(self):
+        super().__init__()
+        self.batched = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func.overloadpacket in (torch.ops.aten.bmm, torch.ops.aten.baddbmm):
+            right = args[-1]
+            assert right.dtype != torch.bfloat16 or right.stride(-1) == 1, "%s of a transposed view" % func
+            self.batched += 1
+        return func(*args, **(kwargs or {}))
+
+
+def test_no_batched_bf16_product_of_a_transposed_operand():
+    """Keys and values straight into their rows, and the dense attention forward and backward."""
+    B, N, dim, H = 2, 64, 128, 2
+    torch.manual_seed(12)
+    m = sa.HierarchicalAttention(dim, H, dropout=0.0, window_size=4).to(DEV).to(torch.bfloat16).eval()
+    m._DIRECT_PROJECTION_MIN_ELEMENTS = 0
+    x, y, z = (torch.randn(B, n, dim, device=DEV).bfloat16() for n in (N, N - 1, N // 2))
+    w = {k: v.detach().double().cpu() for k, v in m.state_dict().items()}
+    with _NoTransposedBatches() as mode, torch.no_grad():
+        out = m.update_X_from_Y(x, y, mask=True)
+        assert mode.batched == 4
+    _within(out, oracle.update_x_from_y_ref(x.double().cpu(), y.double().cpu(), w, H, 4, True), 2e-2, 1e-2, "rows")
+    x.requires_grad_(True)
+    with _NoTransposedBatches() as mode:
+        out, attn = m(x, z, z, return_attention=True)
+        out.float().square().sum().backward()
+        assert mode.batched == 6 and out.dtype == attn.dtype == torch.bfloat16
+    # the same in fp64 on the CPU
+    ref = sa.HierarchicalAttention(dim, H, dropout=0.0, window_size=4).double().eval()
+    ref.load_state_dict(w)
+    xr = x.detach().double().cpu().requires_grad_(True)
+    want = ref(xr, z.double().cpu(), z.double().cpu())
+    want.square().sum().backward()
+    # bf16: a rounding each of the projections, scores, weights and outputs
+    assert (out.double().cpu() - want).norm() <= 0.02 * want.norm()
+    assert (x.grad.double().cpu() - xr.grad).norm() <= 0.04 * xr.grad.norm()
 
 
 def test_lm_generate_appends_a_sampled_token():

@@ -13,6 +13,7 @@ import torch.utils._python_dispatch
 import oracle
 from conftest import error_figures, report
 import sparseattention_amd as sa
+from sparseattention_amd.modules import attention
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -204,21 +205,40 @@ def test_reference_check_configuration_cross_update_y_gradients():
         assert err <= 3e-2 * max(1.0, float(ref.abs().max())), "%s: max abs err %.3e" % (name, err)
 
 
+class _Route:
+    """Sends the leaves' queries, keys and values one of their three ways without autograd and says which ones ran."""
+
+    def __init__(self, monkeypatch, m, route):
+        self.ran, joined, bmm = [], attention.query_key_value, torch.bmm
+
+        def one_launch(*args):
+            r = joined(*args) if route == "one launch" else None
+            self.ran += ["one launch"] * (r is not None)
+            return r
+
+        monkeypatch.setattr(attention, "query_key_value", one_launch)
+        monkeypatch.setattr(torch, "bmm", lambda *a, **k: (self.ran.append("direct"), bmm(*a, **k))[1])
+        m._DIRECT_PROJECTION_MIN_ELEMENTS = 0 if route == "direct" else 1 << 40
+
+
+ROUTES = {"one launch": ["one launch"], "direct": ["direct"] * 4, "concatenation": []}
+
+
 # ---------------------------------------------------------------- autocast (the reference evaluates under it)
 @pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N", [32, 512])
-@pytest.mark.parametrize("direct", [True, False])
-def test_module_under_autocast(amp, N, direct):
+@pytest.mark.parametrize("route", list(ROUTES))
+def test_module_under_autocast(amp, N, route, monkeypatch):
     """fp32 module and fp32 activations inside torch.autocast + no_grad, the way the reference's
     validation loop calls the model (Hierarchical_Transformer_Pretrain.py:607-613): projections
     come out in the autocast type while inputs and weights stay fp32.  N=32 takes the fused upper
-    levels directly from the leaves, N=512 goes through strided levels first.  `direct`: keys and
-    values projected straight into their rows (the branch large inputs take) or from the
-    concatenated input (small inputs)."""
+    levels directly from the leaves, N=512 goes through strided levels first.  `route`: queries, keys
+    and values in one launch, keys and values straight into their rows (larger inputs that the launch
+    does not take), or from the concatenated input."""
     B, dim, H, R = 2, 128, 2, 4
     torch.manual_seed(4)
     m = sa.HierarchicalAttention(dim, H, dropout=0.0, window_size=R).to(DEV).eval()
-    m._DIRECT_PROJECTION_MIN_ELEMENTS = 0 if direct else 1 << 40
+    taken = _Route(monkeypatch, m, route)
     g = torch.Generator().manual_seed(5)
     x = torch.randn(B, N, dim, generator=g).clamp(-1, 1)
     y = torch.randn(B, N - 1, dim, generator=g).clamp(-1, 1)
@@ -227,7 +247,7 @@ def test_module_under_autocast(amp, N, direct):
     with torch.no_grad(), torch.autocast("cuda", dtype=amp):
         y_new = m.cross_update_Y(x.to(DEV), y.to(DEV))
         out = m(x.to(DEV), x.to(DEV), x.to(DEV), y=y.to(DEV), mask=mask)
-    assert y_new.dtype == amp and out.dtype == amp
+    assert y_new.dtype == amp and out.dtype == amp and taken.ran == ROUTES[route]
     _within(y_new, oracle.cross_update_y_ref(x.double(), y.double(), w, H), 8e-3, 0.0, "cross_update_Y")
     _within(out, oracle.update_x_from_y_ref(x.double(), y.double(), w, H, R, True), 8e-3, 0.0, "forward")
     # and with autograd on (the training step runs under autocast as well)
@@ -254,20 +274,26 @@ def test_lm_under_autocast(amp):
     _within(got, want, 2e-2 * stages, 1e-2 * stages, "LM under autocast %s" % amp)
 
 
-def test_update_x_from_y_direct_projection_matches_concatenation():
-    """The no-autograd leaf update projects keys and values either from cat([x, y]) (small inputs)
-    or straight into the rows of the key / value buffers (large inputs): same result."""
-    B, N, dim, H, R = 2, 256, 128, 2, 8
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,dim,H", [(2, 256, 128, 2), (3, 64, 192, 3)])
+def test_update_x_from_y_routes_agree(B, N, dim, H, dtype, monkeypatch):
+    """The no-autograd leaf update projects queries, keys and values in one launch, keys and values straight into
+    the rows of their buffers (larger inputs that the launch does not take) or from cat([x, y]): same result."""
     torch.manual_seed(11)
-    m = sa.HierarchicalAttention(dim, H, dropout=0.0, window_size=R).to(DEV).to(torch.bfloat16).eval()
-    x = torch.randn(B, N, dim, device=DEV).bfloat16()
-    y = torch.randn(B, N - 1, dim, device=DEV).bfloat16()
+    m = sa.HierarchicalAttention(dim, H, dropout=0.0, window_size=8).to(DEV).to(dtype).eval()
+    x, y = (torch.randn(B, n, dim, device=DEV).to(dtype) for n in (N, N - 1))
     outs = []
-    with torch.no_grad():
-        for limit in (0, 1 << 40):
-            m._DIRECT_PROJECTION_MIN_ELEMENTS = limit
-            outs.append(m.update_X_from_Y(x, y, mask=True))
-    assert (outs[0].float() - outs[1].float()).abs().max() <= 2e-2
+    for route, ran in ROUTES.items():
+        for scale in (1.0, 0.5):  # (and again with other weights: none is kept)
+            with monkeypatch.context() as patch, torch.no_grad():
+                m.Wk_x.weight.mul_(scale)
+                taken = _Route(patch, m, route)
+                outs.append(m.update_X_from_Y(x, y, mask=True))
+                m.Wk_x.weight.div_(scale)
+            assert taken.ran == ran
+    for got, want in zip(outs[2:], outs[:2] * 2):
+        assert (got.float() - want.float()).abs().max() <= 2e-2
+    assert (outs[0].float() - outs[1].float()).abs().max() > 2e-2
 
 
 class _NoTransposedBatches(torch.utils._python_dispatch.TorchDispatchMode):

@@ -491,8 +491,9 @@ int hsa_add_split_rows(const void *a, const void *b, const void *c, void *dx, vo
  * (not with w_rows_contract).  Strides multiples of 8, addresses 16-byte aligned (bias: 2-byte).
  * hsa_linear_tile: the tile to take, or -1 where the sizes are not handled or a library's product is as fast.
  * hsa_linear_rectangles: what each workgroup-sized tile of such a launch computes (not tile 3), for checks of the plan without
- * a GPU: segment, batch element, first row, distance between its rows, rows, first column, columns.  Returns the
- * number of tiles, of which the first `capacity` are written, or an error; addresses count with their alignment only.
+ * a GPU, in the order of each XCD's walk: segment, batch element, first row, distance between its rows, rows, first column,
+ * columns, XCD.  Returns the number of tiles, of which the first `capacity` are written, or an error; addresses count with
+ * their alignment only.
  */
 #define HSA_LINEAR_MAX_SEGMENTS 5
 typedef struct {
@@ -502,7 +503,7 @@ typedef struct {
     int batches, rows, cols;
 } hsa_linear_segment;
 int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int dtype);
-int hsa_linear_rectangles(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int (*rects)[7],
+int hsa_linear_rectangles(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int (*rects)[8],
                           int capacity);
 int hsa_linear(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int dtype, void *stream);
 

@@ -89,6 +89,27 @@ __host__ __device__ __forceinline__ LnPlace place_of(const LnArgs &p, int t) {
     return c;
 }
 
+// The tiles of an XCD: consecutive ones, since they share rows of X and W in its L2.  Where rows go through the LDS
+// (ANY == 1) the walks begin in the middle, an eighth of the columns apart: with the same number of row tiles each, all
+// eight XCDs would ask for the same columns' weights at the same time from beginning to end (us, library / together /
+// apart, 48305 columns: 14336 x 256 645 / 804 / 565, 10240 x 256 463 / 578 / 391, 14336 x 512 908 / 1037 / 798).
+struct LnWalk {
+    int first, count, shift;
+    __host__ __device__ __forceinline__ int tile(int t) const {
+        t += shift;
+        return first + (t < count ? t : t - count);
+    }
+};
+template <int ANY> __host__ __device__ __forceinline__ LnWalk walk_of(const LnArgs &p, int xcd) {
+    const int per = p.tiles >> 3, rest = p.tiles & 7;
+    LnWalk w = {xcd * per + (xcd < rest ? xcd : rest), per + (xcd < rest), 0};
+    if (ANY == 1 && w.count) {
+        const int per_group = p.group * p.seg[0].col_tiles, ahead = (xcd * per_group / 8 - w.first) % per_group;
+        w.shift = w.count < per_group ? (int)((long)xcd * w.count / 8) : ahead < 0 ? ahead + per_group : ahead;
+    }
+    return w;
+}
+
 // one transfer of 1 KiB: a scalar base and 32-bit offsets per lane
 __device__ __forceinline__ void lds_dma16_from(const char *base, uint32_t off, uint32_t lds) {
     uint32_t keep;
@@ -141,12 +162,10 @@ __global__ void __launch_bounds__(2 * BM, 2) linear_kernel(LnArgs p) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, r = lane & 15, wm = w >> 1, wn = w & 1;
     const uint32_t lds0 = lds_address(lds);
-    // consecutive tiles on one XCD: they share rows of X and W in its L2
-    const int per = p.tiles >> 3, rest = p.tiles & 7, xcd = blockIdx.x & 7;
-    const int first = xcd * per + (xcd < rest ? xcd : rest), count = per + (xcd < rest);
-    const int slots = gridDim.x >> 3, slot = blockIdx.x >> 3;
+    const LnWalk walk = walk_of<ANY>(p, blockIdx.x & 7);
+    const int count = walk.count, slots = gridDim.x >> 3, slot = blockIdx.x >> 3;
     if (slot >= count) return;
-    auto tile_of = [&](int t) { return place_of<BM, BN, ANY>(p, first + t); };
+    auto tile_of = [&](int t) { return place_of<BM, BN, ANY>(p, walk.tile(t)); };
 
     // ---- transfers.  X: rows 32 w + 8 q + lane / 8, piece lane & 7 of 8.  W likewise (8 QW w + ..), or, TW,
     // rows of the contraction: pieces (w QW + q) 64 + lane of rows of BN / 8.
@@ -656,17 +675,23 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     return best;
 }
 
-int hsa_linear_rectangles(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int (*rects)[7], int capacity) {
+int hsa_linear_rectangles(int nseg, const hsa_linear_segment *seg, int K, int w_rows_contract, int tile, int (*rects)[8], int capacity) {
     using namespace hsa;
     HSA_REQUIRE(tile >= 0 && tile < 5 && tile != 3 && capacity >= 0 && (rects || !capacity), "bad tile %d or no room", tile);
     LnArgs p = {};
     if (!takes(tile, nseg, seg, K, w_rows_contract != 0) || !plan(tile, nseg, seg, K, p))
         return fail(HSA_ERR_UNSUPPORTED, "projection: sizes or alignment not handled by tile %d (K=%d)", tile, K);
-    for (int t = 0; t < p.tiles && t < capacity; ++t) {
-        const LnPlace c = tile == 1 ? place_of<256, 192, 0>(p, t) : tile == 2 ? place_of<128, 128, 0>(p, t)
-                          : tile == 4 && p.seg[0].period > 1 ? place_of<256, 256, 2>(p, t) : place_of<256, 256, 0>(p, t);
-        const int rect[7] = {c.seg, c.b, c.m0, p.seg[c.seg].period, LN_TILES[tile].rows, c.n0, LN_TILES[tile].cols};
-        for (int i = 0; i < 7; ++i) rects[t][i] = rect[i];
+    const bool alike = p.seg[0].period > 1;
+    int at = 0;
+    for (int xcd = 0; xcd < 8; ++xcd) {
+        const LnWalk walk = tile == 4 && !alike ? walk_of<1>(p, xcd) : walk_of<0>(p, xcd);
+        for (int i = 0; i < walk.count && at < capacity; ++i, ++at) {
+            const int t = walk.tile(i);
+            const LnPlace c = tile == 1 ? place_of<256, 192, 0>(p, t) : tile == 2 ? place_of<128, 128, 0>(p, t)
+                              : tile == 4 && alike ? place_of<256, 256, 2>(p, t) : place_of<256, 256, 0>(p, t);
+            const int rect[8] = {c.seg, c.b, c.m0, p.seg[c.seg].period, LN_TILES[tile].rows, c.n0, LN_TILES[tile].cols, xcd};
+            for (int e = 0; e < 8; ++e) rects[at][e] = rect[e];
+        }
     }
     return p.tiles;
 }

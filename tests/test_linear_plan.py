@@ -20,7 +20,7 @@ def _segment(B, R, N, K, ld, first=0):
 
 def _rectangles(tile, K, *segs):
     arr, room = (Segment * len(segs))(*segs), 1 << 16
-    out = np.zeros((room, 7), dtype=np.int32)
+    out = np.zeros((room, 8), dtype=np.int32)
     n = _lib.lib().hsa_linear_rectangles(len(segs), arr, K, 0, tile, out.ctypes.data, room)
     assert 0 < n <= room, n
     return out[:n]
@@ -75,3 +75,18 @@ def test_consecutive_rows(tile, rows, cols):
     for B, R, N in ((1, rows, cols), (3, rows + 1, cols + 8), (2, 5 * rows - 1, 3 * cols - 8), (1, 40 * rows + 7, 2 * cols)):
         segs = [_segment(B, R, N, 192, N + 8, 8), _segment(1, R + 1, N + 8, 192, N + 8)]
         _covered(_rectangles(tile, 192, *segs), *segs)
+
+
+@pytest.mark.parametrize("rows,apart", [(2048, 16), (4096, 8), (5111, 8), (5120, 8), (8192, 8), (10240, 8), (14336, 8), (18432, 8),
+                                        (20480, 8)])
+@pytest.mark.parametrize("cols", [7001, 30001, 48305])
+def test_walks_of_rows_through_the_lds_begin_apart(rows, cols, apart):
+    """The eight XCDs' walks: every tile once, and at any time columns about an eighth apart (a sixteenth where two share a
+    row of tiles): in step, all eight ask for the same weights at once."""
+    s = _segment(1, rows, cols, 256, cols)
+    r = _rectangles(4, 256, s)
+    _covered(r, s)
+    assert len(np.unique(r[:, [2, 5]], axis=0)) == len(r)
+    starts = np.array([r[r[:, 7] == xcd][0, 5] for xcd in range(8)])
+    gaps = np.diff(np.append(np.sort(starts), np.sort(starts)[0] + cols))
+    assert (gaps >= cols / apart - 3 * 256).all(), starts

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..ops.functional import build_parent_nodes, hierarchical_attention, pack_kv_weights
-from ..ops.linear import FORWARDS, linear, project, query_key_value, query_key_value_rows
+from ..ops.linear import FORWARDS, linear, project, query_key_value, query_key_value_rows, weight_and_bias
 from ..ops.topology import build_tree_topology
 
 
@@ -139,8 +139,7 @@ class HierarchicalAttention(nn.Module):
         dimension, so one GEMM computes them all (packed: key / value weights in the operand order
         of the fused upper levels; transposed: one weight with its rows along the contraction); rebuilt
         when any of them has been written to or moved."""
-        # (the parameter dictionary is read directly: Module.__getattr__ costs a microsecond per use)
-        params = [m._parameters["weight"] for m in layers]
+        params = [weight_and_bias(m)[0] for m in layers]
         key = tuple((w.data_ptr(), w._version, w.dtype) for w in params) + (dtype,)
         hit = self._fused.get(name)
         if hit is None or hit[0] != key:

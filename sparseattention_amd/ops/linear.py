@@ -53,6 +53,16 @@ def project(x: torch.Tensor, w: torch.Tensor, contract: bool = False) -> torch.T
     return _lib.ext().project(x, w, None, contract)
 
 
+def weight_and_bias(layer):
+    """(layer.weight, layer.bias), from the parameters' dictionary where they are there (Module.__getattr__ costs half a
+    microsecond a use): sharding and pruning keep plain tensors in their places."""
+    p = layer._parameters
+    try:
+        return p["weight"], p["bias"]
+    except KeyError:
+        return layer.weight, layer.bias
+
+
 def _plain(layer) -> bool:
     """An nn.Linear that may be bypassed."""
     return plain_module(layer, nn.Linear)
@@ -64,31 +74,39 @@ def linear(layer, x: torch.Tensor, wide: bool = False) -> torch.Tensor:
     computes the weight's and the bias's gradient in one contraction over the tokens (csrc/hsa_weight_grad.hip),
     directly in the parameters' type; everything else is the layer itself.  wide: a vocabulary projection, whose
     input gradient is a product with a long contraction (csrc/hsa_linear_long.hip)."""
-    if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer) and not watched(x, layer.weight, layer.bias):
-        y = _lib.ext().linear(x, layer.weight, layer.bias, wide)
-        if y is not None:
-            return y
+    if x.is_cuda and not torch.compiler.is_compiling() and _plain(layer):
+        w, b = weight_and_bias(layer)
+        if not watched(x, w, b):
+            y = _lib.ext().linear(x, w, b, wide)
+            if y is not None:
+                return y
     return layer(x)
+
+
+def _bypassed_weights(layer_q, layer_k, layer_v, x, y):
+    """The weights of three bias-free nn.Linear that may be bypassed for inputs x and y, or None."""
+    if torch.compiler.is_compiling() or not all_plain(((layer_q, nn.Linear), (layer_k, nn.Linear), (layer_v, nn.Linear))):
+        return None
+    (q, bq), (k, bk), (v, bv) = weight_and_bias(layer_q), weight_and_bias(layer_k), weight_and_bias(layer_v)
+    return None if bq is not None or bk is not None or bv is not None or watched(x, y, q, k, v) else (q, k, v)
 
 
 def query_key_value_rows(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
     """(layer_q of x; layer_k, layer_v of cat([x, y], dim=1)) in training on 16-bit types (or under
     autocast to one): the rows are converted and joined in one pass, their gradients added and cut apart
     in one (csrc/hsa_rows.hip).  None where that does not apply."""
-    layers = (layer_q, layer_k, layer_v)
-    if (x.is_cuda and torch.is_grad_enabled() and not torch.compiler.is_compiling()
-            and all(_plain(m) and m.bias is None for m in layers) and not watched(x, y, *(m.weight for m in layers))):
-        return _lib.ext().query_key_value_rows(x, y, *(m.weight for m in layers))
+    if x.is_cuda and torch.is_grad_enabled():
+        ws = _bypassed_weights(layer_q, layer_k, layer_v, x, y)
+        if ws is not None:
+            return _lib.ext().query_key_value_rows(x, y, *ws)
     return None
 
 
 def query_key_value(layer_q, layer_k, layer_v, x: torch.Tensor, y: torch.Tensor):
     """The same without autograd: the rows stay where they are and the five products write into the joined
     results in one launch (csrc/hsa_linear.hip).  None where that does not apply."""
-    if (x.is_cuda and not torch.compiler.is_compiling()
-            and all_plain(((layer_q, nn.Linear), (layer_k, nn.Linear), (layer_v, nn.Linear)))):
-        q, k, v = layer_q._parameters, layer_k._parameters, layer_v._parameters
-        if (q.get("bias") is None and k.get("bias") is None and v.get("bias") is None
-                and not watched(x, y, q["weight"], k["weight"], v["weight"])):
-            return _lib.ext().query_key_value(x, y, q["weight"], k["weight"], v["weight"])
+    if x.is_cuda:
+        ws = _bypassed_weights(layer_q, layer_k, layer_v, x, y)
+        if ws is not None:
+            return _lib.ext().query_key_value(x, y, *ws)
     return None

@@ -20,19 +20,22 @@ from . import _lib
 from .modules import HierarchicalAttention
 from .modules import attention as _attention
 from .ops import generate_span_input_Y
-from .ops.linear import FORWARDS, all_plain, linear, plain_module, watched
+from .ops.linear import FORWARDS, all_plain, linear, plain_module, watched, weight_and_bias
 
 
-def _plain_norm(m) -> bool:
-    """An nn.LayerNorm over the last dimension with weight and bias that may be bypassed."""
-    return (plain_module(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None
-            and m.bias is not None)
+def _norm_weights(m):
+    """Weight and bias of an nn.LayerNorm over the last dimension with both that may be bypassed, else None."""
+    if not plain_module(m, nn.LayerNorm) or len(m.normalized_shape) != 1:
+        return None
+    w, b = weight_and_bias(m)
+    return None if w is None or b is None else (w, b)
 
 
 def layer_norm(x, norm):
     """norm(x) on this package's kernel where it takes the case."""
-    if x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda") and not watched(x, norm.weight, norm.bias):
-        r = _lib.ext().add_layer_norm(x, None, norm.weight, norm.bias, norm.eps)
+    wb = _norm_weights(norm) if x.is_cuda and not torch.is_autocast_enabled("cuda") else None
+    if wb is not None and not watched(x, *wb):
+        r = _lib.ext().add_layer_norm(x, None, *wb, norm.eps)
         if r is not None:
             return r[1]
     return norm(x)
@@ -41,9 +44,9 @@ def layer_norm(x, norm):
 def add_layer_norm(x, branch, norm):
     """(x + branch, norm(x + branch)): one kernel reads both once and writes both results, where it
     takes the case (one GPU, one element type; autocast mixes types and keeps the two steps)."""
-    if (x.is_cuda and _plain_norm(norm) and not torch.is_autocast_enabled("cuda")
-            and not watched(x, branch, norm.weight, norm.bias)):
-        r = _lib.ext().add_layer_norm(x, branch, norm.weight, norm.bias, norm.eps)
+    wb = _norm_weights(norm) if x.is_cuda and not torch.is_autocast_enabled("cuda") else None
+    if wb is not None and not watched(x, branch, *wb):
+        r = _lib.ext().add_layer_norm(x, branch, *wb, norm.eps)
         if r is not None:
             return r
     x = x + branch
@@ -142,14 +145,15 @@ class DecoderLayer(nn.Module):
             return None
         if ff.activation is not F.gelu and ff.activation is not F.relu:
             return None
-        w = [m._parameters["weight"] for m in linears]
-        b = [m._parameters["bias"] for m in linears]
-        n = [p for m in norms for p in (m._parameters["weight"], m._parameters["bias"])]
+        # (None: not there, or a plain tensor in its place)
+        w = [m._parameters.get("weight") for m in linears]
+        b = [m._parameters.get("bias") for m in linears]
+        n = [p for m in norms for p in (m._parameters.get("weight"), m._parameters.get("bias"))]
         if any(t is None for t in n) or any(len(m.normalized_shape) != 1 for m in norms):
             return None
         if any((t is None) != (i in (1, 2, 3)) for i, t in enumerate(b)):
             return None
-        if any(type(t) is not nn.Parameter for t in w + n) or any(type(a[m]._parameters["weight"]) is not nn.Parameter
+        if any(type(t) is not nn.Parameter for t in w + n) or any(type(a[m]._parameters.get("weight")) is not nn.Parameter
                                                                   for m in ("Wq_y", "Wk_y", "Wv_y")):
             return None
         packed, dt = att._chain_weights(x), x.dtype

@@ -134,6 +134,26 @@ def test_steps_replaced_on_their_class_or_module(owner, name, calls, monkeypatch
         assert count.native == 4
 
 
+@pytest.mark.parametrize("name", ["self_attn.Wq_y", "self_attn.Wk_x", "self_attn.out_proj_y", "feed_forward.fc1", "norm2", "norm1"])
+def test_plain_tensors_in_the_parameters_places(name, monkeypatch):
+    """Sharding and pruning take a parameter out of its dictionary and keep a plain tensor under its name: the Python
+    layer reads that, without autograd (to the same bits) and with it (other products: bf16 roundings through two layers)."""
+    net, tok = _lm(), torch.randint(0, 50, (2, 64), device=DEV)
+    with torch.no_grad():
+        want = net(tok)
+    for layer in net.layers:
+        m = layer.get_submodule(name)
+        for n in list(m._parameters):
+            p = m._parameters.pop(n)
+            m.__dict__[n] = p if p is None else p.detach().clone()
+    count = _Count(monkeypatch)
+    with torch.no_grad():
+        # (the first layer's own norm1 is not the native layer's, the second's is taken with the first's sums)
+        assert torch.equal(net(tok), want) and count.native == (1 if name == "norm1" else 0)
+    got = net(tok)
+    assert got.requires_grad and float((got.detach() - want).float().norm()) <= 0.03 * float(want.float().norm())
+
+
 @pytest.mark.parametrize("dim,heads,length", [(768, 12, 1024), (512, 4, 1024), (96, 3, 64)])
 def test_sizes_not_taken_are_not_looked_into(dim, heads, length, monkeypatch):
     """What is known from the sizes alone costs no look at the layer's modules."""

@@ -4,10 +4,10 @@
 // launch, each with row blocks that lie apart in memory on either side (the leaves' and the nodes' rows of
 // the joined key buffer).
 //
-// Why not the library's product: the contraction is short (256 to 1024), so a tile is 8 steps of 64 and then 128 KB
-// of results; the library starts a workgroup per tile, which pays for its first rows and its last stores each
-// time.  Here a workgroup stays on its CU and walks tiles: the rows of the next tile's first two steps are
-// requested before the results of the last one are stored.
+// Why not the library's product: the contraction is short (up to 768; read the other way round up to 2304), so at
+// 512 a tile is 8 steps of 64 and then 128 KB of results; the library starts a workgroup per tile, which pays for
+// its first rows and its last stores each time.  Here a workgroup stays on its CU and walks tiles: the rows of the
+// next tile's first two steps are requested before the results of the last one are stored.
 //
 // Tile 256 x 256 (or 256 x 192 where that leaves fewer CUs idle in the last round), eight wavefronts of 64 rows by
 // 128 (96) columns.  Two stages of 64 contraction steps, both operands straight into LDS; a row's 16-byte pieces are
@@ -22,16 +22,17 @@
 // Results whose rows begin at any element (a vocabulary of odd size): a line that two tiles share costs more
 // than the line.  With rows enough, a tile takes every 64th row: their results lie alike in their lines, so the
 // tiles' columns can begin where the lines do (32768 x 50257 x 512: 1710 us; the library 2160).  Else the rows go
-// through the LDS and are stored as 16-byte pieces where they lie (4096 x 50257 x 512: 283 us; 330 as they come,
-// the library 349).
+// through the LDS and are stored as 16-byte pieces where they lie (4096 x 50257 x 512: 230 to 250 us, the library 330 to
+// 350; stored as they come 330, before the XCDs' walks began apart).
 //
 // The transfers of a stage are requested one by one between the products of a half step: together, behind the
 // barrier, they hold up all wavefronts at once (32768 x 2048 x 512: 73.3 -> 70.2 us, 16376 x 768 x 2304 55.7 -> 50.0).
 //
 // Bound: the matrix cores (1.4 PFLOP/s in the steps) and, not overlapped with them, the stores of the results
-// at the rate of the memory (a third of the time at 32768 x 2048 x 512).  Slower: two workgroups of 128 x 256 on
-// a CU, whose stores would overlap (82 us); four wavefronts for the transfers alone, so that none waits for
-// its stores (72); starts spread over a tile's time (66).
+// at the rate of the memory (a third of the time at 32768 x 2048 x 512; the matrix cores are busy for 46 % of it, and
+// for 63 % at 16384 x 768 x 2304).  Not faster (66 us on the same card): two workgroups of 128 x 256 on a CU, whose
+// stores would overlap (82); four wavefronts for the transfers alone, so that none waits for its stores (72); starts
+// spread over a tile's time (66).
 #include "hsa_lds_dma.h"
 
 #include <cmath>
@@ -530,6 +531,8 @@ void launch(int tile, bool past, const LnArgs &p, hipStream_t st) {
     else if (tile == 1) past ? go(linear_kernel<T, 256, 192, TW, true>, 256) : go(linear_kernel<T, 256, 192, TW, false>, 256);
     else if (tile == 2) go(linear_kernel<T, 128, 128, TW, false>, 128);
     else if constexpr (!TW) {
+        // (rows through the LDS: through the caches as well; past them 1024 x 50257 x 512 74 -> 85 us, 8192 x 30001 x 512 298 ->
+        // 326, before the walks began apart)
         if (p.seg[0].period > 1) past ? go(linear_kernel<T, 256, 256, false, true, 2>, 256) : go(linear_kernel<T, 256, 256, false, false, 2>, 256);
         else go(linear_kernel<T, 256, 256, false, false, 1>, 256);
     }
@@ -599,13 +602,13 @@ bool plan(int tile, int nseg, const hsa_linear_segment *seg, int K, LnArgs &p) {
         t.period = 1;
         t.row_tiles = (s.rows + size.rows - 1) / size.rows;
         t.col_tiles = (s.cols + size.cols - 1) / size.cols;
-        // Tiles of rows that lie alike where whole lines pay for it.  They take 0.8 of the time of consecutive rows
+        // Tiles of rows that lie alike where whole lines pay for it.  They take 0.9 of the time of consecutive rows
         // through the LDS for the same number of tiles, but a row class that does not fill its tiles makes for more of
         // them (us, library / alike / through the LDS, in brackets their tiles by the others': 50257 columns, 32768
-        // rows 2163 / 1710 / 2098 (1), 28672 1890 / 1709 / 1840 (1.14), 24576 1618 / 1705 / 1570 (1.33), 20480 1348 / 1730 /
-        // 1303 (1.6); 50260, 4096 rows 340 / 220 / 280 (1), 5120 420 / 430 / 295 (1.6)), and the first and the last columns'
-        // tiles begin at any element all the same (16384 rows of 3001 73 / 70 / 59, 32768 130 / 137 / 112, of 5001 156 /
-        // 145 / 149, of 8001 395 / 310 / 336, of 10001 285 / 246 / 267).
+        // rows 2180 / 1693 / 1897 (1), 16384 1108 / 866 / 951 (1), 28672 1899 / 1688 / 1668 (1.14), 24576 1635 / 1705 / 1405 (1.33),
+        // 20480 1357 / 1730 / 1169 (1.6); 50260, 4096 rows 342 / 224 / 247 (1), 7168 462 / 426 / 414 (1.14), 5120 415 / 430 /
+        // 296 (1.6)), and the first and the last columns' tiles begin at any element all the same (16384 rows of 3001 75 / 70
+        // / 61, 32768 138 / 137 / 114, of 5001 227 / 210 / 201, of 8001 380 / 298 / 332, of 10001 435 / 364 / 406).
         const int period = tile == 4 && nseg == 1 ? line_period(s.ld_out) : 1;
         if (period > 1 && s.rows / period >= size.rows && t.col_tiles >= 32) {
             const int row_tiles = period * (((s.rows + period - 1) / period + size.rows - 1) / size.rows);
@@ -623,8 +626,8 @@ bool plan(int tile, int nseg, const hsa_linear_segment *seg, int K, LnArgs &p) {
         tiles += (long)n;
     }
     p.tiles = (int)tiles;
-    // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 8 / 32: 2180
-    // / 2200 / 2550 us at 32768 x 50257 x 512)
+    // rows that begin anywhere: neighbours in a row side by side, their common lines meet in one L2 (2 / 4 / 8: 1669 / 2061
+    // / 2138 us at 28672 x 50257 x 512, 428 / 443 / 537 at 7168; 10001 columns 351 / 357 / 345 and 93 / 92 / 91)
     if (tile == 4 && p.seg[0].period == 1) p.group = 2;
     return true;
 }
@@ -641,9 +644,12 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     double results = 0;
     if (nseg < 1 || nseg > HSA_LINEAR_MAX_SEGMENTS || !seg) return -1;
     for (int i = 0; i < nseg; ++i) results += (double)seg[i].batches * seg[i].rows * seg[i].cols;
-    // Few rows (us, library / here; the library's call also takes 15 us more of host time): 64 x 512 x 512 5.6 / 4.0,
-    // 256 x 512 x 512 5.0 / 4.0, 256 x 2048 x 512 5.9 / 6.0, 256 x 1024 x 1024 5.5 / 5.9, 512 x 672 x 672 7.2 / 5.6; beyond: 512
-    // x 2048 x 512 6.4 / 9.7, 256 x 512 x 2048 6.3 / 9.3.  Several projections are several library calls.
+    // Few rows (us on the GPU, library / here; the call takes 20 / 5 us of host time, and sizes like these wait for the
+    // host): 64 x 512 x 512 5.2 / 4.3, 256 x 512 x 512 5.2 / 4.4, 512 x 512 x 256 4.4 / 3.8, 256 x 2048 x 512 6.0 / 6.2, 256 x
+    // 1024 x 1024 5.6 / 6.2, 512 x 672 x 672 7.2 / 5.6.  Replayed from a graph the library is the faster one by up to 2 us
+    // where more than two workgroups meet on a CU or, from contractions of 768 on, more than one: 768 x 768 x 384 5.6 / 6.9,
+    // 512 x 2048 x 256 5.2 / 6.7, 384 x 768 x 768 5.7 / 7.9.  Beyond: 512 x 2048 x 512 6.4 / 9.7, 256 x 512 x 2048 6.3 / 9.3.
+    // Several projections are several library calls.
     if (K <= 1024 && results * K <= (double)(1 << 27) * (nseg + 1) && takes(3, nseg, seg, K, w_rows_contract)) return 3;
     // Tiles: rounds of the chip times the time of a tile, 256 x 256 as 1 (256 x 192 0.8, two of 128 x 128 on one CU 0.74).
     // The library has the better inner loop from contractions of about 1000 on and with its widest tiles at
@@ -652,8 +658,10 @@ int hsa_linear_tile(int nseg, const hsa_linear_segment *seg, int K, int w_rows_c
     // x 512 78 / 70, 4096 x 2048 x 512 15.6 / 15.1, 16384 x 768 x 768 24.2 / 22.8, 32752 x 768 x 768 46.5 / 38; not taken:
     // 4096 x 512 x 512 8.0 / 8.9, 8192 x 768 x 768 15.2 / 17.5, 16384 x 3072 x 768 69 / 72, 16384 x 1024 x 1024 30.5 / 34,
     // 32768 x 512 x 2048 50 / 56.  With the weight's rows along the contraction the library is slower: 16384 x 768 x 768
-    // 26.3 / 23.2, x 1536 41.1 / 36.6, x 2304 57.7 / 50.0.  Rows that begin anywhere (a vocabulary of 50257): 256 x 50257 x 512 31 / 23,
-    // 4096 349 / 281, 32768 2200 / 1800; 8192 x 50257 x 768 593 / 722.
+    // 26.3 / 23.2, x 1536 41.1 / 36.6, x 2304 57.7 / 50.0; not taken although it gains where the tiles fill the chip: 32768 x 768 x
+    // 3072 146 / 125, 16384 x 1024 x 3072 84 / 81, 32768 x 512 x 4096 119 / 113 (but 8192 x 1024 x 3072 53 / 59).  Rows that begin
+    // anywhere (a vocabulary of 50257): 256 x 50257 x 512 34 / 25, 1024 98 / 74, 4096 340 / 240, 8192 576 / 474, 32768 2140 /
+    // 1710; not taken: 4096 x 50257 x 768 346 / 314, 8192 593 / 630, 32768 2321 / 2309.
     int best = -1;
     double least = 0;
     for (int t = 0; t < 3; ++t) {

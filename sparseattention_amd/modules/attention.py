@@ -148,7 +148,9 @@ class HierarchicalAttention(nn.Module):
                 hit = (key, pack_kv_weights(ws[0], ws[1], self.num_heads))
             else:
                 hit = (key, ws[0].t().contiguous() if transposed else torch.cat(ws, dim=0))
-            self._fused[name] = hit
+            # (under capture the copy holds nothing before the first replay: it stays with the graph)
+            if not (params[0].is_cuda and torch.cuda.is_current_stream_capturing()):
+                self._fused[name] = hit
         return hit[1]
 
     def _chain_weights(self, x: torch.Tensor):

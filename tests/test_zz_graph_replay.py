@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import sparseattention_amd as sa
+from sparseattention_amd.modules import attention
 from sparseattention_amd.ops import functional as fn
 
 pytestmark = pytest.mark.gpu
@@ -125,6 +126,43 @@ def test_lm_forward_replays_from_a_hip_graph():
             want = model(tok)
             torch.cuda.synchronize()
             assert torch.equal(got, want), "replay %d differs" % rep
+
+
+@pytest.mark.parametrize("direct", [False, True])
+def test_weights_laid_out_under_capture_stay_with_the_graph(direct):
+    """Changed weights met for the first time under capture: their stacked and transposed copies are not filled
+    before the first replay, and an eager forward before it makes copies of its own."""
+    B, N, dim = 2, 64, 128
+    torch.manual_seed(3)
+    m = sa.HierarchicalAttention(dim, 2, dropout=0.0, window_size=4).to(DEV).to(torch.bfloat16).eval()
+    if direct:
+        m._DIRECT_PROJECTION_MIN_ELEMENTS = 0
+    x, y = (torch.randn(B, n, dim, device=DEV).bfloat16() for n in (N, N - 1))
+    step = lambda: m(x, x, x, y=m.cross_update_Y(x, y), mask=True)
+    with torch.no_grad(), pytest.MonkeyPatch.context() as patch:
+        if direct:
+            patch.setattr(attention, "query_key_value", lambda *a: None)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            step()
+        torch.cuda.current_stream().wait_stream(side)
+        for p in m.parameters():
+            p.mul_(0.5)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = step()
+        eager = step()
+        m.train().eval()
+        assert torch.equal(eager, step())
+        for rep in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), "replay %d differs" % rep
+            x.copy_(torch.randn(B, N, dim, device=DEV))
+            eager = step()
 
 
 def test_lm_full_benchmark_shape_properties():

@@ -710,13 +710,14 @@ bool layer_kind(const Tensor &x, int64_t heads) {
     return B <= (1 << 20) && N >= 2 && N <= (1 << 24) && log2_exact(N) >= 0 && C % heads == 0 && C <= (1 << 16) &&
            hsa_cross_update_level_rows((int)B, (int)heads, (int)(C / heads), type_code(x)) >= N && hsa_add_layer_norm_ok((int)C, type_code(x));
 }
-// larger inputs whose rows' products do not go into one launch: the Python layer has a way without the copy
+// larger inputs whose rows' products do not go into one launch stay with the Python layer, which has a way without the
+// copy for the largest and whose host time is small against their kernels'
 bool layer_rows(const Tensor &x, const Tensor &y, const Tensor &wq, const Tensor &wk, const Tensor &wv) {
     return x.numel() < 1 << 20 || rows_plan(x, y, wq, wk, wv).second >= 0;
 }
 // Whether a layer of these sizes is one that decoder_layer takes, asked before its modules are looked at one by one (a
 // forward of B2 N1024, two layers of 4 heads by 128 channels, which it does not take: 905 us when that is found out last,
-// 845 here, 815 without the native layer)
+// 845 here, 815 without the native layer; since then 818 -> 748 with the rows joined by a copy)
 bool decoder_layer_takes(const Tensor &x, const Tensor &y, const Tensor &w, int64_t heads) {
     return layer_kind(x, heads) && ordinary({&x, &y, &w}) && y.dim() == 3 && y.numel() > 0 && y.size(0) == x.size(0) && layer_rows(x, y, w, w, w);
 }

@@ -107,7 +107,12 @@ class HierarchicalAttention(nn.Module):
             offsets.append(offsets[-1] + s)
         return sizes, offsets
 
-    _DIRECT_PROJECTION_MIN_ELEMENTS = 1 << 20
+    # update_X_from_Y without autograd where the projections do not go into one launch: keys and values straight into
+    # their rows from this many 16-bit elements of x on, or half as many 32-bit ones (us for the whole call, so /
+    # from the joined input, 1024 channels unless said: bf16 B2 N1024 159 / 109, B4 N2048 163 / 138, B8 N2048 242 / 236, B8
+    # N4096 470 / 477; fp16 146 / 109, 151 / 142, 220 / 246, 416 / 495; bf16 autocast 189 / 133, 214 / 201, 337 / 365, 625 /
+    # 713; fp32 B1 N2048 of 512 150 / 115, B8 N1024 of 640 391 / 386, B4 N2048 789 / 809, B8 N4096 3113 / 3205)
+    _DIRECT_PROJECTION_MIN_ELEMENTS = 1 << 24
     # training: levels of at most this many children over the batch run as fused chains, forward and backward
     # (no chain / 1024 / 4096, us forward and backward of one module, fp16: B8 N2048 d768 2034 / 1996 / 1967, B2
     # N512 d512 1503 / 1096 / 1102, B4 N64 d768 1330 / 1084 / 1089, B1 N4096 d1024 1649 / 1232 / 1159)
@@ -134,20 +139,16 @@ class HierarchicalAttention(nn.Module):
         self._fused.clear()
         return super().train(mode)
 
-    def _fused_weight(self, name: str, layers, dtype: torch.dtype, packed: bool = False, transposed: bool = False) -> torch.Tensor:
+    def _fused_weight(self, name: str, layers, dtype: torch.dtype, packed: bool = False) -> torch.Tensor:
         """Weights of several bias-free projections, cast to `dtype` and stacked along the output
         dimension, so one GEMM computes them all (packed: key / value weights in the operand order
-        of the fused upper levels; transposed: one weight with its rows along the contraction); rebuilt
-        when any of them has been written to or moved."""
+        of the fused upper levels); rebuilt when any of them has been written to or moved."""
         params = [weight_and_bias(m)[0] for m in layers]
         key = tuple((w.data_ptr(), w._version, w.dtype) for w in params) + (dtype,)
         hit = self._fused.get(name)
         if hit is None or hit[0] != key:
             ws = [w.detach().to(dtype) for w in params]
-            if packed:
-                hit = (key, pack_kv_weights(ws[0], ws[1], self.num_heads))
-            else:
-                hit = (key, ws[0].t().contiguous() if transposed else torch.cat(ws, dim=0))
+            hit = (key, pack_kv_weights(ws[0], ws[1], self.num_heads) if packed else torch.cat(ws, dim=0))
             # (under capture the copy holds nothing before the first replay: it stays with the graph)
             if not (params[0].is_cuda and torch.cuda.is_current_stream_capturing()):
                 self._fused[name] = hit
@@ -377,11 +378,11 @@ class HierarchicalAttention(nn.Module):
         qkv = join(self.Wq_x, self.Wk_x, self.Wv_x, x, y)
         q = self._heads(linear(self.Wq_x, x) if qkv is None else qkv[0])
         if (qkv is None and not grad and not dropped and y.size(1) == N - 1
-                and B * N * D >= self._DIRECT_PROJECTION_MIN_ELEMENTS):
+                and B * N * D * q.element_size() >= 2 * self._DIRECT_PROJECTION_MIN_ELEMENTS):
             # leaves and span nodes are projected straight into their rows of the [B, 2N-1, D]
             # key / value buffers (batched GEMMs with a strided output): no concatenated input.
-            # (Four GEMM launches instead of a copy and two: small inputs, where the launches cost
-            # more host time than the copy costs the GPU, take the other branch.)
+            # (Four batched GEMM launches instead of a copy and two plain ones: all but large inputs, where the
+            # launches cost more host time than the copy costs the GPU, take the other branch.)
             # Everything is brought to the type of q first (under autocast the activations and
             # weights are fp32 while the projections come out in the autocast type; GEMMs with an
             # `out=` are not autocast)
@@ -390,10 +391,11 @@ class HierarchicalAttention(nn.Module):
             k = torch.empty((B, 2 * N - 1, D), dtype=cdt, device=x.device)
             v = torch.empty_like(k)
             # (bf16: weights laid out along the contraction, since torch's batched bf16 product of a transposed right
-            # operand has faulted on this device; fp16: as they are, 8 x 2048 x 1024 x 1024 33 us against 40)
-            for name, lin, dst in (("k_x_t", self.Wk_x, k), ("v_x_t", self.Wv_x, v)):
-                wt = (self._fused_weight(name, (lin,), cdt, transposed=True) if cdt == torch.bfloat16
-                      else lin.weight.detach().to(cdt).t()).unsqueeze(0).expand(B, D, D)
+            # operand has faulted on this device: 7 us for each of 1024 x 1024, at every call, since a kept copy would miss
+            # writes through .data and in a graph any write; fp16: as they are, 8 x 2048 x 1024 x 1024 33 us against 40)
+            for lin, dst in ((self.Wk_x, k), (self.Wv_x, v)):
+                wt = lin.weight.detach().to(cdt).t()
+                wt = (wt.contiguous() if cdt == torch.bfloat16 else wt).unsqueeze(0).expand(B, D, D)
                 torch.bmm(xc, wt, out=dst[:, :N])
                 torch.bmm(yc, wt, out=dst[:, N:])
             k, v = self._heads(k), self._heads(v)

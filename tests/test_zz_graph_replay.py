@@ -130,7 +130,7 @@ def test_lm_forward_replays_from_a_hip_graph():
 
 @pytest.mark.parametrize("direct", [False, True])
 def test_weights_laid_out_under_capture_stay_with_the_graph(direct):
-    """Changed weights met for the first time under capture: their stacked and transposed copies are not filled
+    """Changed weights met for the first time under capture: their stacked and packed copies are not filled
     before the first replay, and an eager forward before it makes copies of its own."""
     B, N, dim = 2, 64, 128
     torch.manual_seed(3)
@@ -163,6 +163,37 @@ def test_weights_laid_out_under_capture_stay_with_the_graph(direct):
             assert torch.equal(out, eager), "replay %d differs" % rep
             x.copy_(torch.randn(B, N, dim, device=DEV))
             eager = step()
+
+
+def test_leaves_weights_are_read_by_every_call_and_replay(monkeypatch):
+    """Keys and values projected straight into their rows read the weights as they are at the time: after a write
+    through .data, which leaves no trace on the tensor, and in a graph captured before the write."""
+    B, N, dim = 2, 64, 128
+    torch.manual_seed(4)
+    m = sa.HierarchicalAttention(dim, 2, dropout=0.0, window_size=4).to(DEV).to(torch.bfloat16).eval()
+    m._DIRECT_PROJECTION_MIN_ELEMENTS = 0
+    monkeypatch.setattr(attention, "query_key_value", lambda *a: None)
+    x, y = (torch.randn(B, n, dim, device=DEV).bfloat16() for n in (N, N - 1))
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            m.update_X_from_Y(x, y, mask=True)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = m.update_X_from_Y(x, y, mask=True)
+        for rep in range(3):
+            m.Wk_x.weight.data.mul_(-0.75)
+            m.Wv_x.weight.data.mul_(1.5)
+            eager = m.update_X_from_Y(x, y, mask=True)
+            fresh = sa.HierarchicalAttention(dim, 2, dropout=0.0, window_size=4).to(DEV).to(torch.bfloat16).eval()
+            fresh.load_state_dict(m.state_dict())
+            fresh._DIRECT_PROJECTION_MIN_ELEMENTS = 0
+            assert torch.equal(eager, fresh.update_X_from_Y(x, y, mask=True)), "call %d" % rep
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), "replay %d differs" % rep
 
 
 def test_lm_full_benchmark_shape_properties():

@@ -55,8 +55,8 @@ bool same_kind(const Tensor &a, const Tensor &b) {
 }
 
 // Nothing that watches or transforms torch's own calls: no tracing, no dispatch mode, no tensor subclass
-// or functional transform, no forward-mode tangent.  Such calls go the general way, which either
-// supports them or says that it does not.
+// or functional transform, no forward-mode tangent; and nothing without strides (sparse).  Such calls go the general
+// way, which either supports them or says that it does not.
 bool ordinary(std::initializer_list<const Tensor *> ts) {
     constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::Batched,
                                            c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
@@ -64,7 +64,7 @@ bool ordinary(std::initializer_list<const Tensor *> ts) {
     if (at::tracer::impl::is_dispatch_enabled() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python))
         return false;
     for (const Tensor *t : ts)
-        if (t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
+        if (t->layout() != at::kStrided || t->key_set().has_any(wrapped) || t->_fw_grad(0).defined()) return false;
     return true;
 }
 
@@ -485,6 +485,7 @@ struct Linear : public torch::autograd::Function<Linear> {
 // enough to fill the chip by itself) or where the call is not a plain one.  wide: a vocabulary projection, whose
 // input gradient is the long contraction.
 std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias, bool wide) {
+    if (!ordinary({&x, &weight}) || (bias && !ordinary({&*bias}))) return std::nullopt;
     if (!x.is_cuda() || x.dim() < 2 || weight.dim() != 2 || x.numel() == 0 || x.size(-1) != weight.size(1) ||
         x.device() != weight.device() || !weight.is_contiguous())
         return std::nullopt;
@@ -492,7 +493,6 @@ std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::o
     const int64_t O = weight.size(0), I = weight.size(1);
     if (train && (!weight.requires_grad() || (!wide && (O % 8 || I % 8 || !small_result(weight))))) return std::nullopt;
     if (bias && (bias->dim() != 1 || bias->size(0) != O || !same_kind(weight, *bias))) return std::nullopt;
-    if (!ordinary({&x, &weight}) || (bias && !ordinary({&*bias}))) return std::nullopt;
     const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
     const at::ScalarType type = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
     if (type != at::kHalf && type != at::kBFloat16) return std::nullopt;
@@ -615,6 +615,7 @@ struct QueryKeyValueRows : public torch::autograd::Function<QueryKeyValueRows> {
 // autocast state; nullopt where the call is not a plain one on 16-bit types.
 std::optional<at::ScalarType> rows_type(const Tensor &x, const Tensor &y, const Tensor &weight_q, const Tensor &weight_k,
                                         const Tensor &weight_v) {
+    if (!ordinary({&x, &y, &weight_q, &weight_k, &weight_v})) return std::nullopt;
     if (x.dim() != 3 || y.dim() != 3 || x.numel() == 0 || y.numel() == 0 || x.device() != y.device() || y.size(0) != x.size(0) || y.size(2) != x.size(2) || weight_k.device() != x.device() ||
         weight_k.dim() != 2 || weight_k.size(1) != x.size(2))
         return std::nullopt;
@@ -622,7 +623,7 @@ std::optional<at::ScalarType> rows_type(const Tensor &x, const Tensor &y, const 
         if (!same_kind(weight_k, *t) || t->sizes() != weight_k.sizes() || !t->is_contiguous()) return std::nullopt;
     const int64_t O = weight_k.size(0), C = weight_k.size(1);
     if (O % 8 || C % 8 || ((O + 127) / 128) * ((C + 127) / 128) > 256 || x.numel() + y.numel() > (int64_t)1 << 40 ||
-        x.size(1) + y.size(1) > (1 << 30) || !ordinary({&x, &y, &weight_q, &weight_k, &weight_v}))
+        x.size(1) + y.size(1) > (1 << 30))
         return std::nullopt;
     const bool cast = at::autocast::is_autocast_enabled(at::kCUDA);
     const at::ScalarType type = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();

@@ -122,6 +122,19 @@ def test_linear_without_autograd(rows, cols, K, bias):
     assert bool(((got.double() - want).abs() <= _bound(x, wt, want, torch.bfloat16)).all())
 
 
+@pytest.mark.filterwarnings("ignore:Sparse CSR")
+def test_weight_without_strides():
+    """A weight held as compressed sparse rows has no strides to ask for: the layer's own product."""
+    layer = nn.Linear(64, 32, bias=False).to(DEV)
+    layer.weight = nn.Parameter(layer.weight.detach().to_sparse_csr(), requires_grad=False)
+    x = torch.randn(48, 64, device=DEV)
+    with torch.no_grad():
+        got = linear(layer, x)
+    want = x.double() @ layer.weight.to_dense().double().t()
+    # K products and additions in fp32
+    assert bool(((got.double() - want).abs() <= 64 * 2.0 ** -23 * (x.double().abs() @ layer.weight.to_dense().double().abs().t())).all())
+
+
 @pytest.mark.parametrize("rows,K,cols", [(16384, 512, 512), (64, 96, 40)])
 @pytest.mark.parametrize("contract", [False, True])
 def test_products_with_a_bias(rows, K, cols, contract):

@@ -10,6 +10,7 @@ presence is ever looked at (an N x N mask costs 16 MB at N=4096 and is never rea
 from __future__ import annotations
 
 import math
+import operator
 import sys
 
 import torch
@@ -133,31 +134,39 @@ class DecoderLayer(nn.Module):
         wq = a["Wq_x"]._parameters.get("weight")
         if wq is None or not _lib.ext().decoder_layer_takes(x, y, wq, att.num_heads):
             return None
-        drops = (sub["dropout"], a["dropout"], f["dropout"])
+        # (written for its host time, which a short sequence waits for: sets of types and plain loops)
+        drops = [sub["dropout"], a["dropout"], f["dropout"]]
         norms = [sub["norm2"]]
         if following is not None:
             norms += [following._modules["norm_y"], following._modules["norm1"]]
-        linears = [a[n] for n in ("out_proj_y", "Wq_x", "Wk_x", "Wv_x", "out_proj_x")] + [f["fc1"], f["fc2"]]
-        if not all_plain([(att, HierarchicalAttention), (ff, PositionwiseFeedForward)] + [(m, nn.Dropout) for m in drops]
-                         + [(m, nn.LayerNorm) for m in norms] + [(m, nn.Linear) for m in linears]):
+        linears = [a["out_proj_y"], a["Wq_x"], a["Wk_x"], a["Wv_x"], a["out_proj_x"], f["fc1"], f["fc2"]]
+        if not all_plain([(att, HierarchicalAttention), (ff, PositionwiseFeedForward), *zip(drops, _DROPS), *zip(norms, _NORMS),
+                          *zip(linears, _LINEARS)]):
             return None
-        if any(m.training and m.p > 0 for m in drops) or not att.fuse_top_levels or not _own_steps(self, att):
+        for m in drops:
+            if m.training and m.p > 0:
+                return None
+        for m in norms:
+            if len(m.normalized_shape) != 1:
+                return None
+        if not att.fuse_top_levels or not _own_steps(self, att) or (ff.activation is not F.gelu and ff.activation is not F.relu):
             return None
-        if ff.activation is not F.gelu and ff.activation is not F.relu:
+        # (weights and norms: parameters, neither missing nor plain tensors in their places; their type and sizes are
+        # the native call's to check)
+        linears = [m._parameters for m in linears]
+        w, b = [p.get("weight") for p in linears], [p.get("bias") for p in linears]
+        n = []
+        for m in norms:
+            m = m._parameters
+            n += m.get("weight"), m.get("bias")
+        spans = [a["Wq_y"]._parameters.get("weight"), a["Wk_y"]._parameters.get("weight"), a["Wv_y"]._parameters.get("weight")]
+        if {*map(type, w), *map(type, n), *map(type, spans)} != _PARAMETERS:
             return None
-        # (None: not there, or a plain tensor in its place)
-        w = [m._parameters.get("weight") for m in linears]
-        b = [m._parameters.get("bias") for m in linears]
-        n = [p for m in norms for p in (m._parameters.get("weight"), m._parameters.get("bias"))]
-        if any(t is None for t in n) or any(len(m.normalized_shape) != 1 for m in norms):
+        if (b[0] is None or b[1] is not None or b[2] is not None or b[3] is not None or b[4] is None or b[5] is None
+                or b[6] is None):
             return None
-        if any((t is None) != (i in (1, 2, 3)) for i, t in enumerate(b)):
-            return None
-        if any(type(t) is not nn.Parameter for t in w + n) or any(type(a[m]._parameters.get("weight")) is not nn.Parameter
-                                                                  for m in ("Wq_y", "Wk_y", "Wv_y")):
-            return None
-        packed, dt = att._chain_weights(x), x.dtype
-        if packed is None or any(t.dtype != dt for t in w + n):
+        packed = att._chain_weights(x)
+        if packed is None:
             return None
         params = [*packed, w[0], b[0], w[1], w[2], w[3], w[4], b[4], n[0], n[1], w[5], b[5], w[6], b[6], *n[2:]]
         eps = [m.eps for m in norms] + [0.0] * (3 - len(norms))
@@ -178,10 +187,15 @@ _STEPS = tuple((owner, name, getattr(owner, name)) for owner, names in (
     (sys.modules[__name__], ("add_layer_norm", "linear"))) for name in names)
 
 
+_STEP_OWNERS, _STEP_NAMES, _STEP_FUNCTIONS = zip(*_STEPS)
+_ATTENTION_STEPS = [name for owner, name, _ in _STEPS if owner is HierarchicalAttention]
+_DROPS, _NORMS, _LINEARS, _PARAMETERS = (nn.Dropout,) * 3, (nn.LayerNorm,) * 3, (nn.Linear,) * 7, {nn.Parameter}
+
+
 def _own_steps(layer, att) -> bool:
     """Nobody has replaced one of the steps, on its class, on the instance or in its module."""
-    return (all(getattr(owner, name) is f for owner, name, f in _STEPS) and "_chained" not in layer.__dict__
-            and not any(name in att.__dict__ for owner, name, _ in _STEPS if owner is HierarchicalAttention))
+    return (all(map(operator.is_, map(getattr, _STEP_OWNERS, _STEP_NAMES), _STEP_FUNCTIONS))
+            and "_chained" not in layer.__dict__ and att.__dict__.keys().isdisjoint(_ATTENTION_STEPS))
 
 
 class TransformerLM(nn.Module):
